@@ -59,9 +59,9 @@ BATCH_F64_BYTES_PER_POINT = 212
 # write 16 + 16 = 64 B.
 FUSED_MOVED_BYTES_PER_POINT = 99
 BATCH_F32_MOVED_BYTES_PER_POINT = 64
-# With FP32 point storage the batched gathers read each node's velocity as
-# an FP32 pair: 24 B written by the P2G + 8 B read per node.
-BATCH_F32_MOVED_BYTES_PER_NODE = 32
+# The batched substep is one kernel: per node it reads the mass and momentum,
+# adds the next P2G's and clears those of the one after, 24 B each.
+BATCH_MOVED_BYTES_PER_NODE = 72
 METRIC = "particle-updates/s on 1 GPU: batched+learned vs plain MPM at ≤1% force err"
 
 
@@ -404,10 +404,10 @@ def run_batch_learned(args) -> dict:
             log(f"bench: network proposals passing the gate over the probes: tension {ta}/{ta + tf}, shear "
                 f"{sa}/{sa + sf} -> network on for branches {branches} (1 tension, 2 shear)")
         k_avg_s = (ktot / max(klaunch, 1)) / 1e3
-        k_bytes = n_total * BATCH_F32_BYTES_PER_POINT + nodes * FUSED_BYTES_PER_NODE
-        k_moved = n_total * BATCH_F32_MOVED_BYTES_PER_POINT + nodes * BATCH_F32_MOVED_BYTES_PER_NODE
+        k_bytes = n_total * BATCH_F32_BYTES_PER_POINT + nodes * SUBSTEP_BYTES_PER_NODE
+        k_moved = n_total * BATCH_F32_MOVED_BYTES_PER_POINT + nodes * BATCH_MOVED_BYTES_PER_NODE
         achieved = k_bytes / k_avg_s / 1e9 if klaunch else None
-        log(f"bench: fused pass {k_avg_s * 1e6:.1f} us ({klaunch} timed launches), "
+        log(f"bench: substep kernel {k_avg_s * 1e6:.1f} us ({klaunch} timed launches), "
             f"{achieved:.0f} GB/s algorithmic")
 
         # 5. the batched engine with the exact map, same setting
@@ -481,8 +481,8 @@ def run_batch_learned(args) -> dict:
         },
         "roofline": {
             "bound": "hbm",
-            "kernel": (f"k_batch_particles<F32,G2P,P2G,{'learned' if branches else 'exact'}> "
-                       "(fused G2P + P2G, all cases)"),
+            "kernel": (f"k_batch_substep<F32,G2P,{'learned' if branches else 'exact'}> "
+                       "(grid update + G2P + P2G, all cases)"),
             "achieved": achieved,
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
@@ -498,8 +498,8 @@ def run_batch_learned(args) -> dict:
             "timed_launches": klaunch,
             "copy_kernel_gbs": copy_gbs,
         },
-        # the whole substep (grid update and map kernel included) at the
-        # per-unit figure for FP32 state: 108 B per point + 40 B per node
+        # the whole substep (map kernel included) at the per-unit figure for
+        # FP32 state: 108 B per point + 80 B per node
         "substep_effective_gbs": k_bytes * steps / (ms / 1e3) / 1e9,
         "comparison": {
             "plain_single_case_f64_pups": plain_pups,

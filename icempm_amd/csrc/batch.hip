@@ -1,7 +1,7 @@
 // batch.hip -- many independent indentation cases of uneven size advanced
-// together: one launch of the grid update and one of the fused particle pass
-// per substep cover every case, and the substep loop is captured once in a
-// HIP graph and replayed.
+// together: one launch per substep does the grid update, the G2P and the next
+// P2G of every case, and the substep loop is captured once in a HIP graph and
+// replayed.
 //
 // Storage (per batch, cases contiguous, each case in band order):
 //   F64 variant    positions: 2 rows of double; vel(2) Fe(4) Bp(4) Jp_inv(1):
@@ -13,10 +13,9 @@
 //                  from 1 so that float keeps them to ~1e-12 absolute.
 //   crushed        1 byte per point
 //   grain          i16 per point, only when a case has GrainVariability != 0
-//   grids          two grids of 3 rows of double per node (mass, momentum;
-//                  velocity after the update), cases concatenated, swapped
-//                  every substep; the F32 variant also keeps one FP32
-//                  velocity pair per node for the gathers
+//   grids          three grids of 3 rows of double per node (mass, momentum),
+//                  cases concatenated: a substep reads one, scatters into the
+//                  next and clears the third
 // All arithmetic is FP64 in both variants (the return map included); the F32
 // variant only stores less: a fused pass moves 49 B per point instead of 97 B.
 // A case's NACC strengths are uniform (constants per case) or vary per grain
@@ -56,6 +55,8 @@ struct CaseParams {
     double posQ, posInvQ, cellQ, cellQ16, cellInvQ;
     double gxInv;           // 1 / gx: a node's row from its index
     double scm;             // dt V_p D^-1 / m_p: the stress term of the affine momentum per unit mass
+    double vmax;            // the speed limit, half a cell per substep
+    double dtCells;         // dt / h
     int gx, gy, gridTotal, nPts, ptOffset, gridOffset;
     int nbins, binOffset;   // indenter force bins: n_indenter_subdivisions, first double in the bin array
 };
@@ -63,7 +64,6 @@ struct CaseParams {
 #ifndef ICEMPM_BATCH_CHAINS
 #define ICEMPM_BATCH_CHAINS 2   // independent chains of a batched run (groups of cases)
 #endif
-constexpr int kWX = 48, kWS = 52, kWY = 4;   // window width, padded row stride, rows
 
 // Point rows.  FP64 storage: positions FP64.  FP32 storage: positions as
 // 48-bit fixed point in units of h 2^-F, the cell index in the top 48 - F
@@ -127,12 +127,15 @@ static __device__ __forceinline__ double fix_cells(unsigned int hi, unsigned int
 }
 static __device__ __forceinline__ double fix_put_cells(double xr, const CaseParams &cp, unsigned int &hi,
                                                        unsigned int &lo) {
-    double u = rint(xr * cp.cellInvQ);
-    u = (u >= 0.0 && u <= kFix48Max) ? u : (u < 0.0 ? 0.0 : kFix48Max);
-    const double uh = floor(u * (1.0 / 65536.0));
-    hi = (unsigned int)uh;
-    lo = (unsigned int)(u - uh * 65536.0);
-    return u;
+    // clamped (NaN to the top), then u + 2^52: its low 48 mantissa bits are u,
+    // rounded to nearest even as rint would
+    const double top = kFix48Max * cp.cellQ;
+    const double c = xr >= 0.0 ? fmin(xr, top) : (xr < 0.0 ? 0.0 : top);
+    const double s = fma(c, cp.cellInvQ, 0x1p52);
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, s);
+    hi = (unsigned int)(b >> 16);
+    lo = (unsigned int)b & 0xFFFFu;
+    return s - 0x1p52;
 }
 // The quadratic B-spline stencil (gpu_implementation5.cu:185-193) of a
 // coordinate in cell units: base cell floor(xr - 0.5), 0 below xr = 0.5 (as
@@ -196,17 +199,6 @@ typedef float fe4 __attribute__((ext_vector_type(4)));
 static __device__ __forceinline__ fe4 *fe_rec(float *R, size_t pp) { return reinterpret_cast<fe4 *>(R + pp * 2); }
 static __device__ __forceinline__ const fe4 *fe_rec(const float *R, size_t pp) {
     return reinterpret_cast<const fe4 *>(R + pp * 2);
-}
-
-// the velocity of a node (index within its case's grid) as the gathers read it
-static __device__ __forceinline__ void grid_v(const double *g, int node, size_t gpitch, double &v0, double &v1) {
-    v0 = g[gpitch + node];
-    v1 = g[2 * gpitch + node];
-}
-static __device__ __forceinline__ void grid_v(const float2 *g, int node, size_t, float &v0, float &v1) {
-    const float2 a = *at(g, (unsigned)node);
-    v0 = a.x;
-    v1 = a.y;
 }
 
 static __device__ __forceinline__ void wsync() {
@@ -331,14 +323,207 @@ static __device__ __forceinline__ double yield_residual(const KParams &k, const 
     return fmax(fabs(qt - qlim) / k.iss, k.kappa * fabs(dm) / k.ics);
 }
 
-// Bytes of the per-wavefront P2G window.
-constexpr int kWaveWinBytes = 3 * kWY * kWS * 8;
+// A chunk: the up to 256 points of a workgroup, a wavefront a 64 of them, the
+// box of grid nodes their stencils touch, and in it the window of each
+// wavefront.  The workgroup keeps them in the record, renewing them every
+// kBoxEvery substeps (points move far less than a cell in that time; one that
+// has left takes the general paths).
+struct __attribute__((aligned(16))) ChunkRec {
+    int beg, count;   // first slot, points
+    int cs, gofs;     // the case and its first grid node
+    unsigned dims;    // GridX | GridY << 16
+    unsigned org;     // the box: first column | first row << 16
+    unsigned ext;     // columns | rows << 8 | tile stride << 16 (0: no box)
+    unsigned inv;     // ceil(2^16 / columns): a node's row from its index in the box
+    unsigned win[4];  // the windows: first column | first row << 8 (both from the box's) | columns << 16 | rows << 24
+};
+constexpr int kBoxEvery = 8;
 
-// Fused particle pass over all cases (G2P of substep k and/or P2G of k+1).
-// The chunk table, the case table and the point rows lead the arguments,
-// which the kernel receives preloaded in SGPRs: a workgroup's first load is
-// its chunk {first point, end, case}, the point loads follow it at once,
-// and the case's parameters arrive meanwhile.
+// LDS of a workgroup: a window per wavefront for its P2G (three sums per
+// node), the tile of node velocities its G2P reads, and a patch per wavefront
+// for the velocities of kPatch points outside the box.  64 points in band
+// order, four to a cell, touch 10 x 4 nodes and 256 points 34 x 4; the space
+// (25.6 KB, for six workgroups a CU) holds more rows, for points that have moved
+// out of their band.
+constexpr int kWaveWin = 160, kTile = 384;   // nodes x row stride
+constexpr int kWinCols = 40;
+constexpr int kPatch = 7;                // x 9 nodes: one load round of a wavefront
+constexpr int kChunkCols = 58;           // base cells a chunk may span: 60 columns of nodes
+
+// The row stride of a window: rows next to each other lie on different LDS
+// banks (a row of S doubles shifts them by 2 S of 64).
+static __device__ __forceinline__ int win_stride(int w) { return w <= 16 ? 20 : (w <= 32 ? 36 : kWinCols); }
+
+// The box of the base cells [x0, x1] x [y0, y1] as a record's org, ext and
+// inv; false if it does not fit the space.  A tile row of T 16-byte entries, T
+// = 8 mod 16, puts the two cell rows of a band on different LDS banks; a
+// taller box packs its rows.
+static __device__ __forceinline__ bool set_box(ChunkRec &r, int x0, int y0, int x1, int y1) {
+    const int w = x1 + 3 - x0, h = y1 + 3 - y0;
+    if (w > 128 || h > 128 || w * h > kTile) return false;
+    int T = ((w + 7) >> 4) * 16 + 8;
+    if (T * h > kTile) T = w;
+    r.org = (unsigned)x0 | (unsigned)y0 << 16;
+    r.ext = (unsigned)w | (unsigned)h << 8 | (unsigned)T << 16;
+    r.inv = 65535u / (unsigned)w + 1u;
+    return true;
+}
+// A wavefront's window in that box: the stencils of the base cells
+// [x0, x1] x [y0, y1] of its points, as far as they lie in the box and the
+// window has room.
+static __device__ __forceinline__ unsigned win_of(const ChunkRec &r, int x0, int y0, int x1, int y1) {
+    const int ox = (int)(r.org & 0xFFFFu), oy = (int)(r.org >> 16);
+    x0 = max(x0 - ox, 0);
+    y0 = max(y0 - oy, 0);
+    const int w = min(min(x1 - ox + 3, (int)(r.ext & 0xFFu)) - x0, kWinCols);
+    const int h = min(min(y1 - oy + 3, (int)(r.ext >> 8 & 0xFFu)) - y0, kWaveWin / win_stride(w));
+    return w < 3 || h < 3 ? 0u : (unsigned)x0 | (unsigned)y0 << 8 | (unsigned)w << 16 | (unsigned)h << 24;
+}
+
+// The velocity a node has after the grid update (gpu_implementation5.cu:
+// 215-290) from its mass (not zero) and momentum: gravity, the speed limit,
+// the indenter's contact, the walls.  Returns whether the indenter touches
+// it; d is then the velocity the contact takes from it and n the unit normal.
+// 1/m comes from rcp_nr.
+static __device__ __forceinline__ bool node_velocity(const CaseParams &cp, double ind_x, double mass, double p0,
+                                                     double p1, int ix, int iy, double &v0, double &v1, double &d0,
+                                                     double &d1, double &n0, double &n1) {
+    const double rm = rcp_nr(mass);
+    v0 = p0 * rm;
+    v1 = p1 * rm;
+    v1 = v1 - cp.dt * cp.gravity;
+    const double vsq = v0 * v0 + v1 * v1;
+    if (vsq > cp.vmax * cp.vmax) {
+        const double s = cp.vmax / sqrt(vsq);
+        v0 = v0 * s;
+        v1 = v1 * s;
+    }
+    bool hit = false;
+    n0 = ix * cp.h - ind_x;
+    n1 = iy * cp.h - cp.y0;
+    const double z = n0 * n0 + n1 * n1;
+    if (z < cp.indRsq) {
+        const double V = cp.indV, r0 = v0 - V, r1 = v1;
+        if (z > 0) {
+            const double nz = sqrt(z);
+            n0 = n0 / nz;
+            n1 = n1 / nz;
+        }
+        const double vnr = r0 * n0 + r1 * n1;
+        if (vnr < 0) {
+            d0 = v0;
+            d1 = v1;
+            v0 = V + (r0 - n0 * vnr);
+            v1 = r1 - n1 * vnr;
+            d0 -= v0;
+            d1 -= v1;
+            hit = true;
+        }
+    }
+    if (iy <= 2) {
+        v0 = 0;
+        v1 = 0;
+    } else if (iy >= cp.gy - 3 && v1 > 0) {
+        v1 = 0;
+    }
+    if (ix <= 2 && v0 < 0)
+        v0 = 0;
+    else if (ix >= cp.gx - 3 && v0 > 0)
+        v0 = 0;
+    return hit;
+}
+
+// The grid side of a substep: the workgroups after the particle ones each
+// take kNodeBlk nodes of one case.  They clear the grid that the next
+// substep scatters into and add up the indenter's force; nothing else of the
+// grid update is left to them, since every wavefront makes the velocities of
+// its own box.  bounds holds, per case, the box of all nodes that the P2G has
+// ever touched since the run's fresh start (columns and rows of the least and
+// greatest, widened by the passes): outside it (and a border of one) the
+// grids are still zero.
+constexpr int kNodeBlk = 1024;
+struct NodeWork {
+    const int2 *blocks;   // {case, first node} per workgroup
+    double *clear;        // the grid to clear
+    double *hist;         // this substep's force, 2 per case
+    double *bins;
+};
+
+static __device__ __forceinline__ void node_part(const NodeWork &nw, int block, const CaseParams *__restrict__ cases,
+                                                 const double *__restrict__ grid, size_t gpitch, const int4 *bounds,
+                                                 double t, double *lds) {
+    const int2 nb = nw.blocks[block];
+    const CaseParams &cp = cases[nb.x];
+    const int4 bd = bounds[nb.x];
+    const int x0 = bd.x - 1, y0 = bd.y - 1, x1 = bd.z + 1, y1 = bd.w + 1;
+    // rows of the block: (node + 0.5) / gx lies >= 0.5 / gx >= 2^-17 from an
+    // integer and is computed to within 2^-23, so its floor is the row
+    const int first = (int)(((double)nb.y + 0.5) * cp.gxInv);
+    const int last = (int)(((double)min(nb.y + kNodeBlk, cp.gridTotal) - 0.5) * cp.gxInv);
+    if (bd.z < 0 || last < y0 || first > y1) return;   // uniform: nothing was ever touched here
+    if (threadIdx.x < 3) lds[threadIdx.x] = 0;
+    __syncthreads();
+    const double ind_x = cp.x0 + t * cp.indV;
+#pragma unroll
+    for (int q = 0; q < kNodeBlk; q += 256) {
+        const int local = nb.y + q + (int)threadIdx.x;
+        const int iy = (int)(((double)local + 0.5) * cp.gxInv), ix = local - iy * cp.gx;
+        if (local >= cp.gridTotal || ix < x0 || ix > x1 || iy < y0 || iy > y1) continue;
+        const size_t idx = (size_t)cp.gridOffset + local;
+        nw.clear[idx] = 0;
+        nw.clear[gpitch + idx] = 0;
+        nw.clear[2 * gpitch + idx] = 0;
+        const double c0 = ix * cp.h - ind_x, c1 = iy * cp.h - cp.y0;
+        if (c0 * c0 + c1 * c1 < cp.indRsq) {
+            const double mass = grid[idx];
+            if (mass != 0) {
+                double v0, v1, d0, d1, n0, n1;
+                if (node_velocity(cp, ind_x, mass, grid[gpitch + idx], grid[2 * gpitch + idx], ix, iy, v0, v1, d0, d1,
+                                  n0, n1)) {
+                    const double f0 = d0 * mass / cp.dt, f1 = d1 * mass / cp.dt;
+                    atomicAdd(&lds[0], f0);
+                    atomicAdd(&lds[1], f1);
+                    lds[2] = 1;
+                    // the force's angular bin (gpu_implementation5.cu:262-269:
+                    // atan2 of (x, y) of the unit normal, then + pi, scaled)
+                    double angle = atan2(n0, n1);
+                    angle += kPi;
+                    angle *= cp.nbins / (2 * kPi);
+                    int kb = (int)angle;
+                    kb = max(kb, 0);
+                    kb = min(kb, cp.nbins - 1);
+                    unsafeAtomicAdd(&nw.bins[cp.binOffset + 2 * kb], f0);
+                    unsafeAtomicAdd(&nw.bins[cp.binOffset + 2 * kb + 1], f1);
+                }
+            }
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0 && lds[2] != 0) {
+        unsafeAtomicAdd(&nw.hist[2 * nb.x], lds[0]);
+        unsafeAtomicAdd(&nw.hist[2 * nb.x + 1], lds[1]);
+    }
+}
+
+// Node e of a box of the given width: its column and row.
+static __device__ __forceinline__ void box_node(unsigned e, unsigned inv, unsigned w, unsigned &col, unsigned &row) {
+    row = e * inv >> 16;
+    col = e - row * w;
+}
+
+// Widens a case's box of touched nodes to the stencils of base cells
+// [x0, x1] x [y0, y1].  Mostly it holds them already: the atomics of every
+// workgroup on the few cases' boxes would take longer than the substep.
+static __device__ __forceinline__ void widen_bounds(int4 *bounds, int cs, int x0, int y0, int x1, int y1) {
+    int *b = reinterpret_cast<int *>(&bounds[cs]);
+    const auto get = [&](int i) { return __hip_atomic_load(b + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
+    if (x0 >= get(0) && y0 >= get(1) && x1 + 2 <= get(2) && y1 + 2 <= get(3)) return;
+    atomicMin(b, x0);
+    atomicMin(b + 1, y0);
+    atomicMax(b + 2, x1 + 2);
+    atomicMax(b + 3, y1 + 2);
+}
+
 // Quad-level P2G.  A DPP read of a double from another lane of the quad
 // (quad_perm control CTRL; every lane of the quad must be active, so no
 // lane keeps an old value and none is needed)
@@ -387,7 +572,7 @@ static __device__ __forceinline__ void quad_component(int lane, const double (&K
 // lane then adds two or three of the nine node sums per row: 6-9 LDS
 // atomics instead of 27, the nodes of one instruction still distinct
 // within the quad.
-static __device__ __forceinline__ void quad_scatter(int lane, int e0, double h, double fx0, double fx1, double wx0,
+static __device__ __forceinline__ void quad_scatter(int lane, int e0, int S, double h, double fx0, double fx1, double wx0,
                                                     double wx1, double wx2, double wy0, double wy1, double wy2,
                                                     double vx, double vy, double A00, double A01, double A10,
                                                     double A11, double *W0, double *W1, double *W2) {
@@ -415,9 +600,9 @@ static __device__ __forceinline__ void quad_scatter(int lane, int e0, double h, 
     WK[4] = wx1 * wy2;
     // the nodes a lane adds: slot sy's node (2 sx, sy); slot 2 + sy's node,
     // (2 sx, 2) or (1, sx); slot 4's node (1, 2)
-    const int eA = e0 + 2 * sx + sy * kWS;
-    const int eB = e0 + (sy ? 1 + sx * kWS : 2 * sx + 2 * kWS);
-    const int eC = e0 + 1 + 2 * kWS;
+    const int eA = e0 + 2 * sx + sy * S;
+    const int eB = e0 + (sy ? 1 + sx * S : 2 * sx + 2 * S);
+    const int eC = e0 + 1 + 2 * S;
     quad_component(lane, WK, WD, eA, eB, eC, W0);
     double K[5], D[4];
 #pragma unroll
@@ -440,317 +625,406 @@ static __device__ __forceinline__ void quad_scatter(int lane, int e0, double h, 
     quad_component(lane, K, D, eA, eB, eC, W2);
 }
 
-template <bool F32, bool G2P, bool P2G, int RMAP>
-__global__ __launch_bounds__(256) void k_batch_particles(const int4 *__restrict__ chunks, int nChunks,
-                                                         const CaseParams *__restrict__ cases,
-                                                         typename Rows<F32>::P *pos,
-                                                         typename Rows<F32>::V *rest, unsigned char *crushedRow,
-                                                         size_t pitch, const typename Rows<F32>::G *__restrict__ gridV,
-                                                         double *__restrict__ gridOut, size_t gpitch,
-                                                         int *__restrict__ err, const short *__restrict__ grains,
-                                                         LearnArgs la, MapQueue mq, int storeVB) {
+
+// One substep over all cases: grid update, G2P of this substep and P2G of
+// the next (G2P false: a run's first P2G alone).  gridIn holds the masses and
+// momenta of the last P2G; every workgroup turns the nodes of its box into
+// velocities in LDS (a node a thread), its wavefronts gather from there, move
+// their points, sum their contributions in a window of their own and add it to
+// gridOut with one atomic per node and component; the workgroups from pGroups
+// on do the rest of the grid update (node_part).
+//
+// What bounds it is FP64 arithmetic: ~530 vector instructions per 64 points,
+// most of them FP64 at 4 cycles each (HBM is at a third of its rate).  Against
+// a grid update of its own, a particle pass that gathered from global memory
+// and found each wavefront's window anew (625 instructions), a substep of 32
+// cases / 6.98 million points went from 193 to 167 us (FP32 storage), of 12
+// cases / 81 thousand points from 18.4 to 8.9 us, of 8 cases / 671 thousand
+// points from 35 to 25 us (FP64, strengths per grain).  Making a node's
+// velocity in each of the ~2 workgroups that need it costs ~20 instructions per
+// 64 points; it saves a launch, the velocities' trip through memory and the
+// gathers' 6 to 18 loads a point.
+//
+// A window per wavefront, and the points in band order, keep the sums of each
+// node in the order quad, wavefront, grid.  One window per workgroup with the
+// points of a cell spread over its wavefronts (27 LDS atomics a point, none of
+// them at one address) takes 149 us, but adds the terms in another order: the
+// rounding of FP32 storage and the yield branches then carry a study's points
+// past 1e-5 of it within 4000 substeps in most runs, where two runs of this
+// order mostly agree to the bit.
+//
+// The records, the grid and the point rows lead the arguments, which the
+// kernel receives preloaded in SGPRs.
+template <bool F32, bool G2P, int RMAP>
+__global__ __launch_bounds__(256, 5) void k_batch_substep(
+    ChunkRec *__restrict__ recs, const double *__restrict__ gridIn, int nChunks, int pGroups,
+    typename Rows<F32>::P *pos, typename Rows<F32>::V *rest, size_t gpitch, const CaseParams *__restrict__ cases,
+    unsigned char *crushedRow, size_t pitch, double *__restrict__ gridOut, int4 *bounds, int *__restrict__ err,
+    const short *__restrict__ grains, const double *__restrict__ tTab, int step, NodeWork nw, LearnArgs la, MapQueue mq,
+    int storeVB) {
+    __shared__ __attribute__((aligned(16))) double smem[4 * 3 * kWaveWin + 2 * kTile + 4 * (2 * 9 + 1) * kPatch];
+    if constexpr (G2P) {
+        if ((int)blockIdx.x >= pGroups) {
+            node_part(nw, (int)blockIdx.x - pGroups, cases, gridIn, gpitch, bounds, tTab[step], smem);
+            return;
+        }
+    }
     const Rows<F32> S{pos, rest, crushedRow, nullptr, pitch};
-    __shared__ __attribute__((aligned(16))) double smem[4][kWaveWinBytes / 8];
-    const int per = (nChunks + 7) >> 3;
-    const int c = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-    if (c >= nChunks) return;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int4 ch = chunks[c];
-    const int beg = ch.x, end = ch.y;
-    asm volatile("" ::"s"(ch.z));   // all of the chunk in one load, before the branch
-    // FP32 storage: a wavefront issues its point loads and gathers, and later
-    // its window flush, at raised priority, computes at the base one
-    // (measured: -2.6% per substep; FP64 storage measured slower with it)
+    // neighbouring chunks on one XCD (workgroups go round the 8 XCDs)
+    const int chunk = (blockIdx.x & 7) * (pGroups >> 3) + (blockIdx.x >> 3);
+    if (chunk >= nChunks) return;
+    const int lane = threadIdx.x & 63, row = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const ChunkRec rec = recs[chunk];
+    // FP32 storage: a wavefront issues its loads, and later its window flush,
+    // at raised priority, computes at the base one (measured: -2.6% per
+    // substep; FP64 storage measured slower with it)
     if constexpr (F32) __builtin_amdgcn_s_setprio(2);
-    if (beg + wv * 64 >= end) return;
-    const CaseParams cp = cases[ch.z];
+    const CaseParams &cp = cases[rec.cs];
     const KParams k = kp_of(cp, err);
-    const int pt = beg + (int)threadIdx.x;
-    const bool valid = pt < end;
     const size_t pp = S.pitch;
-    const int gx = cp.gx, gy = cp.gy;
-    const auto *__restrict__ gV = gridV + cp.gridOffset;
-    double *__restrict__ gO = gridOut + cp.gridOffset;
+    const int gx = (int)(rec.dims & 0xFFFFu), gy = (int)(rec.dims >> 16);
+    const double *__restrict__ gI = gridIn + rec.gofs;
+    double *__restrict__ gO = gridOut + rec.gofs;
     using V = typename Rows<F32>::V;
     V *__restrict__ R = S.rest;
     constexpr double fe0 = F32 ? 1.0 : 0.0;   // stored Fe = Fe - fe0 * I, Jp_inv - fe0
+    // the wavefront's points: lanes of them (none past the last one)
+    const int lanes = rec.count - row * 64;
+    const bool valid = lane < lanes;
+    const int pt = rec.beg + row * 64 + lane;
+    const unsigned u = (unsigned)pt;
+    // the box with the tile, and the wavefront's window
+    const int ox = (int)(rec.org & 0xFFFFu), oy = (int)(rec.org >> 16);
+    const int bw = (int)(rec.ext & 0xFFu), bh = (int)(rec.ext >> 8 & 0xFFu), tS = (int)(rec.ext >> 16 & 0xFFu);
+    const unsigned nodes = (unsigned)(bw * bh);
+    // base cells whose stencil lies in the box and in the grid: [ox, ox + fw) x [oy, oy + fh)
+    const unsigned fw = (unsigned)max(min(bw, gx - ox) - 2, 0), fh = (unsigned)max(min(bh, gy - oy) - 2, 0);
+    const unsigned win = recs[chunk].win[row];
+    const int wx = ox + (int)(win & 0xFFu), wy = oy + (int)(win >> 8 & 0xFFu);
+    const int ww = (int)(win >> 16 & 0xFFu), wh = (int)(win >> 24), wS = win_stride(ww);
+    const unsigned ww2 = (unsigned)max(min(ww, gx - wx) - 2, 0), wh2 = (unsigned)max(min(wh, gy - wy) - 2, 0);
+    // lanes map onto the window 16, 32 or 64 columns at a time
+    const int wsh = ww <= 16 ? 4 : (ww <= 32 ? 5 : 6);
+    const int wcol = lane & ((1 << wsh) - 1), wrow0 = lane >> wsh, wstep = 64 >> wsh;
+    double *W0 = smem + row * 3 * kWaveWin, *W1 = W0 + kWaveWin, *W2 = W1 + kWaveWin;
+    double2 *tile = reinterpret_cast<double2 *>(smem + 4 * 3 * kWaveWin);
+    const double ind_x = cp.x0 + (G2P ? tTab[step] : 0.0) * cp.indV;
 
-    double px = 0, py = 0, vx = 0, vy = 0;
-    double F00 = 1, F01 = 0, F10 = 0, F11 = 1;
-    double B00 = 0, B01 = 0, B10 = 0, B11 = 0;
-    bool defer = false;   // learned map: projection and P2G done by the map kernel
-    InvSq rt{};           // the trial invariants, and whether the map left F alone
-    bool fresh = false;
+    // The state of the points, streamed once per substep: non-temporal, so the
+    // grid keeps the L2.  A lane without a point reads the chunk's first one
+    // and computes along with the others; only its stores and sums are left out.
+    prec4 pr;
+    fe4 fr;
+    double px, py, F00, F01, F10, F11;
+    unsigned char crushed = 0;
+    short grain = 0;
+    const unsigned us = valid ? u : (unsigned)rec.beg;
+    if constexpr (F32) {
+        pr = __builtin_nontemporal_load(reinterpret_cast<const prec4 *>(S.pos) + us);
+        fr = __builtin_nontemporal_load(fe_rec(R, pp) + us);
+    } else {
+        pos_load<true>(S.pos, pp, (int)us, cp, px, py);
+        F00 = __builtin_nontemporal_load(at(R + pp * 2, us));
+        F01 = __builtin_nontemporal_load(at(R + pp * 3, us));
+        F10 = __builtin_nontemporal_load(at(R + pp * 4, us));
+        F11 = __builtin_nontemporal_load(at(R + pp * 5, us));
+        crushed = __builtin_nontemporal_load(at(S.crushed, us));
+        if (cp.grainVar != 0) grain = __builtin_nontemporal_load(at(grains, us));
+    }
 
-    if constexpr (G2P) {
-        double Jp = 1;
-        unsigned char crushed = 0;
-        short grain = 0;
-        if (valid) {
-            // streamed once per substep: non-temporal, so the grid keeps the L2
-            const unsigned u = (unsigned)pt;
-            if constexpr (F32) {
-                // the record; its coordinates in cell units
-                const prec4 r = __builtin_nontemporal_load(reinterpret_cast<const prec4 *>(S.pos) + pt);
-                px = fix_cells(r.x, r.z & 0xFFFFu, cp);
-                py = fix_cells(r.y, r.z >> 16, cp);
-                crushed = (unsigned char)(r.w & 0xFFu);
-                grain = (short)(r.w >> 16);
-                const fe4 f = __builtin_nontemporal_load(fe_rec(R, pp) + pt);
-                F00 = fe0 + (double)f.x;
-                F01 = (double)f.y;
-                F10 = (double)f.z;
-                F11 = fe0 + (double)f.w;
-            } else {
-                pos_load<true>(S.pos, pp, pt, cp, px, py);
-                F00 = fe0 + (double)__builtin_nontemporal_load(at(R + pp * 2, u));
-                F01 = (double)__builtin_nontemporal_load(at(R + pp * 3, u));
-                F10 = (double)__builtin_nontemporal_load(at(R + pp * 4, u));
-                F11 = fe0 + (double)__builtin_nontemporal_load(at(R + pp * 5, u));
-                crushed = __builtin_nontemporal_load(at(S.crushed, u));
-                if (cp.grainVar != 0) grain = __builtin_nontemporal_load(at(grains, u));
-            }
+    if (wcol < ww) {
+        for (int r = wrow0; r < wh; r += wstep) {
+            const int e = r * wS + wcol;
+            W0[e] = 0;
+            W1[e] = 0;
+            W2[e] = 0;
         }
-        int bx = 0, by = 0;
-        double fx0 = 0, fx1 = 0, wx0, wx1, wx2, wy0, wy1, wy2;
-        bool ok;
-        if constexpr (F32) {   // cell units: a record always has a stencil
-            ok = valid;
-            if (ok) {
+    }
+    // the box's velocities (FP32 storage rounds them to FP32)
+    if constexpr (G2P) {
+        for (unsigned e = threadIdx.x; e < nodes; e += 256) {
+            unsigned c, r;
+            box_node(e, rec.inv, (unsigned)bw, c, r);
+            const int X = ox + (int)c, Y = oy + (int)r;
+            const bool in = X < gx && Y < gy;
+            const unsigned node = in ? (unsigned)(X + Y * gx) : 0u;
+            const double mass = *at(gI, node), m0 = *at(gI + gpitch, node), m1 = *at(gI + 2 * gpitch, node);
+            double n0, n1, e0, e1, e2, e3;
+            node_velocity(cp, ind_x, mass, m0, m1, X, Y, n0, n1, e0, e1, e2, e3);
+            if constexpr (F32) {
+                n0 = (double)(float)n0;
+                n1 = (double)(float)n1;
+            }
+            const bool moves = in && mass != 0;   // a node without mass has no velocity
+            tile[r * (unsigned)tS + c] = make_double2(moves ? n0 : 0.0, moves ? n1 : 0.0);
+        }
+    }
+    if constexpr (F32) __builtin_amdgcn_s_setprio(0);
+    if constexpr (G2P) __syncthreads();
+
+    // the base cells of the points, for the box (when it is renewed)
+    int cellx = -1, celly = -1;
+    if (lanes > 0) {
+        double vx, vy;
+        double B00, B01, B10, B11;   // Bp
+        double t00, t01, t11;        // the Kirchhoff stress
+        bool defer = false;          // learned map: projection and P2G done by the map kernel
+        if constexpr (G2P) {
+            double Jp = 1;
+            if constexpr (F32) {   // the record's coordinates in cell units
+                px = fix_cells(pr.x, pr.z & 0xFFFFu, cp);
+                py = fix_cells(pr.y, pr.z >> 16, cp);
+                crushed = (unsigned char)(pr.w & 0xFFu);
+                grain = (short)(pr.w >> 16);
+                F00 = fe0 + (double)fr.x;
+                F01 = (double)fr.y;
+                F10 = (double)fr.z;
+                F11 = fe0 + (double)fr.w;
+            }
+            int bx = 0, by = 0;
+            double fx0 = 0, fx1 = 0, wx0 = 0, wx1 = 0, wx2 = 0, wy0 = 0, wy1 = 0, wy2 = 0;
+            bool ok = valid;
+            if constexpr (F32) {   // a record always has a stencil
                 stencil_cells(px, bx, fx0, wx0, wx1, wx2);
                 stencil_cells(py, by, fx1, wy0, wy1, wy2);
-            }
-        } else {
-            ok = valid && stencil(px, cp.h_inv, bx, fx0, wx0, wx1, wx2) &&
-                 stencil(py, cp.h_inv, by, fx1, wy0, wy1, wy2);
-            if (valid && !ok) flag_error(k);
-        }
-        InvSq iv{};
-        unsigned char crushed0 = crushed;
-        double Jp0 = Jp;
-        if (ok) {
-            // the gathered velocities stay in their stored type (FP32 pairs
-            // or FP64) and widen at each use: fewer live registers
-            using GT = typename std::conditional<F32, float, double>::type;
-            GT n0[9], n1[9];
-            if (bx + 2 < gx && by + 2 < gy) {
-                if constexpr (F32) {
-                    // a stencil row's three FP32 pairs as one 16-byte load
-                    // (8-byte aligned: the unaligned 16-byte access global
-                    // memory allows) and one 8-byte load: 6 loads instead of
-                    // 9 (measured 2% off the pass)
-                    typedef float v4u __attribute__((ext_vector_type(4), aligned(8)));
-#pragma unroll
-                    for (int j = 0; j < 3; ++j) {
-                        const unsigned node = (unsigned)(bx + (by + j) * gx);
-                        const v4u a = *reinterpret_cast<const v4u *>(at(gV, node));
-                        const float2 c = *at(gV, node + 2);
-                        n0[0 * 3 + j] = a.x;
-                        n1[0 * 3 + j] = a.y;
-                        n0[1 * 3 + j] = a.z;
-                        n1[1 * 3 + j] = a.w;
-                        n0[2 * 3 + j] = c.x;
-                        n1[2 * 3 + j] = c.y;
-                    }
-                } else {
-                    const double *gvx = gV + gpitch + bx + by * gx;
-                    const double *gvy = gvx + gpitch;
-#pragma unroll
-                    for (int i = 0; i < 3; ++i)
-#pragma unroll
-                        for (int j = 0; j < 3; ++j) {
-                            n0[i * 3 + j] = gvx[i + j * gx];
-                            n1[i * 3 + j] = gvy[i + j * gx];
-                        }
-                }
             } else {
-#pragma unroll
-                for (int i = 0; i < 3; ++i)
-#pragma unroll
-                    for (int j = 0; j < 3; ++j) {
-                        const int X = bx + i, Y = by + j;
-                        n0[i * 3 + j] = 0;
-                        n1[i * 3 + j] = 0;
-                        if (X >= gx || Y >= gy) {
-                            flag_error(k);
-                        } else {
-                            grid_v(gV, X + Y * gx, gpitch, n0[i * 3 + j], n1[i * 3 + j]);
-                        }
-                    }
+                const bool st = stencil(px, cp.h_inv, bx, fx0, wx0, wx1, wx2) &&
+                                stencil(py, cp.h_inv, by, fx1, wy0, wy1, wy2);
+                ok = valid && st;
+                if (valid && !st) flag_error(k);
             }
-            if constexpr (F32) __builtin_amdgcn_s_setprio(0);
-            double v0 = 0, v1 = 0, b00 = 0, b01 = 0, b10 = 0, b11 = 0;
+            // the node velocities: in the tile, or for a point outside the box
+            // in the wavefront's patch, where 9 lanes a point put them
+            const int lx0 = bx - ox, ly0 = by - oy;
+            const bool inTile = (unsigned)lx0 < fw && (unsigned)ly0 < fh;
+            const double2 *line = tile + (inTile ? ly0 * tS + lx0 : 0);
+            int ls = tS;
+            bool slow = ok && !inTile;
+            if (const unsigned long long om = __ballot(slow)) {
+                double2 *patch = tile + kTile + row * 9 * kPatch;
+                int2 *cells = reinterpret_cast<int2 *>(tile + kTile + 4 * 9 * kPatch) + row * kPatch;
+                const int rank = __popcll(om & ((1ull << lane) - 1ull));
+                if (slow && rank < kPatch) cells[rank] = make_int2(bx, by);
+                wsync();
+                const int e = lane, o = e / 9, n = e - 9 * o;
+                if (e < 9 * min(__popcll(om), kPatch)) {
+                    const int2 cell = cells[o];
+                    const int X = cell.x + n % 3, Y = cell.y + n / 3;
+                    double n0 = 0, n1 = 0;
+                    if (X >= gx || Y >= gy) {
+                        flag_error(k);
+                    } else {
+                        const unsigned node = (unsigned)(X + Y * gx);
+                        const double mass = *at(gI, node), m0 = *at(gI + gpitch, node), m1 = *at(gI + 2 * gpitch, node);
+                        double e0, e1, e2, e3;
+                        if (mass != 0) node_velocity(cp, ind_x, mass, m0, m1, X, Y, n0, n1, e0, e1, e2, e3);
+                    }
+                    if constexpr (F32) {
+                        n0 = (double)(float)n0;
+                        n1 = (double)(float)n1;
+                    }
+                    patch[e] = make_double2(n0, n1);
+                }
+                wsync();
+                if (slow && rank < kPatch) {
+                    line = patch + 9 * rank;
+                    ls = 3;
+                    slow = false;
+                }
+            }
+            double v0 = 0, v1 = 0, b00 = 0, b01 = 0, b10 = 0, b11 = 0;   // v and Bp
             const double c4 = 4. * cp.h_inv;
-            const double wyd0 = wy0 * (0 - fx1), wyd1 = wy1 * (1 - fx1), wyd2 = wy2 * (2 - fx1);
-            const double wxs[3] = {wx0, wx1, wx2};
+            {
+                const double wyd0 = wy0 * (0 - fx1), wyd1 = wy1 * (1 - fx1), wyd2 = wy2 * (2 - fx1);
+                const double wxs[3] = {wx0, wx1, wx2};
 #pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                const double a0 = n0[i * 3], a1 = n0[i * 3 + 1], a2 = n0[i * 3 + 2];
-                const double c0 = n1[i * 3], c1 = n1[i * 3 + 1], c2 = n1[i * 3 + 2];
-                const double s0 = wy0 * a0 + wy1 * a1 + wy2 * a2;
-                const double s1 = wy0 * c0 + wy1 * c1 + wy2 * c2;
-                const double t0 = wyd0 * a0 + wyd1 * a1 + wyd2 * a2;
-                const double t1 = wyd0 * c0 + wyd1 * c1 + wyd2 * c2;
-                const double wxd = wxs[i] * (i - fx0);
-                v0 += wxs[i] * s0;
-                v1 += wxs[i] * s1;
-                b00 += wxd * s0;
-                b10 += wxd * s1;
-                b01 += wxs[i] * t0;
-                b11 += wxs[i] * t1;
+                for (int i = 0; i < 3; ++i) {
+                    const double2 a = line[i], b = line[ls + i], c = line[2 * ls + i];
+                    const double s0 = wy0 * a.x + wy1 * b.x + wy2 * c.x;
+                    const double s1 = wy0 * a.y + wy1 * b.y + wy2 * c.y;
+                    const double t0 = wyd0 * a.x + wyd1 * b.x + wyd2 * c.x;
+                    const double t1 = wyd0 * a.y + wyd1 * b.y + wyd2 * c.y;
+                    const double wxd = wxs[i] * (i - fx0);
+                    v0 += wxs[i] * s0;
+                    v1 += wxs[i] * s1;
+                    b00 += wxd * s0;
+                    b10 += wxd * s1;
+                    b01 += wxs[i] * t0;
+                    b11 += wxs[i] * t1;
+                }
+            }
+            if (slow) {
+                // more points outside the box than the patch holds: node by node
+                v0 = v1 = b00 = b01 = b10 = b11 = 0;
+#pragma unroll 1
+                for (int e = 0; e < 9; ++e) {
+                    const int i = e % 3, j = e / 3, X = bx + i, Y = by + j;
+                    if (X >= gx || Y >= gy) {
+                        flag_error(k);
+                        continue;
+                    }
+                    const unsigned node = (unsigned)(X + Y * gx);
+                    const double mass = *at(gI, node);
+                    if (mass == 0) continue;
+                    double n0, n1, e0, e1, e2, e3;
+                    node_velocity(cp, ind_x, mass, *at(gI + gpitch, node), *at(gI + 2 * gpitch, node), X, Y, n0, n1,
+                                  e0, e1, e2, e3);
+                    if constexpr (F32) {
+                        n0 = (double)(float)n0;
+                        n1 = (double)(float)n1;
+                    }
+                    const double w = sel3(i, wx0, wx1, wx2) * sel3(j, wy0, wy1, wy2);
+                    v0 += w * n0;
+                    v1 += w * n1;
+                    b00 += w * n0 * (i - fx0);
+                    b01 += w * n0 * (j - fx1);
+                    b10 += w * n1 * (i - fx0);
+                    b11 += w * n1 * (j - fx1);
+                }
             }
             b00 *= c4; b01 *= c4; b10 *= c4; b11 *= c4;
+            B00 = b00; B01 = b01; B10 = b10; B11 = b11;
             const double dt = cp.dt;
-            const double dtp = F32 ? dt * cp.h_inv : dt;   // FP32 storage: cell units
+            const double dtp = F32 ? cp.dtCells : dt;   // FP32 storage: cell units
             px += v0 * dtp;
             py += v1 * dtp;
             const double M00 = 1.0 + dt * b00, M01 = dt * b01, M10 = dt * b10, M11 = 1.0 + dt * b11;
             const double n00 = M00 * F00 + M01 * F10, n01 = M00 * F01 + M01 * F11;
             const double n10 = M10 * F00 + M11 * F10, n11 = M10 * F01 + M11 * F11;
             F00 = n00; F01 = n01; F10 = n10; F11 = n11;
+            vx = v0; vy = v1;
             // p and q^2 of the trial state (q itself is never needed here:
             // every test compares it with a non-negative limit)
-            iv = invariants_sq(F00, F01, F10, F11, cp.mu, cp.kappa);
-            crushed0 = crushed;
-            Jp0 = Jp;
-            if (crushed == 0) {
-                bool f;
-                if (cp.grainVar != 0) {   // GetParametersForGrain's strengths (case-uniform branch)
-                    f = fails_sq(k, grain, iv.p, iv.q2);
-                } else if (iv.p < 0) {
-                    // tension line q > slope (p + 3e6), slope >= 0 and p + 3e6 >= 0 here
-                    const double ql = cp.slope * (iv.p - -3e6);
-                    f = (iv.p < -3e6) || (iv.q2 > ql * ql);
-                } else {
-                    f = cp.onePlus2Beta * iv.q2 + cp.msq * (iv.p + cp.betaPmax) * (iv.p - cp.pmax) > 0;
-                }
-                crushed = f ? 1 : 0;
+            const InvSq iv = invariants_sq(F00, F01, F10, F11, cp.mu, cp.kappa);
+            const unsigned char crushed0 = crushed;
+            if (cp.grainVar != 0) {   // GetParametersForGrain's strengths (case-uniform branch)
+                if (crushed == 0) crushed = fails_sq(k, grain, iv.p, iv.q2) ? 1 : 0;
+            } else {
+                // tension line q > slope (p + 3e6), slope >= 0 and p + 3e6 >= 0 there
+                const double ql = cp.slope * (iv.p - -3e6);
+                const bool ft = (iv.p < -3e6) || (iv.q2 > ql * ql);
+                const bool fc = cp.onePlus2Beta * iv.q2 + cp.msq * (iv.p + cp.betaPmax) * (iv.p - cp.pmax) > 0;
+                if (crushed == 0 && (iv.p < 0 ? ft : fc)) crushed = 1;
             }
-            vx = v0; vy = v1;
-            B00 = b00; B01 = b01; B10 = b10; B11 = b11;
-        }
-        // ---- return map (convergent: the learned map runs wavefront-wide) ----
-        // The trial SVD only for crushed points (few: the wavefront mostly
-        // skips it); p and q for the NACC test came from the invariants.
-        // Jp_inv matters only to the map, so only crushed points load it.
-        const bool crushedOk = ok && crushed == 1;
-        if (crushedOk) {
-            Jp = fe0 + (double)*at(R + pp * 10, (unsigned)pt);
-            Jp0 = Jp;
-        }
-        if constexpr (RMAP == kMapExact) {
-            if (crushedOk && dp_projects_sq(k, iv.p, iv.q2, Jp))
-                dp_return(k, compute_pq_fast(F00, F01, F10, F11, cp.mu, cp.kappa), F00, F01, F10, F11, Jp);
-        } else if constexpr (RMAP == kMapHarvest) {
-            Trial r{};
-            if (crushedOk) r = compute_pq_fast(F00, F01, F10, F11, cp.mu, cp.kappa);
-            double f[5] = {0, 0, 0, 0, 0}, t[3] = {0, 0, 0};
-            bool usable = false;
-            if (crushedOk) {
-                double qlim;
-                const int br = map_branch(k, r, Jp, qlim);
-                map_features(r, Jp, br, f);
-                dp_return(k, r, F00, F01, F10, F11, Jp);
-                if (br != kBrInside) {
-                    const Trial rn = compute_pq(F00, F01, F10, F11, cp.mu, cp.kappa);
-                    usable = r.svd.s1 > 0 && rn.svd.s1 > 0;
-                    t[0] = log(rn.svd.s0) - f[0];
-                    t[1] = log(rn.svd.s1) - f[1];
-                    t[2] = log(Jp) - f[2];
-                }
-            }
-            // one counter update per wavefront
-            const unsigned long long um = __ballot(usable);
-            if (um) {
-                unsigned long long base = 0;
-                if (lane == 0) base = atomicAdd(la.hcount, (unsigned long long)__popcll(um));
-                base = __shfl(base, 0, 64);
-                const unsigned long long slot = base + (unsigned long long)__popcll(um & ((1ull << lane) - 1ull));
-                if (usable && slot < (unsigned long long)la.hcap) {
-                    for (int q = 0; q < 5; ++q) la.hx[slot * 5 + q] = (float)f[q];
-                    for (int q = 0; q < 3; ++q) la.ht[slot * 3 + q] = (float)t[q];
-                }
-            }
-        } else {
-            // the branch is decided exactly; inside the surface the map is
-            // the identity; points that project are queued for the map
-            // kernel (network proposal, residual check, exact fallback) unless
-            // their state is inverted, which takes the exact map here
-            double qlim = 0;
-            Trial r{};
-            if (crushedOk) r = compute_pq_fast(F00, F01, F10, F11, cp.mu, cp.kappa);
-            const int br = crushedOk ? map_branch(k, r, Jp, qlim) : kBrInside;
-            const bool proj = crushedOk && br != kBrInside;
-            // the network proposes only in the branches it is enabled for
-            // (the autotuner switches off a branch whose proposals the yield
-            // gate does not pass); the others take the exact map here
-            const int bit = (br == kBrTension) ? kMapTension : kMapShear;
-            defer = proj && r.svd.s1 > 0 && (la.branches & bit) != 0;
-            if (proj && !defer) dp_return(k, r, F00, F01, F10, F11, Jp);
-            const unsigned long long dm = __ballot(defer);
-            if (dm) {
-                unsigned int base = 0;
-                if (lane == 0) base = atomicAdd(mq.count, (unsigned int)__popcll(dm));
-                base = __shfl(base, 0, 64);
-                const unsigned int slot = base + (unsigned int)__popcll(dm & ((1ull << lane) - 1ull));
-                if (defer) {
-                    if (slot < (unsigned int)mq.cap) {
-                        MapEntry &e = mq.q[slot];
-                        e.pt = pt;
-                        e.cs = ch.z;
-                        e.F[0] = F00; e.F[1] = F01; e.F[2] = F10; e.F[3] = F11;
-                        e.Jp = Jp;
-                        // the position at its stored precision, as the P2G here would take it
-                        if constexpr (F32) {
-                            unsigned int hi, lo;
-                            e.x[0] = fix_put_cells(px, cp, hi, lo) * cp.posQ;
-                            e.x[1] = fix_put_cells(py, cp, hi, lo) * cp.posQ;
-                        } else {
-                            e.x[0] = px;
-                            e.x[1] = py;
-                        }
-                        e.v[0] = vx; e.v[1] = vy;
-                        e.B[0] = B00; e.B[1] = B01; e.B[2] = B10; e.B[3] = B11;
-                    } else {
-                        flag_error(k);
+            // ---- return map (convergent: the learned map runs wavefront-wide) ----
+            // The trial SVD only for crushed points (few: the wavefront mostly
+            // skips it); p and q for the NACC test came from the invariants.
+            // Jp_inv matters only to the map, so only crushed points load it.
+            const bool crushedOk = ok && crushed == 1;
+            if (crushedOk) Jp = fe0 + (double)*at(R + pp * 10, u);
+            const double Jp0 = Jp;
+            if constexpr (RMAP == kMapExact) {
+                if (crushedOk && dp_projects_sq(k, iv.p, iv.q2, Jp))
+                    dp_return(k, compute_pq_fast(F00, F01, F10, F11, cp.mu, cp.kappa), F00, F01, F10, F11, Jp);
+            } else if constexpr (RMAP == kMapHarvest) {
+                Trial r{};
+                if (crushedOk) r = compute_pq_fast(F00, F01, F10, F11, cp.mu, cp.kappa);
+                double f[5] = {0, 0, 0, 0, 0}, t[3] = {0, 0, 0};
+                bool usable = false;
+                if (crushedOk) {
+                    double qlim;
+                    const int br = map_branch(k, r, Jp, qlim);
+                    map_features(r, Jp, br, f);
+                    dp_return(k, r, F00, F01, F10, F11, Jp);
+                    if (br != kBrInside) {
+                        const Trial rn = compute_pq(F00, F01, F10, F11, cp.mu, cp.kappa);
+                        usable = r.svd.s1 > 0 && rn.svd.s1 > 0;
+                        t[0] = log(rn.svd.s0) - f[0];
+                        t[1] = log(rn.svd.s1) - f[1];
+                        t[2] = log(Jp) - f[2];
                     }
                 }
+                // one counter update per wavefront
+                const unsigned long long um = __ballot(usable);
+                if (um) {
+                    unsigned long long base = 0;
+                    if (lane == 0) base = atomicAdd(la.hcount, (unsigned long long)__popcll(um));
+                    base = __shfl(base, 0, 64);
+                    const unsigned long long slot = base + (unsigned long long)__popcll(um & ((1ull << lane) - 1ull));
+                    if (usable && slot < (unsigned long long)la.hcap) {
+                        for (int q = 0; q < 5; ++q) la.hx[slot * 5 + q] = (float)f[q];
+                        for (int q = 0; q < 3; ++q) la.ht[slot * 3 + q] = (float)t[q];
+                    }
+                }
+            } else {
+                // the branch is decided exactly; inside the surface the map is
+                // the identity; points that project are queued for the map
+                // kernel (network proposal, residual check, exact fallback) unless
+                // their state is inverted, which takes the exact map here
+                double qlim = 0;
+                Trial r{};
+                if (crushedOk) r = compute_pq_fast(F00, F01, F10, F11, cp.mu, cp.kappa);
+                const int br = crushedOk ? map_branch(k, r, Jp, qlim) : kBrInside;
+                const bool proj = crushedOk && br != kBrInside;
+                // the network proposes only in the branches it is enabled for
+                // (the autotuner switches off a branch whose proposals the yield
+                // gate does not pass); the others take the exact map here
+                const int bit = (br == kBrTension) ? kMapTension : kMapShear;
+                defer = proj && r.svd.s1 > 0 && (la.branches & bit) != 0;
+                if (proj && !defer) dp_return(k, r, F00, F01, F10, F11, Jp);
+                const unsigned long long dm = __ballot(defer);
+                if (dm) {
+                    unsigned int base = 0;
+                    if (lane == 0) base = atomicAdd(mq.count, (unsigned int)__popcll(dm));
+                    base = __shfl(base, 0, 64);
+                    const unsigned int slot = base + (unsigned int)__popcll(dm & ((1ull << lane) - 1ull));
+                    if (defer) {
+                        if (slot < (unsigned int)mq.cap) {
+                            MapEntry &e = mq.q[slot];
+                            e.pt = pt;
+                            e.cs = rec.cs;
+                            e.F[0] = F00; e.F[1] = F01; e.F[2] = F10; e.F[3] = F11;
+                            e.Jp = Jp;
+                            // the position at its stored precision, as the P2G here would take it
+                            if constexpr (F32) {
+                                unsigned int hi, lo;
+                                e.x[0] = fix_put_cells(px, cp, hi, lo) * cp.posQ;
+                                e.x[1] = fix_put_cells(py, cp, hi, lo) * cp.posQ;
+                            } else {
+                                e.x[0] = px;
+                                e.x[1] = py;
+                            }
+                            e.v[0] = vx; e.v[1] = vy;
+                            e.B[0] = B00; e.B[1] = B01; e.B[2] = B10; e.B[3] = B11;
+                        } else {
+                            flag_error(k);
+                        }
+                    }
+                }
+                const unsigned long long fb = __ballot(proj && !defer), ins = __ballot(crushedOk && !proj);
+                if (lane == 0 && (fb | ins)) {
+                    if (fb) atomicAdd(&la.stats[1], (unsigned long long)__popcll(fb));
+                    if (ins) atomicAdd(&la.stats[2], (unsigned long long)__popcll(ins));
+                }
             }
-            const unsigned long long fb = __ballot(proj && !defer), ins = __ballot(crushedOk && !proj);
-            if (lane == 0 && (fb | ins)) {
-                if (fb) atomicAdd(&la.stats[1], (unsigned long long)__popcll(fb));
-                if (ins) atomicAdd(&la.stats[2], (unsigned long long)__popcll(ins));
+            if (ok) {
+                // px, py become what the rows hold: the P2G takes them at their
+                // stored precision
+                if constexpr (F32) {
+                    // a position outside the grid (or NaN) is an error here, as
+                    // the next stencil of FP64 rows would report it; the fixed
+                    // point clamps it
+                    if (!(px >= 0.0 && px < (double)gx && py >= 0.0 && py < (double)gy)) flag_error(k);
+                }
             }
-        }
-        // a point the map left alone keeps the stress of its trial state: the
-        // P2G takes it from the invariants (with FP32 storage they describe
-        // F before its rounding to the stored FP32, which differs from it by
-        // ~6e-8 of Fe - I)
-        rt = iv;
-        fresh = ok && crushed == 0;
-        if (ok) {
-            // px, py become what the rows hold: the P2G takes them at their
-            // stored precision
             if constexpr (F32) {
-                // a position outside the grid (or NaN) is an error here, as
-                // the next stencil of FP64 rows would report it; the fixed
-                // point clamps it
-                if (!(px >= 0.0 && px < (double)gx && py >= 0.0 && py < (double)gy)) flag_error(k);
                 unsigned int hx, lx, hy, ly;
                 px = fix_put_cells(px, cp, hx, lx) * cp.cellQ;
                 py = fix_put_cells(py, cp, hy, ly) * cp.cellQ;
-                const prec4 r = {hx, hy, lx | (ly << 16),
-                                 (unsigned)crushed | ((unsigned)(unsigned short)grain << 16)};
-                __builtin_nontemporal_store(r, reinterpret_cast<prec4 *>(S.pos) + pt);
-            } else {
+                const prec4 r = {hx, hy, lx | (ly << 16), (unsigned)crushed | ((unsigned)(unsigned short)grain << 16)};
+                const fe4 f = {(float)(F00 - fe0), (float)F01, (float)F10, (float)(F11 - fe0)};
+                if (ok) {
+                    __builtin_nontemporal_store(r, reinterpret_cast<prec4 *>(S.pos) + u);
+                    if (!defer) __builtin_nontemporal_store(f, fe_rec(R, pp) + u);
+                }
+                // a point the map left alone keeps the stress of its trial
+                // state: the P2G takes it from the invariants, which describe F
+                // before its rounding to the stored FP32 (~6e-8 of Fe - I).  A
+                // crushed point's Fe is taken as the next substep reads it back.
+                F00 = f.x; F01 = f.y; F10 = f.z; F11 = f.w;
+            } else if (ok) {
                 pos_store(S.pos, pp, pt, px, py);
-            }
-            const unsigned u = (unsigned)pt;
-            if (!defer) {
-                if constexpr (F32) {
-                    const fe4 f = {(float)(F00 - fe0), (float)F01, (float)F10, (float)(F11 - fe0)};
-                    __builtin_nontemporal_store(f, fe_rec(R, pp) + pt);
-                } else {   // as pos_store
+                if (!defer) {   // as pos_store
                     *at(R + pp * 2, u) = (V)F00;
                     *at(R + pp * 3, u) = (V)F01;
                     *at(R + pp * 4, u) = (V)F10;
@@ -762,7 +1036,7 @@ __global__ __launch_bounds__(256) void k_batch_particles(const int4 *__restrict_
             // recomputes them before any use; the last pass of a run stores
             // them (storeVB), for readback, checkpoints and a P2G that
             // starts afresh
-            if (!P2G || storeVB) {
+            if (storeVB && ok) {
                 R[pt] = (V)vx;
                 R[pp + pt] = (V)vy;
                 R[pp * 6 + pt] = (V)B00;
@@ -770,201 +1044,232 @@ __global__ __launch_bounds__(256) void k_batch_particles(const int4 *__restrict_
                 R[pp * 8 + pt] = (V)B10;
                 R[pp * 9 + pt] = (V)B11;
             }
-            if (Jp != Jp0 && !defer) *at(R + pp * 10, u) = (V)(Jp - fe0);
-            if (!F32 && crushed != crushed0) *at(S.crushed, u) = crushed;   // FP32: in the record
+            if (ok && Jp != Jp0 && !defer) *at(R + pp * 10, u) = (V)(Jp - fe0);
+            if (!F32 && ok && crushed != crushed0) *at(S.crushed, u) = crushed;   // FP32: in the record
+            kirchhoff_from_inv(iv, t00, t01, t11);
+            if (crushedOk) kirchhoff_rcp(fe0 + F00, F01, F10, fe0 + F11, cp.mu, cp.kappa, t00, t01, t11);
+        } else {
             if constexpr (F32) {
-                // Fe is what the next substep reads back: the P2G takes it at
-                // its stored precision.  v and Bp stay FP64: the next G2P
-                // recomputes them (what the last pass of a run stores is
-                // read only by a fresh P2G and the readback).
-                F00 = fe0 + (double)(V)(F00 - fe0); F01 = (double)(V)F01;
-                F10 = (double)(V)F10; F11 = fe0 + (double)(V)(F11 - fe0);
+                px = fix_cells(pr.x, pr.z & 0xFFFFu, cp);
+                py = fix_cells(pr.y, pr.z >> 16, cp);
+                F00 = fe0 + (double)fr.x;
+                F01 = (double)fr.y;
+                F10 = (double)fr.z;
+                F11 = fe0 + (double)fr.w;
             }
+            vx = (double)R[us];
+            vy = (double)R[pp + us];
+            B00 = (double)R[pp * 6 + us];
+            B01 = (double)R[pp * 7 + us];
+            B10 = (double)R[pp * 8 + us];
+            B11 = (double)R[pp * 9 + us];
+            kirchhoff_rcp(F00, F01, F10, F11, cp.mu, cp.kappa, t00, t01, t11);
         }
-    }
 
-    if constexpr (P2G) {
-        bool have = valid;
-        if constexpr (!G2P) {
-            if (valid) {
-                if constexpr (F32) {
-                    const prec4 r = reinterpret_cast<const prec4 *>(S.pos)[pt];
-                    px = fix_cells(r.x, r.z & 0xFFFFu, cp);
-                    py = fix_cells(r.y, r.z >> 16, cp);
-                } else {
-                    pos_load<false>(S.pos, pp, pt, cp, px, py);
-                }
-                vx = (double)R[pt];
-                vy = (double)R[pp + pt];
-                if constexpr (F32) {
-                    const fe4 f = fe_rec(R, pp)[pt];
-                    F00 = fe0 + (double)f.x;
-                    F01 = (double)f.y;
-                    F10 = (double)f.z;
-                    F11 = fe0 + (double)f.w;
-                } else {
-                    F00 = fe0 + (double)R[pp * 2 + pt];
-                    F01 = (double)R[pp * 3 + pt];
-                    F10 = (double)R[pp * 4 + pt];
-                    F11 = fe0 + (double)R[pp * 5 + pt];
-                }
-                B00 = (double)R[pp * 6 + pt];
-                B01 = (double)R[pp * 7 + pt];
-                B10 = (double)R[pp * 8 + pt];
-                B11 = (double)R[pp * 9 + pt];
-            }
-        } else {
-            have = valid && !defer && (F32 || !(px != px || py != py));
-        }
+        // ---- P2G of the points as they now are ----
         int bx = 0, by = 0;
-        double fx0 = 0, fx1 = 0, wx0, wx1, wx2, wy0, wy1, wy2;
-        bool ok;
+        double fx0 = 0, fx1 = 0, wx0 = 0, wx1 = 0, wx2 = 0, wy0 = 0, wy1 = 0, wy2 = 0;
+        bool ok = valid;
         if constexpr (F32) {   // cell units
-            ok = have;
-            if (ok) {
-                stencil_cells(px, bx, fx0, wx0, wx1, wx2);
-                stencil_cells(py, by, fx1, wy0, wy1, wy2);
-            }
+            stencil_cells(px, bx, fx0, wx0, wx1, wx2);
+            stencil_cells(py, by, fx1, wy0, wy1, wy2);
         } else {
-            ok = have && stencil(px, cp.h_inv, bx, fx0, wx0, wx1, wx2) &&
-                 stencil(py, cp.h_inv, by, fx1, wy0, wy1, wy2);
+            const bool st = px == px && py == py && stencil(px, cp.h_inv, bx, fx0, wx0, wx1, wx2) &&
+                            stencil(py, cp.h_inv, by, fx1, wy0, wy1, wy2);
+            ok = valid && st;
+            if (valid && !st) flag_error(k);
         }
-        if (valid && !ok && !defer) flag_error(k);   // deferred points scatter in the map kernel
-        // the box of base cells of the lanes whose stencils can reach the
-        // window (a lane outside the grid touches no node): the window's
-        // origin and the w x hgt nodes the stencils touch, which alone are
-        // cleared and flushed; lanes map onto the box 16, 32 or 64 columns
-        // at a time
-        const bool inb = ok && bx < gx && by < gy;
-        const bool any = __ballot(inb) != 0;
-        const unsigned lx = wave_min_u32(inb ? (unsigned)bx : 0xFFFFFFFFu);
-        const unsigned ly = wave_min_u32(inb ? (unsigned)by : 0xFFFFFFFFu);
-        const unsigned hx = wave_max_u32(inb ? (unsigned)bx : 0u);
-        const unsigned hy = wave_max_u32(inb ? (unsigned)by : 0u);
-        const int ox = any ? (int)lx : INT_MAX;
-        const int oy = any ? (int)ly : INT_MAX;
-        const int bw = any ? min((int)hx + 3 - ox, kWX) : 0;
-        const int bh = any ? min((int)hy + 3 - oy, kWY) : 0;
-        const int bsh = bw <= 16 ? 4 : (bw <= 32 ? 5 : 6);
-        const int bcol = lane & ((1 << bsh) - 1), brow0 = lane >> bsh, bstep = 64 >> bsh;
-        double *W0 = smem[wv];
-        double *W1 = W0 + kWY * kWS, *W2 = W1 + kWY * kWS;
-        if (bcol < bw) {
-            for (int ly = brow0; ly < bh; ly += bstep) {
-                const int e = ly * kWS + bcol;
-                W0[e] = 0;
-                W1[e] = 0;
-                W2[e] = 0;
-            }
+        // the cells of the points in the grid (deferred ones, whose P2G is the
+        // map kernel's, too: the next G2P gathers for them as well)
+        if (ok && bx < gx && by < gy) {
+            cellx = bx;
+            celly = by;
         }
-        wsync();
         // A quad of lanes whose four points share one base cell (in band
         // order most quads, until points cross into other cells) and whose
         // stencil lies in the window sums its contributions in registers
         // before they reach the window.  Every lane is active here.
-        const bool winFits = ok && bx + 2 < gx && by + 2 < gy && (unsigned)(bx - ox) < (unsigned)(kWX - 2) &&
-                             (unsigned)(by - oy) < (unsigned)(kWY - 2);
+        const int lx0 = bx - wx, ly0 = by - wy;
+        const bool winFits = ok && !defer && (unsigned)lx0 < ww2 && (unsigned)ly0 < wh2;
         const bool quad = quad_uniform(winFits ? (unsigned)bx | (unsigned)by << 16 : 0xFFFF0000u | (unsigned)lane);
-        if (ok) {
-            double t00, t01, t11;
-            if (fresh)
-                kirchhoff_from_inv(rt, t00, t01, t11);
-            else
-                kirchhoff_rcp(F00, F01, F10, F11, cp.mu, cp.kappa, t00, t01, t11);
-            // Every point of a case has the same mass m: the window sums the
-            // contributions per unit mass, W (v + (Bp - m^-1 dt V D^-1 tau) d),
-            // and the flush multiplies by m once per node.
-            const double m = cp.mass, h = cp.h;
-            const double A00 = B00 - cp.scm * t00, A01 = B01 - cp.scm * t01;
-            const double A10 = B10 - cp.scm * t01, A11 = B11 - cp.scm * t11;
-            const int lx0 = bx - ox, ly0 = by - oy;
-            // 0 <= lx0 <= kWX - 3 and 0 <= ly0 <= kWY - 3, one unsigned
-            // compare each (the origin is the least base cell of the lanes
-            // that get here, so lx0, ly0 >= 0 already)
-            if (quad) {
-                quad_scatter(lane, ly0 * kWS + lx0, h, fx0, fx1, wx0, wx1, wx2, wy0, wy1, wy2, vx, vy, A00, A01, A10,
-                             A11, W0, W1, W2);
-            } else if (winFits) {
-                const int e0 = ly0 * kWS + lx0;
-                // The four lanes of a quad (in band order mostly the points of
-                // one cell) walk the 3 x 3 stencil from four different nodes,
-                // so their LDS atomics never meet at one address: lane bit 0
-                // shifts the columns, bit 1 the rows, by one.  Step k of an
-                // axis visits node (k + s) mod 3 = s, 1 + s, 2 - 2 s; only the
-                // weights need selecting, the offsets follow from the index.
-                const int sx = lane & 1, sy = (lane >> 1) & 1;
-                const int xe[3] = {sx, 1 + sx, 2 - 2 * sx};
-                const int iy[3] = {sy, 1 + sy, 2 - 2 * sy};
-                const int ye[3] = {iy[0] * kWS, iy[1] * kWS, iy[2] * kWS};
-                const double xw[3] = {sx ? wx1 : wx0, sx ? wx2 : wx1, sx ? wx0 : wx2};
-                const double yw[3] = {sy ? wy1 : wy0, sy ? wy2 : wy1, sy ? wy0 : wy2};
-                double xa[3], xb[3], ya[3], yb[3];
+        // Every point of a case has the same mass m: the window sums the
+        // contributions per unit mass, W (v + (Bp - m^-1 dt V D^-1 tau) d),
+        // and the flush multiplies by m once per node.
+        const double h = cp.h;
+        const double A00 = B00 - cp.scm * t00, A01 = B01 - cp.scm * t01;
+        const double A10 = B10 - cp.scm * t01, A11 = B11 - cp.scm * t11;
+        if (quad) {
+            quad_scatter(lane, ly0 * wS + lx0, wS, h, fx0, fx1, wx0, wx1, wx2, wy0, wy1, wy2, vx, vy, A00, A01, A10,
+                         A11, W0, W1, W2);
+        } else if (winFits) {
+            const int e0 = ly0 * wS + lx0;
+            // The four lanes of a quad (in band order mostly the points of
+            // one cell) walk the 3 x 3 stencil from four different nodes,
+            // so their LDS atomics never meet at one address: lane bit 0
+            // shifts the columns, bit 1 the rows, by one.  Step k of an
+            // axis visits node (k + s) mod 3 = s, 1 + s, 2 - 2 s; only the
+            // weights need selecting, the offsets follow from the index.
+            const int sx = lane & 1, sy = (lane >> 1) & 1;
+            const int xe[3] = {sx, 1 + sx, 2 - 2 * sx};
+            const int iy[3] = {sy, 1 + sy, 2 - 2 * sy};
+            const int ye[3] = {iy[0] * wS, iy[1] * wS, iy[2] * wS};
+            const double xw[3] = {sx ? wx1 : wx0, sx ? wx2 : wx1, sx ? wx0 : wx2};
+            const double yw[3] = {sy ? wy1 : wy0, sy ? wy2 : wy1, sy ? wy0 : wy2};
+            double xa[3], xb[3], ya[3], yb[3];
 #pragma unroll
-                for (int q = 0; q < 3; ++q) {
-                    const double dx = ((double)xe[q] - fx0) * h, dy = ((double)iy[q] - fx1) * h;
-                    xa[q] = vx + A00 * dx;
-                    xb[q] = vy + A10 * dx;
-                    ya[q] = A01 * dy;
-                    yb[q] = A11 * dy;
+            for (int q = 0; q < 3; ++q) {
+                const double dx = ((double)xe[q] - fx0) * h, dy = ((double)iy[q] - fx1) * h;
+                xa[q] = vx + A00 * dx;
+                xb[q] = vy + A10 * dx;
+                ya[q] = A01 * dy;
+                yb[q] = A11 * dy;
+            }
+#pragma unroll
+            for (int a = 0; a < 3; ++a)
+#pragma unroll
+                for (int b = 0; b < 3; ++b) {
+                    const double W = xw[a] * yw[b];
+                    const int e = e0 + xe[a] + ye[b];
+                    atomicAdd(&W0[e], W);
+                    atomicAdd(&W1[e], W * (xa[a] + ya[b]));
+                    atomicAdd(&W2[e], W * (xb[a] + yb[b]));
                 }
-#pragma unroll
-                for (int a = 0; a < 3; ++a)
-#pragma unroll
-                    for (int b = 0; b < 3; ++b) {
-                        const double W = xw[a] * yw[b];
-                        const int e = e0 + xe[a] + ye[b];
-                        atomicAdd(&W0[e], W);
-                        atomicAdd(&W1[e], W * (xa[a] + ya[b]));
-                        atomicAdd(&W2[e], W * (xb[a] + yb[b]));
-                    }
-            } else {
-#pragma unroll
-                for (int i = 0; i < 3; ++i)
-#pragma unroll
-                    for (int j = 0; j < 3; ++j) {
-                        const double Wip = sel3(i, wx0, wx1, wx2) * sel3(j, wy0, wy1, wy2);
-                        const double d0 = (i - fx0) * h, d1 = (j - fx1) * h;
-                        const double incV0 = Wip * (vx + (A00 * d0 + A01 * d1));
-                        const double incV1 = Wip * (vy + (A10 * d0 + A11 * d1));
-                        const int X = bx + i, Y = by + j;
-                        if (X >= gx || Y >= gy) {
-                            flag_error(k);
-                            continue;
-                        }
-                        if ((unsigned)(X - ox) < (unsigned)kWX && (unsigned)(Y - oy) < (unsigned)kWY) {
-                            const int e = (Y - oy) * kWS + (X - ox);
-                            atomicAdd(&W0[e], Wip);
-                            atomicAdd(&W1[e], incV0);
-                            atomicAdd(&W2[e], incV1);
-                        } else {
-                            const int node = X + Y * gx;
-                            unsafeAtomicAdd(&gO[node], Wip * m);
-                            unsafeAtomicAdd(&gO[gpitch + node], incV0 * m);
-                            unsafeAtomicAdd(&gO[2 * gpitch + node], incV1 * m);
-                        }
-                    }
+        }
+        if (ok && !winFits && !defer) {
+            // outside the window, or the stencil leaves the grid: node by node
+            widen_bounds(bounds, rec.cs, bx, by, min(bx, gx), min(by, gy));
+            const double m = cp.mass;
+#pragma unroll 1
+            for (int e = 0; e < 9; ++e) {
+                const int i = e % 3, j = e / 3, X = bx + i, Y = by + j;
+                if (X >= gx || Y >= gy) {
+                    flag_error(k);
+                    continue;
+                }
+                const double W = sel3(i, wx0, wx1, wx2) * sel3(j, wy0, wy1, wy2);
+                const double d0 = (i - fx0) * h, d1 = (j - fx1) * h;
+                const unsigned node = (unsigned)(X + Y * gx);
+                unsafeAtomicAdd(at(gO, node), W * m);
+                unsafeAtomicAdd(at(gO + gpitch, node), W * (vx + (A00 * d0 + A01 * d1)) * m);
+                unsafeAtomicAdd(at(gO + 2 * gpitch, node), W * (vy + (A10 * d0 + A11 * d1)) * m);
             }
         }
         wsync();
         if constexpr (F32) __builtin_amdgcn_s_setprio(2);
-        if (bcol < bw) {
-            for (int ly = brow0; ly < bh; ly += bstep) {
-                const int lx = bcol;
-                const int e = ly * kWS + lx;
+        // the window to the grid
+        if (wcol < ww) {
+            for (int r = wrow0; r < wh; r += wstep) {
+                const int e = r * wS + wcol;
                 // the three sums in one LDS round trip; the atomics address
                 // the rows from their scalar bases with 32-bit offsets
                 const double a = W0[e], a1 = W1[e], a2 = W2[e];
-                if (a != 0) {
-                    const int X = ox + lx, Y = oy + ly;
-                    if (X < gx && Y < gy) {
-                        const unsigned node = (unsigned)(X + Y * gx);
-                        const double m = cp.mass;   // the window holds sums per unit mass
-                        unsafeAtomicAdd(at(gO, node), a * m);
-                        unsafeAtomicAdd(at(gO + gpitch, node), a1 * m);
-                        unsafeAtomicAdd(at(gO + 2 * gpitch, node), a2 * m);
-                    }
+                const int X = wx + wcol, Y = wy + r;
+                if (a != 0 && X < gx && Y < gy) {
+                    const double m = cp.mass;   // the window holds sums per unit mass
+                    const unsigned node = (unsigned)(X + Y * gx);
+                    unsafeAtomicAdd(at(gO, node), a * m);
+                    unsafeAtomicAdd(at(gO + gpitch, node), a1 * m);
+                    unsafeAtomicAdd(at(gO + 2 * gpitch, node), a2 * m);
                 }
             }
+        }
+    }
+    if (step % kBoxEvery == 0) {
+        // the box and the windows of the points as they now are
+        const unsigned x0 = wave_min_u32((unsigned)cellx), y0 = wave_min_u32((unsigned)celly);
+        const unsigned x1 = wave_max_u32((unsigned)(cellx + 1)), y1 = wave_max_u32((unsigned)(celly + 1));
+        __syncthreads();   // the windows have been read
+        unsigned *lim = reinterpret_cast<unsigned *>(smem);
+        if (lane == 0) {
+            lim[row] = x0;
+            lim[4 + row] = y0;
+            lim[8 + row] = x1;
+            lim[12 + row] = y1;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            unsigned q0 = lim[0], q1 = lim[4], q2 = lim[8], q3 = lim[12];
+            for (int q = 1; q < 4; ++q) {
+                q0 = min(q0, lim[q]);
+                q1 = min(q1, lim[4 + q]);
+                q2 = max(q2, lim[8 + q]);
+                q3 = max(q3, lim[12 + q]);
+            }
+            ChunkRec &out = recs[chunk];
+            if (q2 == 0) {   // no point in the grid
+                out.ext = 0;
+                for (int q = 0; q < 4; ++q) out.win[q] = 0;
+            } else if (set_box(out, (int)q0, (int)q1, (int)q2 - 1, (int)q3 - 1)) {
+                for (int q = 0; q < 4; ++q)
+                    out.win[q] = lim[8 + q] ? win_of(out, (int)lim[q], (int)lim[4 + q], (int)lim[8 + q] - 1,
+                                                     (int)lim[12 + q] - 1)
+                                            : 0u;
+                widen_bounds(bounds, rec.cs, (int)q0, (int)q1, (int)q2 - 1, (int)q3 - 1);
+            }
+            // a point far from the others must not take the box away from them:
+            // one that cannot hold all points stays where it was
+        }
+    }
+}
+
+// The boxes of the chunks' points as they are, a wavefront a chunk: what a
+// run's first P2G, or a table rebuilt between two runs, starts from.
+template <bool F32>
+__global__ __launch_bounds__(256) void k_chunk_boxes(ChunkRec *recs, int nChunks, const typename Rows<F32>::P *pos,
+                                                     size_t pitch, const CaseParams *__restrict__ cases, int4 *bounds) {
+    const int ch = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, lane = threadIdx.x & 63;
+    if (ch >= nChunks) return;
+    ChunkRec &rec = recs[ch];
+    const CaseParams &cp = cases[rec.cs];
+    int wx0[4], wy0[4], wx1[4], wy1[4];   // of each wavefront's points
+    int fx = 0, fy = 0, x0 = INT_MAX, y0 = INT_MAX, x1 = -1, y1 = -1;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int i = q * 64 + lane;
+        int bx = -1, by = -1;
+        if (i < rec.count) {
+            double f, a, b, c;
+            if constexpr (F32) {
+                const prec4 r = reinterpret_cast<const prec4 *>(pos)[rec.beg + i];
+                stencil_cells(fix_cells(r.x, r.z & 0xFFFFu, cp), bx, f, a, b, c);
+                stencil_cells(fix_cells(r.y, r.z >> 16, cp), by, f, a, b, c);
+            } else {
+                double x, y;
+                pos_load<false>(pos, pitch, rec.beg + i, cp, x, y);
+                if (!stencil(x, cp.h_inv, bx, f, a, b, c) || !stencil(y, cp.h_inv, by, f, a, b, c)) bx = -1;
+            }
+        }
+        const bool in = (unsigned)bx < (unsigned)cp.gx && (unsigned)by < (unsigned)cp.gy;
+        if (q == 0) {
+            fx = __builtin_amdgcn_readlane(in ? bx : 0, 0);
+            fy = __builtin_amdgcn_readlane(in ? by : 0, 0);
+        }
+        wx0[q] = (int)min(wave_min_u32(in ? (unsigned)bx : 0xFFFFFFFFu), (unsigned)INT_MAX);
+        wy0[q] = (int)min(wave_min_u32(in ? (unsigned)by : 0xFFFFFFFFu), (unsigned)INT_MAX);
+        wx1[q] = (int)wave_max_u32(in ? (unsigned)bx + 1u : 0u) - 1;
+        wy1[q] = (int)wave_max_u32(in ? (unsigned)by + 1u : 0u) - 1;
+        x0 = min(x0, wx0[q]);
+        y0 = min(y0, wy0[q]);
+        x1 = max(x1, wx1[q]);
+        y1 = max(y1, wy1[q]);
+    }
+    if (lane == 0) {
+        // too wide a box (the points of a stale order): the cells of the first
+        // point's surroundings
+        rec.ext = 0;
+        for (int q = 0; q < 4; ++q) rec.win[q] = 0;
+        if (x0 <= x1 && !set_box(rec, x0, y0, x1, y1)) {
+            x0 = max(fx - 7, x0);
+            x1 = min(fx + 7, x1);
+            y0 = max(fy - 7, y0);
+            y1 = min(fy + 7, y1);
+            if (x0 <= x1 && y0 <= y1) (void)set_box(rec, x0, y0, x1, y1);
+        }
+        if (rec.ext) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (wx1[q] >= 0) rec.win[q] = win_of(rec, wx0[q], wy0[q], wx1[q], wy1[q]);
+            widen_bounds(bounds, rec.cs, x0, y0, x1, y1);
         }
     }
 }
@@ -1118,135 +1423,9 @@ __global__ __launch_bounds__(256) void k_batch_map(Rows<F32> S, const CaseParams
     }
 }
 
-// Grid update over all cases: block b handles nodes [nodeBlock[b].y, +256)
-// of case nodeBlock[b].x.  The single-case update (gpu_implementation5.cu:
-// 215-290) with three FAST forms: 1/m from rcp_nr, the speed limit tested on
-// the squared speed, the node's row from a reciprocal of the grid width.
-// The substep's total indenter force of each case goes to hist[case*2 +
-// comp].  The velocities go to rows 1-2 of the grid, or, when vel32 is given
-// (FP32 point storage), to vel32 as FP32 pairs, zero for the nodes without
-// mass.  A node's mass and momentum are loaded together, so that a block
-// waits for memory once.
-// Per-block flags skip the stores that would write zeros over zeros: a
-// block of zeroGrid is cleared only if it took mass in its last P2G
-// (zeroHasMass, recorded when that grid was last updated), and a block of
-// vel32 is rewritten at its massless nodes only if it last held a velocity
-// (velNonzero).  The host sets every flag when a run starts without a
-// P2G left by the previous one.
-__global__ __launch_bounds__(256) void k_batch_update(const CaseParams *__restrict__ cases,
-                                                     const int2 *__restrict__ nodeBlock,
-                                                     double *__restrict__ grid, double *__restrict__ zeroGrid,
-                                                     size_t gpitch, const double *__restrict__ tTab, int step,
-                                                     double *__restrict__ hist, float2 *__restrict__ vel32,
-                                                     int *__restrict__ gridHasMass,
-                                                     const int *__restrict__ zeroHasMass,
-                                                     int *__restrict__ velNonzero, double *__restrict__ bins) {
-    __shared__ double sf[2];
-    __shared__ int any;
-    const int2 nb = nodeBlock[blockIdx.x];
-    const CaseParams &cp = cases[nb.x];
-    const int local = nb.y + (int)threadIdx.x;
-    const bool node = local < cp.gridTotal;
-    const size_t idx = (size_t)cp.gridOffset + (node ? local : 0);
-    double mass = 0, p0 = 0, p1 = 0;
-    if (node) {
-        mass = grid[idx];
-        p0 = grid[gpitch + idx];
-        p1 = grid[2 * gpitch + idx];
-    }
-    if (threadIdx.x == 0) {
-        sf[0] = 0;
-        sf[1] = 0;
-        any = 0;
-    }
-    // a block of zeroGrid that took no mass in its last P2G is still zero,
-    // and a block of vel32 last written with no mass holds zeros
-    const bool zeroIt = zeroGrid && zeroHasMass[blockIdx.x] != 0;
-    const bool velDirty = vel32 && velNonzero[blockIdx.x] != 0;
-    const bool blockMass = __syncthreads_or(mass != 0) != 0;   // also orders sf/any
-    if (threadIdx.x == 0) {
-        gridHasMass[blockIdx.x] = blockMass ? 1 : 0;
-        if (vel32) velNonzero[blockIdx.x] = blockMass ? 1 : 0;
-    }
-    if (node) {
-        if (zeroIt) {
-            zeroGrid[idx] = 0;
-            zeroGrid[gpitch + idx] = 0;
-            zeroGrid[2 * gpitch + idx] = 0;
-        }
-        if (velDirty && mass == 0) vel32[idx] = make_float2(0.f, 0.f);
-        if (mass != 0) {
-            const double dt = cp.dt, h = cp.h, V = cp.indV;
-            const double t = tTab[step];
-            const double ind_x = cp.x0 + t * V, ind_y = cp.y0;
-            const double rm = rcp_nr(mass);
-            double v0 = p0 * rm, v1 = p1 * rm;
-            v1 = v1 - dt * cp.gravity;
-            const double vmax = 0.5 * h / dt;
-            const double vsq = v0 * v0 + v1 * v1;
-            if (vsq > vmax * vmax) {
-                const double s = vmax / sqrt(vsq);
-                v0 = v0 * s;
-                v1 = v1 * s;
-            }
-            // row and column: (local + 0.5) / gx lies >= 0.5 / gx >= 2^-17
-            // from an integer and is computed to within 2^-23, so its floor
-            // is the row
-            const int iy = (int)(((double)local + 0.5) * cp.gxInv);
-            const int ix = local - iy * cp.gx;
-            double n0 = ix * h - ind_x, n1 = iy * h - ind_y;
-            if (n0 * n0 + n1 * n1 < cp.indRsq) {
-                const double r0 = v0 - V, r1 = v1;
-                const double z = n0 * n0 + n1 * n1;
-                if (z > 0) {
-                    const double nz = sqrt(z);
-                    n0 = n0 / nz;
-                    n1 = n1 / nz;
-                }
-                const double vnr = r0 * n0 + r1 * n1;
-                if (vnr < 0) {
-                    const double q0 = v0, q1 = v1;
-                    v0 = V + (r0 - n0 * vnr);
-                    v1 = r1 - n1 * vnr;
-                    const double f0 = (q0 - v0) * mass / dt, f1 = (q1 - v1) * mass / dt;
-                    atomicAdd(&sf[0], f0);
-                    atomicAdd(&sf[1], f1);
-                    any = 1;
-                    // the force's angular bin (gpu_implementation5.cu:262-269:
-                    // atan2 of (x, y) of the unit normal, then + pi, scaled)
-                    double angle = atan2(n0, n1);
-                    angle += kPi;
-                    angle *= cp.nbins / (2 * kPi);
-                    int kb = (int)angle;
-                    kb = max(kb, 0);
-                    kb = min(kb, cp.nbins - 1);
-                    unsafeAtomicAdd(&bins[cp.binOffset + 2 * kb], f0);
-                    unsafeAtomicAdd(&bins[cp.binOffset + 2 * kb + 1], f1);
-                }
-            }
-            if (iy <= 2) {
-                v0 = 0;
-                v1 = 0;
-            } else if (iy >= cp.gy - 3 && v1 > 0) {
-                v1 = 0;
-            }
-            if (ix <= 2 && v0 < 0)
-                v0 = 0;
-            else if (ix >= cp.gx - 3 && v0 > 0)
-                v0 = 0;
-            if (vel32) {
-                vel32[idx] = make_float2((float)v0, (float)v1);
-            } else {
-                grid[gpitch + idx] = v0;
-                grid[2 * gpitch + idx] = v1;
-            }
-        }
-    }
-    __syncthreads();
-    if (threadIdx.x == 0 && any) {
-        unsafeAtomicAdd(&hist[2 * nb.x], sf[0]);
-        unsafeAtomicAdd(&hist[2 * nb.x + 1], sf[1]);
-    }
+__global__ void k_reset_bounds(int4 *bounds, int nCases) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c < nCases) bounds[c] = make_int4(INT_MAX, INT_MAX, -1, -1);
 }
 
 // Cell key of every point of the batch, offset by its case's first node so
@@ -1335,10 +1514,10 @@ struct icempm_batch {
     hipStream_t stream = nullptr;
     // The cases in kChains groups of about equal point counts run their
     // substep loops as independent chains (group g > 0 on side[g - 1]), so
-    // that one group's grid update, bound by memory, overlaps another's
-    // particle pass, bound by issue.  groupCase: each group's first case;
-    // grpChunk / grpBlock: the groups' ranges of the chunk table and of the
-    // node blocks; chains: the number of groups (1 when there is one case).
+    // that one group's launches fill the gaps and the tail of the other's.
+    // groupCase: each group's first case; grpChunk / grpBlock: the groups'
+    // ranges of the chunk records and of the node blocks; chains: the
+    // number of groups (1 when there is one case).
     static constexpr int kChains = ICEMPM_BATCH_CHAINS;
     hipStream_t side[kChains - 1] = {};
     hipEvent_t evFork = nullptr;
@@ -1347,9 +1526,6 @@ struct icempm_batch {
     int groupCase[kChains + 1] = {};
     int grpChunk[kChains + 1] = {};
     int grpBlock[kChains + 1] = {};
-    // the launch target of the next particle pass: its stream and chunk range
-    hipStream_t lstream = nullptr;
-    int lchunk0 = 0, lchunks = 0;
     std::string lastError;
     bool finalized = false;
 
@@ -1372,15 +1548,14 @@ struct icempm_batch {
     int binsTotal = 0;            // doubles
     size_t pitch = 0;
     int nPts = 0;
-    double *gridA = nullptr, *gridB = nullptr;
-    float2 *vel32 = nullptr;   // FP32 storage: the grid velocities the gathers read
-    int *blkFlags = nullptr;   // per node block: grid A took mass, grid B took mass, vel32 nonzero
+    double *grids = nullptr;   // three grids of 3 rows each, used in turn: read, scattered into, cleared
+    int4 *bounds = nullptr;    // per case: the nodes touched since the run's fresh start
     size_t gpitch = 0;
     long nNodes = 0;
     CaseParams *cases = nullptr;
-    int4 *chunks = nullptr;   // {first point, end, case, 0} per chunk
+    ChunkRec *recs = nullptr;   // nChunks records
     int nChunks = 0;
-    size_t chunkCapDev = 0;
+    size_t recCap = 0;
     int2 *nodeBlock = nullptr;
     int nNodeBlocks = 0;
     int *err = nullptr;
@@ -1410,7 +1585,7 @@ struct icempm_batch {
 
     // executable graphs of the substep loop, two per start (of different
     // step counts, the least recently used replaced): fresh (row 0), or the
-    // first substep's P2G already in grid A (row 1) or grid B (row 2); each
+    // first substep's P2G already in grid 0, 1 or 2 (rows 1-3); each
     // with the step count, time table and history rows it was captured
     // with, and the grid that holds the next P2G after it
     struct GraphSlot {
@@ -1421,9 +1596,9 @@ struct icempm_batch {
         int end = -1;
         unsigned long long used = 0;
     };
-    GraphSlot graphs[3][2];
+    GraphSlot graphs[4][2];
     unsigned long long graphTick = 0;
-    // the grid (0: A, 1: B) that holds the P2G of the next substep, made
+    // the grid (0, 1 or 2) that holds the P2G of the next substep, made
     // from the current points by the last pass of the previous run; -1 when
     // there is none, or the points have changed since (restore, re-sort)
     int pending = -1;
@@ -1489,59 +1664,61 @@ void dfree(T *&p) {
 }
 
 constexpr int kMapBlocks = 256;
+// batches of fewer chunks run as one chain
+constexpr int kChainChunks = 2048;
 
-template <bool F32, bool G2P, bool P2G, int RMAP>
-void launch_one(icempm_batch *b, unsigned nb, const void *gV, double *gO, const LearnArgs &la,
-                const MapQueue &mq) {
+// One launch of the substep kernel: a range of the chunks (and of the
+// node blocks) with the grids it reads, scatters into and clears.
+struct Pass {
+    hipStream_t stream;
+    int in, out;              // grids
+    int chunk0, chunks;
+    int block0, blocks;       // node blocks
+    const double *tTab;
+    double *hist;             // of this substep
+    int step;
+    bool storeVB;
+};
+
+template <bool F32, bool G2P, int RMAP>
+void launch_one(icempm_batch *b, const Pass &p, const LearnArgs &la, const MapQueue &mq) {
     Rows<F32> S{static_cast<typename Rows<F32>::P *>(b->pos), reinterpret_cast<typename Rows<F32>::V *>(b->rest),
                 b->crushed, b->grain, b->pitch};
-    hipLaunchKernelGGL((k_batch_particles<F32, G2P, P2G, RMAP>), dim3(nb), dim3(256), 0, b->lstream,
-                       b->chunks + b->lchunk0, b->lchunks, b->cases, S.pos, S.rest, S.crushed, S.pitch,
-                       static_cast<const typename Rows<F32>::G *>(gV), gO, b->gpitch,
-                       b->err, b->grain, la, mq, b->storeVB ? 1 : 0);
-    if (b->evAfter) (void)hipEventRecord(b->evAfter, b->lstream);
+    const size_t grid = 3 * b->gpitch;
+    const int clear = 3 - p.in - p.out;   // the third grid (unused by a first P2G, where in = out)
+    NodeWork nw{b->nodeBlock + p.block0, b->grids + (G2P ? clear * grid : 0), p.hist, b->bins};
+    const int groups = ((p.chunks + 7) / 8) * 8;
+    hipLaunchKernelGGL((k_batch_substep<F32, G2P, RMAP>), dim3((unsigned)(groups + (G2P ? p.blocks : 0))), dim3(256), 0,
+                       p.stream, b->recs + p.chunk0, b->grids + p.in * grid, p.chunks, groups, S.pos, S.rest, b->gpitch,
+                       b->cases, S.crushed, S.pitch, b->grids + p.out * grid, b->bounds, b->err, b->grain, p.tTab, p.step, nw, la, mq,
+                       p.storeVB ? 1 : 0);
+    if (b->evAfter) (void)hipEventRecord(b->evAfter, p.stream);
     if (G2P && RMAP == kMapLearned && la.branches != 0) {
         // the deferred points: map, store, and their P2G into the pass's output grid
-        hipLaunchKernelGGL((k_batch_map<F32>), dim3(kMapBlocks), dim3(256), 0, b->lstream, S, b->cases, mq.q,
-                           mq.count, mq.count == b->mapCount ? b->mapCount + 1 : b->mapCount, gO, b->gpitch,
+        hipLaunchKernelGGL((k_batch_map<F32>), dim3(kMapBlocks), dim3(256), 0, p.stream, S, b->cases, mq.q, mq.count,
+                           mq.count == b->mapCount ? b->mapCount + 1 : b->mapCount, b->grids + p.out * grid, b->gpitch,
                            b->err, la);
     }
 }
 
-template <bool F32, int RMAP>
-void launch_map(icempm_batch *b, unsigned nb, bool g2p, bool p2g, const void *gV, double *gO,
-                const LearnArgs &la, const MapQueue &mq) {
-    if (g2p && p2g)
-        launch_one<F32, true, true, RMAP>(b, nb, gV, gO, la, mq);
-    else if (g2p)
-        launch_one<F32, true, false, RMAP>(b, nb, gV, gO, la, mq);
-    else
-        launch_one<F32, false, true, kMapExact>(b, nb, gV, gO, la, mq);
-}
-
 template <bool F32>
-void launch_prec(icempm_batch *b, unsigned nb, bool g2p, bool p2g, const void *gV, double *gO,
-                 const LearnArgs &la, const MapQueue &mq) {
+void launch_prec(icempm_batch *b, bool g2p, const Pass &p, const LearnArgs &la, const MapQueue &mq) {
     // the learned map with every branch switched off is the exact map: its
     // pass, without the queue logic and the learned map's counters
-    if (b->rmap == kMapHarvest)
-        launch_map<F32, kMapHarvest>(b, nb, g2p, p2g, gV, gO, la, mq);
+    if (!g2p)
+        launch_one<F32, false, kMapExact>(b, p, la, mq);
+    else if (b->rmap == kMapHarvest)
+        launch_one<F32, true, kMapHarvest>(b, p, la, mq);
     else if (b->rmap == kMapLearned && b->mapBranches != 0)
-        launch_map<F32, kMapLearned>(b, nb, g2p, p2g, gV, gO, la, mq);
+        launch_one<F32, true, kMapLearned>(b, p, la, mq);
     else
-        launch_map<F32, kMapExact>(b, nb, g2p, p2g, gV, gO, la, mq);
+        launch_one<F32, true, kMapExact>(b, p, la, mq);
 }
 
-// One particle pass (and, with the learned map, the map kernel after it);
-// parity selects the queue counter the pass appends to.
-// gV: the grid whose rows 1-2 hold the velocities (FP64 storage) or vel32
-hipError_t launch_pass(icempm_batch *b, bool g2p, bool p2g, const void *gV, double *gO, int parity,
-                       hipStream_t st, int chunk0, int chunks) {
-    const unsigned nb = (unsigned)(((chunks + 7) / 8) * 8);
-    if (chunks <= 0) return hipSuccess;
-    b->lstream = st;
-    b->lchunk0 = chunk0;
-    b->lchunks = chunks;
+// One substep of a range of chunks, or (g2p false) the first P2G (and,
+// with the learned map, the map kernel after it).
+hipError_t launch_pass(icempm_batch *b, bool g2p, const Pass &p) {
+    if (p.chunks <= 0) return hipSuccess;
     LearnArgs la{};
     la.wbf = b->mlpW;
     la.pf = b->mlpP;
@@ -1553,18 +1730,20 @@ hipError_t launch_pass(icempm_batch *b, bool g2p, bool p2g, const void *gV, doub
     la.hcap = b->hcap;
     la.stats = b->stats;
     la.branches = b->mapBranches;
-    MapQueue mq{b->mapQ, b->mapCount ? b->mapCount + (parity & 1) : nullptr, b->nPts};
+    // the steps use the two queue counters in turn
+    MapQueue mq{b->mapQ, b->mapCount ? b->mapCount + (p.step & 1) : nullptr, b->nPts};
     if (b->precision == ICEMPM_BATCH_F32)
-        launch_prec<true>(b, nb, g2p, p2g, gV, gO, la, mq);
+        launch_prec<true>(b, g2p, p, la, mq);
     else
-        launch_prec<false>(b, nb, g2p, p2g, gV, gO, la, mq);
+        launch_prec<false>(b, g2p, p, la, mq);
     return hipGetLastError();
 }
 
 // Chunk table from the case-local base cells of the points in slot order
 // (column | row << 16): chunks of <= chunkPoints consecutive points of one
-// case whose base cells span at most two cell rows and 126 columns, so that
-// a wavefront's window (4 node rows) holds all its stencils, cut greedily.
+// case whose base cells span at most two cell rows and kChunkCols columns, so
+// that the workgroup's LDS holds all its stencils, cut greedily.  A chunk that
+// is cut for its columns alone ends at a wavefront's last point if it can.
 // Points in band order give chunks of one band each, until they move.  The
 // cases are independent, so they are cut on several host threads.
 void chunk_table(const icempm_batch *b, const unsigned *cells, std::vector<int> &cstart,
@@ -1578,22 +1757,22 @@ void chunk_table(const icempm_batch *b, const unsigned *cells, std::vector<int> 
         std::vector<int> &st = starts[ci];
         if (n <= 0) return;
         st.reserve((size_t)n / (size_t)cap + 16);
-        st.push_back(o);
-        int cs = 0;
-        int c0 = (int)(cells[o] & 0xFFFFu), r0 = (int)(cells[o] >> 16);
-        int c1 = c0, r1 = r0;
-        for (int i = 1; i < n; ++i) {
-            const unsigned ki = cells[(size_t)o + i];
-            const int cc = (int)(ki & 0xFFFFu), r = (int)(ki >> 16);
-            const int nr0 = std::min(r0, r), nr1 = std::max(r1, r), nc0 = std::min(c0, cc), nc1 = std::max(c1, cc);
-            if ((i - cs >= cap) || nr1 - nr0 > 1 || nc1 - nc0 > 125) {
-                st.push_back(o + i);
-                cs = i;
-                r0 = r1 = r;
-                c0 = c1 = cc;
-            } else {
-                r0 = nr0; r1 = nr1; c0 = nc0; c1 = nc1;
+        for (int cs = 0; cs < n;) {
+            int c0 = INT_MAX, r0 = INT_MAX, c1 = -1, r1 = -1, i = cs;
+            bool wide = false;
+            for (; i < n && i - cs < cap; ++i) {
+                const unsigned ki = cells[(size_t)o + i];
+                const int cc = (int)(ki & 0xFFFFu), r = (int)(ki >> 16);
+                r0 = std::min(r0, r);
+                r1 = std::max(r1, r);
+                c0 = std::min(c0, cc);
+                c1 = std::max(c1, cc);
+                wide = c1 - c0 > kChunkCols - 1;
+                if (r1 - r0 > 1 || wide) break;
             }
+            if (wide && r1 - r0 <= 1 && i - cs > 64) i = cs + (i - cs) / 64 * 64;
+            st.push_back(o + cs);
+            cs = i;
         }
     };
     const unsigned hw = std::thread::hardware_concurrency();
@@ -1646,20 +1825,39 @@ void drop_graph(icempm_batch *b) {
         }
 }
 
-// the host chunk table to the device (grows the device array when needed)
+
+// The boxes of the chunks from the points as they are.
+hipError_t launch_boxes(icempm_batch *b) {
+    const dim3 nb((unsigned)((b->nChunks + 3) / 4));
+    if (b->precision == ICEMPM_BATCH_F32)
+        hipLaunchKernelGGL(k_chunk_boxes<true>, nb, dim3(256), 0, b->stream, b->recs, b->nChunks,
+                           static_cast<const unsigned int *>(b->pos), b->pitch, b->cases, b->bounds);
+    else
+        hipLaunchKernelGGL(k_chunk_boxes<false>, nb, dim3(256), 0, b->stream, b->recs, b->nChunks,
+                           static_cast<const double *>(b->pos), b->pitch, b->cases, b->bounds);
+    return hipGetLastError();
+}
+
+// The host chunk table as records on the device (grown when needed).  Boxes
+// are made when a run starts afresh; a table rebuilt between two runs gets
+// them here.
 int upload_chunks(icempm_batch *b) {
     const size_t n = b->hccase.size();
-    std::vector<int4> t(std::max<size_t>(n, 1));
-    for (size_t c = 0; c < n; ++c) t[c] = make_int4(b->hcstart[c], b->hcstart[c + 1], b->hccase[c], 0);
-    const int4 *before = b->chunks;
-    const int nBefore = b->nChunks;
-    if (t.size() > b->chunkCapDev) {
-        dfree(b->chunks);
-        b->chunkCapDev = 0;
-        BCHK(b, hipMalloc(&b->chunks, t.size() * sizeof(int4)), "chunk table");
-        b->chunkCapDev = t.size();
+    std::vector<ChunkRec> t(n);
+    for (size_t c = 0; c < n; ++c) {
+        const CaseParams &cp = b->hc[(size_t)b->hccase[c]].cp;
+        t[c] = ChunkRec{b->hcstart[c], b->hcstart[c + 1] - b->hcstart[c], b->hccase[c], cp.gridOffset,
+                        (unsigned)cp.gx | (unsigned)cp.gy << 16, 0, 0, 0};
     }
-    BCHK(b, hipMemcpy(b->chunks, t.data(), t.size() * sizeof(int4), hipMemcpyHostToDevice), "chunk table");
+    const ChunkRec *before = b->recs;
+    const int nBefore = b->nChunks;
+    if (n > b->recCap) {
+        dfree(b->recs);
+        b->recCap = 0;
+        BCHK(b, hipMalloc(&b->recs, n * sizeof(ChunkRec)), "chunk table");
+        b->recCap = n;
+    }
+    BCHK(b, hipMemcpy(b->recs, t.data(), n * sizeof(ChunkRec), hipMemcpyHostToDevice), "chunk table");
     b->nChunks = (int)n;
     // each group's first chunk
     bool splitMoved = false;
@@ -1673,7 +1871,8 @@ int upload_chunks(icempm_batch *b) {
     // a captured loop holds the table's address, the chunk count and the
     // groups' ranges (the grid sizes of its launches); the table's contents
     // are read at run time
-    if (b->chunks != before || b->nChunks != nBefore || splitMoved) drop_graph(b);
+    if (b->recs != before || b->nChunks != nBefore || splitMoved) drop_graph(b);
+    if (b->pending >= 0) BCHK(b, launch_boxes(b), "chunk table");
     return ICEMPM_OK;
 }
 
@@ -1790,62 +1989,54 @@ int rebuild_chunks(icempm_batch *b) {
     return upload_chunks(b);
 }
 
-// The substep loop of n substeps starting from grid A, as stream work.
-// The substep loop: n times the grid update and the fused pass (G2P of
-// this substep, P2G of the next into the other grid).  A fresh start (start
-// < 0) clears grid A and scatters the points into it first; start = 0 or 1
-// takes the P2G the previous run's last pass left in grid A or B, with the
-// block flags that run left.  *end receives the grid that then holds the
-// next substep's P2G.
+// The substep loop: n launches of the substep kernel (per group of cases).  A
+// fresh start (start < 0) clears the grids and scatters the points into grid 0
+// first; start = 0, 1 or 2 takes the P2G that the previous run's last pass
+// left in that grid.  Substep i reads grid start + i, scatters into the next
+// and clears the one after (mod 3).  *end receives the grid that then holds
+// the next substep's P2G.
 hipError_t enqueue_loop(icempm_batch *b, int n, const double *tTab, double *hist, int start, int *end) {
     hipError_t e;
-    const size_t nblk = (size_t)b->nNodeBlocks;
-    double *A0 = b->gridA, *B0 = b->gridB;
-    int *fA0 = b->blkFlags, *fB0 = b->blkFlags + nblk, *fV = b->blkFlags + 2 * nblk;
-    if (start < 0 && (e = launch_fill_f64(b->gridA, b->gpitch * 3, 0.0, b->stream)) != hipSuccess) return e;
-    if ((e = launch_fill_f64(hist, 2 * (size_t)n * b->hc.size(), 0.0, b->stream)) != hipSuccess) return e;
+    const size_t nc = b->hc.size();
+    if ((e = launch_fill_f64(hist, 2 * (size_t)n * nc, 0.0, b->stream)) != hipSuccess) return e;
     if (b->mapCount &&
         (e = launch_fill_i32(reinterpret_cast<int *>(b->mapCount), 2, 0, b->stream)) != hipSuccess)
         return e;
-    int cur = 0;   // which grid A is
+    Pass p{};
+    p.stream = b->stream;
     if (start < 0) {
-        if ((e = launch_pass(b, false, true, b->gridA, b->gridA, 0, b->stream, 0, b->nChunks)) != hipSuccess)
-            return e;
-        // the grids' and vel32's contents are unknown at a fresh start
-        if ((e = launch_fill_i32(b->blkFlags, 3 * nblk, 1, b->stream)) != hipSuccess) return e;
-    } else if (start == 1) {
-        std::swap(A0, B0);
-        std::swap(fA0, fB0);
-        cur = 1;
+        // what the grids hold, and where, is unknown at a fresh start
+        start = 0;
+        if ((e = launch_fill_f64(b->grids, 9 * b->gpitch, 0.0, b->stream)) != hipSuccess) return e;
+        hipLaunchKernelGGL(k_reset_bounds, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, b->stream, b->bounds, (int)nc);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        if ((e = launch_boxes(b)) != hipSuccess) return e;
+        p.chunks = b->nChunks;
+        if ((e = launch_pass(b, false, p)) != hipSuccess) return e;
     }
     // The groups of cases as independent chains, when there are several,
     // the map kernel (one queue for all cases) is not in the loop and no
     // pass is being timed: the side chains start after everything above,
     // and the main stream waits for them at the end.
     const bool mapKernel = b->rmap == kMapLearned && b->mapBranches != 0;
-    const int groups = (!mapKernel && b->timingStride <= 0) ? b->chains : 1;
+    const int groups = (!mapKernel && b->timingStride <= 0 && b->nChunks >= kChainChunks) ? b->chains : 1;
     if (groups > 1) {
         if ((e = hipEventRecord(b->evFork, b->stream)) != hipSuccess) return e;
         for (int g = 1; g < groups; ++g)
             if ((e = hipStreamWaitEvent(b->side[g - 1], b->evFork, 0)) != hipSuccess) return e;
     }
-    const size_t nc = b->hc.size();
+    p.tTab = tTab;
     for (int g = 0; g < groups; ++g) {
-        hipStream_t st = g == 0 ? b->stream : b->side[g - 1];
-        const int c0 = groups > 1 ? b->grpChunk[g] : 0;
-        const int nch = groups > 1 ? b->grpChunk[g + 1] - c0 : b->nChunks;
-        const int k0 = groups > 1 ? b->grpBlock[g] : 0;
-        const int nkb = groups > 1 ? b->grpBlock[g + 1] - k0 : b->nNodeBlocks;
-        double *A = A0, *B = B0;
-        int *fA = fA0, *fB = fB0;
+        hipStream_t st = p.stream = g == 0 ? b->stream : b->side[g - 1];
+        p.chunk0 = groups > 1 ? b->grpChunk[g] : 0;
+        p.chunks = (groups > 1 ? b->grpChunk[g + 1] : b->nChunks) - p.chunk0;
+        p.block0 = groups > 1 ? b->grpBlock[g] : 0;
+        p.blocks = (groups > 1 ? b->grpBlock[g + 1] : b->nNodeBlocks) - p.block0;
         for (int i = 0; i < n; ++i) {
-            if (nkb > 0) {
-                hipLaunchKernelGGL(k_batch_update, dim3(nkb), dim3(256), 0, st, b->cases, b->nodeBlock + k0, A, B,
-                                   b->gpitch, tTab, i, hist + 2 * nc * (size_t)i, b->vel32, fA + k0, fB + k0,
-                                   fV + k0, b->bins);
-                if ((e = hipGetLastError()) != hipSuccess) return e;
-            }
-            const void *gV = b->vel32 ? static_cast<const void *>(b->vel32) : static_cast<const void *>(A);
+            p.in = (start + i) % 3;
+            p.out = (start + i + 1) % 3;
+            p.hist = hist + 2 * nc * (size_t)i;
+            p.step = i;
             const bool timeIt = b->timingStride > 0 && i % b->timingStride == 0;
             hipEvent_t t0 = nullptr, t1 = nullptr;
             if (timeIt) {
@@ -1862,20 +2053,17 @@ hipError_t enqueue_loop(icempm_batch *b, int n, const double *tTab, double *hist
                 if ((e = hipEventRecord(t0, st)) != hipSuccess) return e;
             }
             b->evAfter = timeIt ? t1 : nullptr;   // recorded right after the particle kernel
-            b->storeVB = (i == n - 1);
-            e = launch_pass(b, true, true, gV, B, i, st, c0, nch);
+            p.storeVB = (i == n - 1);
+            e = launch_pass(b, true, p);
             b->evAfter = nullptr;
-            b->storeVB = false;
             if (e != hipSuccess) return e;
-            std::swap(A, B);
-            std::swap(fA, fB);
         }
     }
     for (int g = 1; g < groups; ++g) {
         if ((e = hipEventRecord(b->evJoin[g - 1], b->side[g - 1])) != hipSuccess) return e;
         if ((e = hipStreamWaitEvent(b->stream, b->evJoin[g - 1], 0)) != hipSuccess) return e;
     }
-    *end = cur ^ (n & 1);
+    *end = (start + n) % 3;
     return hipSuccess;
 }
 
@@ -1913,9 +2101,8 @@ void icempm_batch_destroy(icempm_batch *b) {
     for (hipStream_t st : b->side)
         if (st) (void)hipStreamSynchronize(st);
     drop_graph(b);
-    dfree(b->pos); dfree(b->rest); dfree(b->crushed); dfree(b->gridA); dfree(b->gridB); dfree(b->vel32);
-    dfree(b->blkFlags);
-    dfree(b->cases); dfree(b->chunks); dfree(b->nodeBlock);
+    dfree(b->pos); dfree(b->rest); dfree(b->crushed); dfree(b->grids); dfree(b->bounds);
+    dfree(b->cases); dfree(b->recs); dfree(b->nodeBlock);
     dfree(b->err); dfree(b->tTab); dfree(b->hist);
     dfree(b->mlpW); dfree(b->mlpP); dfree(b->hx); dfree(b->ht); dfree(b->hcount); dfree(b->stats);
     dfree(b->mapQ); dfree(b->mapCount);
@@ -1990,6 +2177,8 @@ int icempm_batch_add_case(icempm_batch *b, const void *simparams, size_t nbytes,
         c.nbins = P.n_indenter_subdivisions;
         c.binOffset = 0;   // set by finalize
         c.scm = c.dt * c.vol * c.Dinv / c.mass;
+        c.vmax = 0.5 * c.h / c.dt;
+        c.dtCells = c.dt * c.h_inv;
         {
             // FP32 storage: 48 - ib fraction bits, ib the bits a cell index needs
             // (finalize refuses grids beyond 65536 nodes a side: ib <= 16)
@@ -2055,7 +2244,7 @@ int icempm_batch_finalize(icempm_batch *b) {
             for (int i = 0; i < h.cp.nPts; ++i) ord[(size_t)i] = i;
             std::stable_sort(ord.begin(), ord.end(), [&h](int a, int c) { return h.keys[(size_t)a] < h.keys[(size_t)c]; });
             for (int k = 0; k < h.cp.nPts; ++k) keys.push_back(h.keys[(size_t)ord[(size_t)k]]);
-            for (int nd = 0; nd < h.cp.gridTotal; nd += 256) nblk.push_back(make_int2((int)ci, nd));
+            for (int nd = 0; nd < h.cp.gridTotal; nd += kNodeBlk) nblk.push_back(make_int2((int)ci, nd));
             pofs += h.cp.nPts;
             gofs += h.cp.gridTotal;
         }
@@ -2125,13 +2314,10 @@ int icempm_batch_finalize(icempm_batch *b) {
         if (anyGrains) BCHK(b, hipMalloc(&b->grain, b->pitch * sizeof(short)), "batch finalize");
         BCHK(b, hipMalloc(&b->bins, (size_t)b->binsTotal * sizeof(double)), "batch finalize");
         BCHK(b, hipMalloc(&b->orig, b->pitch * sizeof(int)), "batch finalize");
-        BCHK(b, hipMalloc(&b->gridA, 3 * b->gpitch * sizeof(double)), "batch finalize");
-        BCHK(b, hipMalloc(&b->gridB, 3 * b->gpitch * sizeof(double)), "batch finalize");
-        if (b->precision == ICEMPM_BATCH_F32)
-            BCHK(b, hipMalloc(&b->vel32, b->gpitch * sizeof(float2)), "batch finalize");
+        BCHK(b, hipMalloc(&b->grids, 9 * b->gpitch * sizeof(double)), "batch finalize");
+        BCHK(b, hipMalloc(&b->bounds, b->hc.size() * sizeof(int4)), "batch finalize");
         BCHK(b, hipMalloc(&b->cases, b->hc.size() * sizeof(CaseParams)), "batch finalize");
         BCHK(b, hipMalloc(&b->nodeBlock, nblk.size() * sizeof(int2)), "batch finalize");
-        BCHK(b, hipMalloc(&b->blkFlags, 3 * nblk.size() * sizeof(int)), "batch finalize");
         BCHK(b, hipMalloc(&b->err, sizeof(int)), "batch finalize");
         BCHK(b, hipMalloc(&b->hcount, sizeof(unsigned long long)), "batch finalize");
         BCHK(b, hipMalloc(&b->stats, kMapStats * sizeof(unsigned long long)), "batch finalize");
@@ -2216,8 +2402,8 @@ namespace {
 // P2G the previous run left (b->pending) or from a fresh P2G, as one graph
 // launch (captured when the start, the step count or the pointers change)
 // or as stream launches; returns the device time in ms.
-// The executable graph of n substeps from the given start (-1 fresh, 0 or 1:
-// the P2G in grid A or B) with these time-table and history rows, captured,
+// The executable graph of n substeps from the given start (-1 fresh, 0, 1 or
+// 2: the P2G in that grid) with these time-table and history rows, captured,
 // instantiated and put on the device unless its slot already holds it.
 int ensure_graph(icempm_batch *b, int n, const double *tTab, double *hist, int start,
                  const icempm_batch::GraphSlot **out) {
@@ -2359,9 +2545,9 @@ int icempm_batch_prepare(icempm_batch *b, int n) {
         BCHK(b, hipStreamSynchronize(b->stream), "prepare");
         int rc = ensure_capacity(b, n);
         if (rc) return rc;
-        // the first segment of such a run, from each of the three starts
+        // the first segment of such a run, from each of the four starts
         const int len = b->resortEvery > 0 ? std::min(b->resortEvery, n) : n;
-        for (int start = -1; start <= 1; ++start)
+        for (int start = -1; start <= 2; ++start)
             if ((rc = ensure_graph(b, len, b->tTab, b->hist, start, nullptr))) return rc;
         return ICEMPM_OK;
     });

@@ -385,29 +385,25 @@ static __device__ __forceinline__ bool fails(const KParams &k, short grain, doub
     return y > 0;
 }
 
-// fails() from q^2: the tension line's q_limit is >= 0 for qmax >= 0, and
-// q > q_limit iff q^2 > q_limit^2 there; a negative q_limit (qmax < 0, a
-// GrainVariability above 1) is exceeded by every q >= 0
+// fails() from q^2 and without its divisions and square root.  With t = -pmin
+// = beta pmax and s = pmax + t, the ellipse is
+//   (1 + 2 beta) (q^2 + 4 qmax^2 (p + t) (p - pmax) / s^2) > 0,
+// and the tension line's q_limit = 2 sqrt(pmax t) qmax / s (p + 3e6) / 3e6 is
+// exceeded iff q^2 > q_limit^2 when it is >= 0, and always when qmax < 0 (a
+// GrainVariability above 1).  A grain whose pmax or t is not positive (nor
+// then 1 + 2 beta) takes the formula as it stands.
 static __device__ __forceinline__ bool fails_sq(const KParams &k, short grain, double p, double q2) {
-    double var1 = 1.0 + k.grainVar * 0.05 * (-10 + grain % 21);
-    double var2 = 1.0 + k.grainVar * 0.033 * (-15 + (grain + 3) % 30);
-    double var3 = 1.0 + k.grainVar * 0.1 * (-10 + (grain + 4) % 11);
-    double pmax = k.ics * var1;
-    double pmin = -k.its * var2;
-    double qmax = k.iss * var3;
-    double beta = -pmin / pmax;
-    double a = pmax * (1 + beta);
-    double mSq = (4 * qmax * qmax * (1 + 2 * beta)) / (a * a);
-    const double pmin2 = -3e6;
+    const double var1 = 1.0 + k.grainVar * 0.05 * (-10 + grain % 21);
+    const double var2 = 1.0 + k.grainVar * 0.033 * (-15 + (grain + 3) % 30);
+    const double var3 = 1.0 + k.grainVar * 0.1 * (-10 + (grain + 4) % 11);
+    const double pmax = k.ics * var1, t = k.its * var2, qmax = k.iss * var3;
+    if (!(pmax > 0 && t > 0)) return fails(k, grain, p, sqrt(q2));
+    const double s = pmax + t, qs = q2 * (s * s), m4 = 4. * qmax * qmax;
     if (p < 0) {
-        if (p < pmin2) return true;
-        double q0 = 2 * sqrt(-pmax * pmin) * qmax / (pmax - pmin);
-        double kk = -q0 / pmin2;
-        double q_limit = kk * (p - pmin2);
-        return q_limit < 0 || q2 > q_limit * q_limit;
+        const double d = p + 3e6;
+        return d < 0 || qmax < 0 || qs * 9e12 > m4 * (pmax * t) * (d * d);
     }
-    double y = (1. + 2. * beta) * q2 + mSq * (p + beta * pmax) * (p - pmax);
-    return y > 0;
+    return qs + m4 * (p + t) * (p - pmax) > 0;
 }
 
 // Drucker-Prager return map for crushed points (Wolper_Drucker_Prager
