@@ -34,7 +34,7 @@ struct icempm_ctx {
     // device arrays
     double *pts = nullptr, *ptsTmp = nullptr;
     size_t pp = 0, nPtsAlloc = 0;
-    double *gridA = nullptr, *gridB = nullptr;
+    double *gridA = nullptr, *gridB = nullptr, *gridC = nullptr;   // gridC: substep kernel only
     size_t gp = 0, nGridAlloc = 0;
     double *bins = nullptr;
     int nBinsAlloc = 0;   // doubles
@@ -49,6 +49,17 @@ struct icempm_ctx {
     int nChunks = 0;
     size_t chunkCap = 0;
     bool chunksDirty = true;
+
+    // the substep kernel of longer FAST runs: the points' band order and its
+    // chunks (a plan, good until points are loaded), their records and copied
+    // rows, the case's constants (and what was uploaded) with its touched nodes
+    int *perm = nullptr, *bandStart = nullptr;
+    int nBand = 0, bandPoints = 0;
+    bool bandDirty = true;
+    void *recs = nullptr;
+    double *rows = nullptr;
+    unsigned char *caseDev = nullptr;
+    std::vector<unsigned char> caseHost;
 
     // sort scratch
     int *keys = nullptr, *vals = nullptr, *keys2 = nullptr, *vals2 = nullptr, *sortTmp = nullptr;
@@ -322,8 +333,9 @@ int ensure_ordered(icempm_ctx *c) {
 }
 
 void free_all(icempm_ctx *c) {
-    dfree(c->pts); dfree(c->ptsTmp); dfree(c->gridA); dfree(c->gridB); dfree(c->bins);
-    dfree(c->hist); dfree(c->chunkStart);
+    dfree(c->pts); dfree(c->ptsTmp); dfree(c->gridA); dfree(c->gridB); dfree(c->gridC); dfree(c->bins);
+    dfree(c->hist); dfree(c->chunkStart); 
+    dfree(c->perm); dfree(c->bandStart); dfree(c->recs); dfree(c->rows); dfree(c->caseDev);
     dfree(c->keys); dfree(c->vals); dfree(c->keys2); dfree(c->vals2); dfree(c->sortTmp);
     OrderedScratch &o = c->ord;
     dfree(o.contrib); dfree(o.cnode); dfree(o.count); dfree(o.start); dfree(o.cursor);
@@ -331,9 +343,10 @@ void free_all(icempm_ctx *c) {
     dfree(o.contacts); dfree(o.scanTmp);
     o = OrderedScratch{};
     hfree(c->hostPts); hfree(c->hostForce);
-    c->histCap = 0; c->chunkCap = 0; c->sortCap = 0; c->sortTmpCap = 0;
+    c->histCap = 0; c->chunkCap = 0;
+    c->caseHost.clear(); c->sortCap = 0; c->sortTmpCap = 0;
     c->nPtsAlloc = 0; c->nGridAlloc = 0; c->nBinsAlloc = 0; c->nChunks = 0;
-    c->chunksDirty = true;
+    c->chunksDirty = c->bandDirty = true;
 }
 
 // the particle pass of the context's mode: FMA-contracted in FAST mode,
@@ -347,30 +360,109 @@ hipError_t particles(icempm_ctx *c, const KParams &k, bool g2p, bool p2g, const 
                                   recordPQ, c->stream, c->passKind);
 }
 
-// the dominant kernel of a substep, optionally bracketed by timing events
+// brackets the dominant kernel of a substep with timing events: slot < 0 is off
+int timing_begin(icempm_ctx *c, int timeIt, int &slot) {
+    slot = -1;
+    if (!timeIt) return ICEMPM_OK;
+    size_t q = 0;
+    for (; q < c->tevUsed.size(); ++q)
+        if (!c->tevUsed[q]) break;
+    if (q == c->tevUsed.size()) {
+        hipEvent_t a, b;
+        HIPCHK(c, hipEventCreate(&a), "timing events");
+        HIPCHK(c, hipEventCreate(&b), "timing events");
+        c->tev.push_back(a);
+        c->tev.push_back(b);
+        c->tevUsed.push_back(0);
+    }
+    c->tevUsed[q] = 1;
+    HIPCHK(c, hipEventRecord(c->tev[2 * q], c->stream), "timing events");
+    slot = (int)q;
+    return ICEMPM_OK;
+}
+int timing_end(icempm_ctx *c, int slot) {
+    if (slot >= 0) HIPCHK(c, hipEventRecord(c->tev[2 * (size_t)slot + 1], c->stream), "timing events");
+    return ICEMPM_OK;
+}
+
 int launch_particles_timed(icempm_ctx *c, const KParams &k, bool g2p, bool p2g,
                            const double *gridV, double *gridOut, int recordPQ, int timeIt) {
-    hipEvent_t e0 = nullptr, e1 = nullptr;
-    if (timeIt) {
-        size_t slot = 0;
-        for (; slot < c->tevUsed.size(); ++slot)
-            if (!c->tevUsed[slot]) break;
-        if (slot == c->tevUsed.size()) {
-            hipEvent_t a, b;
-            HIPCHK(c, hipEventCreate(&a), "timing events");
-            HIPCHK(c, hipEventCreate(&b), "timing events");
-            c->tev.push_back(a);
-            c->tev.push_back(b);
-            c->tevUsed.push_back(0);
-        }
-        c->tevUsed[slot] = 1;
-        e0 = c->tev[2 * slot];
-        e1 = c->tev[2 * slot + 1];
-        HIPCHK(c, hipEventRecord(e0, c->stream), "timing events");
-    }
+    int slot, rc = timing_begin(c, timeIt, slot);
+    if (rc) return rc;
     HIPCHK(c, particles(c, k, g2p, p2g, gridV, gridOut, recordPQ), "particle pass");
-    if (timeIt) HIPCHK(c, hipEventRecord(e1, c->stream), "timing events");
-    return ICEMPM_OK;
+    return timing_end(c, slot);
+}
+
+// Whether a run of n substeps goes by the substep kernel.  It needs two grids
+// more cleared and a copy of the points in band order, made and taken back: that
+// pays from about 32 substeps and, for the copies, one more per 8192 points.
+// us per substep without -> with it, in runs of 1000 (of 200):
+//   2,400 points   10.9 -> 7.8     400,000 points  24.4 -> 19.0 (32.7 -> 24.6)
+//   60,000 points  11.9 -> 7.8     800,000 points  36.3 -> 33.7 (48.2 -> 42.7)
+//   200,000 points 15.8 -> 11.3    1,204,000       48.1 -> 47.3 (63.7 -> 61.9)
+//   (21.3 -> 14.9)                 1,600,000       54.6 -> 55.8 (76.8 -> 74.1)
+// Beyond, where launches no longer count, the two kernels' smaller working sets
+// are the faster.
+constexpr int kSubstepKernelMaxPts = 1200000;
+bool substep_kernel_pays(int n, int nPts) { return nPts <= kSubstepKernelMaxPts && n >= 32 + nPts / 8192; }
+
+// The substep kernel's plan and arrays for the next run, the indenter starting
+// at (x0, y0); false where the run goes by the grid update and the particle
+// pass instead: another mode or pass kind, constants that the kernel does not
+// take, no memory.
+bool ensure_substep(icempm_ctx *c, double x0, double y0, single::Run &r) {
+    if (c->mode != ICEMPM_MODE_FAST || c->passKind != 2) return false;
+    std::vector<unsigned char> cp(single::kCaseBytes);
+    if (!single::case_constants(c->prms, x0, y0, cp.data())) return false;
+    const icy::SimParams &P = c->prms;
+    const auto get = [](auto *&p, size_t bytes) { return p || hipMalloc(&p, bytes) == hipSuccess; };
+    const auto upload = [c](void *dst, const void *src, size_t bytes) {
+        return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream) == hipSuccess &&
+               hipStreamSynchronize(c->stream) == hipSuccess;
+    };
+    bool ok = get(c->gridC, c->gp * kGridRows * sizeof(double)) && get(c->rows, single::copy_bytes(c->pp)) &&
+              get(c->perm, c->pp * sizeof(int)) && get(c->caseDev, single::kCaseBytes + 64);
+    if (ok && c->caseHost != cp) {
+        c->caseHost.clear();
+        ok = upload(c->caseDev, cp.data(), cp.size());
+        if (ok) c->caseHost = cp;
+    }
+    r = single::Run{};
+    r.cp = c->caseDev;
+    r.bounds = c->caseDev ? c->caseDev + single::kCaseBytes : nullptr;
+    r.pts = c->pts;
+    r.pp = c->pp;
+    r.gp = c->gp;
+    r.n = P.nPts;
+    r.gx = P.GridX;
+    r.gy = P.GridY;
+    r.stream = c->stream;
+    if (ok && (c->bandDirty || c->bandPoints != P.nPts)) {
+        std::vector<int> starts;
+        dfree(c->bandStart);
+        dfree(c->recs);
+        ok = ensure_sort_scratch(c, (size_t)P.nPts) == ICEMPM_OK &&
+             single::plan(r, P.nPts, c->keys, c->vals, c->keys2, c->vals2, c->sortTmp, starts) == hipSuccess &&
+             get(c->bandStart, starts.size() * sizeof(int)) && get(c->recs, starts.size() * single::kRecBytes) &&
+             upload(c->bandStart, starts.data(), starts.size() * sizeof(int)) &&
+             hipMemcpyAsync(c->perm, c->vals, (size_t)P.nPts * sizeof(int), hipMemcpyDeviceToDevice, c->stream) ==
+                 hipSuccess;
+        c->nBand = (int)starts.size() - 1;
+        c->bandPoints = P.nPts;
+        c->bandDirty = !ok;
+    }
+    if (!ok) {
+        (void)hipGetLastError();
+        return false;
+    }
+    r.perm = c->perm;
+    r.starts = c->bandStart;
+    r.recs = c->recs;
+    r.nChunks = c->nBand;
+    r.rows = c->rows;
+    r.bins = c->bins;
+    r.err = c->dErr;
+    return true;
 }
 
 int collect_timing(icempm_ctx *c) {
@@ -547,7 +639,7 @@ int icempm_update_constants(icempm_ctx *c, const void *simparams, size_t nbytes)
             HIPCHK(c, hipStreamSynchronize(c->stream), "cuda_update_constants: gprms");
         }
         c->haveParams = true;
-        c->chunksDirty = true;
+        c->chunksDirty = c->bandDirty = true;
         // gpu_error_indicator <- error_code (gpu_implementation5.cu:474)
         HIPCHK(c, launch_fill_i32(c->dErr, 1, c->errorCode.load(), c->stream),
                "gpu_error_indicator initialization");
@@ -602,7 +694,7 @@ int icempm_transfer_points_to_device(icempm_ctx *c) {
                                  hipMemcpyHostToDevice, c->stream), "transfer_points_to_device");
         HIPCHK(c, hipStreamSynchronize(c->stream), "transfer_points_to_device");
         std::memset(c->hostForce, 0, (size_t)c->nBinsAlloc * sizeof(double));
-        c->chunksDirty = true;
+        c->chunksDirty = c->bandDirty = true;
         return ICEMPM_OK;
     });
 }
@@ -697,9 +789,17 @@ int icempm_run_substeps(icempm_ctx *c, int first_step, int n, double *t,
             if ((rc = ensure_ordered(c))) return rc;
         }
         if ((rc = ensure_chunks(c))) return rc;
+        single::Run run{};
+        const bool one = substep_kernel_pays(n, c->prms.nPts) &&
+                         ensure_substep(c, indenter_x_initial, indenter_y, run);
+        bool copied = false;   // the points are in the substep kernel's copy
         if (!ordered) {
             HIPCHK(c, launch_fill_f64(c->gridA, c->gp * kGridRows, 0.0, c->stream), "run_substeps");
             HIPCHK(c, particles(c, k, false, true, c->gridA, c->gridA, 0), "run_substeps");
+            if (one) {
+                HIPCHK(c, launch_fill_f64(c->gridB, c->gp * kGridRows, 0.0, c->stream), "run_substeps");
+                HIPCHK(c, launch_fill_f64(c->gridC, c->gp * kGridRows, 0.0, c->stream), "run_substeps");
+            }
         }
         for (int i = 0; i < n; ++i) {
             const int s = first_step + i;
@@ -721,12 +821,31 @@ int icempm_run_substeps(icempm_ctx *c, int first_step, int n, double *t,
                     return rc;
             } else {
                 const bool last = (i == n - 1);
-                HIPCHK(c, launch_update(k, c->gridA, ix, indenter_y, h2, last ? nullptr : c->gridB,
+                // P and Q, and the values a run ends with, are the particle pass's
+                if (one && !last && !rec) {
+                    if (!copied) HIPCHK(c, single::enter(run), "run_substeps");
+                    copied = true;
+                    int slot;
+                    if ((rc = timing_begin(c, timeIt, slot))) return rc;
+                    HIPCHK(c, single::substep(run, c->gridA, c->gridB, c->gridC, h2, tt, i), "run_substeps");
+                    if ((rc = timing_end(c, slot))) return rc;
+                    double *done = c->gridA;
+                    c->gridA = c->gridB;
+                    c->gridB = c->gridC;
+                    c->gridC = done;
+                    continue;
+                }
+                if (copied) HIPCHK(c, single::leave(run), "run_substeps");
+                copied = false;
+                // the grid that the next P2G goes to is cleared here, or was
+                // by the substep kernel, whose third grid then is
+                HIPCHK(c, launch_update(k, c->gridA, ix, indenter_y, h2, last ? nullptr : (one ? c->gridC : c->gridB),
                                         false, nullptr, nullptr, c->stream), "run_substeps");
                 if (!last) {
                     if ((rc = launch_particles_timed(c, k, true, true, c->gridA, c->gridB, rec, timeIt)))
                         return rc;
                     std::swap(c->gridA, c->gridB);
+                    if (one) std::swap(c->gridB, c->gridC);
                 } else {
                     if ((rc = launch_particles_timed(c, k, true, false, c->gridA, nullptr, rec, timeIt)))
                         return rc;
@@ -846,7 +965,7 @@ int icempm_sort_points(icempm_ctx *c, int *perm_out, int *keys_out) {
             HIPCHK(c, hipMemcpyAsync(keys_out, c->keys, (size_t)n * sizeof(int), hipMemcpyDeviceToHost,
                                      c->stream), "sort_points");
         HIPCHK(c, hipStreamSynchronize(c->stream), "sort_points");
-        c->chunksDirty = true;
+        c->chunksDirty = c->bandDirty = true;
         return ICEMPM_OK;
     });
 }
@@ -950,7 +1069,7 @@ int icempm_set_tuning(icempm_ctx *c, int knob, int value) {
         switch (knob) {
         case ICEMPM_TUNE_PASS_KIND:
             if (value < 0 || value > 2) return fail(c, ICEMPM_E_ARG, "set_tuning: pass kind is 0, 1 or 2");
-            if ((value == 0) != (c->passKind == 0)) c->chunksDirty = true;   // the chunk rule differs
+            if ((value == 0) != (c->passKind == 0)) c->chunksDirty = c->bandDirty = true;   // the chunk rule differs
             c->passKind = value;
             return ICEMPM_OK;
         default:

@@ -78,9 +78,6 @@ template <bool F32>
 struct Rows {
     using V = typename std::conditional<F32, float, double>::type;
     using P = typename std::conditional<F32, unsigned int, double>::type;
-    // grid velocity as the gathers read it: FP64 rows 1-2 of the grid, or
-    // (FP32 storage) one FP32 pair per node written by the grid update
-    using G = typename std::conditional<F32, float2, double>::type;
     // FP64: rows x, y.  FP32: one 16-byte record per slot, {high 32 bits of
     // x, of y, the two low 16-bit halves, the crushed flag | grain id << 16}
     // (one load and one store per pass; the crushed and grain rows are then
@@ -443,7 +440,7 @@ static __device__ __forceinline__ bool node_velocity(const CaseParams &cp, doubl
 // grids are still zero.
 constexpr int kNodeBlk = 1024;
 struct NodeWork {
-    const int2 *blocks;   // {case, first node} per workgroup
+    const int2 *blocks;   // {case, first node} per workgroup (null: one case's, in order)
     double *clear;        // the grid to clear
     double *hist;         // this substep's force, 2 per case
     double *bins;
@@ -452,7 +449,7 @@ struct NodeWork {
 static __device__ __forceinline__ void node_part(const NodeWork &nw, int block, const CaseParams *__restrict__ cases,
                                                  const double *__restrict__ grid, size_t gpitch, const int4 *bounds,
                                                  double t, double *lds) {
-    const int2 nb = nw.blocks[block];
+    const int2 nb = nw.blocks ? nw.blocks[block] : make_int2(0, block * kNodeBlk);
     const CaseParams &cp = cases[nb.x];
     const int4 bd = bounds[nb.x];
     const int x0 = bd.x - 1, y0 = bd.y - 1, x1 = bd.z + 1, y1 = bd.w + 1;
@@ -660,12 +657,12 @@ __global__ __launch_bounds__(256, 5) void k_batch_substep(
     ChunkRec *__restrict__ recs, const double *__restrict__ gridIn, int nChunks, int pGroups,
     typename Rows<F32>::P *pos, typename Rows<F32>::V *rest, size_t gpitch, const CaseParams *__restrict__ cases,
     unsigned char *crushedRow, size_t pitch, double *__restrict__ gridOut, int4 *bounds, int *__restrict__ err,
-    const short *__restrict__ grains, const double *__restrict__ tTab, int step, NodeWork nw, LearnArgs la, MapQueue mq,
-    int storeVB) {
+    const short *__restrict__ grains, typename Rows<F32>::V *jpRow, const double *__restrict__ tTab, double t0, int step,
+    NodeWork nw, LearnArgs la, MapQueue mq, int storeVB) {
     __shared__ __attribute__((aligned(16))) double smem[4 * 3 * kWaveWin + 2 * kTile + 4 * (2 * 9 + 1) * kPatch];
     if constexpr (G2P) {
         if ((int)blockIdx.x >= pGroups) {
-            node_part(nw, (int)blockIdx.x - pGroups, cases, gridIn, gpitch, bounds, tTab[step], smem);
+            node_part(nw, (int)blockIdx.x - pGroups, cases, gridIn, gpitch, bounds, tTab ? tTab[step] : t0, smem);
             return;
         }
     }
@@ -708,7 +705,7 @@ __global__ __launch_bounds__(256, 5) void k_batch_substep(
     const int wcol = lane & ((1 << wsh) - 1), wrow0 = lane >> wsh, wstep = 64 >> wsh;
     double *W0 = smem + row * 3 * kWaveWin, *W1 = W0 + kWaveWin, *W2 = W1 + kWaveWin;
     double2 *tile = reinterpret_cast<double2 *>(smem + 4 * 3 * kWaveWin);
-    const double ind_x = cp.x0 + (G2P ? tTab[step] : 0.0) * cp.indV;
+    const double ind_x = cp.x0 + (G2P ? (tTab ? tTab[step] : t0) : 0.0) * cp.indV;
 
     // The state of the points, streamed once per substep: non-temporal, so the
     // grid keeps the L2.  A lane without a point reads the chunk's first one
@@ -911,7 +908,7 @@ __global__ __launch_bounds__(256, 5) void k_batch_substep(
             // skips it); p and q for the NACC test came from the invariants.
             // Jp_inv matters only to the map, so only crushed points load it.
             const bool crushedOk = ok && crushed == 1;
-            if (crushedOk) Jp = fe0 + (double)*at(R + pp * 10, u);
+            if (crushedOk) Jp = fe0 + (double)*at(jpRow, u);
             const double Jp0 = Jp;
             if constexpr (RMAP == kMapExact) {
                 if (crushedOk && dp_projects_sq(k, iv.p, iv.q2, Jp))
@@ -1044,7 +1041,7 @@ __global__ __launch_bounds__(256, 5) void k_batch_substep(
                 R[pp * 8 + pt] = (V)B10;
                 R[pp * 9 + pt] = (V)B11;
             }
-            if (ok && Jp != Jp0 && !defer) *at(R + pp * 10, u) = (V)(Jp - fe0);
+            if (ok && Jp != Jp0 && !defer) *at(jpRow, u) = (V)(Jp - fe0);
             if (!F32 && ok && crushed != crushed0) *at(S.crushed, u) = crushed;   // FP32: in the record
             kirchhoff_from_inv(iv, t00, t01, t11);
             if (crushedOk) kirchhoff_rcp(fe0 + F00, F01, F10, fe0 + F11, cp.mu, cp.kappa, t00, t01, t11);
@@ -1214,12 +1211,21 @@ __global__ __launch_bounds__(256, 5) void k_batch_substep(
 
 // The boxes of the chunks' points as they are, a wavefront a chunk: what a
 // run's first P2G, or a table rebuilt between two runs, starts from.
+// starts (one case only, may be null): the chunks' first slots and the end, from
+// which the rest of their records is made first.
 template <bool F32>
 __global__ __launch_bounds__(256) void k_chunk_boxes(ChunkRec *recs, int nChunks, const typename Rows<F32>::P *pos,
-                                                     size_t pitch, const CaseParams *__restrict__ cases, int4 *bounds) {
+                                                     size_t pitch, const CaseParams *__restrict__ cases, int4 *bounds,
+                                                     const int *__restrict__ starts) {
     const int ch = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, lane = threadIdx.x & 63;
     if (ch >= nChunks) return;
-    ChunkRec &rec = recs[ch];
+    ChunkRec rec = recs[ch];
+    if (starts) {
+        rec = ChunkRec{};
+        rec.beg = starts[ch];
+        rec.count = starts[ch + 1] - rec.beg;
+        rec.dims = (unsigned)cases[0].gx | (unsigned)cases[0].gy << 16;
+    }
     const CaseParams &cp = cases[rec.cs];
     int wx0[4], wy0[4], wx1[4], wy1[4];   // of each wavefront's points
     int fx = 0, fy = 0, x0 = INT_MAX, y0 = INT_MAX, x1 = -1, y1 = -1;
@@ -1258,6 +1264,7 @@ __global__ __launch_bounds__(256) void k_chunk_boxes(ChunkRec *recs, int nChunks
         // point's surroundings
         rec.ext = 0;
         for (int q = 0; q < 4; ++q) rec.win[q] = 0;
+        if (x0 <= x1) widen_bounds(bounds, rec.cs, x0, y0, x1, y1);
         if (x0 <= x1 && !set_box(rec, x0, y0, x1, y1)) {
             x0 = max(fx - 7, x0);
             x1 = min(fx + 7, x1);
@@ -1269,8 +1276,8 @@ __global__ __launch_bounds__(256) void k_chunk_boxes(ChunkRec *recs, int nChunks
 #pragma unroll
             for (int q = 0; q < 4; ++q)
                 if (wx1[q] >= 0) rec.win[q] = win_of(rec, wx0[q], wy0[q], wx1[q], wy1[q]);
-            widen_bounds(bounds, rec.cs, x0, y0, x1, y1);
         }
+        recs[ch] = rec;
     }
 }
 
@@ -1646,6 +1653,46 @@ struct icempm_batch {
 
 namespace {
 
+// A case's constants from its parameters, but for the offsets of a batch.
+void fill_case(CaseParams &c, const icy::SimParams &P) {
+    c = CaseParams{};
+    c.dt = P.InitialTimeStep; c.vol = P.ParticleVolume; c.mass = P.ParticleMass; c.h = P.cellsize;
+    c.h_inv = P.cellsize_inv; c.Dinv = P.Dp_inv; c.mu = P.mu; c.kappa = P.kappa; c.gravity = P.Gravity;
+    c.indRsq = P.IndRSq; c.indV = P.IndVelocity; c.ics = P.IceCompressiveStrength;
+    c.its = P.IceTensileStrength; c.iss = P.IceShearStrength; c.tanPhi = P.DP_tan_phi;
+    c.dpThr = P.DP_threshold_p; c.x0 = P.indenter_x_initial; c.y0 = P.indenter_y;
+    {
+        // NACC constants of grain 0 with no variability (gpu_implementation5.cu:97-141)
+        const double pmax = P.IceCompressiveStrength, pmin = -P.IceTensileStrength, qmax = P.IceShearStrength;
+        const double beta = -pmin / pmax;
+        const double a = pmax * (1 + beta);
+        c.pmax = pmax;
+        c.msq = (4 * qmax * qmax * (1 + 2 * beta)) / (a * a);
+        c.betaPmax = beta * pmax;
+        c.onePlus2Beta = 1. + 2. * beta;
+        c.slope = -(2 * std::sqrt(-pmax * pmin) * qmax / (pmax - pmin)) / -3e6;
+    }
+    c.gx = P.GridX; c.gy = P.GridY; c.gridTotal = P.GridTotal; c.nPts = P.nPts;
+    c.gxInv = 1.0 / c.gx;
+    c.grainVar = P.GrainVariability;
+    c.nbins = P.n_indenter_subdivisions;
+    c.scm = c.dt * c.vol * c.Dinv / c.mass;
+    c.vmax = 0.5 * c.h / c.dt;
+    c.dtCells = c.dt * c.h_inv;
+    {
+        // FP32 storage: 48 - ib fraction bits, ib the bits a cell index needs
+        // (finalize refuses grids beyond 65536 nodes a side: ib <= 16)
+        int ib = 0;
+        while (ib < 16 && (1 << ib) < std::max(c.gx, c.gy)) ++ib;
+        const int F = 48 - ib;
+        c.cellQ = std::ldexp(1.0, -F);
+        c.cellQ16 = std::ldexp(1.0, 16 - F);
+        c.cellInvQ = std::ldexp(1.0, F);
+        c.posQ = c.h * c.cellQ;
+        c.posInvQ = c.cellInvQ / c.h;
+    }
+}
+
 int bfail(icempm_batch *b, int code, const std::string &m) {
     if (b) b->lastError = m;
     return code;
@@ -1690,8 +1737,8 @@ void launch_one(icempm_batch *b, const Pass &p, const LearnArgs &la, const MapQu
     const int groups = ((p.chunks + 7) / 8) * 8;
     hipLaunchKernelGGL((k_batch_substep<F32, G2P, RMAP>), dim3((unsigned)(groups + (G2P ? p.blocks : 0))), dim3(256), 0,
                        p.stream, b->recs + p.chunk0, b->grids + p.in * grid, p.chunks, groups, S.pos, S.rest, b->gpitch,
-                       b->cases, S.crushed, S.pitch, b->grids + p.out * grid, b->bounds, b->err, b->grain, p.tTab, p.step, nw, la, mq,
-                       p.storeVB ? 1 : 0);
+                       b->cases, S.crushed, S.pitch, b->grids + p.out * grid, b->bounds, b->err, b->grain,
+                       S.rest + 10 * S.pitch, p.tTab, 0.0, p.step, nw, la, mq, p.storeVB ? 1 : 0);
     if (b->evAfter) (void)hipEventRecord(b->evAfter, p.stream);
     if (G2P && RMAP == kMapLearned && la.branches != 0) {
         // the deferred points: map, store, and their P2G into the pass's output grid
@@ -1739,13 +1786,35 @@ hipError_t launch_pass(icempm_batch *b, bool g2p, const Pass &p) {
     return hipGetLastError();
 }
 
-// Chunk table from the case-local base cells of the points in slot order
-// (column | row << 16): chunks of <= chunkPoints consecutive points of one
-// case whose base cells span at most two cell rows and kChunkCols columns, so
-// that the workgroup's LDS holds all its stencils, cut greedily.  A chunk that
-// is cut for its columns alone ends at a wavefront's last point if it can.
-// Points in band order give chunks of one band each, until they move.  The
-// cases are independent, so they are cut on several host threads.
+// Chunks of n consecutive points with the given base cells (column | row <<
+// 16), the first of them slot o: <= cap points whose cells span at most two
+// cell rows and kChunkCols columns, so that the workgroup's LDS holds all their
+// stencils, cut greedily.  A chunk that is cut for its columns alone ends at a
+// wavefront's last point if it can.  Points in band order give chunks of one
+// band each, until they move.
+void cut_chunks(const unsigned *cells, int n, int o, int cap, std::vector<int> &starts) {
+    starts.reserve((size_t)n / (size_t)cap + 16);
+    for (int cs = 0; cs < n;) {
+        int c0 = INT_MAX, r0 = INT_MAX, c1 = -1, r1 = -1, i = cs;
+        bool wide = false;
+        for (; i < n && i - cs < cap; ++i) {
+            const int cc = (int)(cells[i] & 0xFFFFu), r = (int)(cells[i] >> 16);
+            r0 = std::min(r0, r);
+            r1 = std::max(r1, r);
+            c0 = std::min(c0, cc);
+            c1 = std::max(c1, cc);
+            wide = c1 - c0 > kChunkCols - 1;
+            if (r1 - r0 > 1 || wide) break;
+        }
+        if (wide && r1 - r0 <= 1 && i - cs > 64) i = cs + (i - cs) / 64 * 64;
+        starts.push_back(o + cs);
+        cs = i;
+    }
+}
+
+// Chunk table from the case-local base cells of the points in slot order, the
+// chunks within one case.  The cases are independent, so they are cut on
+// several host threads.
 void chunk_table(const icempm_batch *b, const unsigned *cells, std::vector<int> &cstart,
                  std::vector<int> &ccase) {
     const size_t nc = b->hc.size();
@@ -1753,27 +1822,7 @@ void chunk_table(const icempm_batch *b, const unsigned *cells, std::vector<int> 
     std::vector<std::vector<int>> starts(nc);
     auto cut = [&](size_t ci) {
         const CaseParams &cp = b->hc[ci].cp;
-        const int n = cp.nPts, o = cp.ptOffset;
-        std::vector<int> &st = starts[ci];
-        if (n <= 0) return;
-        st.reserve((size_t)n / (size_t)cap + 16);
-        for (int cs = 0; cs < n;) {
-            int c0 = INT_MAX, r0 = INT_MAX, c1 = -1, r1 = -1, i = cs;
-            bool wide = false;
-            for (; i < n && i - cs < cap; ++i) {
-                const unsigned ki = cells[(size_t)o + i];
-                const int cc = (int)(ki & 0xFFFFu), r = (int)(ki >> 16);
-                r0 = std::min(r0, r);
-                r1 = std::max(r1, r);
-                c0 = std::min(c0, cc);
-                c1 = std::max(c1, cc);
-                wide = c1 - c0 > kChunkCols - 1;
-                if (r1 - r0 > 1 || wide) break;
-            }
-            if (wide && r1 - r0 <= 1 && i - cs > 64) i = cs + (i - cs) / 64 * 64;
-            st.push_back(o + cs);
-            cs = i;
-        }
+        if (cp.nPts > 0) cut_chunks(cells + cp.ptOffset, cp.nPts, cp.ptOffset, cap, starts[ci]);
     };
     const unsigned hw = std::thread::hardware_concurrency();
     const size_t nt = std::min<size_t>(nc, std::min(16u, std::max(1u, hw)));
@@ -1831,10 +1880,10 @@ hipError_t launch_boxes(icempm_batch *b) {
     const dim3 nb((unsigned)((b->nChunks + 3) / 4));
     if (b->precision == ICEMPM_BATCH_F32)
         hipLaunchKernelGGL(k_chunk_boxes<true>, nb, dim3(256), 0, b->stream, b->recs, b->nChunks,
-                           static_cast<const unsigned int *>(b->pos), b->pitch, b->cases, b->bounds);
+                           static_cast<const unsigned int *>(b->pos), b->pitch, b->cases, b->bounds, nullptr);
     else
         hipLaunchKernelGGL(k_chunk_boxes<false>, nb, dim3(256), 0, b->stream, b->recs, b->nChunks,
-                           static_cast<const double *>(b->pos), b->pitch, b->cases, b->bounds);
+                           static_cast<const double *>(b->pos), b->pitch, b->cases, b->bounds, nullptr);
     return hipGetLastError();
 }
 
@@ -2069,6 +2118,109 @@ hipError_t enqueue_loop(icempm_batch *b, int n, const double *tTab, double *hist
 
 }  // namespace
 
+// ---- one case on its context's own arrays -----------------------------------
+namespace icempm {
+namespace single {
+
+static_assert(sizeof(ChunkRec) == kRecBytes && sizeof(CaseParams) <= kCaseBytes, "sizes of internal.h");
+
+bool case_constants(const icy::SimParams &P, double x0, double y0, void *out) {
+    // the substep kernel's premises: 16-bit cell indices, 32-bit byte offsets,
+    // consistent cell sizes, numbers for the strengths
+    if (P.nPts <= 0 || P.nPts >= 1 << 28 || P.GridX > 32767 || P.GridY > 32767 || P.GridTotal >= 1 << 28) return false;
+    if (!(P.cellsize_inv == 1. / P.cellsize) || !(P.Dp_inv == 4. / (P.cellsize * P.cellsize))) return false;
+    if (!(P.GrainVariability == P.GrainVariability)) return false;
+    CaseParams c;
+    fill_case(c, P);
+    c.x0 = x0;
+    c.y0 = y0;
+    std::memset(out, 0, kCaseBytes);
+    std::memcpy(out, &c, sizeof(c));
+    return true;
+}
+
+hipError_t plan(const Run &r, int n, int *keys, int *vals, int *keys2, int *vals2, int *tmp, std::vector<int> &starts) {
+    hipLaunchKernelGGL(k_batch_keys<double>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, r.stream, r.pts + kRowPosX * r.pp,
+                       r.pp, n, static_cast<const CaseParams *>(r.cp), 1, keys, vals);
+    hipError_t e = radix_sort_pairs(keys, vals, keys2, vals2, (size_t)n, tmp, r.stream);
+    if (e != hipSuccess) return e;
+    std::vector<int> hk((size_t)n);
+    std::vector<unsigned> cells((size_t)n);
+    if ((e = hipMemcpyAsync(hk.data(), keys, (size_t)n * sizeof(int), hipMemcpyDeviceToHost, r.stream)) != hipSuccess) return e;
+    if ((e = hipStreamSynchronize(r.stream)) != hipSuccess) return e;
+    for (int i = 0; i < n; ++i) {
+        int x, y;
+        band_cell(hk[(size_t)i], r.gx, r.gy, x, y);
+        cells[(size_t)i] = (unsigned)x | (unsigned)y << 16;
+    }
+    starts.clear();
+    cut_chunks(cells.data(), n, 0, 256, starts);
+    starts.push_back(n);
+    return hipSuccess;
+}
+
+// The rows a substep reads and writes, from the points' own order to band
+// order and back; v and Bp are not among them, since every substep makes its
+// own, and P and Q are not touched.
+__global__ __launch_bounds__(256) void k_pack(const double *__restrict__ pts, size_t pp, int n, const int *__restrict__ perm,
+                                              double *__restrict__ rows) {
+    const int k = blockIdx.x * 256 + threadIdx.x;
+    if (k >= n) return;
+    const int j = perm[k];
+    rows[k] = pts[kRowPosX * pp + j];
+    rows[pp + k] = pts[(kRowPosX + 1) * pp + j];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) rows[(2 + r) * pp + k] = pts[(kRowFe00 + r) * pp + j];
+    rows[6 * pp + k] = pts[kRowJp * pp + j];
+    const unsigned char *u = reinterpret_cast<const unsigned char *>(pts + kRowUtil * pp);
+    unsigned char *v = reinterpret_cast<unsigned char *>(rows + 7 * pp);
+    v[k] = u[j];
+    reinterpret_cast<short *>(v + pp)[k] = reinterpret_cast<const short *>(u + pp)[j];
+}
+__global__ __launch_bounds__(256) void k_unpack(const double *__restrict__ rows, size_t pp, int n,
+                                                const int *__restrict__ perm, double *__restrict__ pts) {
+    const int k = blockIdx.x * 256 + threadIdx.x;
+    if (k >= n) return;
+    const int j = perm[k];
+    pts[kRowPosX * pp + j] = rows[k];
+    pts[(kRowPosX + 1) * pp + j] = rows[pp + k];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) pts[(kRowFe00 + r) * pp + j] = rows[(2 + r) * pp + k];
+    pts[kRowJp * pp + j] = rows[6 * pp + k];
+    reinterpret_cast<unsigned char *>(pts + kRowUtil * pp)[j] = reinterpret_cast<const unsigned char *>(rows + 7 * pp)[k];
+}
+
+hipError_t enter(const Run &r) {
+    int4 *bounds = static_cast<int4 *>(r.bounds);
+    hipLaunchKernelGGL(k_pack, dim3((unsigned)((r.n + 255) / 256)), dim3(256), 0, r.stream, r.pts, r.pp, r.n, r.perm, r.rows);
+    hipLaunchKernelGGL(k_reset_bounds, dim3(1), dim3(64), 0, r.stream, bounds, 1);
+    hipLaunchKernelGGL(k_chunk_boxes<false>, dim3((unsigned)((r.nChunks + 3) / 4)), dim3(256), 0, r.stream,
+                       static_cast<ChunkRec *>(r.recs), r.nChunks, r.rows, r.pp, static_cast<const CaseParams *>(r.cp), bounds,
+                       r.starts);
+    return hipGetLastError();
+}
+
+hipError_t leave(const Run &r) {
+    hipLaunchKernelGGL(k_unpack, dim3((unsigned)((r.n + 255) / 256)), dim3(256), 0, r.stream, r.rows, r.pp, r.n, r.perm, r.pts);
+    return hipGetLastError();
+}
+
+hipError_t substep(const Run &r, const double *in, double *out, double *clear, double *hist2, double t, int step) {
+    const int groups = ((r.nChunks + 7) / 8) * 8, blocks = (r.gx * r.gy + kNodeBlk - 1) / kNodeBlk;
+    const NodeWork nw{nullptr, clear, hist2, r.bins};
+    unsigned char *util = reinterpret_cast<unsigned char *>(r.rows + 7 * r.pp);
+    // rows 2-5 of the kernel's 11 are Fe; without storeVB it takes no other
+    hipLaunchKernelGGL((k_batch_substep<false, true, kMapExact>), dim3((unsigned)(groups + blocks)), dim3(256), 0, r.stream,
+                       static_cast<ChunkRec *>(r.recs), in, r.nChunks, groups, r.rows, r.rows, r.gp,
+                       static_cast<const CaseParams *>(r.cp), util, r.pp, out, static_cast<int4 *>(r.bounds), r.err,
+                       reinterpret_cast<const short *>(util + r.pp), r.rows + 6 * r.pp, nullptr, t, step, nw, LearnArgs{},
+                       MapQueue{}, 0);
+    return hipGetLastError();
+}
+
+}  // namespace single
+}  // namespace icempm
+
 extern "C" {
 
 int icempm_batch_create(icempm_batch **out, int precision) {
@@ -2155,42 +2307,7 @@ int icempm_batch_add_case(icempm_batch *b, const void *simparams, size_t nbytes,
             return -bfail(b, ICEMPM_E_ARG, "add_case: all cases of a batch share one time step");
         icempm_batch::HostCase h{};
         CaseParams &c = h.cp;
-        c.dt = P.InitialTimeStep; c.vol = P.ParticleVolume; c.mass = P.ParticleMass; c.h = P.cellsize;
-        c.h_inv = P.cellsize_inv; c.Dinv = P.Dp_inv; c.mu = P.mu; c.kappa = P.kappa; c.gravity = P.Gravity;
-        c.indRsq = P.IndRSq; c.indV = P.IndVelocity; c.ics = P.IceCompressiveStrength;
-        c.its = P.IceTensileStrength; c.iss = P.IceShearStrength; c.tanPhi = P.DP_tan_phi;
-        c.dpThr = P.DP_threshold_p; c.x0 = P.indenter_x_initial; c.y0 = P.indenter_y;
-        {
-            // NACC constants of grain 0 with no variability (gpu_implementation5.cu:97-141)
-            const double pmax = P.IceCompressiveStrength, pmin = -P.IceTensileStrength, qmax = P.IceShearStrength;
-            const double beta = -pmin / pmax;
-            const double a = pmax * (1 + beta);
-            c.pmax = pmax;
-            c.msq = (4 * qmax * qmax * (1 + 2 * beta)) / (a * a);
-            c.betaPmax = beta * pmax;
-            c.onePlus2Beta = 1. + 2. * beta;
-            c.slope = -(2 * std::sqrt(-pmax * pmin) * qmax / (pmax - pmin)) / -3e6;
-        }
-        c.gx = P.GridX; c.gy = P.GridY; c.gridTotal = P.GridTotal; c.nPts = P.nPts;
-        c.gxInv = 1.0 / c.gx;
-        c.grainVar = P.GrainVariability;
-        c.nbins = P.n_indenter_subdivisions;
-        c.binOffset = 0;   // set by finalize
-        c.scm = c.dt * c.vol * c.Dinv / c.mass;
-        c.vmax = 0.5 * c.h / c.dt;
-        c.dtCells = c.dt * c.h_inv;
-        {
-            // FP32 storage: 48 - ib fraction bits, ib the bits a cell index needs
-            // (finalize refuses grids beyond 65536 nodes a side: ib <= 16)
-            int ib = 0;
-            while (ib < 16 && (1 << ib) < std::max(c.gx, c.gy)) ++ib;
-            const int F = 48 - ib;
-            c.cellQ = std::ldexp(1.0, -F);
-            c.cellQ16 = std::ldexp(1.0, 16 - F);
-            c.cellInvQ = std::ldexp(1.0, F);
-            c.posQ = c.h * c.cellQ;
-            c.posInvQ = c.cellInvQ / c.h;
-        }
+        fill_case(c, P);
         const int n = P.nPts;
         h.pos.resize(2 * (size_t)n);
         h.rest.resize(11 * (size_t)n);

@@ -4,6 +4,9 @@
 
 #include <hip/hip_runtime.h>
 
+#include <vector>
+
+#include "../host/parameters_sim.h"
 #include "host_guard.h"
 #include "mpm_device.h"
 
@@ -68,6 +71,42 @@ struct OrderedScratch {
 hipError_t ordered_p2g(const KParams &k, double *grid, OrderedScratch &o, hipStream_t s);
 hipError_t ordered_fold_forces(const KParams &k, OrderedScratch &o, double *hist2,
                                hipStream_t s);
+
+// ---- batch.hip: the batches' substep kernel for one case ------------------------
+// One launch per substep: grid update, G2P and the next P2G, FP64, exact return
+// map; v, Bp, P and Q are not recorded.  It runs on a copy of the points in
+// band order, which enter makes and leave takes back.  Three grids rotate: a
+// substep reads in (mass and momentum of its P2G), adds the next P2G to out,
+// which must be zero, and clears the third.
+namespace single {
+constexpr size_t kRecBytes = 48, kCaseBytes = 512;   // of a chunk record and of the case's constants
+constexpr size_t copy_bytes(size_t pp) { return pp * (7 * sizeof(double) + 3); }
+struct Run {
+    const void *cp;          // the case's constants (device)
+    void *bounds;            // 16 bytes: the box of touched nodes
+    double *pts;             // 16 rows x pp
+    size_t pp, gp;
+    int n, gx, gy;
+    const int *perm;         // slot in band order -> point
+    const int *starts;       // nChunks + 1 first slots
+    void *recs;              // nChunks records, made by enter
+    int nChunks;
+    double *rows;            // the copy
+    double *bins;
+    int *err;
+    hipStream_t stream;
+};
+// The case's constants, the indenter starting at (x0, y0), in out (kCaseBytes);
+// false where the kernel does not take the case.
+bool case_constants(const icy::SimParams &P, double x0, double y0, void *out);
+// The points' band order as they are (in vals; keys, keys2, vals2: n ints, tmp:
+// radix_tmp_ints(n)) and its chunks' first slots.
+hipError_t plan(const Run &r, int n, int *keys, int *vals, int *keys2, int *vals2, int *tmp, std::vector<int> &starts);
+hipError_t enter(const Run &r);
+hipError_t leave(const Run &r);
+// hist2: this substep's force (added to); t: its time; step: its index in the run.
+hipError_t substep(const Run &r, const double *in, double *out, double *clear, double *hist2, double t, int step);
+}  // namespace single
 
 hipError_t launch_hello(int *flag, hipStream_t s);
 hipError_t launch_copy(const double *src, double *dst, size_t n_doubles, hipStream_t s);

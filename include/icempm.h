@@ -192,15 +192,16 @@ int icempm_get_mode(const icempm_ctx *ctx);
 /* Tuning knobs (no counterpart).  ICEMPM_TUNE_PASS_KIND selects the kernel
  * of the particle pass: 0 workgroup-wide shared-memory windows for gather and
  * scatter, 1 wavefront windows (direct gather, per-wavefront scatter), 2 as 1
- * with the per-lane stencil rotation (default).  Results differ only in the
- * order of the FAST-mode P2G sums. */
+ * with the per-lane stencil rotation (default; longer FAST runs of up to 1.2
+ * million points then do a substep in one kernel, on a copy of the points in
+ * another order).  Results differ only in the order of the FAST-mode P2G sums. */
 enum { ICEMPM_TUNE_PASS_KIND = 0 };
 int icempm_set_tuning(icempm_ctx *ctx, int knob, int value);
 /* current value, or -1 for an unknown knob */
 int icempm_get_tuning(const icempm_ctx *ctx, int knob);
 
-/* Device-side timing of the dominant kernel (the fused G2P+P2G pass, or
- * G2P in ORDERED mode) over icempm_run_substeps calls: when enabled, each
+/* Device-side timing of the dominant kernel (the fused G2P+P2G pass, the
+ * one-kernel substep, or G2P in ORDERED mode) over icempm_run_substeps calls: when enabled, each
  * launch is bracketed by events on the context's stream and the durations
  * are summed.  Returns total milliseconds and the launch count. */
 int icempm_kernel_timing(icempm_ctx *ctx, int enable);
@@ -221,8 +222,8 @@ int icempm_read_bins(icempm_ctx *ctx, double *out);
 
 /* -- batches of independent cases (no counterpart) ----------------------
  * Many indentation cases of uneven size advanced together: every substep is
- * one grid-update launch and one particle-pass launch over all cases, and
- * the substep loop can be captured in a HIP graph and replayed.  Cases are
+ * one launch over all cases (two groups of cases side by side when they are
+ * large; one more launch with the learned map), and the substep loop can be captured in a HIP graph and replayed.  Cases are
  * added from the reference SoA layout (16 rows x pitch doubles, as read back
  * by icempm_read_points after LoadRawPoints); all cases share the time step.
  * A case with GrainVariability != 0 takes each point's NACC strengths from
