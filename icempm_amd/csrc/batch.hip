@@ -1486,6 +1486,54 @@ __global__ void k_batch_cells(const PT *__restrict__ pos, size_t pitch, int nPts
     cells[i] = cx | cy << 16;
 }
 
+// A case's points in the layout they came in: rows 0 and 3-15 of the point SoA
+// (row r > 2 at out + (r - 2) pitch), every point at its index within the case,
+// the padding zero.  bad: set when the slot map is not one.
+template <bool F32>
+__global__ __launch_bounds__(256) void k_read_points(Rows<F32> S, const int *__restrict__ orig, CaseParams cp, int pitch,
+                                                     double *__restrict__ out, int *__restrict__ bad) {
+    const int k = blockIdx.x * 256 + threadIdx.x, n = cp.nPts, o = cp.ptOffset;
+    if (k >= pitch) return;
+    if (k >= n) {
+        for (int r = 1; r < 14; ++r) out[(size_t)r * pitch + k] = 0;
+        return;
+    }
+    const int slot = o + k, i = orig[slot] - o;
+    if (i < 0 || i >= n) {
+        *bad = 1;
+        return;
+    }
+    const size_t pp = S.pitch;
+    const auto *__restrict__ R = S.rest;
+    double v[13];   // Jp, x, y, v, Fe, Bp
+    unsigned char crushed;
+    short grain = 0;
+    if constexpr (F32) {
+        const unsigned w = pos_load<false>(S.pos, pp, slot, cp, v[1], v[2]);
+        crushed = (unsigned char)(w & 0xFFu);
+        grain = (short)(w >> 16);
+        const fe4 f = fe_rec(R, pp)[slot];
+        v[5] = (double)f.x + 1.0;
+        v[6] = (double)f.y;
+        v[7] = (double)f.z;
+        v[8] = (double)f.w + 1.0;
+        v[0] = (double)R[pp * 10 + slot] + 1.0;
+    } else {
+        pos_load<false>(S.pos, pp, slot, cp, v[1], v[2]);
+        crushed = S.crushed[slot];
+        if (S.grain) grain = S.grain[slot];
+        for (int r = 2; r < 6; ++r) v[3 + r] = R[pp * r + slot];
+        v[0] = R[pp * 10 + slot];
+    }
+    v[3] = (double)R[slot];
+    v[4] = (double)R[pp + slot];
+    for (int r = 6; r < 10; ++r) v[3 + r] = (double)R[pp * r + slot];
+    unsigned char *u8 = reinterpret_cast<unsigned char *>(out);
+    u8[i] = crushed;
+    *reinterpret_cast<short *>(u8 + pitch + 2 * (size_t)i) = grain;   // point.cpp:19-23
+    for (int r = 0; r < 13; ++r) out[(size_t)(r + 1) * pitch + i] = v[r];
+}
+
 // Point state permuted: slot k of the destination <- slot perm[k] of the source.
 template <bool F32>
 __global__ void k_batch_permute(Rows<F32> src, Rows<F32> dst, const int *__restrict__ srcOrig,
@@ -1515,6 +1563,8 @@ __global__ void k_batch_permute(Rows<F32> src, Rows<F32> dst, const int *__restr
 
 using namespace icempm;
 using namespace icempm::batch;
+
+constexpr int kReadGroups = 4;   // groups of rows of a readback
 
 struct icempm_batch {
     int precision = ICEMPM_BATCH_F64;
@@ -1640,6 +1690,12 @@ struct icempm_batch {
     std::vector<int> kcstart, kccase;
     int kChunkPoints = 256;
     double runMs = 0;   // device time of the last run's segments + re-sorts
+
+    // scratch of read_points, for cases of up to rbPitch points
+    std::mutex rbLock;
+    double *rbDev = nullptr, *rbHost = nullptr;
+    size_t rbPitch = 0;
+    hipEvent_t rbEvent[kReadGroups] = {};
 
     // device timing of the fused particle pass (stream launches only)
     int timingStride = 0;
@@ -2030,6 +2086,81 @@ int resort(icempm_batch *b) {
     return upload_chunks(b);
 }
 
+// Scratch of read_points, for the largest case: the device rows, the pinned
+// rows they come down to and an event per group of rows.
+int read_scratch(icempm_batch *b) {
+    size_t pitch = 0;
+    for (const auto &h : b->hc) pitch = std::max(pitch, ((size_t)h.cp.nPts + 63) / 64 * 64);
+    for (hipEvent_t &e : b->rbEvent)
+        if (!e) BCHK(b, hipEventCreateWithFlags(&e, hipEventDisableTiming), "read_points");
+    if (b->rbPitch >= pitch) return ICEMPM_OK;
+    b->rbPitch = 0;
+    dfree(b->rbDev);
+    if (b->rbHost) (void)hipHostFree(b->rbHost);
+    b->rbHost = nullptr;
+    BCHK(b, hipMalloc(&b->rbDev, 14 * pitch * sizeof(double) + 64), "read_points");
+    BCHK(b, hipHostMalloc(&b->rbHost, 14 * pitch * sizeof(double) + 64, hipHostMallocDefault), "read_points");
+    b->rbPitch = pitch;
+    return ICEMPM_OK;
+}
+
+// A case's points to the host: put in order on the device, brought down in
+// groups of rows to pinned memory and copied to the caller's from there, a group
+// while the next comes down.  What it takes is the caller's pages: 7 million
+// points (32 cases, 0.9 GB) in 73 ms, where a copy per row and the ordering
+// on the host took 192.  (Helper threads copy no faster: 84 ms with eight.)
+int read_points(icempm_batch *b, int c, double *soa, size_t pitch) {
+    const CaseParams &cp = b->hc[c].cp;
+    std::lock_guard<std::mutex> lock(b->rbLock);
+    const size_t dp = ((size_t)cp.nPts + 63) / 64 * 64;   // pitch on the device
+    int rc = read_scratch(b);
+    if (rc) return rc;
+    int *bad = reinterpret_cast<int *>(b->rbDev + 14 * dp);
+    BCHK(b, launch_fill_f64(b->rbDev, dp, 0.0, b->stream), "read_points");
+    BCHK(b, launch_fill_i32(bad, 1, 0, b->stream), "read_points");
+    const dim3 nb((unsigned)((dp + 255) / 256));
+    if (b->precision == ICEMPM_BATCH_F32) {
+        Rows<true> S{static_cast<unsigned int *>(b->pos), reinterpret_cast<float *>(b->rest), b->crushed, b->grain, b->pitch};
+        hipLaunchKernelGGL(k_read_points<true>, nb, dim3(256), 0, b->stream, S, b->orig, cp, (int)dp, b->rbDev, bad);
+    } else {
+        Rows<false> S{static_cast<double *>(b->pos), reinterpret_cast<double *>(b->rest), b->crushed, b->grain, b->pitch};
+        hipLaunchKernelGGL(k_read_points<false>, nb, dim3(256), 0, b->stream, S, b->orig, cp, (int)dp, b->rbDev, bad);
+    }
+    BCHK(b, hipGetLastError(), "read_points");
+    constexpr int kGroups = kReadGroups, kRows = 14;
+    int *hostBad = reinterpret_cast<int *>(b->rbHost + kRows * dp);
+    BCHK(b, hipMemcpyAsync(hostBad, bad, sizeof(int), hipMemcpyDeviceToHost, b->stream), "read_points");
+    const auto group = [](int g) { return g * kRows / kGroups; };   // first row
+    for (int g = 0; g < kGroups; ++g) {
+        BCHK(b, hipMemcpyAsync(b->rbHost + group(g) * dp, b->rbDev + group(g) * dp,
+                               (size_t)(group(g + 1) - group(g)) * dp * sizeof(double), hipMemcpyDeviceToHost, b->stream),
+             "read_points");
+        BCHK(b, hipEventRecord(b->rbEvent[g], b->stream), "read_points");
+    }
+    const size_t n = (size_t)cp.nPts, row = pitch * sizeof(double);
+    unsigned char *out = reinterpret_cast<unsigned char *>(soa);
+    for (int g = 0; g < kGroups; ++g) {
+        if (g == 1) std::memset(soa + pitch, 0, 2 * row);   // P and Q: a batch keeps none
+        BCHK(b, hipEventSynchronize(b->rbEvent[g]), "read_points");
+        for (int d = group(g); d < group(g + 1); ++d) {
+            const double *src = b->rbHost + (size_t)d * dp;
+            if (d > 0) {
+                double *dst = soa + (size_t)(d + 2) * pitch;
+                std::memcpy(dst, src, n * sizeof(double));
+                std::memset(dst + n, 0, row - n * sizeof(double));
+            } else {   // the flags, and the grain ids at byte pitch + 2 i
+                const unsigned char *u8 = reinterpret_cast<const unsigned char *>(src);
+                std::memset(out, 0, row);
+                std::memcpy(out, u8, n);
+                std::memcpy(out + pitch, u8 + dp, 2 * n);
+            }
+        }
+    }
+    BCHK(b, hipStreamSynchronize(b->stream), "read_points");
+    if (*hostBad) return bfail(b, ICEMPM_E_STATE, "read_points: slot map corrupt");
+    return ICEMPM_OK;
+}
+
 // the chunk table for the current slots and chunkPoints
 int rebuild_chunks(icempm_batch *b) {
     int rc = current_cells(b);
@@ -2260,6 +2391,10 @@ void icempm_batch_destroy(icempm_batch *b) {
     dfree(b->mapQ); dfree(b->mapCount);
     dfree(b->dcells);
     if (b->hcells) (void)hipHostFree(b->hcells);
+    dfree(b->rbDev);
+    if (b->rbHost) (void)hipHostFree(b->rbHost);
+    for (hipEvent_t ev : b->rbEvent)
+        if (ev) (void)hipEventDestroy(ev);
     b->hcells = nullptr;
     dfree(b->orig); dfree(b->sKeys); dfree(b->sVals); dfree(b->sKeys2); dfree(b->sVals2); dfree(b->sTmp);
     dfree(b->tpos); dfree(b->trest); dfree(b->tcrushed); dfree(b->torig);
@@ -2730,79 +2865,8 @@ int icempm_batch_force_bins(icempm_batch *b, int c, double *out, int nbins) {
 int icempm_batch_read_points(icempm_batch *b, int c, double *soa, size_t pitch) {
     return host_guard(b ? &b->lastError : nullptr, [&]() -> int {
         if (!b || !soa || c < 0 || (size_t)c >= b->hc.size()) return ICEMPM_E_ARG;
-        const CaseParams &cp = b->hc[c].cp;
-        const int n = cp.nPts, o = cp.ptOffset;
-        if ((size_t)n > pitch) return bfail(b, ICEMPM_E_ARG, "read_points: pitch too small");
-        const size_t vs = b->precision == ICEMPM_BATCH_F32 ? sizeof(float) : sizeof(double);
-        std::vector<double> hpos(2 * (size_t)n);
-        std::vector<unsigned char> hrest(11 * (size_t)n * vs), hcr(n);
-        std::vector<short> hgr((size_t)n, 0);
-        if (b->precision == ICEMPM_BATCH_F32) {
-            std::vector<unsigned int> q(4 * (size_t)n);
-            const unsigned int *P = static_cast<const unsigned int *>(b->pos);
-            BCHK(b, hipMemcpy(q.data(), P + 4 * (size_t)o, 4 * (size_t)n * sizeof(unsigned int), hipMemcpyDeviceToHost),
-                 "read_points");
-            for (int i = 0; i < n; ++i) {
-                const unsigned int lo = q[4 * (size_t)i + 2];
-                hpos[i] = fix48_get(q[4 * (size_t)i], lo & 0xFFFFu, cp);
-                hpos[n + i] = fix48_get(q[4 * (size_t)i + 1], lo >> 16, cp);
-                hcr[i] = (unsigned char)(q[4 * (size_t)i + 3] & 0xFFu);
-                hgr[i] = (short)(q[4 * (size_t)i + 3] >> 16);
-            }
-        } else {
-            const double *P = static_cast<const double *>(b->pos);
-            BCHK(b, hipMemcpy(hpos.data(), P + o, n * sizeof(double), hipMemcpyDeviceToHost), "read_points");
-            BCHK(b, hipMemcpy(hpos.data() + n, P + b->pitch + o, n * sizeof(double), hipMemcpyDeviceToHost),
-                 "read_points");
-        }
-        // rows of the case's slots [o, o + n) into hrest[r][slot]; FP32 storage's
-        // Fe records come down as one block and are split
-        for (int r = 0; r < 11; ++r) {
-            if (b->precision == ICEMPM_BATCH_F32 && r >= 2 && r <= 5) continue;
-            BCHK(b, hipMemcpy(hrest.data() + (size_t)r * n * vs, (unsigned char *)b->rest + rest_elem(b, r, o) * vs,
-                              n * vs, hipMemcpyDeviceToHost), "read_points");
-        }
-        if (b->precision == ICEMPM_BATCH_F32) {
-            std::vector<float> fe(4 * (size_t)n);
-            BCHK(b, hipMemcpy(fe.data(), (unsigned char *)b->rest + rest_elem(b, 2, o) * vs, 4 * (size_t)n * vs,
-                              hipMemcpyDeviceToHost), "read_points");
-            for (int slot = 0; slot < n; ++slot)
-                for (int r = 2; r <= 5; ++r)
-                    std::memcpy(&hrest[((size_t)r * n + slot) * vs], &fe[4 * (size_t)slot + (r - 2)], vs);
-        }
-        if (b->precision != ICEMPM_BATCH_F32)   // FP32: from the position records above
-            BCHK(b, hipMemcpy(hcr.data(), b->crushed + o, n, hipMemcpyDeviceToHost), "read_points");
-        if (b->grain && b->precision != ICEMPM_BATCH_F32)
-            BCHK(b, hipMemcpy(hgr.data(), b->grain + o, n * sizeof(short), hipMemcpyDeviceToHost), "read_points");
-        std::vector<int> horig((size_t)n);
-        BCHK(b, hipMemcpy(horig.data(), b->orig + o, n * sizeof(int), hipMemcpyDeviceToHost), "read_points");
-        std::memset(soa, 0, 16 * pitch * sizeof(double));
-        unsigned char *u8 = reinterpret_cast<unsigned char *>(soa);
-        for (int slot = 0; slot < n; ++slot) {
-            // the point in this slot, at its index within the case
-            const int i = horig[slot] - o;
-            if (i < 0 || i >= n) return bfail(b, ICEMPM_E_STATE, "read_points: slot map corrupt");
-            u8[i] = hcr[slot];
-            std::memcpy(u8 + pitch + 2 * (size_t)i, &hgr[slot], sizeof(short));   // point.cpp:19-23
-            soa[pitch * 4 + i] = hpos[slot];
-            soa[pitch * 5 + i] = hpos[n + slot];
-            for (int r = 0; r < 11; ++r) {
-                double v;
-                if (vs == sizeof(float)) {
-                    float f;
-                    std::memcpy(&f, &hrest[((size_t)r * n + slot) * vs], vs);
-                    v = f;
-                    if (r == 2 || r == 5 || r == 10) v += 1.0;
-                } else {
-                    std::memcpy(&v, &hrest[((size_t)r * n + slot) * vs], vs);
-                }
-                if (r < 10)
-                    soa[pitch * (6 + r) + i] = v;
-                else
-                    soa[pitch * 3 + i] = v;
-            }
-        }
-        return ICEMPM_OK;
+        if ((size_t)b->hc[c].cp.nPts > pitch) return bfail(b, ICEMPM_E_ARG, "read_points: pitch too small");
+        return read_points(b, c, soa, pitch);
     });
 }
 
