@@ -307,27 +307,26 @@ int ensure_chunks(icempm_ctx *c) { return c->chunksDirty ? build_chunks(c) : ICE
 int ensure_ordered(icempm_ctx *c) {
     OrderedScratch &o = c->ord;
     const size_t N = (size_t)c->prms.nPts, G = (size_t)c->prms.GridTotal;
-    if (o.nPts < N || !o.contrib) {
-        dfree(o.contrib); dfree(o.cnode); dfree(o.list);
+    if (o.nPts < N || !o.next) {
+        dfree(o.rec); dfree(o.next);
         const size_t n = N < 1 ? 1 : N;
-        HIPCHK(c, hipMalloc(&o.contrib, 27 * n * sizeof(double)), "ordered scratch");
-        HIPCHK(c, hipMalloc(&o.cnode, 9 * n * sizeof(int)), "ordered scratch");
-        HIPCHK(c, hipMalloc(&o.list, 9 * n * sizeof(int)), "ordered scratch");
+        HIPCHK(c, hipMalloc(&o.rec, 8 * n * sizeof(double)), "ordered scratch");
+        HIPCHK(c, hipMalloc(&o.next, n * sizeof(int)), "ordered scratch");
         o.nPts = n;
     }
-    if (o.nGrid < G || !o.count) {
-        dfree(o.count); dfree(o.start); dfree(o.cursor); dfree(o.nodeBin); dfree(o.nodeF);
-        dfree(o.flags); dfree(o.cpos); dfree(o.contacts); dfree(o.scanTmp);
-        HIPCHK(c, hipMalloc(&o.count, (G + 1) * sizeof(int)), "ordered scratch");
-        HIPCHK(c, hipMalloc(&o.start, (G + 1) * sizeof(int)), "ordered scratch");
-        HIPCHK(c, hipMalloc(&o.cursor, (G + 1) * sizeof(int)), "ordered scratch");
-        HIPCHK(c, hipMalloc(&o.nodeBin, (G + 1) * sizeof(int)), "ordered scratch");
-        HIPCHK(c, hipMalloc(&o.nodeF, 2 * (G + 1) * sizeof(double)), "ordered scratch");
-        HIPCHK(c, hipMalloc(&o.flags, (G + 1) * sizeof(int)), "ordered scratch");
-        HIPCHK(c, hipMalloc(&o.cpos, (G + 1) * sizeof(int)), "ordered scratch");
-        HIPCHK(c, hipMalloc(&o.contacts, (G + 1) * sizeof(int)), "ordered scratch");
-        HIPCHK(c, hipMalloc(&o.scanTmp, scan_tmp_ints(G + 1) * sizeof(int)), "ordered scratch");
+    if (o.nGrid < G || !o.nodeF) {
+        dfree(o.bucket); dfree(o.cells[0]); dfree(o.cells[1]); dfree(o.nodeBin); dfree(o.nodeF);
+        HIPCHK(c, hipMalloc(&o.bucket, kCellCap * G * sizeof(int)), "ordered scratch");
+        for (int2 *&cells : o.cells) HIPCHK(c, hipMalloc(&cells, G * sizeof(int2)), "ordered scratch");
+        HIPCHK(c, hipMalloc(&o.nodeBin, G * sizeof(int)), "ordered scratch");
+        HIPCHK(c, hipMalloc(&o.nodeF, 2 * G * sizeof(double)), "ordered scratch");
         o.nGrid = G;
+        o.cleared = 0;
+    }
+    if (o.cleared != G) {   // a P2G clears for the next one of the same grid
+        for (int2 *cells : o.cells)
+            HIPCHK(c, launch_fill_i32(reinterpret_cast<int *>(cells), 2 * o.nGrid, 0, c->stream), "ordered scratch");
+        o.cleared = G;
     }
     return ICEMPM_OK;
 }
@@ -338,9 +337,8 @@ void free_all(icempm_ctx *c) {
     dfree(c->perm); dfree(c->bandStart); dfree(c->recs); dfree(c->rows); dfree(c->caseDev);
     dfree(c->keys); dfree(c->vals); dfree(c->keys2); dfree(c->vals2); dfree(c->sortTmp);
     OrderedScratch &o = c->ord;
-    dfree(o.contrib); dfree(o.cnode); dfree(o.count); dfree(o.start); dfree(o.cursor);
-    dfree(o.list); dfree(o.nodeBin); dfree(o.nodeF); dfree(o.flags); dfree(o.cpos);
-    dfree(o.contacts); dfree(o.scanTmp);
+    dfree(o.rec); dfree(o.next); dfree(o.bucket); dfree(o.cells[0]); dfree(o.cells[1]);
+    dfree(o.nodeBin); dfree(o.nodeF);
     o = OrderedScratch{};
     hfree(c->hostPts); hfree(c->hostForce);
     c->histCap = 0; c->chunkCap = 0;
@@ -725,7 +723,7 @@ int icempm_p2g(icempm_ctx *c) {
         const KParams k = make_kparams(c);
         if (c->mode == ICEMPM_MODE_ORDERED) {
             if ((rc = ensure_ordered(c))) return rc;
-            HIPCHK(c, ordered_p2g(k, c->gridA, c->ord, c->stream), "cuda_p2g");
+            HIPCHK(c, ordered_p2g(k, c->gridA, c->ord, false, 0, 0, c->stream), "cuda_p2g");
             return ICEMPM_OK;
         }
         if ((rc = ensure_chunks(c))) return rc;
@@ -743,7 +741,8 @@ int icempm_update_nodes(icempm_ctx *c, double indenter_x, double indenter_y) {
             if ((rc = ensure_ordered(c))) return rc;
             HIPCHK(c, launch_update(k, c->gridA, indenter_x, indenter_y, nullptr, nullptr, true,
                                     c->ord.nodeBin, c->ord.nodeF, c->stream), "cuda_update_nodes");
-            HIPCHK(c, ordered_fold_forces(k, c->ord, nullptr, c->stream), "cuda_update_nodes");
+            HIPCHK(c, ordered_fold_forces(k, c->ord, nullptr, indenter_x, indenter_y, c->stream),
+                   "cuda_update_nodes");
             return ICEMPM_OK;
         }
         HIPCHK(c, launch_update(k, c->gridA, indenter_x, indenter_y, nullptr, nullptr, false, nullptr,
@@ -811,12 +810,8 @@ int icempm_run_substeps(icempm_ctx *c, int first_step, int n, double *t,
             double *h2 = c->hist + 2 * (size_t)i;
             const int timeIt = c->timing && (i % c->timingStride == 0);
             if (ordered) {
-                HIPCHK(c, launch_fill_f64(c->gridA, c->gp * kGridRows, 0.0, c->stream), "run_substeps");
-                k.pts = c->pts;
-                HIPCHK(c, ordered_p2g(k, c->gridA, c->ord, c->stream), "run_substeps");
-                HIPCHK(c, launch_update(k, c->gridA, ix, indenter_y, nullptr, nullptr, true,
-                                        c->ord.nodeBin, c->ord.nodeF, c->stream), "run_substeps");
-                HIPCHK(c, ordered_fold_forces(k, c->ord, h2, c->stream), "run_substeps");
+                HIPCHK(c, ordered_p2g(k, c->gridA, c->ord, true, ix, indenter_y, c->stream), "run_substeps");
+                HIPCHK(c, ordered_fold_forces(k, c->ord, h2, ix, indenter_y, c->stream), "run_substeps");
                 if ((rc = launch_particles_timed(c, k, true, false, c->gridA, nullptr, rec, timeIt)))
                     return rc;
             } else {

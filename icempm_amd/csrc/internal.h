@@ -52,25 +52,30 @@ hipError_t launch_update(const KParams &k, double *grid, double ix, double iy, d
                          double *zeroGrid, bool ordered, int *nodeBin, double *nodeF,
                          hipStream_t s);
 
-// ORDERED-mode P2G: contributions in particle order per node.
+// ORDERED mode: contributions in particle order per node.  cells[0] and cells[1]
+// (in turn, see flip) count the points of every base cell and chain those past
+// kCellCap; the one not in use is zero.
+constexpr int kCellCap = 16;
 struct OrderedScratch {
-    double *contrib = nullptr;   // 27 doubles per particle
-    int *cnode = nullptr;        // 9 node ids per particle (-1: none)
-    int *count = nullptr;        // gridTotal + 1
-    int *start = nullptr;        // gridTotal + 1
-    int *cursor = nullptr;       // gridTotal
-    int *list = nullptr;         // 9 per particle
+    double *rec = nullptr;       // 8 doubles per particle
+    int *next = nullptr;         // chain of a crowded cell: point + 1, or 0
+    int *bucket = nullptr;       // kCellCap points per cell
+    int2 *cells[2] = {};         // {points, first of the chain + 1} per cell
+    int flip = 0;
     int *nodeBin = nullptr;      // gridTotal
     double *nodeF = nullptr;     // 2 per node
-    int *flags = nullptr;        // gridTotal + 1
-    int *cpos = nullptr;         // gridTotal + 1
-    int *contacts = nullptr;     // gridTotal
-    int *scanTmp = nullptr;      // scan scratch
-    size_t nPts = 0, nGrid = 0;
+    size_t nPts = 0, nGrid = 0, cleared = 0;
 };
-hipError_t ordered_p2g(const KParams &k, double *grid, OrderedScratch &o, hipStream_t s);
-hipError_t ordered_fold_forces(const KParams &k, OrderedScratch &o, double *hist2,
+// The P2G into grid; update: with the grid update, for an indenter at (ix, iy),
+// and the padding of the grid's rows cleared.
+hipError_t ordered_p2g(const KParams &k, double *grid, OrderedScratch &o, bool update, double ix, double iy,
+                       hipStream_t s);
+// The contact forces of the last update, with the indenter where it was.
+hipError_t ordered_fold_forces(const KParams &k, OrderedScratch &o, double *hist2, double ix, double iy,
                                hipStream_t s);
+
+hipError_t launch_hello(int *flag, hipStream_t s);
+hipError_t launch_copy(const double *src, double *dst, size_t n_doubles, hipStream_t s);
 
 // ---- batch.hip: the batches' substep kernel for one case ------------------------
 // One launch per substep: grid update, G2P and the next P2G, FP64, exact return
@@ -107,9 +112,6 @@ hipError_t leave(const Run &r);
 // hist2: this substep's force (added to); t: its time; step: its index in the run.
 hipError_t substep(const Run &r, const double *in, double *out, double *clear, double *hist2, double t, int step);
 }  // namespace single
-
-hipError_t launch_hello(int *flag, hipStream_t s);
-hipError_t launch_copy(const double *src, double *dst, size_t n_doubles, hipStream_t s);
 
 // ---- sort.hip -----------------------------------------------------------------
 // Exclusive scan of n ints (in and out may alias).  tmp must hold

@@ -5,9 +5,9 @@
 //   k_update<false>  grid update (FAST mode) with the indenter force reduced
 //       per workgroup in shared memory; also clears the next substep's grid.
 // ORDERED path (bit-reproducible):
-//   k_p2g_contrib / k_p2g_fill / k_p2g_fold  every node sums its
-//       contributions in increasing particle index;
-//   k_update<true> + k_bins_fold  the indenter force is summed in increasing
+//   k_point_records / k_node_fold  every node sums its contributions in
+//       increasing particle index (and, in a run, is updated at once);
+//   k_update<true>, k_bins_fold  the indenter force is summed in increasing
 //       node index.
 #include <climits>
 
@@ -85,6 +85,65 @@ hipError_t launch_hello(int *flag, hipStream_t s) {
 constexpr int kUpdBlock = 256;
 constexpr int kMaxLdsBins = 256;
 
+// A node of the given mass (not zero): v is its momentum, then its velocity; bin
+// and f are set where the indenter touches it.
+static __device__ __forceinline__ void node_update(const KParams &k, int idx, double mass, double ind_x, double ind_y,
+                                                   double &v0, double &v1, int &bin, double &f0, double &f1) {
+    const int nb = k.nbins;
+    const double dt = k.dt, h = k.h, V = k.indV;
+    const int gx = k.gridX, gy = k.gridY;
+    v0 = v0 / mass;
+    v1 = v1 / mass;
+    v1 = v1 - dt * k.gravity;
+    const double vmax = 0.5 * h / dt;
+    const double vn = sqrt(v0 * v0 + v1 * v1);
+    if (vn > vmax) {
+        v0 = v0 / vn * vmax;
+        v1 = v1 / vn * vmax;
+    }
+    const int ix = idx % gx;
+    const int iy = idx / gx;
+    double n0 = ix * h - ind_x;
+    double n1 = iy * h - ind_y;
+    if (n0 * n0 + n1 * n1 < k.indRsq) {
+        const double r0 = v0 - V;
+        const double r1 = v1 - 0.0;
+        const double z = n0 * n0 + n1 * n1;
+        if (z > 0) {
+            const double nz = sqrt(z);
+            n0 = n0 / nz;
+            n1 = n1 / nz;
+        }
+        const double vnr = r0 * n0 + r1 * n1;
+        if (vnr < 0) {
+            const double t0 = r0 - n0 * vnr;
+            const double t1 = r1 - n1 * vnr;
+            const double p0 = v0, p1 = v1;
+            v0 = V + t0;
+            v1 = 0.0 + t1;
+            f0 = (p0 - v0) * mass / dt;
+            f1 = (p1 - v1) * mass / dt;
+            double angle = atan2(n0, n1);
+            angle += kPi;
+            angle *= nb / (2 * kPi);
+            int index = (int)angle;
+            index = max(index, 0);
+            index = min(index, nb - 1);
+            bin = index;
+        }
+    }
+    if (iy <= 2) {
+        v0 = 0;
+        v1 = 0;
+    } else if (iy >= gy - 3 && v1 > 0) {
+        v1 = 0;
+    }
+    if (ix <= 2 && v0 < 0)
+        v0 = 0;
+    else if (ix >= gx - 3 && v0 > 0)
+        v0 = 0;
+}
+
 template <bool ORDERED>
 __global__ __launch_bounds__(kUpdBlock) void k_update(KParams k, double *__restrict__ grid,
                                                       double ind_x, double ind_y,
@@ -115,59 +174,8 @@ __global__ __launch_bounds__(kUpdBlock) void k_update(KParams k, double *__restr
         }
         const double mass = grid[idx];
         if (mass != 0) {
-            const double dt = k.dt, h = k.h, V = k.indV;
-            const int gx = k.gridX, gy = k.gridY;
             double v0 = grid[gp + idx], v1 = grid[2 * gp + idx];
-            v0 = v0 / mass;
-            v1 = v1 / mass;
-            v1 = v1 - dt * k.gravity;
-            const double vmax = 0.5 * h / dt;
-            const double vn = sqrt(v0 * v0 + v1 * v1);
-            if (vn > vmax) {
-                v0 = v0 / vn * vmax;
-                v1 = v1 / vn * vmax;
-            }
-            const int ix = idx % gx;
-            const int iy = idx / gx;
-            double n0 = ix * h - ind_x;
-            double n1 = iy * h - ind_y;
-            if (n0 * n0 + n1 * n1 < k.indRsq) {
-                const double r0 = v0 - V;
-                const double r1 = v1 - 0.0;
-                const double z = n0 * n0 + n1 * n1;
-                if (z > 0) {
-                    const double nz = sqrt(z);
-                    n0 = n0 / nz;
-                    n1 = n1 / nz;
-                }
-                const double vnr = r0 * n0 + r1 * n1;
-                if (vnr < 0) {
-                    const double t0 = r0 - n0 * vnr;
-                    const double t1 = r1 - n1 * vnr;
-                    const double p0 = v0, p1 = v1;
-                    v0 = V + t0;
-                    v1 = 0.0 + t1;
-                    f0 = (p0 - v0) * mass / dt;
-                    f1 = (p1 - v1) * mass / dt;
-                    double angle = atan2(n0, n1);
-                    angle += kPi;
-                    angle *= nb / (2 * kPi);
-                    int index = (int)angle;
-                    index = max(index, 0);
-                    index = min(index, nb - 1);
-                    bin = index;
-                }
-            }
-            if (iy <= 2) {
-                v0 = 0;
-                v1 = 0;
-            } else if (iy >= gy - 3 && v1 > 0) {
-                v1 = 0;
-            }
-            if (ix <= 2 && v0 < 0)
-                v0 = 0;
-            else if (ix >= gx - 3 && v0 > 0)
-                v0 = 0;
+            node_update(k, idx, mass, ind_x, ind_y, v0, v1, bin, f0, f1);
             grid[gp + idx] = v0;
             grid[2 * gp + idx] = v1;
         }
@@ -225,186 +233,348 @@ hipError_t launch_update(const KParams &k, double *grid, double ix, double iy, d
 }
 
 // ---------------------------------------------------------------------------
-// ORDERED P2G
-__global__ __launch_bounds__(256) void k_p2g_contrib(KParams k, double *__restrict__ contrib,
-                                                    int *__restrict__ cnode,
-                                                    int *__restrict__ count) {
+// ORDERED P2G, in two kernels: every point makes the record its contributions
+// follow from and enters its base cell's list; every node then collects the
+// points of its nine cells, puts them in order and sums.  What bounds it is
+// latency, the ~36 terms of a node being one chain: LAT
+struct Terms {   // a point's part of its contributions: weights, distances, affine momentum, momentum
+    double wx[3], wy[3], dx[3], dy[3], A00, A01, A10, A11, mv0, mv1;
+};
+static __device__ __forceinline__ void axis_terms(double fx, double h, double *w, double *d) {
+    // as stencil
+    const double v0 = 1.5 - fx, v1 = fx - 1.0, v2 = fx - 0.5;
+    w[0] = 0.5 * v0 * v0;
+    w[1] = 0.75 - v1 * v1;
+    w[2] = 0.5 * v2 * v2;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) d[i] = (i - fx) * h;
+}
+static __device__ __forceinline__ Terms point_terms(const double *__restrict__ rec, int pt, double h) {
+    const double2 *r = reinterpret_cast<const double2 *>(rec) + 4 * (size_t)pt;
+    const double2 f = r[0], a = r[1], b = r[2], mv = r[3];
+    Terms t;
+    axis_terms(f.x, h, t.wx, t.dx);
+    axis_terms(f.y, h, t.wy, t.dy);
+    t.A00 = a.x; t.A01 = a.y; t.A10 = b.x; t.A11 = b.y;
+    t.mv0 = mv.x; t.mv1 = mv.y;
+    return t;
+}
+static __device__ __forceinline__ void add_term(const Terms &t, int i, int j, double mass, double &m, double &x, double &y) {
+    const double W = t.wx[i] * t.wy[j], d0 = t.dx[i], d1 = t.dy[j];
+    m += W * mass;
+    x += W * (t.mv0 + (t.A00 * d0 + t.A01 * d1));
+    y += W * (t.mv1 + (t.A10 * d0 + t.A11 * d1));
+}
+
+// padGrid (may be null): the padding of its rows is cleared.
+__global__ __launch_bounds__(256) void k_point_records(KParams k, double *__restrict__ rec, int *__restrict__ bucket,
+                                                      int2 *__restrict__ cells, int *__restrict__ next,
+                                                      double *__restrict__ padGrid) {
     const int pt = blockIdx.x * blockDim.x + threadIdx.x;
+    if (padGrid && (size_t)k.gridTotal + pt < k.gp)
+        for (int r = 0; r < kGridRows; ++r) padGrid[r * k.gp + k.gridTotal + pt] = 0;
     if (pt >= k.nPts) return;
     const double *P = k.pts;
     const size_t pp = k.pp;
-    const int gx = k.gridX, gy = k.gridY;
     const double px = P[pp * kRowPosX + pt], py = P[pp * (kRowPosX + 1) + pt];
     const double vx = P[pp * kRowVelX + pt], vy = P[pp * (kRowVelX + 1) + pt];
     const double F00 = P[pp * (kRowFe00 + 0) + pt], F01 = P[pp * (kRowFe00 + 1) + pt];
     const double F10 = P[pp * (kRowFe00 + 2) + pt], F11 = P[pp * (kRowFe00 + 3) + pt];
     const double B00 = P[pp * (kRowBp00 + 0) + pt], B01 = P[pp * (kRowBp00 + 1) + pt];
     const double B10 = P[pp * (kRowBp00 + 2) + pt], B11 = P[pp * (kRowBp00 + 3) + pt];
-    int *cn = cnode + 9 * (size_t)pt;
     int bx, by;
-    double fx0, fx1, wx0, wx1, wx2, wy0, wy1, wy2;
-    if (!stencil(px, k.h_inv, bx, fx0, wx0, wx1, wx2) ||
-        !stencil(py, k.h_inv, by, fx1, wy0, wy1, wy2)) {
+    double fx0, fx1, w0, w1, w2;
+    if (!stencil(px, k.h_inv, bx, fx0, w0, w1, w2) || !stencil(py, k.h_inv, by, fx1, w0, w1, w2)) {
         flag_error(k);
-        for (int e = 0; e < 9; ++e) cn[e] = -1;
         return;
     }
     double t00, t01, t11;
     kirchhoff(F00, F01, F10, F11, k.mu, k.kappa, t00, t01, t11);
-    const double m = k.mass, h = k.h;
+    const double m = k.mass;
     const double sc = k.dt * k.vol * k.Dinv;
-    const double A00 = m * B00 - sc * t00;
-    const double A01 = m * B01 - sc * t01;
-    const double A10 = m * B10 - sc * t01;
-    const double A11 = m * B11 - sc * t11;
-    const double mv0 = vx * m, mv1 = vy * m;
-    double *co = contrib + 27 * (size_t)pt;
+    double2 *r = reinterpret_cast<double2 *>(rec) + 4 * (size_t)pt;
+    r[0] = make_double2(fx0, fx1);
+    r[1] = make_double2(m * B00 - sc * t00, m * B01 - sc * t01);
+    r[2] = make_double2(m * B10 - sc * t01, m * B11 - sc * t11);
+    r[3] = make_double2(vx * m, vy * m);
+    if (bx >= k.gridX - 2 || by >= k.gridY - 2) flag_error(k);   // nodes outside the grid take nothing
+    if (bx >= k.gridX || by >= k.gridY) return;
+    int *cell = reinterpret_cast<int *>(cells + (bx + by * k.gridX));
+    const int slot = atomicAdd(cell, 1);
+    if (slot < kCellCap)
+        bucket[kCellCap * (size_t)(bx + by * k.gridX) + slot] = pt;
+    else
+        next[pt] = atomicExch(cell + 1, pt + 1);
+}
+
+// A wavefront takes a tile of 8 x 8 nodes: the points of its 10 x 10 cells go to
+// LDS with their terms, every lane lists those of its node's nine cells in order
+// (cell by cell they come almost so: points are in cell order until they move)
+// and adds up.  Tiles of more points than kFoldPts, about 4.5 a cell, go by
+// quarters, and where those or a cell's bucket overflow, a node looks its points
+// up one after the other.
+constexpr int kTileN = 8, kFoldPts = 448, kFoldList = 4096;
+struct FoldLds {
+    Terms terms[kFoldPts];
+    int idx[kFoldPts];
+    unsigned short list[kFoldList];                    // entry e of lane t at e lanes + t: cell << 9 | place in idx
+    unsigned short ofs[(kTileN + 2) * (kTileN + 2) + 1];   // a cell's first place in idx
+    double res[kTileN * kTileN][3];
+};
+static_assert(kFoldPts < 512, "list entries hold a place in 9 bits");
+
+// The T x T nodes from (X0, Y0) of the tile at (TX, TY); false if they do not fit.
+static __device__ bool fold_tile(const KParams &k, FoldLds &L, const double *__restrict__ rec,
+                                 const int *__restrict__ bucket, const int2 *__restrict__ cells, int T, int X0, int Y0,
+                                 int TX, int TY) {
+    const int lane = threadIdx.x, E = T + 2, gx = k.gridX, gy = k.gridY;
+    // points per cell, two cells a lane
+    int n[2], sum = 0;
+    bool over = false;
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
+    for (int q = 0; q < 2; ++q) {
+        const int c = 2 * lane + q, X = X0 - 2 + c % E, Y = Y0 - 2 + c / E;
+        n[q] = c < E * E && X >= 0 && X < gx && Y >= 0 && Y < gy ? cells[X + Y * gx].x : 0;
+        over |= n[q] > kCellCap;
+        sum += n[q];
+    }
+    int inc = sum;
 #pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            const int e = i * 3 + j;
-            const double Wip = sel3(i, wx0, wx1, wx2) * sel3(j, wy0, wy1, wy2);
-            const double d0 = (i - fx0) * h;
-            const double d1 = (j - fx1) * h;
-            const double incV0 = Wip * (mv0 + (A00 * d0 + A01 * d1));
-            const double incV1 = Wip * (mv1 + (A10 * d0 + A11 * d1));
-            const double incM = Wip * m;
-            const int X = bx + i, Y = by + j;
-            if (X < 0 || Y < 0 || X >= gx || Y >= gy) {
-                flag_error(k);
-                cn[e] = -1;
-                continue;
+    for (int d = 1; d < 64; d <<= 1) {
+        const int v = __shfl_up(inc, d, 64);
+        if (lane >= d) inc += v;
+    }
+    const int total = __shfl(inc, 63, 64);
+    if (__ballot(over) || total > kFoldPts) return false;
+    __syncthreads();   // the tile before has been used
+    int at = inc - sum;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const int c = 2 * lane + q;
+        if (c <= E * E) L.ofs[c] = (unsigned short)at;
+        if (n[q] > 0) {
+            const int X = X0 - 2 + c % E, Y = Y0 - 2 + c / E;
+            const int *b = bucket + kCellCap * (size_t)(X + Y * gx);
+            for (int e = 0; e < n[q]; ++e) {   // in order
+                const int v = b[e];
+                int j = at + e;
+                for (; j > at && L.idx[j - 1] > v; --j) L.idx[j] = L.idx[j - 1];
+                L.idx[j] = v;
             }
-            const int node = X + Y * gx;
-            cn[e] = node;
-            co[3 * e + 0] = incM;
-            co[3 * e + 1] = incV0;
-            co[3 * e + 2] = incV1;
-            atomicAdd(&count[node], 1);
+            at += n[q];
         }
     }
-}
-
-__global__ void k_p2g_fill(const int *__restrict__ cnode, const int *__restrict__ start,
-                           int *__restrict__ cursor, int *__restrict__ list, size_t n9) {
-    const size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-    if (e >= n9) return;
-    const int node = cnode[e];
-    if (node < 0) return;
-    const int slot = start[node] + atomicAdd(&cursor[node], 1);
-    list[slot] = (int)e;
-}
-
-__global__ void k_p2g_fold(double *__restrict__ grid, size_t gp, const int *__restrict__ start,
-                           int *__restrict__ list, const double *__restrict__ contrib,
-                           int gridTotal) {
-    const int node = blockIdx.x * blockDim.x + threadIdx.x;
-    if (node >= gridTotal) return;
-    const int b = start[node], e = start[node + 1];
-    // insertion sort: the entries are (particle*9 + stencil slot), so the
-    // ascending order is the particle order
-    for (int i = b + 1; i < e; ++i) {
-        const int v = list[i];
-        int j = i - 1;
-        while (j >= b && list[j] > v) {
-            list[j + 1] = list[j];
-            --j;
+    __syncthreads();
+    for (int e = lane; e < total; e += 64) L.terms[e] = point_terms(rec, L.idx[e], k.h);
+    const int lanes = T * T, x = lane % T, y = lane / T;
+    const bool mine = lane < lanes;
+    int cnt = 0;
+    if (mine)
+        for (int r = 0; r < 3; ++r) {   // the cells of a row are next to each other
+            const int c = (y + r) * E + x;
+            cnt += L.ofs[c + 3] - L.ofs[c];
         }
-        list[j + 1] = v;
+    if (__ballot(cnt * lanes > kFoldList)) return false;
+    __syncthreads();
+    if (mine) {
+        unsigned short *list = L.list + lane;
+        int len = 0, last = -1;
+        for (int c9 = 0; c9 < 9; ++c9) {   // cells in order
+            const int c = (y + c9 / 3) * E + x + c9 % 3;
+            for (int p = L.ofs[c]; p < L.ofs[c + 1]; ++p) {
+                const int v = L.idx[p];
+                int j = len++;
+                if (v < last) {   // from another row or column: to its place
+                    for (; j > 0; --j) {
+                        const unsigned short o = list[(j - 1) * lanes];
+                        if (L.idx[o & 511] < v) break;
+                        list[j * lanes] = o;
+                    }
+                } else {
+                    last = v;
+                }
+                list[j * lanes] = (unsigned short)(c9 << 9 | p);
+            }
+        }
+        double m = 0.0, sx = 0.0, sy = 0.0;
+        for (int e = 0; e < len; ++e) {
+            const int o = list[e * lanes], c9 = o >> 9;
+            add_term(L.terms[o & 511], 2 - c9 % 3, 2 - c9 / 3, k.mass, m, sx, sy);
+        }
+        double *res = L.res[(Y0 - TY + y) * kTileN + X0 - TX + x];
+        res[0] = m;
+        res[1] = sx;
+        res[2] = sy;
     }
-    double m = 0.0, x = 0.0, y = 0.0;
-    for (int i = b; i < e; ++i) {
-        const double *c = contrib + 3 * (size_t)list[i];
-        m += c[0];
-        x += c[1];
-        y += c[2];
-    }
-    grid[node] = m;
-    grid[gp + node] = x;
-    grid[2 * gp + node] = y;
+    return true;
 }
 
-hipError_t ordered_p2g(const KParams &k, double *grid, OrderedScratch &o, hipStream_t s) {
-    hipError_t e;
-    const size_t G = (size_t)k.gridTotal, N = (size_t)k.nPts;
-    if ((e = launch_fill_i32(o.count, G + 1, 0, s)) != hipSuccess) return e;
-    if ((e = launch_fill_i32(o.cursor, G, 0, s)) != hipSuccess) return e;
-    if (N > 0) {
-        hipLaunchKernelGGL(k_p2g_contrib, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s, k,
-                           o.contrib, o.cnode, o.count);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
+// The same for crowded cells, in memory: the least index above the last, until there is none.
+static __device__ void fold_slow(const KParams &k, FoldLds &L, const double *__restrict__ rec,
+                                 const int *__restrict__ bucket, const int2 *__restrict__ cells,
+                                 const int *__restrict__ next, int T, int X0, int Y0, int TX, int TY) {
+    const int lane = threadIdx.x;
+    if (lane >= T * T) return;
+    const int x = lane % T, y = lane / T;
+    double m = 0.0, sx = 0.0, sy = 0.0;
+    for (int last = -1;;) {
+        int best = INT_MAX, cell = 0;
+        for (int c9 = 0; c9 < 9; ++c9) {
+            const int X = X0 + x - 2 + c9 % 3, Y = Y0 + y - 2 + c9 / 3;
+            if (X < 0 || X >= k.gridX || Y < 0 || Y >= k.gridY) continue;
+            const int c = X + Y * k.gridX;
+            const int2 h = cells[c];
+            const auto see = [&](int v) {
+                if (v > last && v < best) {
+                    best = v;
+                    cell = c9;
+                }
+            };
+            for (int e = 0; e < min(h.x, kCellCap); ++e) see(bucket[kCellCap * (size_t)c + e]);
+            for (int p = h.y; p > 0; p = next[p - 1]) see(p - 1);
+        }
+        if (best == INT_MAX) break;
+        add_term(point_terms(rec, best, k.h), 2 - cell % 3, 2 - cell / 3, k.mass, m, sx, sy);
+        last = best;
     }
-    if ((e = exclusive_scan(o.count, o.start, G + 1, o.scanTmp, s)) != hipSuccess) return e;
-    if (N > 0) {
-        hipLaunchKernelGGL(k_p2g_fill, dim3((unsigned)((9 * N + 255) / 256)), dim3(256), 0, s,
-                           o.cnode, o.start, o.cursor, o.list, 9 * N);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
+    double *res = L.res[(Y0 - TY + y) * kTileN + X0 - TX + x];
+    res[0] = m;
+    res[1] = sx;
+    res[2] = sy;
+}
+
+// UPDATE: the grid update of the node as well.  Clears the other list of cells
+// for the next P2G.
+template <bool UPDATE>
+__global__ __launch_bounds__(64) void k_node_fold(KParams k, double *__restrict__ grid, const double *__restrict__ rec,
+                                                  const int *__restrict__ bucket, const int2 *__restrict__ cells,
+                                                  int2 *__restrict__ cellsNext, const int *__restrict__ next,
+                                                  double ind_x, double ind_y, int *__restrict__ nodeBin,
+                                                  double *__restrict__ nodeF) {
+    __shared__ FoldLds L;
+    const int TX = (int)blockIdx.x * kTileN, TY = (int)blockIdx.y * kTileN;
+    if (!fold_tile(k, L, rec, bucket, cells, kTileN, TX, TY, TX, TY)) {
+        constexpr int T = kTileN / 2;
+        for (int q = 0; q < 4; ++q) {
+            const int X0 = TX + (q & 1) * T, Y0 = TY + (q >> 1) * T;
+            if (!fold_tile(k, L, rec, bucket, cells, T, X0, Y0, TX, TY))
+                fold_slow(k, L, rec, bucket, cells, next, T, X0, Y0, TX, TY);
+        }
     }
-    hipLaunchKernelGGL(k_p2g_fold, dim3((unsigned)((G + 255) / 256)), dim3(256), 0, s, grid,
-                       k.gp, o.start, o.list, o.contrib, k.gridTotal);
-    return hipGetLastError();
+    __syncthreads();
+    const int lane = threadIdx.x, X = TX + lane % kTileN, Y = TY + lane / kTileN;
+    if (X >= k.gridX || Y >= k.gridY) return;
+    const int idx = X + Y * k.gridX;
+    const double mass = L.res[lane][0];
+    double v0 = L.res[lane][1], v1 = L.res[lane][2];
+    if constexpr (UPDATE) {
+        int bin = -1;
+        double f0 = 0, f1 = 0;
+        if (mass != 0) node_update(k, idx, mass, ind_x, ind_y, v0, v1, bin, f0, f1);
+        nodeBin[idx] = bin;
+        nodeF[2 * (size_t)idx] = f0;
+        nodeF[2 * (size_t)idx + 1] = f1;
+    }
+    grid[idx] = mass;
+    grid[k.gp + idx] = v0;
+    grid[2 * k.gp + idx] = v1;
+    cellsNext[idx] = make_int2(0, 0);
+}
+
+hipError_t ordered_p2g(const KParams &k, double *grid, OrderedScratch &o, bool update, double ix, double iy,
+                       hipStream_t s) {
+    int2 *cells = o.cells[o.flip], *other = o.cells[o.flip ^ 1];
+    const int threads = k.nPts > 64 ? k.nPts : 64;   // 64: the rows' padding
+    hipLaunchKernelGGL(k_point_records, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, k, o.rec, o.bucket,
+                       cells, o.next, update ? grid : nullptr);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    const dim3 tiles((unsigned)((k.gridX + kTileN - 1) / kTileN), (unsigned)((k.gridY + kTileN - 1) / kTileN));
+    if (update)
+        hipLaunchKernelGGL(k_node_fold<true>, tiles, dim3(64), 0, s, k, grid, o.rec, o.bucket, cells, other, o.next, ix, iy,
+                           o.nodeBin, o.nodeF);
+    else
+        hipLaunchKernelGGL(k_node_fold<false>, tiles, dim3(64), 0, s, k, grid, o.rec, o.bucket, cells, other, o.next, ix, iy,
+                           o.nodeBin, o.nodeF);
+    if ((e = hipGetLastError()) == hipSuccess) o.flip ^= 1;
+    return e;
 }
 
 // ---------------------------------------------------------------------------
-// ORDERED indenter force: contact nodes compacted in node order, then each
-// bin (and the substep total) folded sequentially.
-__global__ void k_contact_flags(const int *__restrict__ nodeBin, int *__restrict__ flags, int G) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < G) flags[i] = nodeBin[i] >= 0 ? 1 : 0;
-    if (i == G) flags[i] = 0;
-}
-
-__global__ void k_contact_compact(const int *__restrict__ flags, const int *__restrict__ cpos,
-                                  int *__restrict__ contacts, int G) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < G && flags[i]) contacts[cpos[i]] = i;
-}
-
-__global__ void k_bins_fold(double *__restrict__ bins, int nb, const int *__restrict__ nodeBin,
-                            const double *__restrict__ nodeF, const int *__restrict__ contacts,
-                            const int *__restrict__ countPtr, double *__restrict__ hist2) {
+// ORDERED indenter force: each bin, and the substep's total, summed in node
+// order by one thread each over the nodes in contact.  One workgroup: it looks
+// only at the nodes around the disc, and leaves those in contact in LDS, 1024
+// nodes at a time.
+constexpr int kFoldBlock = 1024;
+__global__ __launch_bounds__(kFoldBlock) void k_bins_fold(double *__restrict__ bins, int nb, const int *__restrict__ nodeBin,
+                                                          const double *__restrict__ nodeF, int gx, int x0, int y0, int w,
+                                                          int h, double *__restrict__ hist2) {
+    __shared__ int bin[kFoldBlock], wave[kFoldBlock / 64];
+    __shared__ double f0[kFoldBlock], f1[kFoldBlock];
     const int t = threadIdx.x;
-    const int count = *countPtr;
+    const bool total = t == nb;
+    double a0 = 0.0, a1 = 0.0;
     if (t < nb) {
-        double a0 = bins[2 * t], a1 = bins[2 * t + 1];
-        for (int e = 0; e < count; ++e) {
-            const int i = contacts[e];
-            if (nodeBin[i] == t) {
-                a0 += nodeF[2 * (size_t)i];
-                a1 += nodeF[2 * (size_t)i + 1];
-            }
+        a0 = bins[2 * t];
+        a1 = bins[2 * t + 1];
+    }
+    const long nodes = (long)w * h;
+    for (long first = 0; first < nodes; first += kFoldBlock) {
+        const long e = first + t;
+        int b = -1, idx = 0;
+        if (e < nodes) {
+            idx = x0 + (int)(e % w) + (y0 + (int)(e / w)) * gx;
+            b = nodeBin[idx];
         }
+        const unsigned long long hit = __ballot(b >= 0);
+        if ((t & 63) == 0) wave[t >> 6] = __popcll(hit);
+        __syncthreads();
+        int at = __popcll(hit & ((1ull << (t & 63)) - 1ull)), count = 0;
+        for (int q = 0; q < kFoldBlock / 64; ++q) {
+            if (q < t >> 6) at += wave[q];
+            count += wave[q];
+        }
+        if (b >= 0) {
+            bin[at] = b;
+            f0[at] = nodeF[2 * (size_t)idx];
+            f1[at] = nodeF[2 * (size_t)idx + 1];
+        }
+        __syncthreads();
+        if (t <= nb)
+            for (int q = 0; q < count; ++q)
+                if (total || bin[q] == t) {
+                    a0 += f0[q];
+                    a1 += f1[q];
+                }
+        __syncthreads();
+    }
+    if (t < nb) {
         bins[2 * t] = a0;
         bins[2 * t + 1] = a1;
-    } else if (t == nb && hist2) {
-        double s0 = 0.0, s1 = 0.0;
-        for (int e = 0; e < count; ++e) {
-            const int i = contacts[e];
-            s0 += nodeF[2 * (size_t)i];
-            s1 += nodeF[2 * (size_t)i + 1];
-        }
-        hist2[0] = s0;
-        hist2[1] = s1;
+    } else if (total && hist2) {
+        hist2[0] = a0;
+        hist2[1] = a1;
     }
 }
 
-hipError_t ordered_fold_forces(const KParams &k, OrderedScratch &o, double *hist2,
+hipError_t ordered_fold_forces(const KParams &k, OrderedScratch &o, double *hist2, double ix, double iy,
                                hipStream_t s) {
-    hipError_t e;
-    const int G = k.gridTotal;
-    const unsigned nbk = (unsigned)((G + 1 + 255) / 256);
-    hipLaunchKernelGGL(k_contact_flags, dim3(nbk), dim3(256), 0, s, o.nodeBin, o.flags, G);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    if ((e = exclusive_scan(o.flags, o.cpos, (size_t)G + 1, o.scanTmp, s)) != hipSuccess)
-        return e;
-    hipLaunchKernelGGL(k_contact_compact, dim3(nbk), dim3(256), 0, s, o.flags, o.cpos,
-                       o.contacts, G);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    const int threads = ((k.nbins + 1 + 63) / 64) * 64;
-    if (threads > 1024) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_bins_fold, dim3(1), dim3(threads), 0, s, k.bins, k.nbins, o.nodeBin,
-                       o.nodeF, o.contacts, o.cpos + G, hist2);
+    if (k.nbins + 1 > kFoldBlock) return hipErrorInvalidValue;
+    // the nodes in contact lie within the disc; two nodes of margin for the rounding
+    const double R = sqrt(k.indRsq);
+    const auto range = [&](double c, int g, int &lo, int &n) {
+        const double a = floor((c - R) * k.h_inv) - 2, b = ceil((c + R) * k.h_inv) + 2;
+        lo = 0;
+        n = g;
+        if (!(a <= b)) return;   // not a number: all
+        lo = (int)fmin(fmax(a, 0.0), (double)(g - 1));
+        n = (int)fmin(fmax(b, 0.0), (double)(g - 1)) - lo + 1;
+    };
+    int x0, y0, w, h;
+    range(ix, k.gridX, x0, w);
+    range(iy, k.gridY, y0, h);
+    hipLaunchKernelGGL(k_bins_fold, dim3(1), dim3(kFoldBlock), 0, s, k.bins, k.nbins, o.nodeBin, o.nodeF, k.gridX, x0, y0, w,
+                       h, hist2);
     return hipGetLastError();
 }
 
