@@ -236,7 +236,12 @@ hipError_t launch_update(const KParams &k, double *grid, double ix, double iy, d
 // ORDERED P2G, in two kernels: every point makes the record its contributions
 // follow from and enters its base cell's list; every node then collects the
 // points of its nine cells, puts them in order and sums.  What bounds it is
-// latency, the ~36 terms of a node being one chain: LAT
+// latency: few workgroups, each a chain of LDS passes (counts and points 1.5 us,
+// order 6.5, lists 6.4, sums 3.9 at 60,000 points).  A substep there takes 45 us
+// of which the records 10 and the fold 25; through memory, with a counting sort
+// and an insertion sort per node, it took 249 (contributions 20, sort 60, fold
+// 165).  An insertion sort of each node's list in LDS took up to 20 us: the
+// points of one row of the load's order lie in two rows of cells.
 struct Terms {   // a point's part of its contributions: weights, distances, affine momentum, momentum
     double wx[3], wy[3], dx[3], dy[3], A00, A01, A10, A11, mv0, mv1;
 };
@@ -249,25 +254,27 @@ static __device__ __forceinline__ void axis_terms(double fx, double h, double *w
 #pragma unroll
     for (int i = 0; i < 3; ++i) d[i] = (i - fx) * h;
 }
-static __device__ __forceinline__ Terms point_terms(const double *__restrict__ rec, int pt, double h) {
-    const double2 *r = reinterpret_cast<const double2 *>(rec) + 4 * (size_t)pt;
-    const double2 f = r[0], a = r[1], b = r[2], mv = r[3];
+struct PointRec {   // what they follow from, 64 bytes
+    double2 f, a, b, mv;
+};
+static __device__ __forceinline__ Terms terms_of(const PointRec &r, double h) {
     Terms t;
-    axis_terms(f.x, h, t.wx, t.dx);
-    axis_terms(f.y, h, t.wy, t.dy);
-    t.A00 = a.x; t.A01 = a.y; t.A10 = b.x; t.A11 = b.y;
-    t.mv0 = mv.x; t.mv1 = mv.y;
+    axis_terms(r.f.x, h, t.wx, t.dx);
+    axis_terms(r.f.y, h, t.wy, t.dy);
+    t.A00 = r.a.x; t.A01 = r.a.y; t.A10 = r.b.x; t.A11 = r.b.y;
+    t.mv0 = r.mv.x; t.mv1 = r.mv.y;
     return t;
 }
-static __device__ __forceinline__ void add_term(const Terms &t, int i, int j, double mass, double &m, double &x, double &y) {
-    const double W = t.wx[i] * t.wy[j], d0 = t.dx[i], d1 = t.dy[j];
-    m += W * mass;
-    x += W * (t.mv0 + (t.A00 * d0 + t.A01 * d1));
-    y += W * (t.mv1 + (t.A10 * d0 + t.A11 * d1));
+// The contribution to node (i, j) of the stencil: mass (part 0) or momentum (1, 2).
+static __device__ __forceinline__ double term(const Terms &t, int i, int j, int part, double mass) {
+    const double W = t.wx[i] * t.wy[j];
+    if (part == 0) return W * mass;
+    const double d0 = t.dx[i], d1 = t.dy[j];
+    return part == 1 ? W * (t.mv0 + (t.A00 * d0 + t.A01 * d1)) : W * (t.mv1 + (t.A10 * d0 + t.A11 * d1));
 }
 
 // padGrid (may be null): the padding of its rows is cleared.
-__global__ __launch_bounds__(256) void k_point_records(KParams k, double *__restrict__ rec, int *__restrict__ bucket,
+__global__ __launch_bounds__(256) void k_point_records(KParams k, PointRec *__restrict__ rec, int *__restrict__ bucket,
                                                       int2 *__restrict__ cells, int *__restrict__ next,
                                                       double *__restrict__ padGrid) {
     const int pt = blockIdx.x * blockDim.x + threadIdx.x;
@@ -292,11 +299,8 @@ __global__ __launch_bounds__(256) void k_point_records(KParams k, double *__rest
     kirchhoff(F00, F01, F10, F11, k.mu, k.kappa, t00, t01, t11);
     const double m = k.mass;
     const double sc = k.dt * k.vol * k.Dinv;
-    double2 *r = reinterpret_cast<double2 *>(rec) + 4 * (size_t)pt;
-    r[0] = make_double2(fx0, fx1);
-    r[1] = make_double2(m * B00 - sc * t00, m * B01 - sc * t01);
-    r[2] = make_double2(m * B10 - sc * t01, m * B11 - sc * t11);
-    r[3] = make_double2(vx * m, vy * m);
+    rec[pt] = PointRec{make_double2(fx0, fx1), make_double2(m * B00 - sc * t00, m * B01 - sc * t01),
+                       make_double2(m * B10 - sc * t01, m * B11 - sc * t11), make_double2(vx * m, vy * m)};
     if (bx >= k.gridX - 2 || by >= k.gridY - 2) flag_error(k);   // nodes outside the grid take nothing
     if (bx >= k.gridX || by >= k.gridY) return;
     int *cell = reinterpret_cast<int *>(cells + (bx + by * k.gridX));
@@ -307,110 +311,152 @@ __global__ __launch_bounds__(256) void k_point_records(KParams k, double *__rest
         next[pt] = atomicExch(cell + 1, pt + 1);
 }
 
-// A wavefront takes a tile of 8 x 8 nodes: the points of its 10 x 10 cells go to
-// LDS with their terms, every lane lists those of its node's nine cells in order
-// (cell by cell they come almost so: points are in cell order until they move)
-// and adds up.  Tiles of more points than kFoldPts, about 4.5 a cell, go by
-// quarters, and where those or a cell's bucket overflow, a node looks its points
-// up one after the other.
-constexpr int kTileN = 8, kFoldPts = 448, kFoldList = 4096;
+// A workgroup takes a tile of 8 x 8 nodes: the points of its 10 x 10 cells, put in
+// order by counting the smaller ones, a bit mask of them per cell, a node's list
+// from the bits of its nine cells, and a wavefront per component that adds up.
+// Tiles of more points than kFoldPts, about 4.4 a cell, go by quarters, and
+// where those or a cell's bucket overflow, a node looks its points up one after
+// the other.
+constexpr int kTileN = 8, kTileNodes = kTileN * kTileN, kTileCells = (kTileN + 2) * (kTileN + 2);
+constexpr int kFoldPts = 440, kFoldWords = (kFoldPts + 63) / 64, kFoldList = 4096;
 struct FoldLds {
-    Terms terms[kFoldPts];
-    int idx[kFoldPts];
-    unsigned short list[kFoldList];                    // entry e of lane t at e lanes + t: cell << 9 | place in idx
-    unsigned short ofs[(kTileN + 2) * (kTileN + 2) + 1];   // a cell's first place in idx
-    double res[kTileN * kTileN][3];
+    union {
+        struct {
+            unsigned long long mask[kTileCells][kFoldWords];   // a cell's points, by their places in order
+            unsigned char bits[kFoldWords][kTileNodes];        // of a node, per word
+        };
+        struct {
+            Terms t;
+            double pad;   // 19 doubles: the places of a wavefront spread over the banks
+        } terms[kFoldPts];
+    };
+    __attribute__((aligned(16))) int idx[kFoldPts + 8];   // the points as found
+    unsigned char cell[2][kFoldPts];  // the cells of the points as found, and in order: column | row << 4
+    unsigned short list[kFoldList];   // entry e of node t at e nodes + t: its cell among the nine << 9 | place
+    int wave[2], over, crowded;
+    double res[3][kTileNodes];
 };
-static_assert(kFoldPts < 512, "list entries hold a place in 9 bits");
+static_assert(kFoldPts < 512 && kTileCells <= 128, "list entries hold a place in 9 bits; two wavefronts hold the cells");
 
 // The T x T nodes from (X0, Y0) of the tile at (TX, TY); false if they do not fit.
-static __device__ bool fold_tile(const KParams &k, FoldLds &L, const double *__restrict__ rec,
+static __device__ bool fold_tile(const KParams &k, FoldLds &L, const PointRec *__restrict__ rec,
                                  const int *__restrict__ bucket, const int2 *__restrict__ cells, int T, int X0, int Y0,
                                  int TX, int TY) {
-    const int lane = threadIdx.x, E = T + 2, gx = k.gridX, gy = k.gridY;
-    // points per cell, two cells a lane
-    int n[2], sum = 0;
-    bool over = false;
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-        const int c = 2 * lane + q, X = X0 - 2 + c % E, Y = Y0 - 2 + c / E;
-        n[q] = c < E * E && X >= 0 && X < gx && Y >= 0 && Y < gy ? cells[X + Y * gx].x : 0;
-        over |= n[q] > kCellCap;
-        sum += n[q];
+    const int t = threadIdx.x, lane = t & 63, E = T + 2, gx = k.gridX, gy = k.gridY;
+    // a cell a thread: its count, and the first of its points at the same time
+    int n = 0;
+    int4 head = make_int4(0, 0, 0, 0);
+    const int4 *b = nullptr;
+    if (t < E * E) {
+        const int X = X0 - 2 + t % E, Y = Y0 - 2 + t / E;
+        if (X >= 0 && X < gx && Y >= 0 && Y < gy) {
+            const size_t c = (size_t)X + (size_t)Y * gx;
+            b = reinterpret_cast<const int4 *>(bucket) + kCellCap / 4 * c;
+            n = cells[c].x;
+            head = b[0];
+        }
     }
-    int inc = sum;
+    int inc = n;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
         const int v = __shfl_up(inc, d, 64);
         if (lane >= d) inc += v;
     }
-    const int total = __shfl(inc, 63, 64);
-    if (__ballot(over) || total > kFoldPts) return false;
     __syncthreads();   // the tile before has been used
-    int at = inc - sum;
+    if (t < 128 && lane == 63) L.wave[t >> 6] = inc;
+    if (t == 0) L.over = L.crowded = 0;
+    for (int e = t; e < kTileCells * kFoldWords; e += 256) L.mask[0][e] = 0;
+    __syncthreads();
+    const int total = L.wave[0] + L.wave[1];
+    if (n > kCellCap) L.over = 1;
+    __syncthreads();
+    if (L.over || total > kFoldPts) return false;
+    const int at = inc - n + (t >= 64 ? L.wave[0] : 0);
+    for (int e = 0; e < n; ++e) {
+        if (e > 0 && (e & 3) == 0) head = b[e >> 2];
+        L.idx[at + e] = (e & 3) == 0 ? head.x : ((e & 3) == 1 ? head.y : ((e & 3) == 2 ? head.z : head.w));
+        L.cell[0][at + e] = (unsigned char)(t % E | t / E << 4);
+    }
+    if (t < 8) L.idx[total + t] = INT_MAX;
+    __syncthreads();
+    // the records of the points found at t and t + 256 are on their way while
+    // the lists are made
+    PointRec r[2];
+    int v[2], place[2] = {0, 0};
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
-        const int c = 2 * lane + q;
-        if (c <= E * E) L.ofs[c] = (unsigned short)at;
-        if (n[q] > 0) {
-            const int X = X0 - 2 + c % E, Y = Y0 - 2 + c / E;
-            const int *b = bucket + kCellCap * (size_t)(X + Y * gx);
-            for (int e = 0; e < n[q]; ++e) {   // in order
-                const int v = b[e];
-                int j = at + e;
-                for (; j > at && L.idx[j - 1] > v; --j) L.idx[j] = L.idx[j - 1];
-                L.idx[j] = v;
-            }
-            at += n[q];
+        const int e = t + 256 * q;
+        v[q] = e < total ? L.idx[e] : -1;
+        r[q] = rec[e < total ? v[q] : 0];
+    }
+#pragma unroll 2
+    for (int o = 0; o < total; o += 8) {
+        const int4 w0 = *reinterpret_cast<const int4 *>(&L.idx[o]), w1 = *reinterpret_cast<const int4 *>(&L.idx[o + 4]);
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+            place[q] += (w0.x < v[q]) + (w0.y < v[q]) + (w0.z < v[q]) + (w0.w < v[q]) + (w1.x < v[q]) + (w1.y < v[q]) +
+                        (w1.z < v[q]) + (w1.w < v[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const int e = t + 256 * q, p = place[q];
+        if (e >= total) continue;
+        const unsigned char c = L.cell[0][e];
+        L.cell[1][p] = c;
+        atomicOr(&L.mask[(c >> 4) * E + (c & 15)][p >> 6], 1ull << (p & 63));
+    }
+    __syncthreads();
+    const int nodes = T * T, words = (total + 63) >> 6;
+    unsigned long long mine[2] = {0, 0};   // item t (and t + 256): a word of a node's points
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const int e = t + 256 * q, node = e % nodes, w = e / nodes;
+        if (w >= words) continue;
+        const int c = node / T * E + node % T;
+#pragma unroll
+        for (int c9 = 0; c9 < 9; ++c9) mine[q] |= L.mask[c + c9 / 3 * E + c9 % 3][w];
+        L.bits[w][node] = (unsigned char)__popcll(mine[q]);
+    }
+    __syncthreads();
+    int len = 0;   // of the node lane's list
+    if (lane < nodes)
+        for (int w = 0; w < words; ++w) len += L.bits[w][lane];
+    if (len * nodes > kFoldList) L.crowded = 1;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const int e = t + 256 * q, node = e % nodes, w = e / nodes;
+        if (w >= words) continue;
+        int at = 0;
+        for (int p = 0; p < w; ++p) at += L.bits[p][node];
+        const int X = node % T, Y = node / T;
+        for (unsigned long long m = mine[q]; m; m &= m - 1, ++at) {
+            const int p = w * 64 + __builtin_ctzll(m), c = L.cell[1][p];
+            if (at * nodes < kFoldList)
+                L.list[at * nodes + node] = (unsigned short)((((c >> 4) - Y) * 3 + (c & 15) - X) << 9 | p);
         }
     }
     __syncthreads();
-    for (int e = lane; e < total; e += 64) L.terms[e] = point_terms(rec, L.idx[e], k.h);
-    const int lanes = T * T, x = lane % T, y = lane / T;
-    const bool mine = lane < lanes;
-    int cnt = 0;
-    if (mine)
-        for (int r = 0; r < 3; ++r) {   // the cells of a row are next to each other
-            const int c = (y + r) * E + x;
-            cnt += L.ofs[c + 3] - L.ofs[c];
-        }
-    if (__ballot(cnt * lanes > kFoldList)) return false;
+    if (L.crowded) return false;
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+        if (t + 256 * q < total) L.terms[place[q]].t = terms_of(r[q], k.h);
     __syncthreads();
-    if (mine) {
-        unsigned short *list = L.list + lane;
-        int len = 0, last = -1;
-        for (int c9 = 0; c9 < 9; ++c9) {   // cells in order
-            const int c = (y + c9 / 3) * E + x + c9 % 3;
-            for (int p = L.ofs[c]; p < L.ofs[c + 1]; ++p) {
-                const int v = L.idx[p];
-                int j = len++;
-                if (v < last) {   // from another row or column: to its place
-                    for (; j > 0; --j) {
-                        const unsigned short o = list[(j - 1) * lanes];
-                        if (L.idx[o & 511] < v) break;
-                        list[j * lanes] = o;
-                    }
-                } else {
-                    last = v;
-                }
-                list[j * lanes] = (unsigned short)(c9 << 9 | p);
-            }
-        }
-        double m = 0.0, sx = 0.0, sy = 0.0;
+    if (lane < nodes && t < 3 * 64) {
+        const unsigned short *list = L.list + lane;
+        const int part = t >> 6;
+        double sum = 0.0;
+#pragma unroll 4
         for (int e = 0; e < len; ++e) {
-            const int o = list[e * lanes], c9 = o >> 9;
-            add_term(L.terms[o & 511], 2 - c9 % 3, 2 - c9 / 3, k.mass, m, sx, sy);
+            const int o = list[e * nodes], c9 = o >> 9;
+            sum += term(L.terms[o & 511].t, 2 - c9 % 3, 2 - c9 / 3, part, k.mass);
         }
-        double *res = L.res[(Y0 - TY + y) * kTileN + X0 - TX + x];
-        res[0] = m;
-        res[1] = sx;
-        res[2] = sy;
+        L.res[part][(Y0 - TY + lane / T) * kTileN + X0 - TX + lane % T] = sum;
     }
     return true;
 }
 
 // The same for crowded cells, in memory: the least index above the last, until there is none.
-static __device__ void fold_slow(const KParams &k, FoldLds &L, const double *__restrict__ rec,
+static __device__ void fold_slow(const KParams &k, FoldLds &L, const PointRec *__restrict__ rec,
                                  const int *__restrict__ bucket, const int2 *__restrict__ cells,
                                  const int *__restrict__ next, int T, int X0, int Y0, int TX, int TY) {
     const int lane = threadIdx.x;
@@ -434,19 +480,23 @@ static __device__ void fold_slow(const KParams &k, FoldLds &L, const double *__r
             for (int p = h.y; p > 0; p = next[p - 1]) see(p - 1);
         }
         if (best == INT_MAX) break;
-        add_term(point_terms(rec, best, k.h), 2 - cell % 3, 2 - cell / 3, k.mass, m, sx, sy);
+        const Terms t = terms_of(rec[best], k.h);
+        const int i = 2 - cell % 3, j = 2 - cell / 3;
+        m += term(t, i, j, 0, k.mass);
+        sx += term(t, i, j, 1, k.mass);
+        sy += term(t, i, j, 2, k.mass);
         last = best;
     }
-    double *res = L.res[(Y0 - TY + y) * kTileN + X0 - TX + x];
-    res[0] = m;
-    res[1] = sx;
-    res[2] = sy;
+    const int node = (Y0 - TY + y) * kTileN + X0 - TX + x;
+    L.res[0][node] = m;
+    L.res[1][node] = sx;
+    L.res[2][node] = sy;
 }
 
 // UPDATE: the grid update of the node as well.  Clears the other list of cells
 // for the next P2G.
 template <bool UPDATE>
-__global__ __launch_bounds__(64) void k_node_fold(KParams k, double *__restrict__ grid, const double *__restrict__ rec,
+__global__ __launch_bounds__(256) void k_node_fold(KParams k, double *__restrict__ grid, const PointRec *__restrict__ rec,
                                                   const int *__restrict__ bucket, const int2 *__restrict__ cells,
                                                   int2 *__restrict__ cellsNext, const int *__restrict__ next,
                                                   double ind_x, double ind_y, int *__restrict__ nodeBin,
@@ -463,10 +513,10 @@ __global__ __launch_bounds__(64) void k_node_fold(KParams k, double *__restrict_
     }
     __syncthreads();
     const int lane = threadIdx.x, X = TX + lane % kTileN, Y = TY + lane / kTileN;
-    if (X >= k.gridX || Y >= k.gridY) return;
+    if (lane >= kTileNodes || X >= k.gridX || Y >= k.gridY) return;
     const int idx = X + Y * k.gridX;
-    const double mass = L.res[lane][0];
-    double v0 = L.res[lane][1], v1 = L.res[lane][2];
+    const double mass = L.res[0][lane];
+    double v0 = L.res[1][lane], v1 = L.res[2][lane];
     if constexpr (UPDATE) {
         int bin = -1;
         double f0 = 0, f1 = 0;
@@ -483,18 +533,19 @@ __global__ __launch_bounds__(64) void k_node_fold(KParams k, double *__restrict_
 
 hipError_t ordered_p2g(const KParams &k, double *grid, OrderedScratch &o, bool update, double ix, double iy,
                        hipStream_t s) {
+    PointRec *rec = reinterpret_cast<PointRec *>(o.rec);
     int2 *cells = o.cells[o.flip], *other = o.cells[o.flip ^ 1];
     const int threads = k.nPts > 64 ? k.nPts : 64;   // 64: the rows' padding
-    hipLaunchKernelGGL(k_point_records, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, k, o.rec, o.bucket,
+    hipLaunchKernelGGL(k_point_records, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, k, rec, o.bucket,
                        cells, o.next, update ? grid : nullptr);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const dim3 tiles((unsigned)((k.gridX + kTileN - 1) / kTileN), (unsigned)((k.gridY + kTileN - 1) / kTileN));
     if (update)
-        hipLaunchKernelGGL(k_node_fold<true>, tiles, dim3(64), 0, s, k, grid, o.rec, o.bucket, cells, other, o.next, ix, iy,
+        hipLaunchKernelGGL(k_node_fold<true>, tiles, dim3(256), 0, s, k, grid, rec, o.bucket, cells, other, o.next, ix, iy,
                            o.nodeBin, o.nodeF);
     else
-        hipLaunchKernelGGL(k_node_fold<false>, tiles, dim3(64), 0, s, k, grid, o.rec, o.bucket, cells, other, o.next, ix, iy,
+        hipLaunchKernelGGL(k_node_fold<false>, tiles, dim3(256), 0, s, k, grid, rec, o.bucket, cells, other, o.next, ix, iy,
                            o.nodeBin, o.nodeF);
     if ((e = hipGetLastError()) == hipSuccess) o.flip ^= 1;
     return e;
