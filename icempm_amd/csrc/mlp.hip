@@ -73,61 +73,6 @@ __global__ void k_mfma_probe(const float *A, const float *B, float *D, int K) {
     for (int i = 0; i < 4; ++i) D[(4 * g + i) * 16 + c] = acc[i];
 }
 
-// Per-wavefront scratch in shared memory (floats).
-struct WaveScratch {
-    float x[16][kIn];
-    float h1[16][kH];
-    float h2[16][kH];
-    float y[16][kOut];
-    float d2[16][kH];   // dL/d(pre-activation 2)
-    float d1[16][kH];   // dL/d(pre-activation 1)
-};
-
-// store a D tile (lane l: rows 4g+i, column c) into a row-major array
-template <int LD>
-static __device__ __forceinline__ void put(float (*dst)[LD], int n0, f4 v) {
-    const int l = threadIdx.x & 63, g = l >> 4, c = l & 15;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) dst[4 * g + i][n0 + c] = v[i];
-}
-
-// forward of one 16-row tile held in s.x; parameters P (float, shared or global)
-template <class PW>
-static __device__ __forceinline__ void forward16(WaveScratch &s, const PW &P) {
-    const int l = threadIdx.x & 63, g = l >> 4, c = l & 15;
-    for (int nt = 0; nt < kH / 16; ++nt) {
-        f4 acc = {0, 0, 0, 0};
-        acc = tile([&](int m, int k) { return s.x[m][k]; },
-                   [&](int k, int n) { return P[oW1 + (nt * 16 + n) * kIn + k]; }, kIn, acc);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[i] = tanhf(acc[i] + P[oB1 + nt * 16 + c]);
-        put<kH>(s.h1, nt * 16, acc);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    for (int nt = 0; nt < kH / 16; ++nt) {
-        f4 acc = {0, 0, 0, 0};
-        acc = tile([&](int m, int k) { return s.h1[m][k]; },
-                   [&](int k, int n) { return P[oW2 + (nt * 16 + n) * kH + k]; }, kH, acc);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[i] = tanhf(acc[i] + P[oB2 + nt * 16 + c]);
-        put<kH>(s.h2, nt * 16, acc);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    {
-        f4 acc = {0, 0, 0, 0};
-        acc = tile([&](int m, int k) { return s.h2[m][k]; },
-                   [&](int k, int n) { return P[oW3 + n * kH + k]; }, kH, acc);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[i] += P[oB3 + c];
-        put<kOut>(s.y, 0, acc);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    (void)g;
-}
-
 // Inference: rows of normalised inputs (n x 5) -> normalised outputs (n x 3),
 // by the same wavefront routine as the learned return map of the batch pass.
 __global__ __launch_bounds__(256) void k_mlp_infer(const unsigned short *__restrict__ wbf,
@@ -153,20 +98,103 @@ __global__ __launch_bounds__(256) void k_mlp_infer(const unsigned short *__restr
     }
 }
 
+// LDS of the gradient kernel: the weights and a tile's activations as BF16 bits,
+// every matrix stored so that a lane's operands of a product are one read (both
+// ways round where both are needed).  Rows of 64 are padded to 72 and rows of 16
+// to 20, so that the 16 rows of a fetch lie on different banks.
+constexpr int kLong = kH + 8, kShort = 16 + 4;
+struct GradWeights {
+    alignas(16) unsigned short W1[kH][kShort], W2[kH][kLong], W2t[kH][kLong], W3[kOut][kLong], W3t[kH][kShort];
+    float b1[kH], b2[kH], b3[kOut];
+};
+struct GradScratch {
+    alignas(16) unsigned short x[16][kShort], xt[kIn][kShort];
+    alignas(16) unsigned short h1[16][kLong], h1t[kH][kShort], h2[16][kLong], h2t[kH][kShort];
+    alignas(16) unsigned short y[16][kShort], yt[kOut][kShort];   // dL/dy
+    alignas(16) unsigned short d2[16][kLong], d2t[kH][kShort], d1t[kH][kShort];   // dL/d(pre-activation)
+    float f[16][kH + 16], yf[16][kOut + 4];   // d2, then d1, and dL/dy, for the biases
+};
+
+// One 16 x 16 tile: A row-major, B given by its columns (row n of B holds
+// B[..][n]), K = 16 or a multiple of 32.
+template <int K, int LDA, int LDB>
+static __device__ __forceinline__ f4 tile_of(const unsigned short (*A)[LDA], const unsigned short (*B)[LDB], f4 acc) {
+    const int l = threadIdx.x & 63, r = l & 15, g = l >> 4;
+    if constexpr (K == 16) {
+        const s4 av = *reinterpret_cast<const s4 *>(&A[r][4 * g]), bv = *reinterpret_cast<const s4 *>(&B[r][4 * g]);
+        return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc, 0, 0, 0);
+    } else {
+#pragma unroll
+        for (int k0 = 0; k0 < K; k0 += 32)
+            acc = mfma32(*reinterpret_cast<const s8 *>(&A[r][k0 + 8 * g]), *reinterpret_cast<const s8 *>(&B[r][k0 + 8 * g]),
+                         acc);
+        return acc;
+    }
+}
+// A D tile (lane l: rows 4g + i, column n0 + c) as BF16 bits into a row-major
+// array and its transpose.
+template <int LD>
+static __device__ __forceinline__ void put_bits(unsigned short (*rows)[LD], unsigned short (*cols)[kShort], int n0, f4 v) {
+    const int l = threadIdx.x & 63, g = l >> 4, c = l & 15;
+    s4 b;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        b[i] = (short)to_bf16(v[i]);
+        if (rows) rows[4 * g + i][n0 + c] = (unsigned short)b[i];
+    }
+    *reinterpret_cast<s4 *>(&cols[n0 + c][4 * g]) = b;
+}
+
 // Gradient of L = 1/(2B) sum_rows sum_{k<3} (y_k - t_k)^2 over rows
 // [r0, r0 + B): every wavefront accumulates its tiles' gradient in registers
-// and writes one partial vector (kParams floats) to part[wave].  Also adds
-// the tiles' loss to *loss.
-__global__ __launch_bounds__(256) void k_mlp_grad(const float *__restrict__ params,
-                                                  const float *__restrict__ X,
-                                                  const float *__restrict__ T, int r0, int B,
-                                                  float *__restrict__ part, float *__restrict__ loss) {
-    __shared__ WaveScratch ws[4];
-    __shared__ float P[kParams];
-    for (int e = threadIdx.x; e < kParams; e += 256) P[e] = params[e];
+// and writes one partial vector (kParams floats) to part[wave], and the tiles'
+// loss to lossPart[wave].  A step of 8192 rows is one tile a wavefront, so the
+// kernel takes what one tile's chain of products takes: 20 us, against 45 with
+// the operands in FP32 (converted at every use, 550 conversions a tile, most
+// of their reads 16 lanes on one bank).
+constexpr int kGradWaves = 2;   // per workgroup: 512 wavefronts cover the chip's 256 CUs
+__global__ __launch_bounds__(64 * kGradWaves) void k_mlp_grad(const float *__restrict__ params,
+                                                              const unsigned short *__restrict__ wbf,
+                                                              const float *__restrict__ X, const float *__restrict__ T,
+                                                              int r0, int B, float *__restrict__ part,
+                                                              float *__restrict__ lossPart) {
+    __shared__ GradScratch ws[kGradWaves];
+    __shared__ GradWeights P;
+    // the weights, eight at a time
+    const s8 *wv = reinterpret_cast<const s8 *>(wbf);
+    static_assert(oW1 % 8 == 0 && oW2 % 8 == 0 && oW3 % 8 == 0, "16-byte reads");
+    const auto halves = [](unsigned short *dst, s8 v) {   // rows of kShort are 8-byte aligned
+        *reinterpret_cast<s4 *>(dst) = s4{v[0], v[1], v[2], v[3]};
+        *reinterpret_cast<s4 *>(dst + 4) = s4{v[4], v[5], v[6], v[7]};
+    };
+    constexpr int kThreads = 64 * kGradWaves;
+    static_assert(kH * kIn / 8 == kThreads && kOut * kH / 8 == kThreads && kH * kH / 8 == 4 * kThreads, "loads per thread");
+    {
+        const int t = threadIdx.x;
+        const s8 v1 = wv[oW1 / 8 + t], v3 = wv[oW3 / 8 + t];
+        s8 v2[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v2[q] = wv[oW2 / 8 + q * kThreads + t];
+        halves(&P.W1[t >> 1][(t & 1) * 8], v1);
+        *reinterpret_cast<s8 *>(&P.W3[t >> 3][(t & 7) * 8]) = v3;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) P.W3t[(t & 7) * 8 + j][t >> 3] = (unsigned short)v3[j];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int r = (q * kThreads + t) >> 3, k = (t & 7) * 8;
+            *reinterpret_cast<s8 *>(&P.W2[r][k]) = v2[q];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) P.W2t[k + j][r] = (unsigned short)v2[q][j];
+        }
+    }
+    for (int e = threadIdx.x; e < kH; e += 64 * kGradWaves) {
+        P.b1[e] = params[oB1 + e];
+        P.b2[e] = params[oB2 + e];
+        if (e < kOut) P.b3[e] = params[oB3 + e];
+    }
     __syncthreads();
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63, g = l >> 4, c = l & 15;
-    WaveScratch &s = ws[w];
+    GradScratch &s = ws[w];
     const float invB = 1.f / (float)B;
     f4 gW1[4], gW2[16], gW3[4];
     float gb1[4], gb2[4], gb3 = 0;
@@ -179,93 +207,99 @@ __global__ __launch_bounds__(256) void k_mlp_grad(const float *__restrict__ para
     for (int i = 0; i < 16; ++i) gW2[i] = f4{0, 0, 0, 0};
     float lsum = 0;
     const int tiles = (B + 15) / 16;
-    const int wave = blockIdx.x * 4 + w, nwave = gridDim.x * 4;
+    const int wave = blockIdx.x * kGradWaves + w, nwave = gridDim.x * kGradWaves;
+    // column sums of f (lanes with g == 0 keep them)
+    const auto columns = [&](const float *f, int ld) {
+        float a = 0;
+        for (int m = g; m < 16; m += 4) a += f[m * ld + c];
+        a += __shfl_xor(a, 16, 64);
+        a += __shfl_xor(a, 32, 64);
+        return a;
+    };
     for (int t = wave; t < tiles; t += nwave) {
         for (int e = l; e < 16 * kIn; e += 64) {
             const int m = e / kIn, k = e % kIn, row = t * 16 + m;
-            s.x[m][k] = (row < B && k < kRealIn) ? X[(size_t)(r0 + row) * kRealIn + k] : 0.f;
+            const unsigned short v = to_bf16((row < B && k < kRealIn) ? X[(size_t)(r0 + row) * kRealIn + k] : 0.f);
+            s.x[m][k] = v;
+            s.xt[k][m] = v;
         }
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        forward16(s, P);
-        // dY (kept in s.y), zero for padded outputs and rows
-        for (int e = l; e < 16 * kOut; e += 64) {
-            const int m = e / kOut, k = e % kOut, row = t * 16 + m;
-            float d = 0;
-            if (row < B && k < kRealOut) {
-                d = s.y[m][k] - T[(size_t)(r0 + row) * kRealOut + k];
-                lsum += 0.5f * d * d;
-                d *= invB;
-            }
-            s.y[m][k] = d;
-        }
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        // layer 3: gW3[o][h] += sum_m dY[m][o] h2[m][h]; gb3[o] += sum_m dY[m][o]
-        for (int ht = 0; ht < 4; ++ht)
-            gW3[ht] = tile([&](int o, int m) { return s.y[m][o]; },
-                           [&](int m, int h) { return s.h2[m][ht * 16 + h]; }, 16, gW3[ht]);
-        // d2 = (dY W3) * (1 - h2^2)
-        for (int ht = 0; ht < 4; ++ht) {
-            f4 acc = {0, 0, 0, 0};
-            acc = tile([&](int m, int o) { return s.y[m][o]; },
-                       [&](int o, int h) { return P[oW3 + o * kH + ht * 16 + h]; }, 16, acc);
+        wave_fence();
+        f4 h1[4], h2[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float hv = s.h2[4 * g + i][ht * 16 + c];
-                acc[i] *= (1.f - hv * hv);
-            }
-            put<kH>(s.d2, ht * 16, acc);
-        }
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        // layer 2: gW2[o][h] += sum_m d2[m][o] h1[m][h]
-        for (int ot = 0; ot < 4; ++ot)
-            for (int ht = 0; ht < 4; ++ht)
-                gW2[ot * 4 + ht] = tile([&](int o, int m) { return s.d2[m][ot * 16 + o]; },
-                                        [&](int m, int h) { return s.h1[m][ht * 16 + h]; }, 16,
-                                        gW2[ot * 4 + ht]);
-        // d1 = (d2 W2) * (1 - h1^2)
-        for (int ht = 0; ht < 4; ++ht) {
-            f4 acc = {0, 0, 0, 0};
-            acc = tile([&](int m, int o) { return s.d2[m][o]; },
-                       [&](int o, int h) { return P[oW2 + o * kH + ht * 16 + h]; }, kH, acc);
+        for (int nt = 0; nt < 4; ++nt) {
+            h1[nt] = tile_of<kIn>(s.x, &P.W1[nt * 16], f4{0, 0, 0, 0});
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float hv = s.h1[4 * g + i][ht * 16 + c];
-                acc[i] *= (1.f - hv * hv);
-            }
-            put<kH>(s.d1, ht * 16, acc);
+            for (int i = 0; i < 4; ++i) h1[nt][i] = tanhf(h1[nt][i] + P.b1[nt * 16 + c]);
+            put_bits(s.h1, s.h1t, nt * 16, h1[nt]);
         }
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        // layer 1: gW1[o][k] += sum_m d1[m][o] x[m][k]
-        for (int ot = 0; ot < 4; ++ot)
-            gW1[ot] = tile([&](int o, int m) { return s.d1[m][ot * 16 + o]; },
-                           [&](int m, int k) { return s.x[m][k]; }, 16, gW1[ot]);
-        // biases: column sums (lanes with g == 0 keep them)
-        for (int i = 0; i < 4; ++i) {
-            float a = 0, b = 0;
-            for (int m = g; m < 16; m += 4) {
-                a += s.d1[m][i * 16 + c];
-                b += s.d2[m][i * 16 + c];
-            }
-            a += __shfl_xor(a, 16, 64);
-            a += __shfl_xor(a, 32, 64);
-            b += __shfl_xor(b, 16, 64);
-            b += __shfl_xor(b, 32, 64);
-            gb1[i] += a;
-            gb2[i] += b;
+        wave_fence();
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) {
+            h2[nt] = tile_of<kH>(s.h1, &P.W2[nt * 16], f4{0, 0, 0, 0});
+#pragma unroll
+            for (int i = 0; i < 4; ++i) h2[nt][i] = tanhf(h2[nt][i] + P.b2[nt * 16 + c]);
+            put_bits(s.h2, s.h2t, nt * 16, h2[nt]);
         }
+        wave_fence();
         {
-            float a = 0;
-            for (int m = g; m < 16; m += 4) a += s.y[m][c];
-            a += __shfl_xor(a, 16, 64);
-            a += __shfl_xor(a, 32, 64);
-            gb3 += a;
+            f4 y = tile_of<kH>(s.h2, P.W3, f4{0, 0, 0, 0});
+            // dY, zero for padded outputs and rows
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int row = t * 16 + 4 * g + i;
+                float d = 0;
+                if (row < B && c < kRealOut) {
+                    d = (y[i] + P.b3[c]) - T[(size_t)(r0 + row) * kRealOut + c];
+                    lsum += 0.5f * d * d;
+                    d *= invB;
+                }
+                y[i] = d;
+                s.yf[4 * g + i][c] = d;
+            }
+            put_bits(s.y, s.yt, 0, y);
         }
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+        wave_fence();
+        // layer 3: gW3[o][h] += sum_m dY[m][o] h2[m][h]; gb3[o] += sum_m dY[m][o];
+        // d2 = (dY W3) * (1 - h2^2)
+#pragma unroll
+        for (int ht = 0; ht < 4; ++ht) {
+            gW3[ht] = tile_of<16>(s.yt, &s.h2t[ht * 16], gW3[ht]);
+            f4 acc = tile_of<16>(s.y, &P.W3t[ht * 16], f4{0, 0, 0, 0});
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                acc[i] *= (1.f - h2[ht][i] * h2[ht][i]);
+                s.f[4 * g + i][ht * 16 + c] = acc[i];
+            }
+            put_bits(s.d2, s.d2t, ht * 16, acc);
+        }
+        gb3 += columns(&s.yf[0][0], kOut + 4);
+        wave_fence();
+        // layer 2: gW2[o][h] += sum_m d2[m][o] h1[m][h]; d1 = (d2 W2) * (1 - h1^2)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) gb2[i] += columns(&s.f[0][i * 16], kH + 16);
+#pragma unroll
+        for (int ot = 0; ot < 4; ++ot)
+#pragma unroll
+            for (int ht = 0; ht < 4; ++ht)
+                gW2[ot * 4 + ht] = tile_of<16>(&s.d2t[ot * 16], &s.h1t[ht * 16], gW2[ot * 4 + ht]);
+        wave_fence();
+#pragma unroll
+        for (int ht = 0; ht < 4; ++ht) {
+            f4 acc = tile_of<kH>(s.d2, &P.W2t[ht * 16], f4{0, 0, 0, 0});
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                acc[i] *= (1.f - h1[ht][i] * h1[ht][i]);
+                s.f[4 * g + i][ht * 16 + c] = acc[i];
+            }
+            put_bits<kLong>(nullptr, s.d1t, ht * 16, acc);
+        }
+        wave_fence();
+        // layer 1: gW1[o][k] += sum_m d1[m][o] x[m][k]
+#pragma unroll
+        for (int ot = 0; ot < 4; ++ot) gW1[ot] = tile_of<16>(&s.d1t[ot * 16], s.xt, gW1[ot]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) gb1[i] += columns(&s.f[0][i * 16], kH + 16);
+        wave_fence();
     }
     // write this wavefront's partial gradient
     float *out = part + (size_t)wave * kParams;
@@ -286,27 +320,46 @@ __global__ __launch_bounds__(256) void k_mlp_grad(const float *__restrict__ para
     }
     // the loss of this wavefront's rows
     for (int off = 32; off > 0; off >>= 1) lsum += __shfl_xor(lsum, off, 64);
-    if (l == 0) atomicAdd(loss, lsum);
+    if (l == 0) lossPart[wave] = lsum;
 }
 
 // grad = sum over the partial vectors; then one Adam step on the FP32
 // master parameters.  Parameters that are padding stay zero.
 // The BF16 copy used by inference is refreshed from the result.
 // A workgroup of 256 handles 64 parameters: its four wavefronts each sum a
-// quarter of the partial vectors (64 consecutive floats per load), then the
-// first wavefront adds the four sums and takes the step.
+// quarter of the partial vectors (64 consecutive floats per load, 32 loads in
+// flight: one by one they took 35 us, so they take 10), then the first
+// wavefront adds the four sums and takes the step.  One more wavefront adds up
+// the loss.
 __global__ __launch_bounds__(256) void k_mlp_adam(float *__restrict__ params, unsigned short *__restrict__ wbf,
                                                   float *__restrict__ mom1, float *__restrict__ mom2,
                                                   const float *__restrict__ part, int nparts,
                                                   float *__restrict__ grad, float lr, float b1, float b2,
-                                                  float eps, float c1, float c2) {
+                                                  float eps, float c1, float c2,
+                                                  const float *__restrict__ lossPart, float *__restrict__ loss) {
     __shared__ float qs[4][64];
     const int l = threadIdx.x & 63, q = threadIdx.x >> 6;
     const int i = blockIdx.x * 64 + l;
     float g4 = 0;
-    if (i < kParams)
-        for (int p = q; p < nparts; p += 4) g4 += part[(size_t)p * kParams + i];
+    if (i < kParams) {
+        constexpr int kAhead = 32;
+        int p = q;
+        for (; p + 4 * (kAhead - 1) < nparts; p += 4 * kAhead) {
+            float v[kAhead];
+#pragma unroll
+            for (int j = 0; j < kAhead; ++j) v[j] = part[(size_t)(p + 4 * j) * kParams + i];
+#pragma unroll
+            for (int j = 0; j < kAhead; ++j) g4 += v[j];
+        }
+        for (; p < nparts; p += 4) g4 += part[(size_t)p * kParams + i];
+    }
     qs[q][l] = g4;
+    if (blockIdx.x == 0 && q == 1) {
+        float s = 0;
+        for (int p = l; p < nparts; p += 64) s += lossPart[p];
+        for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+        if (l == 0) *loss = s;
+    }
     __syncthreads();
     if (q != 0 || i >= kParams) return;
     const float gsum = (qs[0][l] + qs[1][l]) + (qs[2][l] + qs[3][l]);
@@ -340,14 +393,14 @@ struct icempm_mlp {
     hipStream_t stream = nullptr;
     float *params = nullptr, *m1 = nullptr, *m2 = nullptr, *grad = nullptr, *part = nullptr;
     unsigned short *wbf = nullptr;   // params as BF16 bits
-    float *loss = nullptr;
+    float *loss = nullptr, *lossPart = nullptr;
     int nparts = 0;
     int t = 0;   // Adam step
     std::string lastError;
 };
 
 namespace {
-constexpr int kGradBlocks = 128;
+constexpr int kGradBlocks = 256;
 
 int mfail(icempm_mlp *m, hipError_t e, const char *tag) {
     if (m) m->lastError = std::string(tag) + ": " + hipGetErrorString(e);
@@ -367,7 +420,7 @@ int icempm_mlp_num_params(void) { return kParams; }
 int icempm_mlp_create(icempm_mlp **out, const float *init) {
     if (!out || !init) return ICEMPM_E_ARG;
     icempm_mlp *m = new icempm_mlp();
-    m->nparts = kGradBlocks * 4;
+    m->nparts = kGradBlocks * kGradWaves;
     hipError_t e = hipSetDevice(0);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipMalloc(&m->params, kParams * sizeof(float));
@@ -376,6 +429,7 @@ int icempm_mlp_create(icempm_mlp **out, const float *init) {
     if (e == hipSuccess) e = hipMalloc(&m->grad, kParams * sizeof(float));
     if (e == hipSuccess) e = hipMalloc(&m->part, (size_t)m->nparts * kParams * sizeof(float));
     if (e == hipSuccess) e = hipMalloc(&m->loss, sizeof(float));
+    if (e == hipSuccess) e = hipMalloc(&m->lossPart, (size_t)m->nparts * sizeof(float));
     if (e == hipSuccess) e = hipMalloc(&m->wbf, kParams * sizeof(unsigned short));
     if (e == hipSuccess) e = hipMemcpy(m->params, init, kParams * sizeof(float), hipMemcpyHostToDevice);
     std::vector<unsigned short> wb(kParams);
@@ -395,7 +449,7 @@ int icempm_mlp_create(icempm_mlp **out, const float *init) {
 void icempm_mlp_destroy(icempm_mlp *m) {
     if (!m) return;
     if (m->stream) (void)hipStreamSynchronize(m->stream);
-    for (float *p : {m->params, m->m1, m->m2, m->grad, m->part, m->loss})
+    for (float *p : {m->params, m->m1, m->m2, m->grad, m->part, m->loss, m->lossPart})
         if (p) (void)hipFree(p);
     if (m->wbf) (void)hipFree(m->wbf);
     if (m->stream) (void)hipStreamDestroy(m->stream);
@@ -412,23 +466,35 @@ int icempm_mlp_get_params(icempm_mlp *m, float *out) {
 
 const float *icempm_mlp_device_params(const icempm_mlp *m) { return m ? m->params : nullptr; }
 
-// X: n x 5 normalised inputs, T: n x 3 normalised targets (device pointers).
-// Gradient over rows [r0, r0+B) into *grad_out (host, may be NULL) and the
-// mean loss; lr > 0 also takes one Adam step.
-int icempm_mlp_step(icempm_mlp *m, const float *X, const float *T, int r0, int B, float lr,
-                    float *grad_out, float *loss_out) {
-    if (!m || !X || !T || B <= 0 || r0 < 0) return ICEMPM_E_ARG;
-    MCHK(m, icempm::launch_fill_i32(reinterpret_cast<int *>(m->loss), 1, 0, m->stream), "mlp step");
-    hipLaunchKernelGGL(k_mlp_grad, dim3(kGradBlocks), dim3(256), 0, m->stream, m->params, X, T, r0, B,
-                       m->part, m->loss);
+}  // extern "C"
+
+namespace {
+// The kernels of a step: gradient over rows [r0, r0 + B) and, lr > 0, one Adam step.
+int enqueue_step(icempm_mlp *m, const float *X, const float *T, int r0, int B, float lr) {
+    hipLaunchKernelGGL(k_mlp_grad, dim3(kGradBlocks), dim3(64 * kGradWaves), 0, m->stream, m->params, m->wbf, X, T, r0, B,
+                       m->part, m->lossPart);
     MCHK(m, hipGetLastError(), "mlp grad");
     const float b1 = 0.9f, b2 = 0.999f;
     if (lr > 0) m->t += 1;
     const float c1 = 1 - std::pow(b1, (float)(m->t > 0 ? m->t : 1));
     const float c2 = 1 - std::pow(b2, (float)(m->t > 0 ? m->t : 1));
     hipLaunchKernelGGL(k_mlp_adam, dim3((kParams + 63) / 64), dim3(256), 0, m->stream, m->params, m->wbf,
-                       m->m1, m->m2, m->part, m->nparts, m->grad, lr, b1, b2, 1e-8f, c1, c2);
+                       m->m1, m->m2, m->part, m->nparts, m->grad, lr, b1, b2, 1e-8f, c1, c2, m->lossPart, m->loss);
     MCHK(m, hipGetLastError(), "mlp adam");
+    return ICEMPM_OK;
+}
+}  // namespace
+
+extern "C" {
+
+// X: n x 5 normalised inputs, T: n x 3 normalised targets (device pointers).
+// Gradient over rows [r0, r0+B) into *grad_out (host, may be NULL) and the
+// mean loss; lr > 0 also takes one Adam step.
+int icempm_mlp_step(icempm_mlp *m, const float *X, const float *T, int r0, int B, float lr,
+                    float *grad_out, float *loss_out) {
+    if (!m || !X || !T || B <= 0 || r0 < 0) return ICEMPM_E_ARG;
+    const int rc = enqueue_step(m, X, T, r0, B, lr);
+    if (rc) return rc;
     if (grad_out)
         MCHK(m, hipMemcpyAsync(grad_out, m->grad, kParams * sizeof(float), hipMemcpyDeviceToHost, m->stream),
              "mlp step");
@@ -575,9 +641,11 @@ int icempm_mlp_train(const float *X, const float *T, int n, int steps, int batch
             const int r0 = (it % windows) * B;
             const double a =
                 (double)lr * (0.05 + 0.95 * 0.5 * (1.0 + std::cos(3.141592653589793 * it / (steps > 0 ? steps : 1))));
-            float l = 0;
-            rc = icempm_mlp_step(m, dX, dT, r0, B, (float)a, nullptr, &l);
-            if (rc == ICEMPM_OK && trace && it % trace_every == 0) trace[it / trace_every] = l;
+            // only a step whose loss is traced is waited for
+            if (trace && it % trace_every == 0)
+                rc = icempm_mlp_step(m, dX, dT, r0, B, (float)a, nullptr, &trace[it / trace_every]);
+            else
+                rc = enqueue_step(m, dX, dT, r0, B, (float)a);
         }
         float full = 0;
         if (rc == ICEMPM_OK) rc = icempm_mlp_step(m, dX, dT, 0, n, 0.f, nullptr, &full);
