@@ -392,17 +392,15 @@ int launch_particles_timed(icempm_ctx *c, const KParams &k, bool g2p, bool p2g,
 }
 
 // Whether a run of n substeps goes by the substep kernel.  It needs two grids
-// more cleared and a copy of the points in band order, made and taken back: that
-// pays from about 32 substeps and, for the copies, one more per 8192 points.
-// us per substep without -> with it, in runs of 1000 (of 200):
-//   2,400 points   10.9 -> 7.8     400,000 points  24.4 -> 19.0 (32.7 -> 24.6)
-//   60,000 points  11.9 -> 7.8     800,000 points  36.3 -> 33.7 (48.2 -> 42.7)
-//   200,000 points 15.8 -> 11.3    1,204,000       48.1 -> 47.3 (63.7 -> 61.9)
-//   (21.3 -> 14.9)                 1,600,000       54.6 -> 55.8 (76.8 -> 74.1)
-// Beyond, where launches no longer count, the two kernels' smaller working sets
-// are the faster.
-constexpr int kSubstepKernelMaxPts = 1200000;
-bool substep_kernel_pays(int n, int nPts) { return nPts <= kSubstepKernelMaxPts && n >= 32 + nPts / 8192; }
+// more cleared and a copy of the points in the kernel's order, made and taken
+// back.  us per substep by the two kernels -> by this one, in runs of 16, 32, 128
+// and 1000:
+//       2,400 points   18.5 -> 13.5  14.9 -> 10.4  14.4 ->  8.3  10.9 ->  7.5
+//      60,000          27.1 -> 22.1  20.3 -> 14.8  16.7 ->  9.3  11.9 ->  7.3
+//     400,000          86.2 -> 83.3  55.6 -> 50.1  34.1 -> 24.9  24.4 -> 16.0
+//   1,600,000           285 ->  290   171 ->  168    88 ->   81  54.7 -> 47.7
+//   6,400,000          1133 -> 1140   688 ->  678   336 ->  311   220 ->  181
+bool substep_kernel_pays(int n, int nPts) { return n >= (nPts < 1000000 ? 16 : 32); }
 
 // The substep kernel's plan and arrays for the next run, the indenter starting
 // at (x0, y0); false where the run goes by the grid update and the particle
@@ -440,12 +438,13 @@ bool ensure_substep(icempm_ctx *c, double x0, double y0, single::Run &r) {
         dfree(c->bandStart);
         dfree(c->recs);
         ok = ensure_sort_scratch(c, (size_t)P.nPts) == ICEMPM_OK &&
-             single::plan(r, P.nPts, c->keys, c->vals, c->keys2, c->vals2, c->sortTmp, starts) == hipSuccess &&
+             single::plan(r, c->keys, c->vals, c->keys2, c->vals2, c->sortTmp, starts) == hipSuccess &&
              get(c->bandStart, starts.size() * sizeof(int)) && get(c->recs, starts.size() * single::kRecBytes) &&
-             upload(c->bandStart, starts.data(), starts.size() * sizeof(int)) &&
-             hipMemcpyAsync(c->perm, c->vals, (size_t)P.nPts * sizeof(int), hipMemcpyDeviceToDevice, c->stream) ==
-                 hipSuccess;
+             upload(c->bandStart, starts.data(), starts.size() * sizeof(int));
         c->nBand = (int)starts.size() - 1;
+        r.starts = c->bandStart;
+        r.nChunks = c->nBand;
+        ok = ok && single::slots(r, c->vals, c->perm) == hipSuccess;
         c->bandPoints = P.nPts;
         c->bandDirty = !ok;
     }

@@ -27,6 +27,7 @@
 #include <cmath>
 #include <cstring>
 #include <exception>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <system_error>
@@ -151,30 +152,18 @@ static __device__ __forceinline__ void stencil_cells(double xr, int &base, doubl
 
 // Point position of slot pt (both storage formats) as FP64; store it back,
 // and the value the stored form holds.
-template <bool NT>
 static __device__ __forceinline__ void pos_load(const double *pos, size_t pp, int pt, const CaseParams &,
                                                 double &x, double &y) {
     const unsigned u = (unsigned)pt;
-    if constexpr (NT) {
-        x = __builtin_nontemporal_load(at(pos, u));
-        y = __builtin_nontemporal_load(at(pos + pp, u));
-    } else {
-        x = *at(pos, u);
-        y = *at(pos + pp, u);
-    }
+    x = *at(pos, u);
+    y = *at(pos + pp, u);
 }
 typedef unsigned int prec4 __attribute__((ext_vector_type(4)));
 // FP32 storage: the slot's record, its coordinates in metres; returns its
 // last word (crushed flag in bits 0-7, grain id in bits 16-31)
-template <bool NT>
 static __device__ __forceinline__ unsigned pos_load(const unsigned int *pos, size_t, int pt, const CaseParams &cp,
                                                     double &x, double &y) {
-    const prec4 *rec = reinterpret_cast<const prec4 *>(pos) + pt;
-    prec4 v;
-    if constexpr (NT)
-        v = __builtin_nontemporal_load(rec);
-    else
-        v = *rec;
+    const prec4 v = reinterpret_cast<const prec4 *>(pos)[pt];
     x = fix48_get(v.x, v.z & 0xFFFFu, cp);
     y = fix48_get(v.y, v.z >> 16, cp);
     return v.w;
@@ -320,48 +309,81 @@ static __device__ __forceinline__ double yield_residual(const KParams &k, const 
     return fmax(fabs(qt - qlim) / k.iss, k.kappa * fabs(dm) / k.ics);
 }
 
-// A chunk: the up to 256 points of a workgroup, a wavefront a 64 of them, the
-// box of grid nodes their stencils touch, and in it the window of each
-// wavefront.  The workgroup keeps them in the record, renewing them every
+// A chunk: the up to 256 points of a workgroup and the box of grid nodes their
+// stencils touch.  The workgroup keeps the box in the record, renewing it every
 // kBoxEvery substeps (points move far less than a cell in that time; one that
-// has left takes the general paths).
+// has left it takes the general paths).
 struct __attribute__((aligned(16))) ChunkRec {
-    int beg, count;   // first slot, points
+    int beg;          // first slot
+    unsigned shape;   // FP32 storage: points; FP64: lanes per row | rows with one lane more << 8 | rows << 16
     int cs, gofs;     // the case and its first grid node
     unsigned dims;    // GridX | GridY << 16
     unsigned org;     // the box: first column | first row << 16
-    unsigned ext;     // columns | rows << 8 | tile stride << 16 (0: no box)
+    unsigned ext;     // columns | rows << 8 | tile stride << 16 | FP64: window stride << 24 (0: no box)
     unsigned inv;     // ceil(2^16 / columns): a node's row from its index in the box
-    unsigned win[4];  // the windows: first column | first row << 8 (both from the box's) | columns << 16 | rows << 24
+    unsigned win[4];  // FP32: the windows: first column | first row << 8 (both from the box's) | columns << 16 | rows << 24
 };
 constexpr int kBoxEvery = 8;
 
-// LDS of a workgroup: a window per wavefront for its P2G (three sums per
-// node), the tile of node velocities its G2P reads, and a patch per wavefront
-// for the velocities of kPatch points outside the box.  64 points in band
-// order, four to a cell, touch 10 x 4 nodes and 256 points 34 x 4; the space
-// (25.6 KB, for six workgroups a CU) holds more rows, for points that have moved
-// out of their band.
-constexpr int kWaveWin = 160, kTile = 384;   // nodes x row stride
+// The points of a chunk, FP32 storage: in band order, 64 a wavefront.  The four
+// lanes of a quad mostly hold the points of a cell and add up their
+// contributions before these reach the wavefront's window.  That keeps the sums
+// of a node in the order quad, wavefront, grid.
+//
+// FP64 storage: in rows of a wavefront each, as few as hold them and filled
+// evenly; slot s holds the point that band order puts at chunk_point(s, shape).
+// Consecutive points go to the same lane of consecutive rows, so that the 64
+// lanes of a wavefront hold different cells and their LDS atomics, 27 a point
+// into one window for the workgroup, go to different nodes (four lanes of one
+// cell at one node take five times as long).
+//
+// The latter takes fewer instructions (8 cases FP64, 671 thousand points: 22.6
+// us a substep, 25.0 in band order; 1.6 million points FP64: 50 and 51), but
+// adds the terms in another order.  FP64 points differ by rounding then; the rounding of FP32 storage and
+// the yield branches carry a study's points past 1e-5 of the other order's
+// within 4000 substeps in most runs, where two runs of one order mostly agree
+// to the bit.
+static __host__ __device__ inline unsigned chunk_shape(int n) {
+    const int rows = (n + 63) / 64;
+    return (unsigned)(n / rows) | (unsigned)(n % rows) << 8 | (unsigned)rows << 16;
+}
+static __host__ __device__ inline int chunk_count(unsigned shape) {
+    return (int)((shape & 0xFFu) * (shape >> 16) + (shape >> 8 & 0xFFu));
+}
+static __host__ __device__ inline int chunk_point(int slot, unsigned shape) {
+    const int lanes = (int)(shape & 0xFFu), more = (int)(shape >> 8 & 0xFFu), rows = (int)(shape >> 16);
+    const int wide = more * (lanes + 1);   // slots of the rows with one lane more
+    const int row = slot < wide ? slot / (lanes + 1) : more + (slot - wide) / lanes;
+    return rows * (slot - row * lanes - (row < more ? row : more)) + row;
+}
+
+// LDS of a workgroup: the windows of its P2G (three sums per node), the tile of
+// node velocities its G2P reads, and a patch per wavefront for the velocities of
+// kPatch points outside the box.  64 points in band order, four to a cell, touch
+// 10 x 4 nodes and 256 points 34 x 4; the space (25.6 KB with a window per
+// wavefront, 19.6 KB with one) holds more rows, for points that have moved out
+// of their band.
+constexpr int kWaveWin = 160, kWin = 384, kTile = 384;   // nodes x row stride
 constexpr int kWinCols = 40;
 constexpr int kPatch = 7;                // x 9 nodes: one load round of a wavefront
 constexpr int kChunkCols = 58;           // base cells a chunk may span: 60 columns of nodes
 
-// The row stride of a window: rows next to each other lie on different LDS
-// banks (a row of S doubles shifts them by 2 S of 64).
+// The row stride of a wavefront's window: rows next to each other lie on
+// different LDS banks (a row of S doubles shifts them by 2 S of 64).
 static __device__ __forceinline__ int win_stride(int w) { return w <= 16 ? 20 : (w <= 32 ? 36 : kWinCols); }
 
 // The box of the base cells [x0, x1] x [y0, y1] as a record's org, ext and
 // inv; false if it does not fit the space.  A tile row of T 16-byte entries, T
-// = 8 mod 16, puts the two cell rows of a band on different LDS banks; a
-// taller box packs its rows.
+// = 8 mod 16, and a window row of S doubles, S = 16 mod 32, put the two cell
+// rows of a band on different LDS banks; a taller box packs its rows.
 static __device__ __forceinline__ bool set_box(ChunkRec &r, int x0, int y0, int x1, int y1) {
     const int w = x1 + 3 - x0, h = y1 + 3 - y0;
     if (w > 128 || h > 128 || w * h > kTile) return false;
-    int T = ((w + 7) >> 4) * 16 + 8;
+    int T = ((w + 7) >> 4) * 16 + 8, S = ((w + 15) >> 5) * 32 + 16;
     if (T * h > kTile) T = w;
+    if (S * h > kWin) S = w;
     r.org = (unsigned)x0 | (unsigned)y0 << 16;
-    r.ext = (unsigned)w | (unsigned)h << 8 | (unsigned)T << 16;
+    r.ext = (unsigned)w | (unsigned)h << 8 | (unsigned)T << 16 | (unsigned)S << 24;
     r.inv = 65535u / (unsigned)w + 1u;
     return true;
 }
@@ -631,24 +653,18 @@ static __device__ __forceinline__ void quad_scatter(int lane, int e0, int S, dou
 // gridOut with one atomic per node and component; the workgroups from pGroups
 // on do the rest of the grid update (node_part).
 //
-// What bounds it is FP64 arithmetic: ~530 vector instructions per 64 points,
-// most of them FP64 at 4 cycles each (HBM is at a third of its rate).  Against
-// a grid update of its own, a particle pass that gathered from global memory
-// and found each wavefront's window anew (625 instructions), a substep of 32
-// cases / 6.98 million points went from 193 to 167 us (FP32 storage), of 12
-// cases / 81 thousand points from 18.4 to 8.9 us, of 8 cases / 671 thousand
-// points from 35 to 25 us (FP64, strengths per grain).  Making a node's
-// velocity in each of the ~2 workgroups that need it costs ~20 instructions per
-// 64 points; it saves a launch, the velocities' trip through memory and the
-// gathers' 6 to 18 loads a point.
-//
-// A window per wavefront, and the points in band order, keep the sums of each
-// node in the order quad, wavefront, grid.  One window per workgroup with the
-// points of a cell spread over its wavefronts (27 LDS atomics a point, none of
-// them at one address) takes 149 us, but adds the terms in another order: the
-// rounding of FP32 storage and the yield branches then carry a study's points
-// past 1e-5 of it within 4000 substeps in most runs, where two runs of this
-// order mostly agree to the bit.
+// What bounds it is instruction issue (660 vector instructions per 64 points in
+// FP32 storage, half of them FP64 at 4 cycles each; HBM is at half a copy's
+// rate) and, below ~100 thousand points, the launch and one chain of memory
+// latencies.  Against a grid update of its own and a particle pass that
+// gathered from global memory and found each wavefront's window anew, a substep
+// of 32 cases / 6.98 million points went from 193 to 167 us (FP32 storage), of
+// 12 cases / 81 thousand points from 18.4 to 9, of 8 cases / 671 thousand points
+// from 35 to 21 (FP64, strengths per grain).  Making a node's velocity in each
+// of the ~2 workgroups that need it costs ~50 instructions per 64 points; it
+// saves a launch, the velocities' trip through memory and the gathers' 6 to 18
+// loads a point.  Four or five wavefronts per SIMD are equally fast, six (80
+// registers) slower.
 //
 // The records, the grid and the point rows lead the arguments, which the
 // kernel receives preloaded in SGPRs.
@@ -659,7 +675,8 @@ __global__ __launch_bounds__(256, 5) void k_batch_substep(
     unsigned char *crushedRow, size_t pitch, double *__restrict__ gridOut, int4 *bounds, int *__restrict__ err,
     const short *__restrict__ grains, typename Rows<F32>::V *jpRow, const double *__restrict__ tTab, double t0, int step,
     NodeWork nw, LearnArgs la, MapQueue mq, int storeVB) {
-    __shared__ __attribute__((aligned(16))) double smem[4 * 3 * kWaveWin + 2 * kTile + 4 * (2 * 9 + 1) * kPatch];
+    constexpr int kWindows = 3 * (F32 ? 4 * kWaveWin : kWin);   // doubles
+    __shared__ __attribute__((aligned(16))) double smem[kWindows + 2 * kTile + 4 * (2 * 9 + 1) * kPatch];
     if constexpr (G2P) {
         if ((int)blockIdx.x >= pGroups) {
             node_part(nw, (int)blockIdx.x - pGroups, cases, gridIn, gpitch, bounds, tTab ? tTab[step] : t0, smem);
@@ -686,30 +703,53 @@ __global__ __launch_bounds__(256, 5) void k_batch_substep(
     V *__restrict__ R = S.rest;
     constexpr double fe0 = F32 ? 1.0 : 0.0;   // stored Fe = Fe - fe0 * I, Jp_inv - fe0
     // the wavefront's points: lanes of them (none past the last one)
-    const int lanes = rec.count - row * 64;
+    int lanes, first;
+    if constexpr (F32) {
+        lanes = (int)rec.shape - row * 64;
+        first = row * 64;
+    } else {
+        const int lanesRow = (int)(rec.shape & 0xFFu), more = (int)(rec.shape >> 8 & 0xFFu);
+        lanes = row < (int)(rec.shape >> 16) ? lanesRow + (row < more ? 1 : 0) : 0;
+        first = row * lanesRow + min(row, more);
+    }
     const bool valid = lane < lanes;
-    const int pt = rec.beg + row * 64 + lane;
+    const int pt = rec.beg + first + lane;
     const unsigned u = (unsigned)pt;
-    // the box with the tile, and the wavefront's window
+    // the box with the tile
     const int ox = (int)(rec.org & 0xFFFFu), oy = (int)(rec.org >> 16);
     const int bw = (int)(rec.ext & 0xFFu), bh = (int)(rec.ext >> 8 & 0xFFu), tS = (int)(rec.ext >> 16 & 0xFFu);
     const unsigned nodes = (unsigned)(bw * bh);
     // base cells whose stencil lies in the box and in the grid: [ox, ox + fw) x [oy, oy + fh)
     const unsigned fw = (unsigned)max(min(bw, gx - ox) - 2, 0), fh = (unsigned)max(min(bh, gy - oy) - 2, 0);
-    const unsigned win = recs[chunk].win[row];
-    const int wx = ox + (int)(win & 0xFFu), wy = oy + (int)(win >> 8 & 0xFFu);
-    const int ww = (int)(win >> 16 & 0xFFu), wh = (int)(win >> 24), wS = win_stride(ww);
-    const unsigned ww2 = (unsigned)max(min(ww, gx - wx) - 2, 0), wh2 = (unsigned)max(min(wh, gy - wy) - 2, 0);
-    // lanes map onto the window 16, 32 or 64 columns at a time
+    // the window: FP64 storage, the box; FP32, the wavefront's part of it
+    int wx = ox, wy = oy, ww = bw, wh = bh, wS = (int)(rec.ext >> 24);
+    unsigned ww2 = fw, wh2 = fh;
+    double *W0 = smem;
+    constexpr int kWinSize = F32 ? kWaveWin : kWin;
+    if constexpr (F32) {
+        const unsigned win = recs[chunk].win[row];
+        wx += (int)(win & 0xFFu);
+        wy += (int)(win >> 8 & 0xFFu);
+        ww = (int)(win >> 16 & 0xFFu);
+        wh = (int)(win >> 24);
+        wS = win_stride(ww);
+        ww2 = (unsigned)max(min(ww, gx - wx) - 2, 0);
+        wh2 = (unsigned)max(min(wh, gy - wy) - 2, 0);
+        W0 += row * 3 * kWaveWin;
+    }
+    double *W1 = W0 + kWinSize, *W2 = W1 + kWinSize;
+    // lanes map onto a wavefront's window 16, 32 or 64 columns at a time
     const int wsh = ww <= 16 ? 4 : (ww <= 32 ? 5 : 6);
     const int wcol = lane & ((1 << wsh) - 1), wrow0 = lane >> wsh, wstep = 64 >> wsh;
-    double *W0 = smem + row * 3 * kWaveWin, *W1 = W0 + kWaveWin, *W2 = W1 + kWaveWin;
-    double2 *tile = reinterpret_cast<double2 *>(smem + 4 * 3 * kWaveWin);
+    double2 *tile = reinterpret_cast<double2 *>(smem + kWindows);
     const double ind_x = cp.x0 + (G2P ? (tTab ? tTab[step] : t0) : 0.0) * cp.indV;
 
-    // The state of the points, streamed once per substep: non-temporal, so the
-    // grid keeps the L2.  A lane without a point reads the chunk's first one
-    // and computes along with the others; only its stores and sums are left out.
+    // The state of the points, read once per substep.  FP32 records
+    // non-temporally, so the grid keeps the L2 (167 us for 6.98 million points,
+    // 178 without); FP64 rows, whose wavefronts' 512 B straddle cache lines that
+    // the neighbours complete, through it (1.6 million points 44 us, 50
+    // non-temporally).  A lane without a point reads the chunk's first one and
+    // computes along with the others; only its stores and sums are left out.
     prec4 pr;
     fe4 fr;
     double px, py, F00, F01, F10, F11;
@@ -720,28 +760,37 @@ __global__ __launch_bounds__(256, 5) void k_batch_substep(
         pr = __builtin_nontemporal_load(reinterpret_cast<const prec4 *>(S.pos) + us);
         fr = __builtin_nontemporal_load(fe_rec(R, pp) + us);
     } else {
-        pos_load<true>(S.pos, pp, (int)us, cp, px, py);
-        F00 = __builtin_nontemporal_load(at(R + pp * 2, us));
-        F01 = __builtin_nontemporal_load(at(R + pp * 3, us));
-        F10 = __builtin_nontemporal_load(at(R + pp * 4, us));
-        F11 = __builtin_nontemporal_load(at(R + pp * 5, us));
-        crushed = __builtin_nontemporal_load(at(S.crushed, us));
-        if (cp.grainVar != 0) grain = __builtin_nontemporal_load(at(grains, us));
+        pos_load(S.pos, pp, (int)us, cp, px, py);
+        F00 = (*at(R + pp * 2, us));
+        F01 = (*at(R + pp * 3, us));
+        F10 = (*at(R + pp * 4, us));
+        F11 = (*at(R + pp * 5, us));
+        crushed = (*at(S.crushed, us));
+        if (cp.grainVar != 0) grain = (*at(grains, us));
     }
 
-    if (wcol < ww) {
-        for (int r = wrow0; r < wh; r += wstep) {
-            const int e = r * wS + wcol;
-            W0[e] = 0;
-            W1[e] = 0;
-            W2[e] = 0;
+    if constexpr (F32) {
+        if (wcol < ww) {
+            for (int r = wrow0; r < wh; r += wstep) {
+                const int e = r * wS + wcol;
+                W0[e] = 0;
+                W1[e] = 0;
+                W2[e] = 0;
+            }
         }
     }
     // the box's velocities (FP32 storage rounds them to FP32)
-    if constexpr (G2P) {
+    if constexpr (G2P || !F32) {
         for (unsigned e = threadIdx.x; e < nodes; e += 256) {
             unsigned c, r;
             box_node(e, rec.inv, (unsigned)bw, c, r);
+            if constexpr (!F32) {
+                const unsigned w = r * (unsigned)wS + c;
+                W0[w] = 0;
+                W1[w] = 0;
+                W2[w] = 0;
+            }
+            if constexpr (!G2P) continue;
             const int X = ox + (int)c, Y = oy + (int)r;
             const bool in = X < gx && Y < gy;
             const unsigned node = in ? (unsigned)(X + Y * gx) : 0u;
@@ -757,7 +806,7 @@ __global__ __launch_bounds__(256, 5) void k_batch_substep(
         }
     }
     if constexpr (F32) __builtin_amdgcn_s_setprio(0);
-    if constexpr (G2P) __syncthreads();
+    if constexpr (G2P || !F32) __syncthreads();
 
     // the base cells of the points, for the box (when it is renewed)
     int cellx = -1, celly = -1;
@@ -1082,55 +1131,72 @@ __global__ __launch_bounds__(256, 5) void k_batch_substep(
             cellx = bx;
             celly = by;
         }
-        // A quad of lanes whose four points share one base cell (in band
-        // order most quads, until points cross into other cells) and whose
-        // stencil lies in the window sums its contributions in registers
-        // before they reach the window.  Every lane is active here.
         const int lx0 = bx - wx, ly0 = by - wy;
         const bool winFits = ok && !defer && (unsigned)lx0 < ww2 && (unsigned)ly0 < wh2;
-        const bool quad = quad_uniform(winFits ? (unsigned)bx | (unsigned)by << 16 : 0xFFFF0000u | (unsigned)lane);
         // Every point of a case has the same mass m: the window sums the
         // contributions per unit mass, W (v + (Bp - m^-1 dt V D^-1 tau) d),
         // and the flush multiplies by m once per node.
         const double h = cp.h;
         const double A00 = B00 - cp.scm * t00, A01 = B01 - cp.scm * t01;
         const double A10 = B10 - cp.scm * t01, A11 = B11 - cp.scm * t11;
-        if (quad) {
-            quad_scatter(lane, ly0 * wS + lx0, wS, h, fx0, fx1, wx0, wx1, wx2, wy0, wy1, wy2, vx, vy, A00, A01, A10,
-                         A11, W0, W1, W2);
-        } else if (winFits) {
-            const int e0 = ly0 * wS + lx0;
-            // The four lanes of a quad (in band order mostly the points of
-            // one cell) walk the 3 x 3 stencil from four different nodes,
-            // so their LDS atomics never meet at one address: lane bit 0
-            // shifts the columns, bit 1 the rows, by one.  Step k of an
-            // axis visits node (k + s) mod 3 = s, 1 + s, 2 - 2 s; only the
-            // weights need selecting, the offsets follow from the index.
-            const int sx = lane & 1, sy = (lane >> 1) & 1;
-            const int xe[3] = {sx, 1 + sx, 2 - 2 * sx};
-            const int iy[3] = {sy, 1 + sy, 2 - 2 * sy};
-            const int ye[3] = {iy[0] * wS, iy[1] * wS, iy[2] * wS};
-            const double xw[3] = {sx ? wx1 : wx0, sx ? wx2 : wx1, sx ? wx0 : wx2};
-            const double yw[3] = {sy ? wy1 : wy0, sy ? wy2 : wy1, sy ? wy0 : wy2};
-            double xa[3], xb[3], ya[3], yb[3];
-#pragma unroll
-            for (int q = 0; q < 3; ++q) {
-                const double dx = ((double)xe[q] - fx0) * h, dy = ((double)iy[q] - fx1) * h;
-                xa[q] = vx + A00 * dx;
-                xb[q] = vy + A10 * dx;
-                ya[q] = A01 * dy;
-                yb[q] = A11 * dy;
-            }
-#pragma unroll
-            for (int a = 0; a < 3; ++a)
-#pragma unroll
-                for (int b = 0; b < 3; ++b) {
-                    const double W = xw[a] * yw[b];
-                    const int e = e0 + xe[a] + ye[b];
-                    atomicAdd(&W0[e], W);
-                    atomicAdd(&W1[e], W * (xa[a] + ya[b]));
-                    atomicAdd(&W2[e], W * (xb[a] + yb[b]));
+        if constexpr (F32) {
+            // A quad of lanes whose four points share one base cell (in band
+            // order most quads, until points cross into other cells) and whose
+            // stencil lies in the window sums its contributions in registers
+            // before they reach the window.  Every lane is active here.
+            const bool quad = quad_uniform(winFits ? (unsigned)bx | (unsigned)by << 16 : 0xFFFF0000u | (unsigned)lane);
+            if (quad) {
+                quad_scatter(lane, ly0 * wS + lx0, wS, h, fx0, fx1, wx0, wx1, wx2, wy0, wy1, wy2, vx, vy, A00, A01, A10,
+                             A11, W0, W1, W2);
+            } else if (winFits) {
+                const int e0 = ly0 * wS + lx0;
+                // The four lanes of a quad (in band order mostly the points of
+                // one cell) walk the 3 x 3 stencil from four different nodes,
+                // so their LDS atomics never meet at one address: lane bit 0
+                // shifts the columns, bit 1 the rows, by one.  Step k of an
+                // axis visits node (k + s) mod 3 = s, 1 + s, 2 - 2 s; only the
+                // weights need selecting, the offsets follow from the index.
+                const int sx = lane & 1, sy = (lane >> 1) & 1;
+                const int xe[3] = {sx, 1 + sx, 2 - 2 * sx};
+                const int iy[3] = {sy, 1 + sy, 2 - 2 * sy};
+                const int ye[3] = {iy[0] * wS, iy[1] * wS, iy[2] * wS};
+                const double xw[3] = {sx ? wx1 : wx0, sx ? wx2 : wx1, sx ? wx0 : wx2};
+                const double yw[3] = {sy ? wy1 : wy0, sy ? wy2 : wy1, sy ? wy0 : wy2};
+                double xa[3], xb[3], ya[3], yb[3];
+    #pragma unroll
+                for (int q = 0; q < 3; ++q) {
+                    const double dx = ((double)xe[q] - fx0) * h, dy = ((double)iy[q] - fx1) * h;
+                    xa[q] = vx + A00 * dx;
+                    xb[q] = vy + A10 * dx;
+                    ya[q] = A01 * dy;
+                    yb[q] = A11 * dy;
                 }
+    #pragma unroll
+                for (int a = 0; a < 3; ++a)
+    #pragma unroll
+                    for (int b = 0; b < 3; ++b) {
+                        const double W = xw[a] * yw[b];
+                        const int e = e0 + xe[a] + ye[b];
+                        atomicAdd(&W0[e], W);
+                        atomicAdd(&W1[e], W * (xa[a] + ya[b]));
+                        atomicAdd(&W2[e], W * (xb[a] + yb[b]));
+                    }
+            }
+        } else if (winFits) {
+            const double wxs[3] = {wx0, wx1, wx2}, wys[3] = {wy0, wy1, wy2};
+            double *w0 = W0 + ly0 * wS + lx0, *w1 = w0 + wS, *w2 = w1 + wS;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const double dx = (i - fx0) * h, xa = vx + A00 * dx, xb = vy + A10 * dx;
+#pragma unroll
+                for (int j = 0; j < 3; ++j) {
+                    double *w = (j == 0 ? w0 : (j == 1 ? w1 : w2)) + i;
+                    const double W = wxs[i] * wys[j], dy = (j - fx1) * h;
+                    atomicAdd(w, W);
+                    atomicAdd(w + kWin, W * (xa + A01 * dy));
+                    atomicAdd(w + 2 * kWin, W * (xb + A11 * dy));
+                }
+            }
         }
         if (ok && !winFits && !defer) {
             // outside the window, or the stencil leaves the grid: node by node
@@ -1151,24 +1217,33 @@ __global__ __launch_bounds__(256, 5) void k_batch_substep(
                 unsafeAtomicAdd(at(gO + 2 * gpitch, node), W * (vy + (A10 * d0 + A11 * d1)) * m);
             }
         }
+    }
+
+    if constexpr (F32)
         wsync();
-        if constexpr (F32) __builtin_amdgcn_s_setprio(2);
-        // the window to the grid
-        if (wcol < ww) {
-            for (int r = wrow0; r < wh; r += wstep) {
-                const int e = r * wS + wcol;
-                // the three sums in one LDS round trip; the atomics address
-                // the rows from their scalar bases with 32-bit offsets
-                const double a = W0[e], a1 = W1[e], a2 = W2[e];
-                const int X = wx + wcol, Y = wy + r;
-                if (a != 0 && X < gx && Y < gy) {
-                    const double m = cp.mass;   // the window holds sums per unit mass
-                    const unsigned node = (unsigned)(X + Y * gx);
-                    unsafeAtomicAdd(at(gO, node), a * m);
-                    unsafeAtomicAdd(at(gO + gpitch, node), a1 * m);
-                    unsafeAtomicAdd(at(gO + 2 * gpitch, node), a2 * m);
-                }
-            }
+    else
+        __syncthreads();
+    if constexpr (F32) __builtin_amdgcn_s_setprio(2);
+    // the window to the grid: the three sums of a node in one LDS round trip; the
+    // atomics address the rows from their scalar bases with 32-bit offsets
+    const auto flush = [&](int e, int X, int Y) {
+        const double a = W0[e], a1 = W1[e], a2 = W2[e];
+        if (a != 0 && X < gx && Y < gy) {
+            const double m = cp.mass;   // the window holds sums per unit mass
+            const unsigned node = (unsigned)(X + Y * gx);
+            unsafeAtomicAdd(at(gO, node), a * m);
+            unsafeAtomicAdd(at(gO + gpitch, node), a1 * m);
+            unsafeAtomicAdd(at(gO + 2 * gpitch, node), a2 * m);
+        }
+    };
+    if constexpr (F32) {
+        if (lanes > 0 && wcol < ww)
+            for (int r = wrow0; r < wh; r += wstep) flush(r * wS + wcol, wx + wcol, wy + r);
+    } else {
+        for (unsigned e = threadIdx.x; e < nodes; e += 256) {
+            unsigned c, r;
+            box_node(e, rec.inv, (unsigned)bw, c, r);
+            flush((int)(r * (unsigned)wS + c), ox + (int)c, oy + (int)r);
         }
     }
     if (step % kBoxEvery == 0) {
@@ -1223,17 +1298,18 @@ __global__ __launch_bounds__(256) void k_chunk_boxes(ChunkRec *recs, int nChunks
     if (starts) {
         rec = ChunkRec{};
         rec.beg = starts[ch];
-        rec.count = starts[ch + 1] - rec.beg;
+        rec.shape = chunk_shape(starts[ch + 1] - rec.beg);
         rec.dims = (unsigned)cases[0].gx | (unsigned)cases[0].gy << 16;
     }
     const CaseParams &cp = cases[rec.cs];
+    const int count = F32 ? (int)rec.shape : chunk_count(rec.shape);
     int wx0[4], wy0[4], wx1[4], wy1[4];   // of each wavefront's points
     int fx = 0, fy = 0, x0 = INT_MAX, y0 = INT_MAX, x1 = -1, y1 = -1;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         const int i = q * 64 + lane;
         int bx = -1, by = -1;
-        if (i < rec.count) {
+        if (i < count) {
             double f, a, b, c;
             if constexpr (F32) {
                 const prec4 r = reinterpret_cast<const prec4 *>(pos)[rec.beg + i];
@@ -1241,7 +1317,7 @@ __global__ __launch_bounds__(256) void k_chunk_boxes(ChunkRec *recs, int nChunks
                 stencil_cells(fix_cells(r.y, r.z >> 16, cp), by, f, a, b, c);
             } else {
                 double x, y;
-                pos_load<false>(pos, pitch, rec.beg + i, cp, x, y);
+                pos_load(pos, pitch, rec.beg + i, cp, x, y);
                 if (!stencil(x, cp.h_inv, bx, f, a, b, c) || !stencil(y, cp.h_inv, by, f, a, b, c)) bx = -1;
             }
         }
@@ -1450,7 +1526,7 @@ __global__ void k_batch_keys(const PT *__restrict__ pos, size_t pitch, int nPts,
     }
     const CaseParams &cp = cases[lo];
     double x, y;
-    pos_load<false>(pos, pitch, i, cp, x, y);
+    pos_load(pos, pitch, i, cp, x, y);
     int key = cp.gridTotal - 1;
     if (x == x && y == y) {
         const double bx = fmin(fmax(x * cp.h_inv - 0.5, 0.0), (double)(cp.gx - 1));
@@ -1461,12 +1537,14 @@ __global__ void k_batch_keys(const PT *__restrict__ pos, size_t pitch, int nPts,
     vals[i] = i;
 }
 
-// The case-local base cell of every slot, packed as column | row << 16
+// The case-local base cell of every slot (of slot order[i], when an order that
+// keeps the cases apart is given), packed as column | row << 16
 // (finalize keeps every grid within 65536 columns and rows): what the chunk
 // table is built from, without the band key's divisions on the host.
 template <class PT>
 __global__ void k_batch_cells(const PT *__restrict__ pos, size_t pitch, int nPts,
-                              const CaseParams *__restrict__ cases, int nCases, unsigned *__restrict__ cells) {
+                              const CaseParams *__restrict__ cases, int nCases, const int *__restrict__ order,
+                              unsigned *__restrict__ cells) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nPts) return;
     int lo = 0, hi = nCases - 1;   // the last case with ptOffset <= i
@@ -1476,7 +1554,7 @@ __global__ void k_batch_cells(const PT *__restrict__ pos, size_t pitch, int nPts
     }
     const CaseParams &cp = cases[lo];
     double x, y;
-    pos_load<false>(pos, pitch, i, cp, x, y);
+    pos_load(pos, pitch, order ? order[i] : i, cp, x, y);
     // the cell k_batch_keys keys the slot by (a NaN position: the last cell)
     unsigned cx = (unsigned)(cp.gx - 1), cy = (unsigned)(cp.gy - 1);
     if (x == x && y == y) {
@@ -1484,6 +1562,15 @@ __global__ void k_batch_cells(const PT *__restrict__ pos, size_t pitch, int nPts
         cy = (unsigned)fmin(fmax(y * cp.h_inv - 0.5, 0.0), (double)(cp.gy - 1));
     }
     cells[i] = cx | cy << 16;
+}
+
+// An order of the points in band order, rearranged into the chunks' slot orders.
+__global__ void k_chunk_order(const ChunkRec *__restrict__ recs, int nChunks, const int *__restrict__ in,
+                              int *__restrict__ out) {
+    const int ch = blockIdx.x;
+    if (ch >= nChunks) return;
+    const int beg = recs[ch].beg, n = chunk_count(recs[ch].shape);
+    if ((int)threadIdx.x < n) out[beg + threadIdx.x] = in[beg + chunk_point((int)threadIdx.x, recs[ch].shape)];
 }
 
 // A case's points in the layout they came in: rows 0 and 3-15 of the point SoA
@@ -1509,7 +1596,7 @@ __global__ __launch_bounds__(256) void k_read_points(Rows<F32> S, const int *__r
     unsigned char crushed;
     short grain = 0;
     if constexpr (F32) {
-        const unsigned w = pos_load<false>(S.pos, pp, slot, cp, v[1], v[2]);
+        const unsigned w = pos_load(S.pos, pp, slot, cp, v[1], v[2]);
         crushed = (unsigned char)(w & 0xFFu);
         grain = (short)(w >> 16);
         const fe4 f = fe_rec(R, pp)[slot];
@@ -1519,7 +1606,7 @@ __global__ __launch_bounds__(256) void k_read_points(Rows<F32> S, const int *__r
         v[8] = (double)f.w + 1.0;
         v[0] = (double)R[pp * 10 + slot] + 1.0;
     } else {
-        pos_load<false>(S.pos, pp, slot, cp, v[1], v[2]);
+        pos_load(S.pos, pp, slot, cp, v[1], v[2]);
         crushed = S.crushed[slot];
         if (S.grain) grain = S.grain[slot];
         for (int r = 2; r < 6; ++r) v[3 + r] = R[pp * r + slot];
@@ -1951,8 +2038,9 @@ int upload_chunks(icempm_batch *b) {
     std::vector<ChunkRec> t(n);
     for (size_t c = 0; c < n; ++c) {
         const CaseParams &cp = b->hc[(size_t)b->hccase[c]].cp;
-        t[c] = ChunkRec{b->hcstart[c], b->hcstart[c + 1] - b->hcstart[c], b->hccase[c], cp.gridOffset,
-                        (unsigned)cp.gx | (unsigned)cp.gy << 16, 0, 0, 0};
+        const int count = b->hcstart[c + 1] - b->hcstart[c];
+        t[c] = ChunkRec{b->hcstart[c], b->precision == ICEMPM_BATCH_F32 ? (unsigned)count : chunk_shape(count),
+                        b->hccase[c], cp.gridOffset, (unsigned)cp.gx | (unsigned)cp.gy << 16, 0, 0, 0, {}};
     }
     const ChunkRec *before = b->recs;
     const int nBefore = b->nChunks;
@@ -2001,8 +2089,9 @@ int sort_keys(icempm_batch *b) {
     return ICEMPM_OK;
 }
 
-// the base cells of the current slots, in b->hcells on the host
-int current_cells(icempm_batch *b) {
+// the base cells of the current slots (or of the slots in the given order), in
+// b->hcells on the host
+int current_cells(icempm_batch *b, const int *order = nullptr) {
     const int n = b->nPts;
     if (!b->dcells) {
         BCHK(b, hipMalloc(&b->dcells, (size_t)n * sizeof(unsigned)), "cells");
@@ -2011,10 +2100,11 @@ int current_cells(icempm_batch *b) {
     if (b->precision == ICEMPM_BATCH_F32)
         hipLaunchKernelGGL(k_batch_cells<unsigned int>, dim3((n + 255) / 256), dim3(256), 0, b->stream,
                            static_cast<const unsigned int *>(b->pos), b->pitch, n, b->cases, (int)b->hc.size(),
-                           b->dcells);
+                           order, b->dcells);
     else
         hipLaunchKernelGGL(k_batch_cells<double>, dim3((n + 255) / 256), dim3(256), 0, b->stream,
-                           static_cast<const double *>(b->pos), b->pitch, n, b->cases, (int)b->hc.size(), b->dcells);
+                           static_cast<const double *>(b->pos), b->pitch, n, b->cases, (int)b->hc.size(), order,
+                           b->dcells);
     BCHK(b, hipGetLastError(), "cells");
     BCHK(b, hipMemcpyAsync(b->hcells, b->dcells, (size_t)n * sizeof(unsigned), hipMemcpyDeviceToHost, b->stream),
          "cells");
@@ -2058,21 +2148,34 @@ int resort(icempm_batch *b) {
         if (b->grain) BCHK(b, hipMalloc(&b->tgrain, b->pitch * sizeof(short)), "re-sort");
     }
     BCHK(b, radix_sort_pairs(b->sKeys, b->sVals, b->sKeys2, b->sVals2, (size_t)n, b->sTmp, b->stream), "re-sort");
+    // the cells in sorted order give the new chunk table, whose chunks then
+    // (FP64 storage) arrange their points
+    if ((rc = current_cells(b, b->sVals))) return rc;
+    chunk_table(b, b->hcells, b->hcstart, b->hccase);
+    if ((rc = upload_chunks(b))) return rc;
+    const int *from = b->sVals;
+    if (b->precision != ICEMPM_BATCH_F32) {
+        hipLaunchKernelGGL(k_chunk_order, dim3((unsigned)b->nChunks), dim3(256), 0, b->stream, b->recs, b->nChunks,
+                           b->sVals, b->sVals2);
+        BCHK(b, hipGetLastError(), "re-sort");
+        from = b->sVals2;
+    }
     const unsigned nb = (unsigned)((n + 255) / 256);
     if (b->precision == ICEMPM_BATCH_F32) {
         Rows<true> a{static_cast<unsigned int *>(b->pos), reinterpret_cast<float *>(b->rest), b->crushed, b->grain,
                      b->pitch};
         Rows<true> t{static_cast<unsigned int *>(b->tpos), reinterpret_cast<float *>(b->trest), b->tcrushed,
                      b->tgrain, b->pitch};
-        hipLaunchKernelGGL(k_batch_permute<true>, dim3(nb), dim3(256), 0, b->stream, a, t, b->orig, b->torig, b->sVals, n);
+        hipLaunchKernelGGL(k_batch_permute<true>, dim3(nb), dim3(256), 0, b->stream, a, t, b->orig, b->torig, from, n);
     } else {
         Rows<false> a{static_cast<double *>(b->pos), reinterpret_cast<double *>(b->rest), b->crushed, b->grain,
                       b->pitch};
         Rows<false> t{static_cast<double *>(b->tpos), reinterpret_cast<double *>(b->trest), b->tcrushed,
                       b->tgrain, b->pitch};
-        hipLaunchKernelGGL(k_batch_permute<false>, dim3(nb), dim3(256), 0, b->stream, a, t, b->orig, b->torig, b->sVals, n);
+        hipLaunchKernelGGL(k_batch_permute<false>, dim3(nb), dim3(256), 0, b->stream, a, t, b->orig, b->torig, from, n);
     }
     BCHK(b, hipGetLastError(), "re-sort");
+    BCHK(b, hipStreamSynchronize(b->stream), "re-sort");
     std::swap(b->pos, b->tpos);
     std::swap(b->rest, b->trest);
     std::swap(b->crushed, b->tcrushed);
@@ -2080,10 +2183,7 @@ int resort(icempm_batch *b) {
     std::swap(b->orig, b->torig);
     drop_graph(b);   // the captured launches hold the old row addresses
     b->pending = -1;   // a P2G in a grid scattered the points from their old slots
-    // the cells of the sorted slots give the new chunk table
-    if ((rc = current_cells(b))) return rc;
-    chunk_table(b, b->hcells, b->hcstart, b->hccase);
-    return upload_chunks(b);
+    return ICEMPM_OK;
 }
 
 // Scratch of read_points, for the largest case: the device rows, the pinned
@@ -2270,24 +2370,51 @@ bool case_constants(const icy::SimParams &P, double x0, double y0, void *out) {
     return true;
 }
 
-hipError_t plan(const Run &r, int n, int *keys, int *vals, int *keys2, int *vals2, int *tmp, std::vector<int> &starts) {
+hipError_t plan(const Run &r, int *keys, int *vals, int *keys2, int *vals2, int *tmp, std::vector<int> &starts) {
+    const int n = r.n;
     hipLaunchKernelGGL(k_batch_keys<double>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, r.stream, r.pts + kRowPosX * r.pp,
                        r.pp, n, static_cast<const CaseParams *>(r.cp), 1, keys, vals);
     hipError_t e = radix_sort_pairs(keys, vals, keys2, vals2, (size_t)n, tmp, r.stream);
     if (e != hipSuccess) return e;
-    std::vector<int> hk((size_t)n);
-    std::vector<unsigned> cells((size_t)n);
-    if ((e = hipMemcpyAsync(hk.data(), keys, (size_t)n * sizeof(int), hipMemcpyDeviceToHost, r.stream)) != hipSuccess) return e;
+    const std::unique_ptr<int[]> hk(new int[(size_t)n]);
+    if ((e = hipMemcpyAsync(hk.get(), keys, (size_t)n * sizeof(int), hipMemcpyDeviceToHost, r.stream)) != hipSuccess) return e;
     if ((e = hipStreamSynchronize(r.stream)) != hipSuccess) return e;
-    for (int i = 0; i < n; ++i) {
-        int x, y;
-        band_cell(hk[(size_t)i], r.gx, r.gy, x, y);
-        cells[(size_t)i] = (unsigned)x | (unsigned)y << 16;
-    }
+    // cut_chunks' cuts, for points that are in band order: a chunk's points lie
+    // in one band, their columns ascending, so only its ends are looked at
     starts.clear();
-    cut_chunks(cells.data(), n, 0, 256, starts);
+    const auto fits = [&](int a, int b) {
+        int xa, ya, xb, yb;
+        band_cell(hk[(size_t)a], r.gx, r.gy, xa, ya);
+        band_cell(hk[(size_t)b], r.gx, r.gy, xb, yb);
+        return ya >> 1 == yb >> 1 && xb - xa <= kChunkCols - 1;
+    };
+    for (int cs = 0; cs < n;) {
+        starts.push_back(cs);
+        int lo = cs + 1, hi = std::min(cs + 256, n);   // the chunk's end lies in [lo, hi]
+        if (!fits(cs, hi - 1)) {
+            while (lo < hi) {
+                const int mid = (lo + hi) / 2;
+                if (fits(cs, mid))
+                    lo = mid + 1;
+                else
+                    hi = mid;
+            }
+        }
+        cs = hi;
+    }
     starts.push_back(n);
     return hipSuccess;
+}
+
+__global__ __launch_bounds__(256) void k_slots(const int *__restrict__ starts, const int *__restrict__ sorted,
+                                               int *__restrict__ perm) {
+    const int beg = starts[blockIdx.x], n = starts[blockIdx.x + 1] - beg, l = threadIdx.x;
+    if (l < n) perm[beg + l] = sorted[beg + chunk_point(l, chunk_shape(n))];
+}
+
+hipError_t slots(const Run &r, const int *sorted, int *perm) {
+    hipLaunchKernelGGL(k_slots, dim3((unsigned)r.nChunks), dim3(256), 0, r.stream, r.starts, sorted, perm);
+    return hipGetLastError();
 }
 
 // The rows a substep reads and writes, from the points' own order to band
@@ -2558,6 +2685,15 @@ int icempm_batch_finalize(icempm_batch *b) {
                 }
             }
             chunk_table(b, cells.data(), b->hcstart, b->hccase);
+            // FP64 storage: every chunk's points in its slot order
+            std::vector<int> sorted;
+            for (size_t c = 0; c < b->hccase.size() && b->precision != ICEMPM_BATCH_F32; ++c) {
+                std::vector<int> &ord = order[(size_t)b->hccase[c]];
+                const int o = b->hc[(size_t)b->hccase[c]].cp.ptOffset;
+                const int p = b->hcstart[c] - o, n = b->hcstart[c + 1] - b->hcstart[c];
+                sorted.assign(ord.begin() + p, ord.begin() + p + n);
+                for (int l = 0; l < n; ++l) ord[(size_t)(p + l)] = sorted[(size_t)chunk_point(l, chunk_shape(n))];
+            }
         }
         const size_t vs = b->precision == ICEMPM_BATCH_F32 ? sizeof(float) : sizeof(double);
         BCHK(b, hipMalloc(&b->pos, pos_bytes(b)), "batch finalize");

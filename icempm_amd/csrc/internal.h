@@ -92,7 +92,7 @@ struct Run {
     double *pts;             // 16 rows x pp
     size_t pp, gp;
     int n, gx, gy;
-    const int *perm;         // slot in band order -> point
+    const int *perm;         // slot -> point
     const int *starts;       // nChunks + 1 first slots
     void *recs;              // nChunks records, made by enter
     int nChunks;
@@ -104,9 +104,11 @@ struct Run {
 // The case's constants, the indenter starting at (x0, y0), in out (kCaseBytes);
 // false where the kernel does not take the case.
 bool case_constants(const icy::SimParams &P, double x0, double y0, void *out);
-// The points' band order as they are (in vals; keys, keys2, vals2: n ints, tmp:
-// radix_tmp_ints(n)) and its chunks' first slots.
-hipError_t plan(const Run &r, int n, int *keys, int *vals, int *keys2, int *vals2, int *tmp, std::vector<int> &starts);
+// The points' band order as they are (in vals; keys, keys2, vals2: scratch of n
+// ints, tmp: of radix_tmp_ints(n)) and its chunks' first slots.
+hipError_t plan(const Run &r, int *keys, int *vals, int *keys2, int *vals2, int *tmp, std::vector<int> &starts);
+// The points of the slots, from that order.
+hipError_t slots(const Run &r, const int *sorted, int *perm);
 hipError_t enter(const Run &r);
 hipError_t leave(const Run &r);
 // hist2: this substep's force (added to); t: its time; step: its index in the run.

@@ -192,9 +192,9 @@ int icempm_get_mode(const icempm_ctx *ctx);
 /* Tuning knobs (no counterpart).  ICEMPM_TUNE_PASS_KIND selects the kernel
  * of the particle pass: 0 workgroup-wide shared-memory windows for gather and
  * scatter, 1 wavefront windows (direct gather, per-wavefront scatter), 2 as 1
- * with the per-lane stencil rotation (default; longer FAST runs of up to 1.2
- * million points then do a substep in one kernel, on a copy of the points in
- * another order).  Results differ only in the order of the FAST-mode P2G sums. */
+ * with the per-lane stencil rotation (default; longer FAST runs then do a
+ * substep in one kernel, on a copy of the points in another order).  Results
+ * differ only in the order of the FAST-mode P2G sums. */
 enum { ICEMPM_TUNE_PASS_KIND = 0 };
 int icempm_set_tuning(icempm_ctx *ctx, int knob, int value);
 /* current value, or -1 for an unknown knob */
