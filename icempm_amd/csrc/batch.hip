@@ -1425,12 +1425,14 @@ __global__ __launch_bounds__(256) void k_batch_map(Rows<F32> S, const CaseParams
     __shared__ __attribute__((aligned(16))) unsigned short wsh[mlpdev::kParams];   // the weights, BF16
     using V = typename Rows<F32>::V;
     constexpr double fe0 = F32 ? 1.0 : 0.0;
+    __shared__ unsigned int counts[kMapStats];
     if (blockIdx.x == 0 && threadIdx.x == 0) qCountNext[0] = 0u;
     const unsigned int n = qCount[0];
     if (blockIdx.x * 64u >= n) return;   // no entry for this block (uniform)
     static_assert(mlpdev::kParams % 8 == 0, "weights are staged 8 at a time");
     for (int x = threadIdx.x; x < mlpdev::kParams / 8; x += 256)
         reinterpret_cast<uint4 *>(wsh)[x] = reinterpret_cast<const uint4 *>(la.wbf)[x];
+    if (threadIdx.x < kMapStats) counts[threadIdx.x] = 0;
     __syncthreads();
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const size_t pp = S.pitch;
@@ -1483,12 +1485,12 @@ __global__ __launch_bounds__(256) void k_batch_map(Rows<F32> S, const CaseParams
         const unsigned long long acc = __ballot(accepted), fb = __ballot(have && !accepted);
         const unsigned long long ten = __ballot(have && br == kBrTension);
         if (lane == 0) {
-            if (acc) atomicAdd(&la.stats[0], (unsigned long long)__popcll(acc));
-            if (fb) atomicAdd(&la.stats[1], (unsigned long long)__popcll(fb));
-            if (acc & ten) atomicAdd(&la.stats[3], (unsigned long long)__popcll(acc & ten));
-            if (fb & ten) atomicAdd(&la.stats[4], (unsigned long long)__popcll(fb & ten));
-            if (acc & ~ten) atomicAdd(&la.stats[5], (unsigned long long)__popcll(acc & ~ten));
-            if (fb & ~ten) atomicAdd(&la.stats[6], (unsigned long long)__popcll(fb & ~ten));
+            if (acc) atomicAdd(&counts[0], (unsigned)__popcll(acc));
+            if (fb) atomicAdd(&counts[1], (unsigned)__popcll(fb));
+            if (acc & ten) atomicAdd(&counts[3], (unsigned)__popcll(acc & ten));
+            if (fb & ten) atomicAdd(&counts[4], (unsigned)__popcll(fb & ten));
+            if (acc & ~ten) atomicAdd(&counts[5], (unsigned)__popcll(acc & ~ten));
+            if (fb & ~ten) atomicAdd(&counts[6], (unsigned)__popcll(fb & ~ten));
         }
         if (have) {
             const int pt = e.pt;
@@ -1504,6 +1506,9 @@ __global__ __launch_bounds__(256) void k_batch_map(Rows<F32> S, const CaseParams
             if (gridOut) scatter_point<F32>(e, cp, k, F00, F01, F10, F11, gridOut, gpitch);
         }
     }
+    __syncthreads();
+    if (threadIdx.x < kMapStats && counts[threadIdx.x])
+        atomicAdd(&la.stats[threadIdx.x], (unsigned long long)counts[threadIdx.x]);
 }
 
 __global__ void k_reset_bounds(int4 *bounds, int nCases) {
