@@ -722,7 +722,7 @@ int icempm_p2g(icempm_ctx *c) {
         const KParams k = make_kparams(c);
         if (c->mode == ICEMPM_MODE_ORDERED) {
             if ((rc = ensure_ordered(c))) return rc;
-            HIPCHK(c, ordered_p2g(k, c->gridA, c->ord, false, 0, 0, c->stream), "cuda_p2g");
+            HIPCHK(c, ordered_p2g(k, c->gridA, c->ord, false, 0, 0, nullptr, c->stream), "cuda_p2g");
             return ICEMPM_OK;
         }
         if ((rc = ensure_chunks(c))) return rc;
@@ -790,7 +790,9 @@ int icempm_run_substeps(icempm_ctx *c, int first_step, int n, double *t,
         single::Run run{};
         const bool one = substep_kernel_pays(n, c->prms.nPts) &&
                          ensure_substep(c, indenter_x_initial, indenter_y, run);
-        bool copied = false;   // the points are in the substep kernel's copy
+        bool copied = false;    // the points are in the substep kernel's copy
+        OrderedForce force{};   // of the last ORDERED substep, folded with the next one
+        bool pending = false;
         if (!ordered) {
             HIPCHK(c, launch_fill_f64(c->gridA, c->gp * kGridRows, 0.0, c->stream), "run_substeps");
             HIPCHK(c, particles(c, k, false, true, c->gridA, c->gridA, 0), "run_substeps");
@@ -801,16 +803,22 @@ int icempm_run_substeps(icempm_ctx *c, int first_step, int n, double *t,
         }
         for (int i = 0; i < n; ++i) {
             const int s = first_step + i;
-            if (reset_bins_at_cycle && s % N == 0)
+            if (reset_bins_at_cycle && s % N == 0) {
+                if (pending)
+                    HIPCHK(c, ordered_fold_forces(k, c->ord, force.hist2, force.ix, force.iy, c->stream), "run_substeps");
+                pending = false;
                 HIPCHK(c, launch_fill_f64(c->bins, (size_t)c->nBinsAlloc, 0.0, c->stream), "run_substeps");
+            }
             tt += dt;
             const double ix = indenter_x_initial + tt * V;
             const int rec = ((s + 1) % N == 0) ? 1 : 0;
             double *h2 = c->hist + 2 * (size_t)i;
             const int timeIt = c->timing && (i % c->timingStride == 0);
             if (ordered) {
-                HIPCHK(c, ordered_p2g(k, c->gridA, c->ord, true, ix, indenter_y, c->stream), "run_substeps");
-                HIPCHK(c, ordered_fold_forces(k, c->ord, h2, ix, indenter_y, c->stream), "run_substeps");
+                HIPCHK(c, ordered_p2g(k, c->gridA, c->ord, true, ix, indenter_y, pending ? &force : nullptr, c->stream),
+                       "run_substeps");
+                force = OrderedForce{h2, ix, indenter_y};
+                pending = true;
                 if ((rc = launch_particles_timed(c, k, true, false, c->gridA, nullptr, rec, timeIt)))
                     return rc;
             } else {
@@ -846,6 +854,8 @@ int icempm_run_substeps(icempm_ctx *c, int first_step, int n, double *t,
                 }
             }
         }
+        if (pending)
+            HIPCHK(c, ordered_fold_forces(k, c->ord, force.hist2, force.ix, force.iy, c->stream), "run_substeps");
         *t = tt;
         if (c->timing) {
             if ((rc = collect_timing(c))) return rc;

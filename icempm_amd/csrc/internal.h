@@ -66,10 +66,15 @@ struct OrderedScratch {
     double *nodeF = nullptr;     // 2 per node
     size_t nPts = 0, nGrid = 0, cleared = 0;
 };
+// A substep's contact forces to add up: its history entry, the indenter where it was.
+struct OrderedForce {
+    double *hist2, ix, iy;
+};
 // The P2G into grid; update: with the grid update, for an indenter at (ix, iy),
-// and the padding of the grid's rows cleared.
+// and the padding of the grid's rows cleared.  force (may be null): the last
+// update's, which are folded before this one's take their place.
 hipError_t ordered_p2g(const KParams &k, double *grid, OrderedScratch &o, bool update, double ix, double iy,
-                       hipStream_t s);
+                       const OrderedForce *force, hipStream_t s);
 // The contact forces of the last update, with the indenter where it was.
 hipError_t ordered_fold_forces(const KParams &k, OrderedScratch &o, double *hist2, double ix, double iy,
                                hipStream_t s);

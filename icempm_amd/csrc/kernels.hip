@@ -236,12 +236,13 @@ hipError_t launch_update(const KParams &k, double *grid, double ix, double iy, d
 // ORDERED P2G, in two kernels: every point makes the record its contributions
 // follow from and enters its base cell's list; every node then collects the
 // points of its nine cells, puts them in order and sums.  What bounds it is
-// latency: few workgroups, each a chain of LDS passes (counts and points 1.5 us,
-// order 6.5, lists 6.4, sums 3.9 at 60,000 points).  A substep there takes 45 us
-// of which the records 10 and the fold 25; through memory, with a counting sort
-// and an insertion sort per node, it took 249 (contributions 20, sort 60, fold
-// 165).  An insertion sort of each node's list in LDS took up to 20 us: the
-// points of one row of the load's order lie in two rows of cells.
+// latency: few workgroups, each a chain of loads and LDS passes.  A substep of
+// 60,000 points takes 32 us, of which the records 9, the fold 16 (found, ranked,
+// listed and summed in about equal parts) and the G2P 7; through memory, with a
+// counting sort and an insertion sort per node, it took 249 (contributions 20,
+// sort 60, fold 165).  An insertion sort of each node's list in LDS took up to 20
+// us (the points of one row of the load's order lie in two rows of cells), a rank
+// by comparing all points of a tile 6.
 struct Terms {   // a point's part of its contributions: weights, distances, affine momentum, momentum
     double wx[3], wy[3], dx[3], dy[3], A00, A01, A10, A11, mv0, mv1;
 };
@@ -273,10 +274,119 @@ static __device__ __forceinline__ double term(const Terms &t, int i, int j, int 
     return part == 1 ? W * (t.mv0 + (t.A00 * d0 + t.A01 * d1)) : W * (t.mv1 + (t.A10 * d0 + t.A11 * d1));
 }
 
-// padGrid (may be null): the padding of its rows is cleared.
+// ORDERED indenter force: each bin, and the substep's total, summed in node
+// order by one thread each over the nodes in contact.  One workgroup: it looks
+// only at the w x h nodes around the disc, and leaves those in contact in LDS,
+// 256 nodes at a time.  In a run it is one more workgroup of the next substep's
+// k_point_records (a launch of its own takes 4.5 us).
+struct BinsFold {
+    double *bins;   // null: nothing to do
+    const int *nodeBin;
+    const double *nodeF;
+    double *hist2;
+    int nb, gx, x0, y0, w, h;
+};
+constexpr int kFoldBlock = 256, kFoldBinsMax = 1024;   // bins and the total
+struct BinsLds {
+    int bin[kFoldBlock], wave[kFoldBlock / 64];
+    double f0[kFoldBlock], f1[kFoldBlock];
+};
+static __device__ void fold_bins(const BinsFold &B, BinsLds &L) {
+    constexpr int kPer = kFoldBinsMax / kFoldBlock;
+    const int t = threadIdx.x, nb = B.nb;
+    double a0[kPer], a1[kPer];
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        const int b = t + kFoldBlock * q;
+        a0[q] = b < nb ? B.bins[2 * b] : 0.0;
+        a1[q] = b < nb ? B.bins[2 * b + 1] : 0.0;
+    }
+    const long nodes = (long)B.w * B.h;
+    for (long first = 0; first < nodes; first += kFoldBlock) {
+        const long e = first + t;
+        int b = -1, idx = 0;
+        if (e < nodes) {
+            idx = B.x0 + (int)(e % B.w) + (B.y0 + (int)(e / B.w)) * B.gx;
+            b = B.nodeBin[idx];
+        }
+        const unsigned long long hit = __ballot(b >= 0);
+        if ((t & 63) == 0) L.wave[t >> 6] = __popcll(hit);
+        __syncthreads();
+        int at = __popcll(hit & ((1ull << (t & 63)) - 1ull)), count = 0;
+        for (int q = 0; q < kFoldBlock / 64; ++q) {
+            if (q < t >> 6) at += L.wave[q];
+            count += L.wave[q];
+        }
+        if (b >= 0) {
+            L.bin[at] = b;
+            L.f0[at] = B.nodeF[2 * (size_t)idx];
+            L.f1[at] = B.nodeF[2 * (size_t)idx + 1];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < kPer; ++q) {
+            const int mine = t + kFoldBlock * q;
+            if (mine <= nb)
+                for (int c = 0; c < count; ++c)
+                    if (mine == nb || L.bin[c] == mine) {
+                        a0[q] += L.f0[c];
+                        a1[q] += L.f1[c];
+                    }
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        const int b = t + kFoldBlock * q;
+        if (b < nb) {
+            B.bins[2 * b] = a0[q];
+            B.bins[2 * b + 1] = a1[q];
+        } else if (b == nb && B.hist2) {
+            B.hist2[0] = a0[q];
+            B.hist2[1] = a1[q];
+        }
+    }
+}
+__global__ __launch_bounds__(kFoldBlock) void k_bins_fold(BinsFold B) {
+    __shared__ BinsLds L;
+    fold_bins(B, L);
+}
+
+// The forces of a substep with the indenter at (ix, iy).
+static BinsFold bins_fold(const KParams &k, const OrderedScratch &o, double *hist2, double ix, double iy) {
+    // the nodes in contact lie within the disc; two nodes of margin for the rounding
+    const double R = sqrt(k.indRsq);
+    const auto range = [&](double c, int g, int &lo, int &n) {
+        const double a = floor((c - R) * k.h_inv) - 2, b = ceil((c + R) * k.h_inv) + 2;
+        lo = 0;
+        n = g;
+        if (!(a <= b)) return;   // not a number: all
+        lo = (int)fmin(fmax(a, 0.0), (double)(g - 1));
+        n = (int)fmin(fmax(b, 0.0), (double)(g - 1)) - lo + 1;
+    };
+    BinsFold B{k.bins, o.nodeBin, o.nodeF, hist2, k.nbins, k.gridX, 0, 0, 0, 0};
+    range(ix, k.gridX, B.x0, B.w);
+    range(iy, k.gridY, B.y0, B.h);
+    return B;
+}
+
+hipError_t ordered_fold_forces(const KParams &k, OrderedScratch &o, double *hist2, double ix, double iy,
+                               hipStream_t s) {
+    if (k.nbins + 1 > kFoldBinsMax) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_bins_fold, dim3(1), dim3(kFoldBlock), 0, s, bins_fold(k, o, hist2, ix, iy));
+    return hipGetLastError();
+}
+
+// padGrid (may be null): the padding of its rows is cleared.  force: the forces of
+// the substep before, by the last workgroup.
 __global__ __launch_bounds__(256) void k_point_records(KParams k, PointRec *__restrict__ rec, int *__restrict__ bucket,
                                                       int2 *__restrict__ cells, int *__restrict__ next,
-                                                      double *__restrict__ padGrid) {
+                                                      double *__restrict__ padGrid, BinsFold force) {
+    __shared__ BinsLds L;
+    if (force.bins && blockIdx.x == gridDim.x - 1) {
+        fold_bins(force, L);
+        return;
+    }
     const int pt = blockIdx.x * blockDim.x + threadIdx.x;
     if (padGrid && (size_t)k.gridTotal + pt < k.gp)
         for (int r = 0; r < kGridRows; ++r) padGrid[r * k.gp + k.gridTotal + pt] = 0;
@@ -295,18 +405,22 @@ __global__ __launch_bounds__(256) void k_point_records(KParams k, PointRec *__re
         flag_error(k);
         return;
     }
+    // the cell's list first: the place in it is on its way while the stress is made
+    if (bx >= k.gridX - 2 || by >= k.gridY - 2) flag_error(k);   // nodes outside the grid take nothing
+    const bool in = bx < k.gridX && by < k.gridY;
+    const int at = in ? bx + by * k.gridX : 0;
+    int *cell = reinterpret_cast<int *>(cells + at);
+    int slot = 0;
+    if (in) slot = atomicAdd(cell, 1);
     double t00, t01, t11;
     kirchhoff(F00, F01, F10, F11, k.mu, k.kappa, t00, t01, t11);
     const double m = k.mass;
     const double sc = k.dt * k.vol * k.Dinv;
     rec[pt] = PointRec{make_double2(fx0, fx1), make_double2(m * B00 - sc * t00, m * B01 - sc * t01),
                        make_double2(m * B10 - sc * t01, m * B11 - sc * t11), make_double2(vx * m, vy * m)};
-    if (bx >= k.gridX - 2 || by >= k.gridY - 2) flag_error(k);   // nodes outside the grid take nothing
-    if (bx >= k.gridX || by >= k.gridY) return;
-    int *cell = reinterpret_cast<int *>(cells + (bx + by * k.gridX));
-    const int slot = atomicAdd(cell, 1);
+    if (!in) return;
     if (slot < kCellCap)
-        bucket[kCellCap * (size_t)(bx + by * k.gridX) + slot] = pt;
+        bucket[kCellCap * (size_t)at + slot] = pt;
     else
         next[pt] = atomicExch(cell + 1, pt + 1);
 }
@@ -318,22 +432,26 @@ __global__ __launch_bounds__(256) void k_point_records(KParams k, PointRec *__re
 // where those or a cell's bucket overflow, a node looks its points up one after
 // the other.
 constexpr int kTileN = 8, kTileNodes = kTileN * kTileN, kTileCells = (kTileN + 2) * (kTileN + 2);
+constexpr int kBuckets = 1024;   // of the ranking
 constexpr int kFoldPts = 440, kFoldWords = (kFoldPts + 63) / 64, kFoldList = 4096;
 struct FoldLds {
     union {
         struct {
             unsigned long long mask[kTileCells][kFoldWords];   // a cell's points, by their places in order
-            unsigned char bits[kFoldWords][kTileNodes];        // of a node, per word
+            unsigned long long node[kFoldWords][kTileNodes];   // a node's
+            unsigned short before[kFoldWords][kTileNodes];     // how many of them are in the words before
+            __attribute__((aligned(16))) int count[kBuckets];  // points per bucket of the ranking, then its first place
+            int sorted[kFoldPts];                              // the points, bucket by bucket
         };
         struct {
             Terms t;
             double pad;   // 19 doubles: the places of a wavefront spread over the banks
         } terms[kFoldPts];
     };
-    __attribute__((aligned(16))) int idx[kFoldPts + 8];   // the points as found
-    unsigned char cell[2][kFoldPts];  // the cells of the points as found, and in order: column | row << 4
+    int idx[kFoldPts];                // the points as found
+    unsigned char cell[kFoldPts];     // their cells: column | row << 4
     unsigned short list[kFoldList];   // entry e of node t at e nodes + t: its cell among the nine << 9 | place
-    int wave[2], over, crowded;
+    int wave[4], low[4], high[4], over, crowded;
     double res[3][kTileNodes];
 };
 static_assert(kFoldPts < 512 && kTileCells <= 128, "list entries hold a place in 9 bits; two wavefronts hold the cells");
@@ -366,6 +484,7 @@ static __device__ bool fold_tile(const KParams &k, FoldLds &L, const PointRec *_
     if (t < 128 && lane == 63) L.wave[t >> 6] = inc;
     if (t == 0) L.over = L.crowded = 0;
     for (int e = t; e < kTileCells * kFoldWords; e += 256) L.mask[0][e] = 0;
+    *reinterpret_cast<int4 *>(&L.count[4 * t]) = make_int4(0, 0, 0, 0);
     __syncthreads();
     const int total = L.wave[0] + L.wave[1];
     if (n > kCellCap) L.over = 1;
@@ -375,68 +494,115 @@ static __device__ bool fold_tile(const KParams &k, FoldLds &L, const PointRec *_
     for (int e = 0; e < n; ++e) {
         if (e > 0 && (e & 3) == 0) head = b[e >> 2];
         L.idx[at + e] = (e & 3) == 0 ? head.x : ((e & 3) == 1 ? head.y : ((e & 3) == 2 ? head.z : head.w));
-        L.cell[0][at + e] = (unsigned char)(t % E | t / E << 4);
+        L.cell[at + e] = (unsigned char)(t % E | t / E << 4);
     }
-    if (t < 8) L.idx[total + t] = INT_MAX;
     __syncthreads();
     // the records of the points found at t and t + 256 are on their way while
     // the lists are made
     PointRec r[2];
     int v[2], place[2] = {0, 0};
+    int low = INT_MAX, high = 0;
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
         const int e = t + 256 * q;
         v[q] = e < total ? L.idx[e] : -1;
         r[q] = rec[e < total ? v[q] : 0];
+        if (e < total) {
+            low = min(low, v[q]);
+            high = max(high, v[q]);
+        }
     }
-#pragma unroll 2
-    for (int o = 0; o < total; o += 8) {
-        const int4 w0 = *reinterpret_cast<const int4 *>(&L.idx[o]), w1 = *reinterpret_cast<const int4 *>(&L.idx[o + 4]);
+    // their places in order: buckets over the range of the indices, and within
+    // a bucket the smaller ones counted
 #pragma unroll
-        for (int q = 0; q < 2; ++q)
-            place[q] += (w0.x < v[q]) + (w0.y < v[q]) + (w0.z < v[q]) + (w0.w < v[q]) + (w1.x < v[q]) + (w1.y < v[q]) +
-                        (w1.z < v[q]) + (w1.w < v[q]);
+    for (int d = 32; d > 0; d >>= 1) {
+        low = min(low, __shfl_xor(low, d, 64));
+        high = max(high, __shfl_xor(high, d, 64));
     }
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-        const int e = t + 256 * q, p = place[q];
-        if (e >= total) continue;
-        const unsigned char c = L.cell[0][e];
-        L.cell[1][p] = c;
-        atomicOr(&L.mask[(c >> 4) * E + (c & 15)][p >> 6], 1ull << (p & 63));
+    if (lane == 0) {
+        L.low[t >> 6] = low;
+        L.high[t >> 6] = high;
     }
     __syncthreads();
+    low = min(min(L.low[0], L.low[1]), min(L.low[2], L.low[3]));
+    high = max(max(L.high[0], L.high[1]), max(L.high[2], L.high[3]));
+    const float scale = (float)kBuckets / ((float)(high - low) + 1.f);
+    int bin[2], pos[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+        if (t + 256 * q < total) {
+            bin[q] = min((int)((float)(v[q] - low) * scale), kBuckets - 1);
+            pos[q] = atomicAdd(&L.count[bin[q]], 1);
+        }
+    __syncthreads();
+    {
+        const int4 c = *reinterpret_cast<const int4 *>(&L.count[4 * t]);
+        const int sum = c.x + c.y + c.z + c.w;
+        int run = sum;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(run, d, 64);
+            if (lane >= d) run += o;
+        }
+        if (lane == 63) L.wave[t >> 6] = run;
+        __syncthreads();
+        for (int w = 0; w < t >> 6; ++w) run += L.wave[w];
+        run -= sum;
+        *reinterpret_cast<int4 *>(&L.count[4 * t]) = make_int4(run, run + c.x, run + c.x + c.y, run + c.x + c.y + c.z);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+        if (t + 256 * q < total) L.sorted[L.count[bin[q]] + pos[q]] = v[q];
+    __syncthreads();
     const int nodes = T * T, words = (total + 63) >> 6;
-    unsigned long long mine[2] = {0, 0};   // item t (and t + 256): a word of a node's points
+    int cx[2], cy[2];
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
-        const int e = t + 256 * q, node = e % nodes, w = e / nodes;
-        if (w >= words) continue;
-        const int c = node / T * E + node % T;
+        const int e = t + 256 * q;
+        if (e >= total) continue;
+        const int from = L.count[bin[q]], to = bin[q] + 1 < kBuckets ? L.count[bin[q] + 1] : total;
+        int p = from;
+        for (int o = from; o < to; ++o) p += L.sorted[o] < v[q];
+        place[q] = p;
+        cx[q] = L.cell[e] & 15;
+        cy[q] = L.cell[e] >> 4;
+        atomicOr(&L.mask[cy[q] * E + cx[q]][p >> 6], 1ull << (p & 63));
+    }
+    __syncthreads();
+    for (int e = t; e < nodes * words; e += 256) {
+        const int node = e % nodes, w = e / nodes, c = node / T * E + node % T;
+        unsigned long long m = 0;
 #pragma unroll
-        for (int c9 = 0; c9 < 9; ++c9) mine[q] |= L.mask[c + c9 / 3 * E + c9 % 3][w];
-        L.bits[w][node] = (unsigned char)__popcll(mine[q]);
+        for (int c9 = 0; c9 < 9; ++c9) m |= L.mask[c + c9 / 3 * E + c9 % 3][w];
+        L.node[w][node] = m;
     }
     __syncthreads();
     int len = 0;   // of the node lane's list
     if (lane < nodes)
-        for (int w = 0; w < words; ++w) len += L.bits[w][lane];
+        for (int w = 0; w < words; ++w) {
+            if (t < 64) L.before[w][lane] = (unsigned short)len;
+            len += __popcll(L.node[w][lane]);
+        }
     if (len * nodes > kFoldList) L.crowded = 1;
+    __syncthreads();
+    if (L.crowded) return false;
+    // every point enters the lists of the nodes around it, at the place its
+    // place in order gives
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
-        const int e = t + 256 * q, node = e % nodes, w = e / nodes;
-        if (w >= words) continue;
-        int at = 0;
-        for (int p = 0; p < w; ++p) at += L.bits[p][node];
-        const int X = node % T, Y = node / T;
-        for (unsigned long long m = mine[q]; m; m &= m - 1, ++at) {
-            const int p = w * 64 + __builtin_ctzll(m), c = L.cell[1][p];
-            if (at * nodes < kFoldList)
-                L.list[at * nodes + node] = (unsigned short)((((c >> 4) - Y) * 3 + (c & 15) - X) << 9 | p);
+        if (t + 256 * q >= total) continue;
+        const int p = place[q], w = p >> 6;
+        const unsigned long long smaller = (1ull << (p & 63)) - 1ull;
+#pragma unroll
+        for (int c9 = 0; c9 < 9; ++c9) {
+            const int x = cx[q] - c9 % 3, y = cy[q] - c9 / 3;
+            if (x < 0 || x >= T || y < 0 || y >= T) continue;
+            const int node = y * T + x, at = L.before[w][node] + __popcll(L.node[w][node] & smaller);
+            L.list[at * nodes + node] = (unsigned short)(c9 << 9 | p);
         }
     }
     __syncthreads();
-    if (L.crowded) return false;
 #pragma unroll
     for (int q = 0; q < 2; ++q)
         if (t + 256 * q < total) L.terms[place[q]].t = terms_of(r[q], k.h);
@@ -532,12 +698,14 @@ __global__ __launch_bounds__(256) void k_node_fold(KParams k, double *__restrict
 }
 
 hipError_t ordered_p2g(const KParams &k, double *grid, OrderedScratch &o, bool update, double ix, double iy,
-                       hipStream_t s) {
+                       const OrderedForce *force, hipStream_t s) {
+    if (force && k.nbins + 1 > kFoldBinsMax) return hipErrorInvalidValue;
+    const BinsFold before = force ? bins_fold(k, o, force->hist2, force->ix, force->iy) : BinsFold{};
     PointRec *rec = reinterpret_cast<PointRec *>(o.rec);
     int2 *cells = o.cells[o.flip], *other = o.cells[o.flip ^ 1];
     const int threads = k.nPts > 64 ? k.nPts : 64;   // 64: the rows' padding
-    hipLaunchKernelGGL(k_point_records, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, k, rec, o.bucket,
-                       cells, o.next, update ? grid : nullptr);
+    hipLaunchKernelGGL(k_point_records, dim3((unsigned)((threads + 255) / 256 + (force ? 1 : 0))), dim3(256), 0, s, k, rec,
+                       o.bucket, cells, o.next, update ? grid : nullptr, before);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const dim3 tiles((unsigned)((k.gridX + kTileN - 1) / kTileN), (unsigned)((k.gridY + kTileN - 1) / kTileN));
@@ -549,84 +717,6 @@ hipError_t ordered_p2g(const KParams &k, double *grid, OrderedScratch &o, bool u
                            o.nodeBin, o.nodeF);
     if ((e = hipGetLastError()) == hipSuccess) o.flip ^= 1;
     return e;
-}
-
-// ---------------------------------------------------------------------------
-// ORDERED indenter force: each bin, and the substep's total, summed in node
-// order by one thread each over the nodes in contact.  One workgroup: it looks
-// only at the nodes around the disc, and leaves those in contact in LDS, 1024
-// nodes at a time.
-constexpr int kFoldBlock = 1024;
-__global__ __launch_bounds__(kFoldBlock) void k_bins_fold(double *__restrict__ bins, int nb, const int *__restrict__ nodeBin,
-                                                          const double *__restrict__ nodeF, int gx, int x0, int y0, int w,
-                                                          int h, double *__restrict__ hist2) {
-    __shared__ int bin[kFoldBlock], wave[kFoldBlock / 64];
-    __shared__ double f0[kFoldBlock], f1[kFoldBlock];
-    const int t = threadIdx.x;
-    const bool total = t == nb;
-    double a0 = 0.0, a1 = 0.0;
-    if (t < nb) {
-        a0 = bins[2 * t];
-        a1 = bins[2 * t + 1];
-    }
-    const long nodes = (long)w * h;
-    for (long first = 0; first < nodes; first += kFoldBlock) {
-        const long e = first + t;
-        int b = -1, idx = 0;
-        if (e < nodes) {
-            idx = x0 + (int)(e % w) + (y0 + (int)(e / w)) * gx;
-            b = nodeBin[idx];
-        }
-        const unsigned long long hit = __ballot(b >= 0);
-        if ((t & 63) == 0) wave[t >> 6] = __popcll(hit);
-        __syncthreads();
-        int at = __popcll(hit & ((1ull << (t & 63)) - 1ull)), count = 0;
-        for (int q = 0; q < kFoldBlock / 64; ++q) {
-            if (q < t >> 6) at += wave[q];
-            count += wave[q];
-        }
-        if (b >= 0) {
-            bin[at] = b;
-            f0[at] = nodeF[2 * (size_t)idx];
-            f1[at] = nodeF[2 * (size_t)idx + 1];
-        }
-        __syncthreads();
-        if (t <= nb)
-            for (int q = 0; q < count; ++q)
-                if (total || bin[q] == t) {
-                    a0 += f0[q];
-                    a1 += f1[q];
-                }
-        __syncthreads();
-    }
-    if (t < nb) {
-        bins[2 * t] = a0;
-        bins[2 * t + 1] = a1;
-    } else if (total && hist2) {
-        hist2[0] = a0;
-        hist2[1] = a1;
-    }
-}
-
-hipError_t ordered_fold_forces(const KParams &k, OrderedScratch &o, double *hist2, double ix, double iy,
-                               hipStream_t s) {
-    if (k.nbins + 1 > kFoldBlock) return hipErrorInvalidValue;
-    // the nodes in contact lie within the disc; two nodes of margin for the rounding
-    const double R = sqrt(k.indRsq);
-    const auto range = [&](double c, int g, int &lo, int &n) {
-        const double a = floor((c - R) * k.h_inv) - 2, b = ceil((c + R) * k.h_inv) + 2;
-        lo = 0;
-        n = g;
-        if (!(a <= b)) return;   // not a number: all
-        lo = (int)fmin(fmax(a, 0.0), (double)(g - 1));
-        n = (int)fmin(fmax(b, 0.0), (double)(g - 1)) - lo + 1;
-    };
-    int x0, y0, w, h;
-    range(ix, k.gridX, x0, w);
-    range(iy, k.gridY, y0, h);
-    hipLaunchKernelGGL(k_bins_fold, dim3(1), dim3(kFoldBlock), 0, s, k.bins, k.nbins, o.nodeBin, o.nodeF, k.gridX, x0, y0, w,
-                       h, hist2);
-    return hipGetLastError();
 }
 
 }  // namespace icempm

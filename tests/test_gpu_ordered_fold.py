@@ -39,3 +39,23 @@ def test_fold_matches_the_oracle(gpu_available, squeeze, shuffled):
     assert err == m.error_flag() == 0
     assert np.array_equal(m.points()[:, :n], pts[:, :n], equal_nan=True)
     assert np.array_equal(got, want)
+
+
+def test_forces_of_one_run_and_of_single_substeps(gpu_available):
+    """A run folds a substep's forces with the next one's P2G; the last one's, and
+    those before the bins are cleared at a cycle's start, by themselves."""
+    out = []
+    for runs in ((11,), (1,) * 11, (4, 7)):
+        m = Model(MODE_ORDERED)
+        configure_params(m.prms, INDENT_TINY)
+        m.prms.UpdateEveryNthStep = 4
+        xy, _ = lattice_points(INDENT_TINY)
+        m.load_raw_points(xy, np.zeros(xy.shape[0], np.int16), INDENT_TINY.volume)
+        m.prms.indenter_x_initial += 0.02   # into the block's side
+        m.prms.indenter_y -= 0.03
+        hist = np.concatenate([m.run(n) for n in runs])
+        out.append((hist, m.bins(), m.points()))
+    assert np.abs(out[0][0]).max() > 0 and np.abs(out[0][1]).max() > 0
+    for other in out[1:]:
+        for a, b in zip(out[0], other):
+            assert np.array_equal(a.view(np.uint64), b.view(np.uint64))
