@@ -327,8 +327,8 @@ __global__ __launch_bounds__(64 * kGradWaves) void k_mlp_grad(const float *__res
 // master parameters.  Parameters that are padding stay zero.
 // The BF16 copy used by inference is refreshed from the result.
 // A workgroup of 256 handles 64 parameters: its four wavefronts each sum a
-// quarter of the partial vectors (64 consecutive floats per load, 32 loads in
-// flight: one by one they took 35 us, so they take 10), then the first
+// quarter of the partial vectors (64 consecutive floats per load, 64 loads in
+// flight: one by one they took 35 us, so they take 7), then the first
 // wavefront adds the four sums and takes the step.  One more wavefront adds up
 // the loss.
 __global__ __launch_bounds__(256) void k_mlp_adam(float *__restrict__ params, unsigned short *__restrict__ wbf,
@@ -342,7 +342,7 @@ __global__ __launch_bounds__(256) void k_mlp_adam(float *__restrict__ params, un
     const int i = blockIdx.x * 64 + l;
     float g4 = 0;
     if (i < kParams) {
-        constexpr int kAhead = 32;
+        constexpr int kAhead = 64;
         int p = q;
         for (; p + 4 * (kAhead - 1) < nparts; p += 4 * kAhead) {
             float v[kAhead];
