@@ -722,7 +722,8 @@ int icempm_p2g(icempm_ctx *c) {
         const KParams k = make_kparams(c);
         if (c->mode == ICEMPM_MODE_ORDERED) {
             if ((rc = ensure_ordered(c))) return rc;
-            HIPCHK(c, ordered_p2g(k, c->gridA, c->ord, false, 0, 0, nullptr, c->stream), "cuda_p2g");
+            HIPCHK(c, ordered_records(k, c->ord, nullptr, c->stream), "cuda_p2g");
+            HIPCHK(c, ordered_fold(k, c->gridA, c->ord, false, 0, 0, c->stream), "cuda_p2g");
             return ICEMPM_OK;
         }
         if ((rc = ensure_chunks(c))) return rc;
@@ -790,9 +791,9 @@ int icempm_run_substeps(icempm_ctx *c, int first_step, int n, double *t,
         single::Run run{};
         const bool one = substep_kernel_pays(n, c->prms.nPts) &&
                          ensure_substep(c, indenter_x_initial, indenter_y, run);
-        bool copied = false;    // the points are in the substep kernel's copy
-        OrderedForce force{};   // of the last ORDERED substep, folded with the next one
-        bool pending = false;
+        bool copied = false;   // the points are in the substep kernel's copy
+        // ORDERED: the wavefront kernel's G2P also makes the next substep's records
+        const bool records = c->passKind != 0;
         if (!ordered) {
             HIPCHK(c, launch_fill_f64(c->gridA, c->gp * kGridRows, 0.0, c->stream), "run_substeps");
             HIPCHK(c, particles(c, k, false, true, c->gridA, c->gridA, 0), "run_substeps");
@@ -803,24 +804,31 @@ int icempm_run_substeps(icempm_ctx *c, int first_step, int n, double *t,
         }
         for (int i = 0; i < n; ++i) {
             const int s = first_step + i;
-            if (reset_bins_at_cycle && s % N == 0) {
-                if (pending)
-                    HIPCHK(c, ordered_fold_forces(k, c->ord, force.hist2, force.ix, force.iy, c->stream), "run_substeps");
-                pending = false;
+            if (reset_bins_at_cycle && s % N == 0)
                 HIPCHK(c, launch_fill_f64(c->bins, (size_t)c->nBinsAlloc, 0.0, c->stream), "run_substeps");
-            }
             tt += dt;
             const double ix = indenter_x_initial + tt * V;
             const int rec = ((s + 1) % N == 0) ? 1 : 0;
             double *h2 = c->hist + 2 * (size_t)i;
             const int timeIt = c->timing && (i % c->timingStride == 0);
             if (ordered) {
-                HIPCHK(c, ordered_p2g(k, c->gridA, c->ord, true, ix, indenter_y, pending ? &force : nullptr, c->stream),
-                       "run_substeps");
-                force = OrderedForce{h2, ix, indenter_y};
-                pending = true;
-                if ((rc = launch_particles_timed(c, k, true, false, c->gridA, nullptr, rec, timeIt)))
-                    return rc;
+                if (i == 0 || !records)
+                    HIPCHK(c, ordered_records(k, c->ord, c->gridA, c->stream), "run_substeps");
+                HIPCHK(c, ordered_fold(k, c->gridA, c->ord, true, ix, indenter_y, c->stream), "run_substeps");
+                if (records) {
+                    PassExtra extra{};
+                    if (i + 1 < n) extra.lists = ordered_lists(c->ord);
+                    extra.force = ordered_force(k, c->ord, h2, ix, indenter_y);
+                    int slot;
+                    if ((rc = timing_begin(c, timeIt, slot))) return rc;
+                    HIPCHK(c, exact::launch_g2p_records(k, c->gridA, c->chunkStart, c->nChunks, rec, c->stream, c->passKind,
+                                                        extra), "particle pass");
+                    if ((rc = timing_end(c, slot))) return rc;
+                } else {
+                    HIPCHK(c, ordered_fold_forces(k, c->ord, h2, ix, indenter_y, c->stream), "run_substeps");
+                    if ((rc = launch_particles_timed(c, k, true, false, c->gridA, nullptr, rec, timeIt)))
+                        return rc;
+                }
             } else {
                 const bool last = (i == n - 1);
                 // P and Q, and the values a run ends with, are the particle pass's
@@ -854,8 +862,6 @@ int icempm_run_substeps(icempm_ctx *c, int first_step, int n, double *t,
                 }
             }
         }
-        if (pending)
-            HIPCHK(c, ordered_fold_forces(k, c->ord, force.hist2, force.ix, force.iy, c->stream), "run_substeps");
         *t = tt;
         if (c->timing) {
             if ((rc = collect_timing(c))) return rc;

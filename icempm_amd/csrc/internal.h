@@ -24,6 +24,27 @@ constexpr int kWinY = 4;
 hipError_t launch_fill_f64(double *p, size_t n, double v, hipStream_t s);
 hipError_t launch_fill_i32(int *p, size_t n, int v, hipStream_t s);
 
+// ORDERED mode: where a particle pass leaves the points' records, and the
+// indenter force that one workgroup folds (see ordered_device.h).
+struct PointRec;
+struct PointLists {
+    PointRec *rec;   // null: none
+    int *bucket;
+    int2 *cells;
+    int *next;
+};
+struct BinsFold {
+    double *bins;    // null: nothing to do
+    const int *nodeBin;
+    const double *nodeF;
+    double *hist2;
+    int nb, gx, x0, y0, w, h;
+};
+struct PassExtra {
+    PointLists lists;
+    BinsFold force;
+};
+
 // ---- particles_exact.hip / particles_fast.hip ---------------------------------
 // The particle pass.  do_g2p: gather from gridV (velocities in rows 1-2) and
 // update the particles; do_p2g: scatter the (updated) particles into gridOut
@@ -37,6 +58,9 @@ namespace exact {
 hipError_t launch_particles(const KParams &k, bool do_g2p, bool do_p2g, const double *gridV,
                             double *gridOut, const int *chunkStart, int nChunks, int recordPQ,
                             hipStream_t s, int kind);
+// The G2P of an ORDERED substep (kind 1 or 2) with what the next one needs.
+hipError_t launch_g2p_records(const KParams &k, const double *gridV, const int *chunkStart, int nChunks,
+                              int recordPQ, hipStream_t s, int kind, const PassExtra &extra);
 }
 namespace fast {
 hipError_t launch_particles(const KParams &k, bool do_g2p, bool do_p2g, const double *gridV,
@@ -66,16 +90,17 @@ struct OrderedScratch {
     double *nodeF = nullptr;     // 2 per node
     size_t nPts = 0, nGrid = 0, cleared = 0;
 };
-// A substep's contact forces to add up: its history entry, the indenter where it was.
-struct OrderedForce {
-    double *hist2, ix, iy;
-};
-// The P2G into grid; update: with the grid update, for an indenter at (ix, iy),
-// and the padding of the grid's rows cleared.  force (may be null): the last
-// update's, which are folded before this one's take their place.
-hipError_t ordered_p2g(const KParams &k, double *grid, OrderedScratch &o, bool update, double ix, double iy,
-                       const OrderedForce *force, hipStream_t s);
-// The contact forces of the last update, with the indenter where it was.
+// The points' records and cell lists for the next fold, in the list not in use.
+PointLists ordered_lists(const OrderedScratch &o);
+// Makes them; padGrid (may be null): the padding of its rows is cleared.
+hipError_t ordered_records(const KParams &k, const OrderedScratch &o, double *padGrid, hipStream_t s);
+// The P2G of the records into grid; update: with the grid update, for an
+// indenter at (ix, iy).
+hipError_t ordered_fold(const KParams &k, double *grid, OrderedScratch &o, bool update, double ix, double iy,
+                        hipStream_t s);
+// The contact forces of the last update, with the indenter where it was: as
+// arguments of a fold, and folded by a launch of its own.
+BinsFold ordered_force(const KParams &k, const OrderedScratch &o, double *hist2, double ix, double iy);
 hipError_t ordered_fold_forces(const KParams &k, OrderedScratch &o, double *hist2, double ix, double iy,
                                hipStream_t s);
 

@@ -12,6 +12,7 @@
 #include <climits>
 
 #include "internal.h"
+#include "ordered_device.h"
 
 namespace icempm {
 
@@ -237,8 +238,8 @@ hipError_t launch_update(const KParams &k, double *grid, double ix, double iy, d
 // follow from and enters its base cell's list; every node then collects the
 // points of its nine cells, puts them in order and sums.  What bounds it is
 // latency: few workgroups, each a chain of loads and LDS passes.  A substep of
-// 60,000 points takes 32 us, of which the records 9, the fold 16 (found, ranked,
-// listed and summed in about equal parts) and the G2P 7; through memory, with a
+// 60,000 points takes 31 us, of which the fold 16 (found, ranked, listed and
+// summed in about equal parts) and the G2P with the records 14; through memory, with a
 // counting sort and an insertion sort per node, it took 249 (contributions 20,
 // sort 60, fold 165).  An insertion sort of each node's list in LDS took up to 20
 // us (the points of one row of the load's order lie in two rows of cells), a rank
@@ -255,9 +256,6 @@ static __device__ __forceinline__ void axis_terms(double fx, double h, double *w
 #pragma unroll
     for (int i = 0; i < 3; ++i) d[i] = (i - fx) * h;
 }
-struct PointRec {   // what they follow from, 64 bytes
-    double2 f, a, b, mv;
-};
 static __device__ __forceinline__ Terms terms_of(const PointRec &r, double h) {
     Terms t;
     axis_terms(r.f.x, h, t.wx, t.dx);
@@ -274,86 +272,12 @@ static __device__ __forceinline__ double term(const Terms &t, int i, int j, int 
     return part == 1 ? W * (t.mv0 + (t.A00 * d0 + t.A01 * d1)) : W * (t.mv1 + (t.A10 * d0 + t.A11 * d1));
 }
 
-// ORDERED indenter force: each bin, and the substep's total, summed in node
-// order by one thread each over the nodes in contact.  One workgroup: it looks
-// only at the w x h nodes around the disc, and leaves those in contact in LDS,
-// 256 nodes at a time.  In a run it is one more workgroup of the next substep's
-// k_point_records (a launch of its own takes 4.5 us).
-struct BinsFold {
-    double *bins;   // null: nothing to do
-    const int *nodeBin;
-    const double *nodeF;
-    double *hist2;
-    int nb, gx, x0, y0, w, h;
-};
-constexpr int kFoldBlock = 256, kFoldBinsMax = 1024;   // bins and the total
-struct BinsLds {
-    int bin[kFoldBlock], wave[kFoldBlock / 64];
-    double f0[kFoldBlock], f1[kFoldBlock];
-};
-static __device__ void fold_bins(const BinsFold &B, BinsLds &L) {
-    constexpr int kPer = kFoldBinsMax / kFoldBlock;
-    const int t = threadIdx.x, nb = B.nb;
-    double a0[kPer], a1[kPer];
-#pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-        const int b = t + kFoldBlock * q;
-        a0[q] = b < nb ? B.bins[2 * b] : 0.0;
-        a1[q] = b < nb ? B.bins[2 * b + 1] : 0.0;
-    }
-    const long nodes = (long)B.w * B.h;
-    for (long first = 0; first < nodes; first += kFoldBlock) {
-        const long e = first + t;
-        int b = -1, idx = 0;
-        if (e < nodes) {
-            idx = B.x0 + (int)(e % B.w) + (B.y0 + (int)(e / B.w)) * B.gx;
-            b = B.nodeBin[idx];
-        }
-        const unsigned long long hit = __ballot(b >= 0);
-        if ((t & 63) == 0) L.wave[t >> 6] = __popcll(hit);
-        __syncthreads();
-        int at = __popcll(hit & ((1ull << (t & 63)) - 1ull)), count = 0;
-        for (int q = 0; q < kFoldBlock / 64; ++q) {
-            if (q < t >> 6) at += L.wave[q];
-            count += L.wave[q];
-        }
-        if (b >= 0) {
-            L.bin[at] = b;
-            L.f0[at] = B.nodeF[2 * (size_t)idx];
-            L.f1[at] = B.nodeF[2 * (size_t)idx + 1];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int q = 0; q < kPer; ++q) {
-            const int mine = t + kFoldBlock * q;
-            if (mine <= nb)
-                for (int c = 0; c < count; ++c)
-                    if (mine == nb || L.bin[c] == mine) {
-                        a0[q] += L.f0[c];
-                        a1[q] += L.f1[c];
-                    }
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-        const int b = t + kFoldBlock * q;
-        if (b < nb) {
-            B.bins[2 * b] = a0[q];
-            B.bins[2 * b + 1] = a1[q];
-        } else if (b == nb && B.hist2) {
-            B.hist2[0] = a0[q];
-            B.hist2[1] = a1[q];
-        }
-    }
-}
 __global__ __launch_bounds__(kFoldBlock) void k_bins_fold(BinsFold B) {
     __shared__ BinsLds L;
     fold_bins(B, L);
 }
 
-// The forces of a substep with the indenter at (ix, iy).
-static BinsFold bins_fold(const KParams &k, const OrderedScratch &o, double *hist2, double ix, double iy) {
+BinsFold ordered_force(const KParams &k, const OrderedScratch &o, double *hist2, double ix, double iy) {
     // the nodes in contact lie within the disc; two nodes of margin for the rounding
     const double R = sqrt(k.indRsq);
     const auto range = [&](double c, int g, int &lo, int &n) {
@@ -373,56 +297,21 @@ static BinsFold bins_fold(const KParams &k, const OrderedScratch &o, double *his
 hipError_t ordered_fold_forces(const KParams &k, OrderedScratch &o, double *hist2, double ix, double iy,
                                hipStream_t s) {
     if (k.nbins + 1 > kFoldBinsMax) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_bins_fold, dim3(1), dim3(kFoldBlock), 0, s, bins_fold(k, o, hist2, ix, iy));
+    hipLaunchKernelGGL(k_bins_fold, dim3(1), dim3(kFoldBlock), 0, s, ordered_force(k, o, hist2, ix, iy));
     return hipGetLastError();
 }
 
-// padGrid (may be null): the padding of its rows is cleared.  force: the forces of
-// the substep before, by the last workgroup.
-__global__ __launch_bounds__(256) void k_point_records(KParams k, PointRec *__restrict__ rec, int *__restrict__ bucket,
-                                                      int2 *__restrict__ cells, int *__restrict__ next,
-                                                      double *__restrict__ padGrid, BinsFold force) {
-    __shared__ BinsLds L;
-    if (force.bins && blockIdx.x == gridDim.x - 1) {
-        fold_bins(force, L);
-        return;
-    }
+// padGrid (may be null): the padding of its rows is cleared.
+__global__ __launch_bounds__(256) void k_point_records(KParams k, PointLists lists, double *__restrict__ padGrid) {
     const int pt = blockIdx.x * blockDim.x + threadIdx.x;
     if (padGrid && (size_t)k.gridTotal + pt < k.gp)
         for (int r = 0; r < kGridRows; ++r) padGrid[r * k.gp + k.gridTotal + pt] = 0;
     if (pt >= k.nPts) return;
-    const double *P = k.pts;
+    const double *P = k.pts + pt;
     const size_t pp = k.pp;
-    const double px = P[pp * kRowPosX + pt], py = P[pp * (kRowPosX + 1) + pt];
-    const double vx = P[pp * kRowVelX + pt], vy = P[pp * (kRowVelX + 1) + pt];
-    const double F00 = P[pp * (kRowFe00 + 0) + pt], F01 = P[pp * (kRowFe00 + 1) + pt];
-    const double F10 = P[pp * (kRowFe00 + 2) + pt], F11 = P[pp * (kRowFe00 + 3) + pt];
-    const double B00 = P[pp * (kRowBp00 + 0) + pt], B01 = P[pp * (kRowBp00 + 1) + pt];
-    const double B10 = P[pp * (kRowBp00 + 2) + pt], B11 = P[pp * (kRowBp00 + 3) + pt];
-    int bx, by;
-    double fx0, fx1, w0, w1, w2;
-    if (!stencil(px, k.h_inv, bx, fx0, w0, w1, w2) || !stencil(py, k.h_inv, by, fx1, w0, w1, w2)) {
-        flag_error(k);
-        return;
-    }
-    // the cell's list first: the place in it is on its way while the stress is made
-    if (bx >= k.gridX - 2 || by >= k.gridY - 2) flag_error(k);   // nodes outside the grid take nothing
-    const bool in = bx < k.gridX && by < k.gridY;
-    const int at = in ? bx + by * k.gridX : 0;
-    int *cell = reinterpret_cast<int *>(cells + at);
-    int slot = 0;
-    if (in) slot = atomicAdd(cell, 1);
-    double t00, t01, t11;
-    kirchhoff(F00, F01, F10, F11, k.mu, k.kappa, t00, t01, t11);
-    const double m = k.mass;
-    const double sc = k.dt * k.vol * k.Dinv;
-    rec[pt] = PointRec{make_double2(fx0, fx1), make_double2(m * B00 - sc * t00, m * B01 - sc * t01),
-                       make_double2(m * B10 - sc * t01, m * B11 - sc * t11), make_double2(vx * m, vy * m)};
-    if (!in) return;
-    if (slot < kCellCap)
-        bucket[kCellCap * (size_t)at + slot] = pt;
-    else
-        next[pt] = atomicExch(cell + 1, pt + 1);
+    point_record(k, lists, pt, P[pp * kRowPosX], P[pp * (kRowPosX + 1)], P[pp * kRowVelX], P[pp * (kRowVelX + 1)],
+                 P[pp * (kRowFe00 + 0)], P[pp * (kRowFe00 + 1)], P[pp * (kRowFe00 + 2)], P[pp * (kRowFe00 + 3)],
+                 P[pp * (kRowBp00 + 0)], P[pp * (kRowBp00 + 1)], P[pp * (kRowBp00 + 2)], P[pp * (kRowBp00 + 3)]);
 }
 
 // A workgroup takes a tile of 8 x 8 nodes: the points of its 10 x 10 cells, put in
@@ -697,25 +586,30 @@ __global__ __launch_bounds__(256) void k_node_fold(KParams k, double *__restrict
     cellsNext[idx] = make_int2(0, 0);
 }
 
-hipError_t ordered_p2g(const KParams &k, double *grid, OrderedScratch &o, bool update, double ix, double iy,
-                       const OrderedForce *force, hipStream_t s) {
-    if (force && k.nbins + 1 > kFoldBinsMax) return hipErrorInvalidValue;
-    const BinsFold before = force ? bins_fold(k, o, force->hist2, force->ix, force->iy) : BinsFold{};
-    PointRec *rec = reinterpret_cast<PointRec *>(o.rec);
-    int2 *cells = o.cells[o.flip], *other = o.cells[o.flip ^ 1];
+PointLists ordered_lists(const OrderedScratch &o) {
+    return PointLists{reinterpret_cast<PointRec *>(o.rec), o.bucket, o.cells[o.flip], o.next};
+}
+
+hipError_t ordered_records(const KParams &k, const OrderedScratch &o, double *padGrid, hipStream_t s) {
     const int threads = k.nPts > 64 ? k.nPts : 64;   // 64: the rows' padding
-    hipLaunchKernelGGL(k_point_records, dim3((unsigned)((threads + 255) / 256 + (force ? 1 : 0))), dim3(256), 0, s, k, rec,
-                       o.bucket, cells, o.next, update ? grid : nullptr, before);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_point_records, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, k, ordered_lists(o),
+                       padGrid);
+    return hipGetLastError();
+}
+
+hipError_t ordered_fold(const KParams &k, double *grid, OrderedScratch &o, bool update, double ix, double iy,
+                        hipStream_t s) {
+    const PointLists l = ordered_lists(o);
+    int2 *other = o.cells[o.flip ^ 1];
     const dim3 tiles((unsigned)((k.gridX + kTileN - 1) / kTileN), (unsigned)((k.gridY + kTileN - 1) / kTileN));
     if (update)
-        hipLaunchKernelGGL(k_node_fold<true>, tiles, dim3(256), 0, s, k, grid, rec, o.bucket, cells, other, o.next, ix, iy,
+        hipLaunchKernelGGL(k_node_fold<true>, tiles, dim3(256), 0, s, k, grid, l.rec, l.bucket, l.cells, other, l.next, ix, iy,
                            o.nodeBin, o.nodeF);
     else
-        hipLaunchKernelGGL(k_node_fold<false>, tiles, dim3(256), 0, s, k, grid, rec, o.bucket, cells, other, o.next, ix, iy,
+        hipLaunchKernelGGL(k_node_fold<false>, tiles, dim3(256), 0, s, k, grid, l.rec, l.bucket, l.cells, other, l.next, ix, iy,
                            o.nodeBin, o.nodeF);
-    if ((e = hipGetLastError()) == hipSuccess) o.flip ^= 1;
+    const hipError_t e = hipGetLastError();
+    if (e == hipSuccess) o.flip ^= 1;
     return e;
 }
 
