@@ -653,18 +653,21 @@ static __device__ __forceinline__ void quad_scatter(int lane, int e0, int S, dou
 // gridOut with one atomic per node and component; the workgroups from pGroups
 // on do the rest of the grid update (node_part).
 //
-// What bounds it is instruction issue (660 vector instructions per 64 points in
-// FP32 storage, half of them FP64 at 4 cycles each; HBM is at half a copy's
-// rate) and, below ~100 thousand points, the launch and one chain of memory
-// latencies.  Against a grid update of its own and a particle pass that
-// gathered from global memory and found each wavefront's window anew, a substep
-// of 32 cases / 6.98 million points went from 193 to 167 us (FP32 storage), of
-// 12 cases / 81 thousand points from 18.4 to 9, of 8 cases / 671 thousand points
-// from 35 to 21 (FP64, strengths per grain).  Making a node's velocity in each
-// of the ~2 workgroups that need it costs ~50 instructions per 64 points; it
-// saves a launch, the velocities' trip through memory and the gathers' 6 to 18
-// loads a point.  Four or five wavefronts per SIMD are equally fast, six (80
-// registers) slower.
+// What bounds it: at 7 million points in FP32 storage the memory (647 MB a
+// substep, 131 us at a copy's rate, of which 123 to 194 MB are atomic requests of
+// 64 bytes) and the vector units (660 instructions per 64 points, half of them
+// FP64 at 4 cycles each, 108 us), which overlap in part; below ~100 thousand
+// points the launch and one chain of memory latencies (3.9 us).  Against a grid
+// update of its own and a particle pass that gathered from global memory and
+// found each wavefront's window anew, a substep of 32 cases / 6.98 million points
+// went from 193 to 168 us (FP32 storage), of 12 cases / 81 thousand points from
+// 18.4 to 8.2, of 8 cases / 671 thousand points from 35 to 21 (FP64, strengths
+// per grain).  Making a node's velocity in each of the ~2 workgroups that need it
+// costs ~50 instructions per 64 points; it saves a launch, the velocities' trip
+// through memory and the gathers' 6 to 18 loads a point.  Four or five wavefronts
+// per SIMD are equally fast, six (80 registers) slower.  The grid's workgroups
+// come last: spread among the others their writes slow these down (1.6 million
+// points FP64 47 us against 44).
 //
 // The records, the grid and the point rows lead the arguments, which the
 // kernel receives preloaded in SGPRs.
