@@ -3037,6 +3037,7 @@ int icempm_batch_force_bins(icempm_batch *b, int c, double *out, int nbins) {
 int icempm_batch_read_points(icempm_batch *b, int c, double *soa, size_t pitch) {
     return host_guard(b ? &b->lastError : nullptr, [&]() -> int {
         if (!b || !soa || c < 0 || (size_t)c >= b->hc.size()) return ICEMPM_E_ARG;
+        if (!b->finalized) return bfail(b, ICEMPM_E_STATE, "read_points: batch not finalized");
         if ((size_t)b->hc[c].cp.nPts > pitch) return bfail(b, ICEMPM_E_ARG, "read_points: pitch too small");
         return read_points(b, c, soa, pitch);
     });

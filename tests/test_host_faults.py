@@ -1,0 +1,102 @@
+"""The host code's refusals and its way out of failed allocations, without a
+GPU: the library runs on a stand-in for the HIP runtime (tests/cpp/fake_hip.cpp)
+that counts the launches and fails allocations on request.  What these calls
+must not do is launch a kernel on arrays that are not there."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PRELUDE = r"""
+import ctypes, sys
+import numpy as np
+sys.path.insert(0, ROOT)
+from icempm_amd import SimParams, _lib
+from icempm_amd._lib import *
+F = ctypes.CDLL(None)
+F.fake_hip_live_bytes.restype = F.fake_hip_launches.restype = F.fake_hip_nulls.restype = ctypes.c_long
+F.fake_hip_pending_failure.restype = ctypes.c_long
+H = _lib.hip()
+
+def fail_at(k):
+    F.fake_hip_fail_at(ctypes.c_long(k))
+
+def launches(part):
+    return F.fake_hip_launches(part.encode())
+
+def params(n, gx=64, gy=32):
+    p = SimParams()
+    _lib.host().icempm_simparams_reset(ctypes.byref(p))
+    p.GridX, p.GridY, p.GridTotal, p.nPts, p.nPtsPitch = gx, gy, gx * gy, n, (n + 63) // 64 * 64
+    p.cellsize, p.InitialTimeStep = 0.01, 1e-6
+    p.cellsize_inv, p.Dp_inv = 1. / p.cellsize, 4. / (p.cellsize * p.cellsize)
+    p.ParticleVolume, p.ParticleMass = 1e-4 / 4, 1e-4 / 4 * 900
+    return p
+
+def soa(p):
+    s = np.zeros((16, p.nPtsPitch))
+    i = np.arange(p.nPts)
+    s[3, :p.nPts] = s[8, :p.nPts] = s[11, :p.nPts] = 1
+    s[4, :p.nPts] = (4 + 0.5 * (i % 80)) * p.cellsize
+    s[5, :p.nPts] = (4 + 0.5 * (i // 80)) * p.cellsize
+    return s
+
+def batch(precision, n=700, finalize=True):
+    b = ctypes.c_void_p()
+    assert H.icempm_batch_create(ctypes.byref(b), precision) == 0
+    p = params(n)
+    a = soa(p)
+    assert H.icempm_batch_add_case(b, ctypes.byref(p), ctypes.sizeof(p),
+                                   a.ctypes.data_as(ctypes.POINTER(ctypes.c_double)), p.nPtsPitch) == 0
+    if finalize:
+        assert H.icempm_batch_finalize(b) == 0
+    return b, p
+"""
+
+
+@pytest.fixture(scope="module")
+def fake_hip(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("fake") / "libfake_hip.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-o", so,
+                    os.path.join(ROOT, "tests", "cpp", "fake_hip.cpp")], check=True)
+
+    def run(body):
+        preload = ":".join(x for x in (so, os.environ.get("LD_PRELOAD")) if x)
+        r = subprocess.run([sys.executable, "-c", f"ROOT = {ROOT!r}\n{PRELUDE}\n{body}"], timeout=120,
+                           env=dict(os.environ, LD_PRELOAD=preload), capture_output=True, text=True)
+        assert r.returncode == 0 and "passed" in r.stdout, r.stdout + r.stderr
+    return run
+
+
+@pytest.mark.parametrize("precision", ["BATCH_F64", "BATCH_F32"])
+def test_read_points_of_a_batch_that_is_not_finalized(fake_hip, precision):
+    """The points of a batch before finalize, or after a finalize that failed
+    at any of its allocations: refused, and nothing launched."""
+    fake_hip(f"""
+def refused(b, p):
+    out = np.zeros((16, p.nPtsPitch))
+    before = launches("")
+    rc = H.icempm_batch_read_points(b, 0, out.ctypes.data_as(ctypes.POINTER(ctypes.c_double)), p.nPtsPitch)
+    assert rc == ICEMPM_E_STATE and b"not finalized" in H.icempm_batch_last_error(b), rc
+    assert launches("") == before
+
+b, p = batch({precision}, finalize=False)
+refused(b, p)
+H.icempm_batch_destroy(b)
+for k in range(100):
+    b, p = batch({precision}, finalize=False)
+    fail_at(k)
+    rc = H.icempm_batch_finalize(b)
+    hit = F.fake_hip_pending_failure() < 0
+    fail_at(-1)
+    if not hit:
+        break
+    assert rc == ICEMPM_E_HIP
+    refused(b, p)
+    H.icempm_batch_destroy(b)
+assert rc == 0 and k > 8
+print("passed")
+""")
