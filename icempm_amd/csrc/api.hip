@@ -226,6 +226,7 @@ int ensure_sort_scratch(icempm_ctx *c, size_t n) {
     const size_t tneed = radix_tmp_ints(need);
     if (c->sortTmpCap < tneed) {
         dfree(c->sortTmp);
+        c->sortTmpCap = 0;
         HIPCHK(c, hipMalloc(&c->sortTmp, tneed * sizeof(int)), "sort scratch");
         c->sortTmpCap = tneed;
     }

@@ -100,3 +100,33 @@ for k in range(100):
 assert rc == 0 and k > 8
 print("passed")
 """)
+
+
+def test_sort_after_a_failed_allocation(fake_hip):
+    """A sort that fails at any of its allocations leaves none of its scratch
+    taken for granted: a smaller one afterwards sorts with a workspace."""
+    fake_hip("""
+def sort(ctx, n):
+    xy, g = np.ones((n, 2), np.float32), np.zeros(n, np.int16)
+    return H.icempm_sort_raw_points(ctx, xy.ctypes.data_as(ctypes.POINTER(ctypes.c_float)),
+                                    g.ctypes.data_as(ctypes.POINTER(ctypes.c_int16)), n, ctypes.c_double(100.), 64)
+for k in range(20):
+    ctx = ctypes.c_void_p()
+    assert H.icempm_create(ctypes.byref(ctx)) == 0
+    assert sort(ctx, 5000) == 0
+    fail_at(k)
+    rc = sort(ctx, 100000)
+    hit = F.fake_hip_pending_failure() < 0
+    fail_at(-1)
+    if not hit:
+        break
+    assert rc == ICEMPM_E_HIP
+    for arg in (0, 2):   # the keys, the workspace
+        F.fake_hip_watch(b"k_minmax_key", arg)
+        before = launches("k_minmax_key")
+        assert sort(ctx, 5000) == 0
+        assert launches("k_minmax_key") > before and F.fake_hip_nulls() == 0, (k, arg)
+    H.icempm_destroy(ctx)
+assert rc == 0 and k >= 3
+print("passed")
+""")
