@@ -300,6 +300,7 @@ int build_chunks(icempm_ctx *c) {
     const size_t need = starts.size();
     if (c->chunkCap < need) {
         dfree(c->chunkStart);
+        c->chunkCap = 0;
         HIPCHK(c, hipMalloc(&c->chunkStart, need * sizeof(int)), "chunk table");
         c->chunkCap = need;
     }
@@ -782,6 +783,7 @@ int icempm_run_substeps(icempm_ctx *c, int first_step, int n, double *t,
         const size_t histNeed = 2 * (size_t)n;
         if (histNeed > c->histCap) {
             dfree(c->hist);
+            c->histCap = 0;
             const size_t cap = histNeed < 64 ? 64 : histNeed;
             HIPCHK(c, hipMalloc(&c->hist, cap * sizeof(double)), "run_substeps");
             c->histCap = cap;

@@ -130,3 +130,55 @@ for k in range(20):
 assert rc == 0 and k >= 3
 print("passed")
 """)
+
+
+def test_run_after_a_failed_allocation(fake_hip):
+    """The same for runs: after one that fails at any of its allocations, a
+    shorter one on fewer points has its force history, chunk table and grids."""
+    fake_hip("""
+def load(ctx, n):
+    p = params(n)
+    assert H.icempm_update_constants(ctx, ctypes.byref(p), ctypes.sizeof(p)) == 0
+    return p
+def setup(mode):
+    ctx = ctypes.c_void_p()
+    assert H.icempm_create(ctypes.byref(ctx)) == 0
+    assert H.icempm_set_mode(ctx, mode) == 0
+    p = load(ctx, 300)
+    pg, pp = ctypes.c_size_t(), ctypes.c_size_t()
+    hp, hf = (ctypes.POINTER(ctypes.c_double)() for _ in range(2))
+    assert H.icempm_allocate_arrays(ctx, p.GridTotal, 9000, 2 * p.n_indenter_subdivisions, ctypes.byref(pg),
+                                    ctypes.byref(pp), ctypes.byref(hp), ctypes.byref(hf)) == 0
+    return ctx
+def run(ctx, n):
+    t = ctypes.c_double(0)
+    return H.icempm_run_substeps(ctx, 0, n, ctypes.byref(t), ctypes.c_double(0), ctypes.c_double(0), 1)
+# kernels and the arguments that must be there
+PRESENT = [("k_fill_f64", 0), ("k_update", 4), ("k_particles_wave", 3), ("k_batch_substep", 0), ("k_batch_substep", 11),
+           ("k_chunk_boxes", 5), ("k_pack", 3), ("k_minmax_key", 2), ("k_node_fold", 2), ("k_node_fold", 3),
+           ("k_node_fold", 4), ("k_node_fold", 5)]
+seen = set()
+for mode, short, long in ((MODE_FAST, 40, 4000), (MODE_ORDERED, 4, 4000)):
+    for k in range(40):
+        for name, arg in PRESENT:
+            ctx = setup(mode)
+            assert run(ctx, short) == 0
+            load(ctx, 9000)
+            fail_at(k)
+            run(ctx, long)   # may also go by another path
+            hit = F.fake_hip_pending_failure() < 0
+            fail_at(-1)
+            load(ctx, 300)
+            F.fake_hip_watch(name.encode(), arg)
+            before = launches(name)
+            assert run(ctx, short) == 0, (mode, k)
+            if launches(name) > before:
+                seen.add(name)
+            assert F.fake_hip_nulls() == 0, (mode, k, name, arg)
+            H.icempm_destroy(ctx)
+        if not hit:
+            break
+    assert k > 2
+assert seen == {name for name, _ in PRESENT}, seen
+print("passed")
+""")
