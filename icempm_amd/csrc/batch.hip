@@ -1882,6 +1882,13 @@ void dfree(T *&p) {
     p = nullptr;
 }
 
+// An array that is allocated once: an earlier call may have failed after some of
+// those it needs.
+template <class T>
+hipError_t once(T *&p, size_t bytes) {
+    return p ? hipSuccess : hipMalloc(&p, bytes);
+}
+
 constexpr int kMapBlocks = 256;
 // batches of fewer chunks run as one chain
 constexpr int kChainChunks = 2048;
@@ -2081,9 +2088,11 @@ int upload_chunks(icempm_batch *b) {
     const ChunkRec *before = b->recs;
     const int nBefore = b->nChunks;
     if (n > b->recCap) {
+        // (where it cannot be had, the former table stays: any cut into chunks is correct)
+        ChunkRec *recs = nullptr;
+        BCHK(b, hipMalloc(&recs, n * sizeof(ChunkRec)), "chunk table");
         dfree(b->recs);
-        b->recCap = 0;
-        BCHK(b, hipMalloc(&b->recs, n * sizeof(ChunkRec)), "chunk table");
+        b->recs = recs;
         b->recCap = n;
     }
     BCHK(b, hipMemcpy(b->recs, t.data(), n * sizeof(ChunkRec), hipMemcpyHostToDevice), "chunk table");
@@ -2109,10 +2118,8 @@ int upload_chunks(icempm_batch *b) {
 // slots in sKeys / sVals
 int sort_keys(icempm_batch *b) {
     const int n = b->nPts;
-    if (!b->sKeys) {
-        BCHK(b, hipMalloc(&b->sKeys, (size_t)n * sizeof(int)), "keys");
-        BCHK(b, hipMalloc(&b->sVals, (size_t)n * sizeof(int)), "keys");
-    }
+    BCHK(b, once(b->sKeys, (size_t)n * sizeof(int)), "keys");
+    BCHK(b, once(b->sVals, (size_t)n * sizeof(int)), "keys");
     if (b->precision == ICEMPM_BATCH_F32)
         hipLaunchKernelGGL(k_batch_keys<unsigned int>, dim3((n + 255) / 256), dim3(256), 0, b->stream,
                            static_cast<const unsigned int *>(b->pos), b->pitch, n, b->cases, (int)b->hc.size(),
@@ -2129,10 +2136,8 @@ int sort_keys(icempm_batch *b) {
 // b->hcells on the host
 int current_cells(icempm_batch *b, const int *order = nullptr) {
     const int n = b->nPts;
-    if (!b->dcells) {
-        BCHK(b, hipMalloc(&b->dcells, (size_t)n * sizeof(unsigned)), "cells");
-        BCHK(b, hipHostMalloc(&b->hcells, (size_t)n * sizeof(unsigned), hipHostMallocDefault), "cells");
-    }
+    BCHK(b, once(b->dcells, (size_t)n * sizeof(unsigned)), "cells");
+    if (!b->hcells) BCHK(b, hipHostMalloc(&b->hcells, (size_t)n * sizeof(unsigned), hipHostMallocDefault), "cells");
     if (b->precision == ICEMPM_BATCH_F32)
         hipLaunchKernelGGL(k_batch_cells<unsigned int>, dim3((n + 255) / 256), dim3(256), 0, b->stream,
                            static_cast<const unsigned int *>(b->pos), b->pitch, n, b->cases, (int)b->hc.size(),
@@ -2173,16 +2178,14 @@ int resort(icempm_batch *b) {
     if (n <= 1) return ICEMPM_OK;
     int rc = sort_keys(b);
     if (rc) return rc;
-    if (!b->sKeys2) {
-        BCHK(b, hipMalloc(&b->sKeys2, (size_t)n * sizeof(int)), "re-sort");
-        BCHK(b, hipMalloc(&b->sVals2, (size_t)n * sizeof(int)), "re-sort");
-        BCHK(b, hipMalloc(&b->sTmp, radix_tmp_ints((size_t)n) * sizeof(int)), "re-sort");
-        BCHK(b, hipMalloc(&b->tpos, pos_bytes(b)), "re-sort");
-        BCHK(b, hipMalloc(&b->trest, rest_bytes(b)), "re-sort");
-        BCHK(b, hipMalloc(&b->tcrushed, b->pitch), "re-sort");
-        BCHK(b, hipMalloc(&b->torig, b->pitch * sizeof(int)), "re-sort");
-        if (b->grain) BCHK(b, hipMalloc(&b->tgrain, b->pitch * sizeof(short)), "re-sort");
-    }
+    BCHK(b, once(b->sKeys2, (size_t)n * sizeof(int)), "re-sort");
+    BCHK(b, once(b->sVals2, (size_t)n * sizeof(int)), "re-sort");
+    BCHK(b, once(b->sTmp, radix_tmp_ints((size_t)n) * sizeof(int)), "re-sort");
+    BCHK(b, once(b->tpos, pos_bytes(b)), "re-sort");
+    BCHK(b, once(b->trest, rest_bytes(b)), "re-sort");
+    BCHK(b, once(b->tcrushed, b->pitch), "re-sort");
+    BCHK(b, once(b->torig, b->pitch * sizeof(int)), "re-sort");
+    if (b->grain) BCHK(b, once(b->tgrain, b->pitch * sizeof(short)), "re-sort");
     BCHK(b, radix_sort_pairs(b->sKeys, b->sVals, b->sKeys2, b->sVals2, (size_t)n, b->sTmp, b->stream), "re-sort");
     // the cells in sorted order give the new chunk table, whose chunks then
     // (FP64 storage) arrange their points
@@ -3128,10 +3131,13 @@ int icempm_batch_set_tuning(icempm_batch *b, int knob, int value) {
             if (value != 64 && value != 128 && value != 256)
                 return bfail(b, ICEMPM_E_ARG, "set_tuning: points per chunk is 64, 128 or 256");
             if (value != b->chunkPoints) {
+                const int before = b->chunkPoints;
                 b->chunkPoints = value;
                 if (b->finalized) {
                     BCHK(b, hipStreamSynchronize(b->stream), "set_tuning");
-                    return rebuild_chunks(b);
+                    const int rc = rebuild_chunks(b);
+                    if (rc) b->chunkPoints = before;
+                    return rc;
                 }
             }
             return ICEMPM_OK;
@@ -3172,13 +3178,11 @@ int icempm_batch_checkpoint(icempm_batch *b) {
     return host_guard(b ? &b->lastError : nullptr, [&]() -> int {
         if (!b) return ICEMPM_E_ARG;
         if (!b->finalized) return bfail(b, ICEMPM_E_STATE, "checkpoint: batch not finalized");
-        if (!b->kpos) {
-            BCHK(b, hipMalloc(&b->kpos, pos_bytes(b)), "checkpoint");
-            BCHK(b, hipMalloc(&b->krest, rest_bytes(b)), "checkpoint");
-            BCHK(b, hipMalloc(&b->kcrushed, b->pitch), "checkpoint");
-            BCHK(b, hipMalloc(&b->korig, b->pitch * sizeof(int)), "checkpoint");
-            if (b->grain) BCHK(b, hipMalloc(&b->kgrain, b->pitch * sizeof(short)), "checkpoint");
-        }
+        BCHK(b, once(b->kpos, pos_bytes(b)), "checkpoint");
+        BCHK(b, once(b->krest, rest_bytes(b)), "checkpoint");
+        BCHK(b, once(b->kcrushed, b->pitch), "checkpoint");
+        BCHK(b, once(b->korig, b->pitch * sizeof(int)), "checkpoint");
+        if (b->grain) BCHK(b, once(b->kgrain, b->pitch * sizeof(short)), "checkpoint");
         BCHK(b, hipMemcpyAsync(b->kpos, b->pos, pos_bytes(b), hipMemcpyDeviceToDevice, b->stream), "checkpoint");
         BCHK(b, hipMemcpyAsync(b->krest, b->rest, rest_bytes(b), hipMemcpyDeviceToDevice, b->stream), "checkpoint");
         BCHK(b, hipMemcpyAsync(b->kcrushed, b->crushed, b->pitch, hipMemcpyDeviceToDevice, b->stream), "checkpoint");

@@ -182,3 +182,45 @@ for mode, short, long in ((MODE_FAST, 40, 4000), (MODE_ORDERED, 4, 4000)):
 assert seen == {name for name, _ in PRESENT}, seen
 print("passed")
 """)
+
+
+@pytest.mark.parametrize("precision", ["BATCH_F64", "BATCH_F32"])
+def test_batch_after_a_failed_allocation(fake_hip, precision):
+    """A re-sort, a finer chunk table, a checkpoint, a readback or a run that
+    fails at any of its allocations can be asked for again, and the substeps in
+    between have their chunk table."""
+    fake_hip(f"""
+def calls(b, p):
+    out = np.zeros((16, p.nPtsPitch))
+    return {{"resort": lambda: H.icempm_batch_resort(b),
+             "chunks": lambda: H.icempm_batch_set_tuning(b, BATCH_TUNE_CHUNK, 64),
+             "checkpoint": lambda: H.icempm_batch_checkpoint(b) or H.icempm_batch_restore(b),
+             "points": lambda: H.icempm_batch_read_points(b, 0, out.ctypes.data_as(ctypes.POINTER(ctypes.c_double)),
+                                                          p.nPtsPitch),
+             "run": lambda: H.icempm_batch_run(b, 20, 0)}}
+# kernels of what comes after, and the argument that must be there
+PRESENT = {{"resort": [("k_minmax_key", 0), ("k_minmax_key", 2), ("k_batch_permute", 4), ("k_batch_substep", 0)],
+            "chunks": [("k_batch_cells", 6), ("k_batch_substep", 0)], "checkpoint": [("k_batch_substep", 0)],
+            "points": [("k_read_points", 4)], "run": [("k_batch_substep", 0), ("k_batch_substep", 11)]}}
+for call, watch in PRESENT.items():
+    for name, arg in watch:
+        for k in range(20):
+            b, p = batch({precision}, n=3000)
+            fail_at(k)
+            rc = calls(b, p)[call]()
+            hit = F.fake_hip_pending_failure() < 0
+            fail_at(-1)
+            if hit:
+                assert rc == ICEMPM_E_HIP, (call, k, rc)
+            F.fake_hip_watch(name.encode(), arg)
+            before = launches(name)
+            assert H.icempm_batch_run(b, 8, 0) == 0
+            assert calls(b, p)[call]() == 0, (call, k, H.icempm_batch_last_error(b))
+            assert H.icempm_batch_run(b, 8, 0) == 0
+            assert (launches(name) > before or not hit) and F.fake_hip_nulls() == 0, (call, k, name, arg)
+            H.icempm_batch_destroy(b)
+            if not hit:
+                break
+        assert not hit and k > 0, (call, k)
+print("passed")
+""")
