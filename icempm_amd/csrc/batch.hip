@@ -1135,7 +1135,8 @@ __global__ __launch_bounds__(256, 5) void k_batch_substep(
             celly = by;
         }
         const int lx0 = bx - wx, ly0 = by - wy;
-        const bool winFits = ok && !defer && (unsigned)lx0 < ww2 && (unsigned)ly0 < wh2;
+        const bool inWin = ok && (unsigned)lx0 < ww2 && (unsigned)ly0 < wh2;
+        const bool winFits = inWin && !defer;
         // Every point of a case has the same mass m: the window sums the
         // contributions per unit mass, W (v + (Bp - m^-1 dt V D^-1 tau) d),
         // and the flush multiplies by m once per node.
@@ -1201,9 +1202,11 @@ __global__ __launch_bounds__(256, 5) void k_batch_substep(
                 }
             }
         }
-        if (ok && !winFits && !defer) {
-            // outside the window, or the stencil leaves the grid: node by node
-            widen_bounds(bounds, rec.cs, bx, by, min(bx, gx), min(by, gy));
+        // outside the window, or the stencil leaves the grid: the box of touched
+        // nodes has to hold these (deferred points too, which the map kernel
+        // scatters), and they are added node by node
+        if (ok && !inWin) widen_bounds(bounds, rec.cs, bx, by, min(bx, gx), min(by, gy));
+        if (ok && !inWin && !defer) {
             const double m = cp.mass;
 #pragma unroll 1
             for (int e = 0; e < 9; ++e) {
