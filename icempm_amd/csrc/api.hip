@@ -333,7 +333,9 @@ int ensure_ordered(icempm_ctx *c) {
         o.nGrid = G;
         o.cleared = 0;
     }
-    if (o.cleared != G) {   // a P2G clears for the next one of the same grid
+    // a P2G clears for the next one of the same grid; callers take the mark away
+    // while lists are made, so that a failure in between has them cleared here
+    if (o.cleared != G) {
         for (int2 *cells : o.cells)
             HIPCHK(c, launch_fill_i32(reinterpret_cast<int *>(cells), 2 * o.nGrid, 0, c->stream), "ordered scratch");
         o.cleared = G;
@@ -732,8 +734,10 @@ int icempm_p2g(icempm_ctx *c) {
         const KParams k = make_kparams(c);
         if (c->mode == ICEMPM_MODE_ORDERED) {
             if ((rc = ensure_ordered(c))) return rc;
+            c->ord.cleared = 0;
             HIPCHK(c, ordered_records(k, c->ord, nullptr, c->stream), "cuda_p2g");
             HIPCHK(c, ordered_fold(k, c->gridA, c->ord, false, 0, 0, c->stream), "cuda_p2g");
+            c->ord.cleared = (size_t)c->prms.GridTotal;
             return ICEMPM_OK;
         }
         if ((rc = ensure_chunks(c))) return rc;
@@ -797,6 +801,7 @@ int icempm_run_substeps(icempm_ctx *c, int first_step, int n, double *t,
         const bool ordered = c->mode == ICEMPM_MODE_ORDERED;
         if (ordered) {
             if ((rc = ensure_ordered(c))) return rc;
+            c->ord.cleared = 0;
         }
         if ((rc = ensure_chunks(c))) return rc;
         single::Run run{};
@@ -874,6 +879,7 @@ int icempm_run_substeps(icempm_ctx *c, int first_step, int n, double *t,
             }
         }
         *t = tt;
+        if (ordered) c->ord.cleared = (size_t)c->prms.GridTotal;
         if (c->timing) {
             if ((rc = collect_timing(c))) return rc;
         }

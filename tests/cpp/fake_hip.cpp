@@ -1,6 +1,7 @@
 // A stand-in for the HIP runtime, preloaded by tests of the host code where
 // there is no GPU: device memory is the host's (zeroed), copies copy, kernels
-// are counted by name and not run, and an allocation fails when it is asked to.
+// are counted by name and not run, and an allocation or a launch fails when it is
+// asked to.
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
@@ -23,8 +24,9 @@ std::map<void *, size_t> &blocks() {
     static std::map<void *, size_t> m;
     return m;
 }
-std::string watched;
-int watchedArg = -1;
+std::string watched, failing;
+int watchedArg = -1, lastError = 0;
+long failLaunchAt = -1;
 long nulls = 0, failAt = -1, live = 0;
 int handle;   // what every stream, event and graph is
 constexpr int kOk = 0, kOutOfMemory = 2;
@@ -73,6 +75,11 @@ void fake_hip_watch(const char *part, int arg) {
     nulls = 0;
 }
 long fake_hip_nulls() { return nulls; }
+// the k-th launch from now on of such a kernel fails
+void fake_hip_fail_launch(const char *part, long k) {
+    failing = part;
+    failLaunchAt = k;
+}
 
 void **__hipRegisterFatBinary(const void *) {
     static void *h;
@@ -92,6 +99,7 @@ int __hipPopCallConfiguration(dim3_t *g, dim3_t *b, size_t *s, void **st) {
 }
 int hipLaunchKernel(const void *fn, dim3_t, dim3_t, void **args, size_t, void *) {
     const std::string &name = names()[fn];
+    if (failLaunchAt >= 0 && name.find(failing) != std::string::npos && failLaunchAt-- == 0) return lastError = 719;
     ++launches()[name];
     if (watchedArg >= 0 && name.find(watched) != std::string::npos && !*static_cast<void **>(args[watchedArg])) ++nulls;
     return kOk;
@@ -108,7 +116,11 @@ int hipGetDeviceCount(int *n) {
 }
 int hipSetDevice(int) { return kOk; }
 int hipDeviceSynchronize() { return kOk; }
-int hipGetLastError() { return kOk; }
+int hipGetLastError() {
+    const int e = lastError;
+    lastError = kOk;
+    return e;
+}
 const char *hipGetErrorString(int) { return "an error of the stand-in"; }
 int hipGetSymbolAddress(void **p, const void *) {
     static void *area = std::calloc(1 << 20, 1);

@@ -44,6 +44,23 @@ def soa(p):
     s[5, :p.nPts] = (4 + 0.5 * (i // 80)) * p.cellsize
     return s
 
+def load(ctx, n):
+    p = params(n)
+    assert H.icempm_update_constants(ctx, ctypes.byref(p), ctypes.sizeof(p)) == 0
+    return p
+def setup(mode):
+    ctx = ctypes.c_void_p()
+    assert H.icempm_create(ctypes.byref(ctx)) == 0
+    assert H.icempm_set_mode(ctx, mode) == 0
+    p = load(ctx, 300)
+    pg, pp = ctypes.c_size_t(), ctypes.c_size_t()
+    hp, hf = (ctypes.POINTER(ctypes.c_double)() for _ in range(2))
+    assert H.icempm_allocate_arrays(ctx, p.GridTotal, 9000, 2 * p.n_indenter_subdivisions, ctypes.byref(pg),
+                                    ctypes.byref(pp), ctypes.byref(hp), ctypes.byref(hf)) == 0
+    return ctx
+def run(ctx, n):
+    t = ctypes.c_double(0)
+    return H.icempm_run_substeps(ctx, 0, n, ctypes.byref(t), ctypes.c_double(0), ctypes.c_double(0), 1)
 def batch(precision, n=700, finalize=True):
     b = ctypes.c_void_p()
     assert H.icempm_batch_create(ctypes.byref(b), precision) == 0
@@ -136,23 +153,6 @@ def test_run_after_a_failed_allocation(fake_hip):
     """The same for runs: after one that fails at any of its allocations, a
     shorter one on fewer points has its force history, chunk table and grids."""
     fake_hip("""
-def load(ctx, n):
-    p = params(n)
-    assert H.icempm_update_constants(ctx, ctypes.byref(p), ctypes.sizeof(p)) == 0
-    return p
-def setup(mode):
-    ctx = ctypes.c_void_p()
-    assert H.icempm_create(ctypes.byref(ctx)) == 0
-    assert H.icempm_set_mode(ctx, mode) == 0
-    p = load(ctx, 300)
-    pg, pp = ctypes.c_size_t(), ctypes.c_size_t()
-    hp, hf = (ctypes.POINTER(ctypes.c_double)() for _ in range(2))
-    assert H.icempm_allocate_arrays(ctx, p.GridTotal, 9000, 2 * p.n_indenter_subdivisions, ctypes.byref(pg),
-                                    ctypes.byref(pp), ctypes.byref(hp), ctypes.byref(hf)) == 0
-    return ctx
-def run(ctx, n):
-    t = ctypes.c_double(0)
-    return H.icempm_run_substeps(ctx, 0, n, ctypes.byref(t), ctypes.c_double(0), ctypes.c_double(0), 1)
 # kernels and the arguments that must be there
 PRESENT = [("k_fill_f64", 0), ("k_update", 4), ("k_particles_wave", 3), ("k_batch_substep", 0), ("k_batch_substep", 11),
            ("k_chunk_boxes", 5), ("k_pack", 3), ("k_minmax_key", 2), ("k_node_fold", 2), ("k_node_fold", 3),
@@ -222,5 +222,29 @@ for call, watch in PRESENT.items():
             if not hit:
                 break
         assert not hit and k > 0, (call, k)
+print("passed")
+""")
+
+
+def test_ordered_run_after_a_failed_launch(fake_hip):
+    """An ORDERED run that fails between making the cells' lists and folding them
+    leaves points in the lists: the next call clears them before it adds its own."""
+    fake_hip("""
+def fills(call, *args):
+    before = launches("k_fill_i32")
+    rc = call(*args)
+    return rc, launches("k_fill_i32") - before
+for fails in ("k_particles_wave", "k_node_fold", "k_point_records"):
+    for again in (lambda c: run(c, 4), H.icempm_p2g):
+        ctx = setup(MODE_ORDERED)
+        assert run(ctx, 4) == 0
+        rc, usual = fills(again, ctx)
+        assert rc == 0
+        F.fake_hip_fail_launch(fails.encode(), ctypes.c_long(0))
+        assert run(ctx, 4) == ICEMPM_E_HIP
+        rc, now = fills(again, ctx)
+        assert rc == 0 and now == usual + 2, (fails, now, usual)
+        assert fills(again, ctx) == (0, usual)
+        H.icempm_destroy(ctx)
 print("passed")
 """)
