@@ -51,10 +51,12 @@ struct icempm_ctx {
     bool chunksDirty = true;
 
     // the substep kernel of longer FAST runs: the points' band order and its
-    // chunks (a plan, good until points are loaded), their records and copied
-    // rows, the case's constants (and what was uploaded) with its touched nodes
+    // chunks (a plan, good until points are loaded, for a point count and a grid),
+    // their records and copied rows, the case's constants (and what was uploaded)
+    // with its touched nodes
     int *perm = nullptr, *bandStart = nullptr;
-    int nBand = 0, bandPoints = 0;
+    int nBand = 0, bandPoints = 0, bandX = 0, bandY = 0;
+    double bandCell = 0;
     bool bandDirty = true;
     void *recs = nullptr;
     double *rows = nullptr;
@@ -445,7 +447,8 @@ bool ensure_substep(icempm_ctx *c, double x0, double y0, single::Run &r) {
     r.gx = P.GridX;
     r.gy = P.GridY;
     r.stream = c->stream;
-    if (ok && (c->bandDirty || c->bandPoints != P.nPts)) {
+    if (ok && (c->bandDirty || c->bandPoints != P.nPts || c->bandX != P.GridX || c->bandY != P.GridY ||
+               c->bandCell != P.cellsize)) {
         std::vector<int> starts;
         dfree(c->bandStart);
         dfree(c->recs);
@@ -458,6 +461,9 @@ bool ensure_substep(icempm_ctx *c, double x0, double y0, single::Run &r) {
         r.nChunks = c->nBand;
         ok = ok && single::slots(r, c->vals, c->perm) == hipSuccess;
         c->bandPoints = P.nPts;
+        c->bandX = P.GridX;
+        c->bandY = P.GridY;
+        c->bandCell = P.cellsize;
         c->bandDirty = !ok;
     }
     if (!ok) {
@@ -648,7 +654,7 @@ int icempm_update_constants(icempm_ctx *c, const void *simparams, size_t nbytes)
             HIPCHK(c, hipStreamSynchronize(c->stream), "cuda_update_constants: gprms");
         }
         c->haveParams = true;
-        c->chunksDirty = c->bandDirty = true;
+        c->chunksDirty = true;
         // gpu_error_indicator <- error_code (gpu_implementation5.cu:474)
         HIPCHK(c, launch_fill_i32(c->dErr, 1, c->errorCode.load(), c->stream),
                "gpu_error_indicator initialization");
@@ -1098,7 +1104,7 @@ int icempm_set_tuning(icempm_ctx *c, int knob, int value) {
         switch (knob) {
         case ICEMPM_TUNE_PASS_KIND:
             if (value < 0 || value > 2) return fail(c, ICEMPM_E_ARG, "set_tuning: pass kind is 0, 1 or 2");
-            if ((value == 0) != (c->passKind == 0)) c->chunksDirty = c->bandDirty = true;   // the chunk rule differs
+            if ((value == 0) != (c->passKind == 0)) c->chunksDirty = true;   // the chunk rule differs
             c->passKind = value;
             return ICEMPM_OK;
         default:

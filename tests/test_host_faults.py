@@ -248,3 +248,30 @@ for fails in ("k_particles_wave", "k_node_fold", "k_point_records"):
         H.icempm_destroy(ctx)
 print("passed")
 """)
+
+
+def test_new_constants_keep_the_order_of_the_points(fake_hip):
+    """The band order of a longer FAST run depends on the points and the grid
+    alone: constants uploaded between runs do not have it made again, points do,
+    and so do another point count and another grid."""
+    fake_hip("""
+def plans(ctx, change):
+    before = launches("k_slots")
+    assert change() == 0 and run(ctx, 40) == 0
+    return launches("k_slots") - before
+def constants(**kw):
+    p = params(300, **{k: kw.pop(k) for k in ("gx", "gy") if k in kw})
+    for name, value in kw.items():
+        setattr(p, name, value)
+    return lambda: H.icempm_update_constants(ctx, ctypes.byref(p), ctypes.sizeof(p))
+ctx = setup(MODE_FAST)
+assert plans(ctx, lambda: 0) == 1 and plans(ctx, lambda: 0) == 0
+assert plans(ctx, constants()) == 0
+assert plans(ctx, constants(IceTensileStrength=2e6, IndVelocity=0.3, InitialTimeStep=2e-6)) == 0
+assert plans(ctx, constants(nPts=299)) == 1
+assert plans(ctx, constants()) == 1
+assert plans(ctx, lambda: H.icempm_transfer_points_to_device(ctx)) == 1
+assert plans(ctx, constants(gx=32, gy=64)) == 1
+assert plans(ctx, constants(gx=32, gy=64, cellsize=0.02, cellsize_inv=1. / 0.02, Dp_inv=4. / (0.02 * 0.02))) == 1
+print("passed")
+""")
