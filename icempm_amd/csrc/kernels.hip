@@ -281,7 +281,8 @@ BinsFold ordered_force(const KParams &k, const OrderedScratch &o, double *hist2,
     // the nodes in contact lie within the disc; two nodes of margin for the rounding
     const double R = sqrt(k.indRsq);
     const auto range = [&](double c, int g, int &lo, int &n) {
-        const double a = floor((c - R) * k.h_inv) - 2, b = ceil((c + R) * k.h_inv) + 2;
+        // (by h, which places the nodes; h_inv places the points)
+        const double a = floor((c - R) / k.h) - 2, b = ceil((c + R) / k.h) + 2;
         lo = 0;
         n = g;
         if (!(a <= b)) return;   // not a number: all
