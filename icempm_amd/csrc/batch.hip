@@ -2405,6 +2405,7 @@ bool case_constants(const icy::SimParams &P, double x0, double y0, void *out) {
     if (!(P.GrainVariability == P.GrainVariability)) return false;
     CaseParams c;
     fill_case(c, P);
+    if (c.slope < 0) return false;   // its tension line is compared by squares
     c.x0 = x0;
     c.y0 = y0;
     std::memset(out, 0, kCaseBytes);

@@ -275,3 +275,21 @@ assert plans(ctx, constants(gx=32, gy=64)) == 1
 assert plans(ctx, constants(gx=32, gy=64, cellsize=0.02, cellsize_inv=1. / 0.02, Dp_inv=4. / (0.02 * 0.02))) == 1
 print("passed")
 """)
+
+
+def test_strengths_of_the_one_kernel_substep(fake_hip):
+    """A negative shear strength puts the tension line below every q, which the
+    one-kernel substep's comparison of squares does not hold for: such a run takes
+    the grid update and the particle pass, others of its length the one kernel."""
+    fake_hip("""
+for shear, one in ((1e6, True), (0., True), (-1e6, False)):
+    ctx = setup(MODE_FAST)
+    p = params(300)
+    p.IceCompressiveStrength, p.IceTensileStrength, p.IceShearStrength = 1e7, 1e6, shear
+    assert H.icempm_update_constants(ctx, ctypes.byref(p), ctypes.sizeof(p)) == 0
+    before = launches("k_batch_substep")
+    assert run(ctx, 40) == 0
+    assert (launches("k_batch_substep") > before) == one, shear
+    H.icempm_destroy(ctx)
+print("passed")
+""")
