@@ -1605,23 +1605,20 @@ __global__ void k_chunk_order(const ChunkRec *__restrict__ recs, int nChunks, co
     if ((int)threadIdx.x < n) out[beg + threadIdx.x] = in[beg + chunk_point((int)threadIdx.x, recs[ch].shape)];
 }
 
-// A case's points in the layout they came in: rows 0 and 3-15 of the point SoA
-// (row r > 2 at out + (r - 2) pitch), every point at its index within the case,
-// the padding zero.  bad: set when the slot map is not one.
+// Points [first, first + pitch) of a case in the layout they came in: rows 0 and
+// 3-15 of the point SoA (row r > 2 at out + (r - 2) pitch), every point at its
+// index within the case less first.  bad: set when the slot map is not one.
 template <bool F32>
-__global__ __launch_bounds__(256) void k_read_points(Rows<F32> S, const int *__restrict__ orig, CaseParams cp, int pitch,
-                                                     double *__restrict__ out, int *__restrict__ bad) {
+__global__ __launch_bounds__(256) void k_read_points(Rows<F32> S, const int *__restrict__ orig, CaseParams cp, int first,
+                                                     int pitch, double *__restrict__ out, int *__restrict__ bad) {
     const int k = blockIdx.x * 256 + threadIdx.x, n = cp.nPts, o = cp.ptOffset;
-    if (k >= pitch) return;
-    if (k >= n) {
-        for (int r = 1; r < 14; ++r) out[(size_t)r * pitch + k] = 0;
-        return;
-    }
-    const int slot = o + k, i = orig[slot] - o;
-    if (i < 0 || i >= n) {
+    if (k >= n) return;
+    const int slot = o + k, i = orig[slot] - o - first;
+    if (i < -first || i >= n - first) {
         *bad = 1;
         return;
     }
+    if (i < 0 || i >= pitch) return;   // of another part
     const size_t pp = S.pitch;
     const auto *__restrict__ R = S.rest;
     double v[13];   // Jp, x, y, v, Fe, Bp
@@ -1683,7 +1680,8 @@ __global__ void k_batch_permute(Rows<F32> src, Rows<F32> dst, const int *__restr
 using namespace icempm;
 using namespace icempm::batch;
 
-constexpr int kReadGroups = 4;   // groups of rows of a readback
+constexpr int kReadGroups = 4;       // groups of rows of a readback
+constexpr int kReadPart = 1 << 20;   // points of a case it brings down at a time (a multiple of 64)
 
 struct icempm_batch {
     int precision = ICEMPM_BATCH_F64;
@@ -1810,7 +1808,7 @@ struct icempm_batch {
     int kChunkPoints = 256;
     double runMs = 0;   // device time of the last run's segments + re-sorts
 
-    // scratch of read_points, for cases of up to rbPitch points
+    // scratch of read_points, for up to rbPitch points at a time
     std::mutex rbLock;
     double *rbDev = nullptr, *rbHost = nullptr;
     size_t rbPitch = 0;
@@ -2228,11 +2226,12 @@ int resort(icempm_batch *b) {
     return ICEMPM_OK;
 }
 
-// Scratch of read_points, for the largest case: the device rows, the pinned
-// rows they come down to and an event per group of rows.
+// Scratch of read_points, for the largest case or kReadPart of its points: the
+// device rows, the pinned rows they come down to and an event per group of rows.
 int read_scratch(icempm_batch *b) {
     size_t pitch = 0;
     for (const auto &h : b->hc) pitch = std::max(pitch, ((size_t)h.cp.nPts + 63) / 64 * 64);
+    pitch = std::min(pitch, (size_t)kReadPart);
     for (hipEvent_t &e : b->rbEvent)
         if (!e) BCHK(b, hipEventCreateWithFlags(&e, hipEventDisableTiming), "read_points");
     if (b->rbPitch >= pitch) return ICEMPM_OK;
@@ -2250,56 +2249,65 @@ int read_scratch(icempm_batch *b) {
 // groups of rows to pinned memory and copied to the caller's from there, a group
 // while the next comes down.  What it takes is the caller's pages: 7 million
 // points (32 cases, 0.9 GB) in 73 ms, where a copy per row and the ordering
-// on the host took 192.  (Helper threads copy no faster: 84 ms with eight.)
+// on the host took 192.  (Helper threads copy no faster: 84 ms with eight.)  A
+// case of more than kReadPart points goes by parts of that many, which bounds the
+// scratch (112 bytes a point on either side); the kernel looks at all slots for
+// each, 4 bytes a slot.
 int read_points(icempm_batch *b, int c, double *soa, size_t pitch) {
     const CaseParams &cp = b->hc[c].cp;
     std::lock_guard<std::mutex> lock(b->rbLock);
-    const size_t dp = ((size_t)cp.nPts + 63) / 64 * 64;   // pitch on the device
     int rc = read_scratch(b);
     if (rc) return rc;
-    int *bad = reinterpret_cast<int *>(b->rbDev + 14 * dp);
-    BCHK(b, launch_fill_f64(b->rbDev, dp, 0.0, b->stream), "read_points");
-    BCHK(b, launch_fill_i32(bad, 1, 0, b->stream), "read_points");
-    const dim3 nb((unsigned)((dp + 255) / 256));
-    if (b->precision == ICEMPM_BATCH_F32) {
-        Rows<true> S{static_cast<unsigned int *>(b->pos), reinterpret_cast<float *>(b->rest), b->crushed, b->grain, b->pitch};
-        hipLaunchKernelGGL(k_read_points<true>, nb, dim3(256), 0, b->stream, S, b->orig, cp, (int)dp, b->rbDev, bad);
-    } else {
-        Rows<false> S{static_cast<double *>(b->pos), reinterpret_cast<double *>(b->rest), b->crushed, b->grain, b->pitch};
-        hipLaunchKernelGGL(k_read_points<false>, nb, dim3(256), 0, b->stream, S, b->orig, cp, (int)dp, b->rbDev, bad);
-    }
-    BCHK(b, hipGetLastError(), "read_points");
     constexpr int kGroups = kReadGroups, kRows = 14;
-    int *hostBad = reinterpret_cast<int *>(b->rbHost + kRows * dp);
-    BCHK(b, hipMemcpyAsync(hostBad, bad, sizeof(int), hipMemcpyDeviceToHost, b->stream), "read_points");
     const auto group = [](int g) { return g * kRows / kGroups; };   // first row
-    for (int g = 0; g < kGroups; ++g) {
-        BCHK(b, hipMemcpyAsync(b->rbHost + group(g) * dp, b->rbDev + group(g) * dp,
-                               (size_t)(group(g + 1) - group(g)) * dp * sizeof(double), hipMemcpyDeviceToHost, b->stream),
-             "read_points");
-        BCHK(b, hipEventRecord(b->rbEvent[g], b->stream), "read_points");
-    }
-    const size_t n = (size_t)cp.nPts, row = pitch * sizeof(double);
+    const size_t n = (size_t)cp.nPts;
     unsigned char *out = reinterpret_cast<unsigned char *>(soa);
-    for (int g = 0; g < kGroups; ++g) {
-        if (g == 1) std::memset(soa + pitch, 0, 2 * row);   // P and Q: a batch keeps none
-        BCHK(b, hipEventSynchronize(b->rbEvent[g]), "read_points");
-        for (int d = group(g); d < group(g + 1); ++d) {
-            const double *src = b->rbHost + (size_t)d * dp;
-            if (d > 0) {
-                double *dst = soa + (size_t)(d + 2) * pitch;
-                std::memcpy(dst, src, n * sizeof(double));
-                std::memset(dst + n, 0, row - n * sizeof(double));
-            } else {   // the flags, and the grain ids at byte pitch + 2 i
-                const unsigned char *u8 = reinterpret_cast<const unsigned char *>(src);
-                std::memset(out, 0, row);
-                std::memcpy(out, u8, n);
-                std::memcpy(out + pitch, u8 + dp, 2 * n);
+    for (size_t first = 0; first < n; first += kReadPart) {
+        const size_t count = std::min(n - first, (size_t)kReadPart), dp = (count + 63) / 64 * 64;   // points, pitch on the device
+        int *bad = reinterpret_cast<int *>(b->rbDev + kRows * dp);
+        BCHK(b, launch_fill_f64(b->rbDev, dp, 0.0, b->stream), "read_points");
+        BCHK(b, launch_fill_i32(bad, 1, 0, b->stream), "read_points");
+        const dim3 nb((unsigned)((n + 255) / 256));
+        if (b->precision == ICEMPM_BATCH_F32) {
+            Rows<true> S{static_cast<unsigned int *>(b->pos), reinterpret_cast<float *>(b->rest), b->crushed, b->grain, b->pitch};
+            hipLaunchKernelGGL(k_read_points<true>, nb, dim3(256), 0, b->stream, S, b->orig, cp, (int)first, (int)dp, b->rbDev,
+                               bad);
+        } else {
+            Rows<false> S{static_cast<double *>(b->pos), reinterpret_cast<double *>(b->rest), b->crushed, b->grain, b->pitch};
+            hipLaunchKernelGGL(k_read_points<false>, nb, dim3(256), 0, b->stream, S, b->orig, cp, (int)first, (int)dp, b->rbDev,
+                               bad);
+        }
+        BCHK(b, hipGetLastError(), "read_points");
+        int *hostBad = reinterpret_cast<int *>(b->rbHost + kRows * dp);
+        BCHK(b, hipMemcpyAsync(hostBad, bad, sizeof(int), hipMemcpyDeviceToHost, b->stream), "read_points");
+        for (int g = 0; g < kGroups; ++g) {
+            BCHK(b, hipMemcpyAsync(b->rbHost + group(g) * dp, b->rbDev + group(g) * dp,
+                                   (size_t)(group(g + 1) - group(g)) * dp * sizeof(double), hipMemcpyDeviceToHost, b->stream),
+                 "read_points");
+            BCHK(b, hipEventRecord(b->rbEvent[g], b->stream), "read_points");
+        }
+        const bool end = first + count == n;   // the rows' padding with the last points
+        const size_t pad = end ? (pitch - n) * sizeof(double) : 0;
+        for (int g = 0; g < kGroups; ++g) {
+            if (g == 1 && first == 0) std::memset(soa + pitch, 0, 2 * pitch * sizeof(double));   // P and Q: a batch keeps none
+            BCHK(b, hipEventSynchronize(b->rbEvent[g]), "read_points");
+            for (int d = group(g); d < group(g + 1); ++d) {
+                const double *src = b->rbHost + (size_t)d * dp;
+                if (d > 0) {
+                    double *dst = soa + (size_t)(d + 2) * pitch + first;
+                    std::memcpy(dst, src, count * sizeof(double));
+                    std::memset(dst + count, 0, pad);
+                } else {   // the flags, and the grain ids at byte pitch + 2 i
+                    const unsigned char *u8 = reinterpret_cast<const unsigned char *>(src);
+                    if (first == 0) std::memset(out, 0, pitch * sizeof(double));
+                    std::memcpy(out + first, u8, count);
+                    std::memcpy(out + pitch + 2 * first, u8 + dp, 2 * count);
+                }
             }
         }
+        BCHK(b, hipStreamSynchronize(b->stream), "read_points");
+        if (*hostBad) return bfail(b, ICEMPM_E_STATE, "read_points: slot map corrupt");
     }
-    BCHK(b, hipStreamSynchronize(b->stream), "read_points");
-    if (*hostBad) return bfail(b, ICEMPM_E_STATE, "read_points: slot map corrupt");
     return ICEMPM_OK;
 }
 
