@@ -315,7 +315,7 @@ static __device__ __forceinline__ double yield_residual(const KParams &k, const 
 // has left it takes the general paths).
 struct __attribute__((aligned(16))) ChunkRec {
     int beg;          // first slot
-    unsigned shape;   // FP32 storage: points; FP64: lanes per row | rows with one lane more << 8 | rows << 16
+    unsigned shape;   // points in band order: their number; else lanes per row | rows with one lane more << 8 | rows << 16
     int cs, gofs;     // the case and its first grid node
     unsigned dims;    // GridX | GridY << 16
     unsigned org;     // the box: first column | first row << 16
@@ -325,24 +325,28 @@ struct __attribute__((aligned(16))) ChunkRec {
 };
 constexpr int kBoxEvery = 8;
 
-// The points of a chunk, FP32 storage: in band order, 64 a wavefront.  The four
-// lanes of a quad mostly hold the points of a cell and add up their
-// contributions before these reach the wavefront's window.  That keeps the sums
-// of a node in the order quad, wavefront, grid.
+// The points of a chunk, FP32 storage, or workgroups of fewer than four
+// wavefronts: in band order, 64 a wavefront.  The four lanes of a quad mostly hold
+// the points of a cell and add up their contributions before these reach the
+// window (FP32: the wavefront's, which keeps the sums of a node in the order quad,
+// wavefront, grid).
 //
-// FP64 storage: in rows of a wavefront each, as few as hold them and filled
-// evenly; slot s holds the point that band order puts at chunk_point(s, shape).
-// Consecutive points go to the same lane of consecutive rows, so that the 64
+// FP64 storage, four wavefronts: in rows of a wavefront each, as few as hold them
+// and filled evenly; slot s holds the point that band order puts at chunk_point(s,
+// shape).  Consecutive points go to the same lane of consecutive rows, so that the 64
 // lanes of a wavefront hold different cells and their LDS atomics, 27 a point
 // into one window for the workgroup, go to different nodes (four lanes of one
 // cell at one node take five times as long).
 //
 // The latter takes fewer instructions (8 cases FP64, 671 thousand points: 22.6
 // us a substep, 25.0 in band order; 1.6 million points FP64: 50 and 51), but
-// adds the terms in another order.  FP64 points differ by rounding then; the rounding of FP32 storage and
-// the yield branches carry a study's points past 1e-5 of the other order's
-// within 4000 substeps in most runs, where two runs of one order mostly agree
-// to the bit.
+// adds the terms in another order.  FP64 points differ by rounding then; the
+// rounding of FP32 storage and the yield branches carry a study's points past 1e-5
+// of the other order's within 4000 substeps in most runs, where two runs of one
+// order mostly agree to the bit.  Chunks of 64 points keep band order: in one row
+// their cells' points are neighbours anyway (32 cases, 6.98 million points: 242 us,
+// 480 with an LDS atomic for each of a point's 27 sums).
+constexpr bool band_order(bool f32, int waves) { return f32 || waves < 4; }
 static __host__ __device__ inline unsigned chunk_shape(int n) {
     const int rows = (n + 63) / 64;
     return (unsigned)(n / rows) | (unsigned)(n % rows) << 8 | (unsigned)rows << 16;
@@ -362,26 +366,30 @@ static __host__ __device__ inline int chunk_point(int slot, unsigned shape) {
 // kPatch points outside the box.  64 points in band order, four to a cell, touch
 // 10 x 4 nodes and 256 points 34 x 4; the space (25.6 KB with a window per
 // wavefront, 19.6 KB with one) holds more rows, for points that have moved out
-// of their band.
-constexpr int kWaveWin = 160, kWin = 384, kTile = 384;   // nodes x row stride
+// of their band.  Workgroups of one or two wavefronts, for chunks of at most 64
+// or 128 points, have room for the box of a chunk's two rows and no more, so that
+// as many wavefronts fit a CU.
+constexpr int kWaveWin = 160;            // of a wavefront's window (FP32): nodes x row stride
+constexpr int box_space(int waves) { return waves == 4 ? 384 : 240; }   // of the tile, and of the window (FP64)
 constexpr int kWinCols = 40;
 constexpr int kPatch = 7;                // x 9 nodes: one load round of a wavefront
 constexpr int kChunkCols = 58;           // base cells a chunk may span: 60 columns of nodes
+static_assert(4 * (kChunkCols + 2) <= box_space(1), "the box of two rows of cells fits");
 
 // The row stride of a wavefront's window: rows next to each other lie on
 // different LDS banks (a row of S doubles shifts them by 2 S of 64).
 static __device__ __forceinline__ int win_stride(int w) { return w <= 16 ? 20 : (w <= 32 ? 36 : kWinCols); }
 
 // The box of the base cells [x0, x1] x [y0, y1] as a record's org, ext and
-// inv; false if it does not fit the space.  A tile row of T 16-byte entries, T
+// inv; false if it does not fit the space (of box_space).  A tile row of T 16-byte entries, T
 // = 8 mod 16, and a window row of S doubles, S = 16 mod 32, put the two cell
 // rows of a band on different LDS banks; a taller box packs its rows.
-static __device__ __forceinline__ bool set_box(ChunkRec &r, int x0, int y0, int x1, int y1) {
+static __device__ __forceinline__ bool set_box(ChunkRec &r, int x0, int y0, int x1, int y1, int space) {
     const int w = x1 + 3 - x0, h = y1 + 3 - y0;
-    if (w > 128 || h > 128 || w * h > kTile) return false;
+    if (w > 128 || h > 128 || w * h > space) return false;
     int T = ((w + 7) >> 4) * 16 + 8, S = ((w + 15) >> 5) * 32 + 16;
-    if (T * h > kTile) T = w;
-    if (S * h > kWin) S = w;
+    if (T * h > space) T = w;
+    if (S * h > space) S = w;
     r.org = (unsigned)x0 | (unsigned)y0 << 16;
     r.ext = (unsigned)w | (unsigned)h << 8 | (unsigned)T << 16 | (unsigned)S << 24;
     r.inv = 65535u / (unsigned)w + 1u;
@@ -455,7 +463,7 @@ static __device__ __forceinline__ bool node_velocity(const CaseParams &cp, doubl
 // The grid side of a substep: the workgroups after the particle ones each
 // take kNodeBlk nodes of one case.  They clear the grid that the next
 // substep scatters into and add up the indenter's force; nothing else of the
-// grid update is left to them, since every wavefront makes the velocities of
+// grid update is left to them, since every workgroup makes the velocities of
 // its own box.  bounds holds, per case, the box of all nodes that the P2G has
 // ever touched since the run's fresh start (columns and rows of the least and
 // greatest, widened by the passes): outside it (and a border of one) the
@@ -468,23 +476,26 @@ struct NodeWork {
     double *bins;
 };
 
+template <int kWaves>
 static __device__ __forceinline__ void node_part(const NodeWork &nw, int block, const CaseParams *__restrict__ cases,
                                                  const double *__restrict__ grid, size_t gpitch, const int4 *bounds,
                                                  double t, double *lds) {
-    const int2 nb = nw.blocks ? nw.blocks[block] : make_int2(0, block * kNodeBlk);
+    constexpr int kParts = 4 / kWaves, kNodes = kNodeBlk / kParts;   // smaller workgroups take a part of a block
+    int2 nb = nw.blocks ? nw.blocks[block / kParts] : make_int2(0, block / kParts * kNodeBlk);
+    if constexpr (kParts > 1) nb.y += block % kParts * kNodes;
     const CaseParams &cp = cases[nb.x];
     const int4 bd = bounds[nb.x];
     const int x0 = bd.x - 1, y0 = bd.y - 1, x1 = bd.z + 1, y1 = bd.w + 1;
     // rows of the block: (node + 0.5) / gx lies >= 0.5 / gx >= 2^-17 from an
     // integer and is computed to within 2^-23, so its floor is the row
     const int first = (int)(((double)nb.y + 0.5) * cp.gxInv);
-    const int last = (int)(((double)min(nb.y + kNodeBlk, cp.gridTotal) - 0.5) * cp.gxInv);
-    if (bd.z < 0 || last < y0 || first > y1) return;   // uniform: nothing was ever touched here
+    const int last = (int)(((double)min(nb.y + kNodes, cp.gridTotal) - 0.5) * cp.gxInv);
+    if ((kParts > 1 && nb.y >= cp.gridTotal) || bd.z < 0 || last < y0 || first > y1) return;   // uniform: nothing was ever touched here
     if (threadIdx.x < 3) lds[threadIdx.x] = 0;
     __syncthreads();
     const double ind_x = cp.x0 + t * cp.indV;
 #pragma unroll
-    for (int q = 0; q < kNodeBlk; q += 256) {
+    for (int q = 0; q < kNodes; q += 64 * kWaves) {
         const int local = nb.y + q + (int)threadIdx.x;
         const int iy = (int)(((double)local + 0.5) * cp.gxInv), ix = local - iy * cp.gx;
         if (local >= cp.gridTotal || ix < x0 || ix > x1 || iy < y0 || iy > y1) continue;
@@ -671,18 +682,26 @@ static __device__ __forceinline__ void quad_scatter(int lane, int e0, int S, dou
 //
 // The records, the grid and the point rows lead the arguments, which the
 // kernel receives preloaded in SGPRs.
-template <bool F32, bool G2P, int RMAP>
-__global__ __launch_bounds__(256, 5) void k_batch_substep(
+//
+// kWaves: wavefronts of a workgroup, for chunks of at most 64 kWaves points.  Fewer
+// than four only where a caller asks for smaller chunks.  us a substep in chunks of
+// 256, 128 and 64: 32 cases / 6.98 million points 178, 178 and 189 (FP32), 210, 224
+// and 242 (FP64); 12 cases / 81 thousand points 8.2, 8.1 and 9.4, 7.5, 8.1 and 8.4.
+// With four wavefronts for all of them 176, 233 and 356, 212, 287 and 486; 8.1, 8.1
+// and 10.5, 7.5, 8.2 and 13.
+template <bool F32, bool G2P, int RMAP, int kWaves>
+__global__ __launch_bounds__(64 * kWaves, kWaves == 1 ? 4 : 5) void k_batch_substep(
     ChunkRec *__restrict__ recs, const double *__restrict__ gridIn, int nChunks, int pGroups,
     typename Rows<F32>::P *pos, typename Rows<F32>::V *rest, size_t gpitch, const CaseParams *__restrict__ cases,
     unsigned char *crushedRow, size_t pitch, double *__restrict__ gridOut, int4 *bounds, int *__restrict__ err,
     const short *__restrict__ grains, typename Rows<F32>::V *jpRow, const double *__restrict__ tTab, double t0, int step,
     NodeWork nw, LearnArgs la, MapQueue mq, int storeVB, int joint) {
-    constexpr int kWindows = 3 * (F32 ? 4 * kWaveWin : kWin);   // doubles
-    __shared__ __attribute__((aligned(16))) double smem[kWindows + 2 * kTile + 4 * (2 * 9 + 1) * kPatch];
+    constexpr int kWin = box_space(kWaves), kTile = kWin;
+    constexpr int kWindows = 3 * (F32 ? kWaves * kWaveWin : kWin);   // doubles
+    __shared__ __attribute__((aligned(16))) double smem[kWindows + 2 * kTile + kWaves * (2 * 9 + 1) * kPatch];
     if constexpr (G2P) {
         if ((int)blockIdx.x >= pGroups) {
-            node_part(nw, (int)blockIdx.x - pGroups, cases, gridIn, gpitch, bounds, tTab ? tTab[step] : t0, smem);
+            node_part<kWaves>(nw, (int)blockIdx.x - pGroups, cases, gridIn, gpitch, bounds, tTab ? tTab[step] : t0, smem);
             return;
         }
     }
@@ -707,7 +726,7 @@ __global__ __launch_bounds__(256, 5) void k_batch_substep(
     constexpr double fe0 = F32 ? 1.0 : 0.0;   // stored Fe = Fe - fe0 * I, Jp_inv - fe0
     // the wavefront's points: lanes of them (none past the last one)
     int lanes, first;
-    if constexpr (F32) {
+    if constexpr (band_order(F32, kWaves)) {
         lanes = (int)rec.shape - row * 64;
         first = row * 64;
     } else {
@@ -784,7 +803,7 @@ __global__ __launch_bounds__(256, 5) void k_batch_substep(
     }
     // the box's velocities (FP32 storage rounds them to FP32)
     if constexpr (G2P || !F32) {
-        for (unsigned e = threadIdx.x; e < nodes; e += 256) {
+        for (unsigned e = threadIdx.x; e < nodes; e += 64 * kWaves) {
             unsigned c, r;
             box_node(e, rec.inv, (unsigned)bw, c, r);
             if constexpr (!F32) {
@@ -851,7 +870,7 @@ __global__ __launch_bounds__(256, 5) void k_batch_substep(
             bool slow = ok && !inTile;
             if (const unsigned long long om = __ballot(slow)) {
                 double2 *patch = tile + kTile + row * 9 * kPatch;
-                int2 *cells = reinterpret_cast<int2 *>(tile + kTile + 4 * 9 * kPatch) + row * kPatch;
+                int2 *cells = reinterpret_cast<int2 *>(tile + kTile + kWaves * 9 * kPatch) + row * kPatch;
                 const int rank = __popcll(om & ((1ull << lane) - 1ull));
                 if (slow && rank < kPatch) cells[rank] = make_int2(bx, by);
                 wsync();
@@ -1143,7 +1162,7 @@ __global__ __launch_bounds__(256, 5) void k_batch_substep(
         const double h = cp.h;
         const double A00 = B00 - cp.scm * t00, A01 = B01 - cp.scm * t01;
         const double A10 = B10 - cp.scm * t01, A11 = B11 - cp.scm * t11;
-        if constexpr (F32) {
+        if constexpr (band_order(F32, kWaves)) {
             // A quad of lanes whose four points share one base cell (in band
             // order most quads, until points cross into other cells) and whose
             // stencil lies in the window sums its contributions in registers
@@ -1242,14 +1261,14 @@ __global__ __launch_bounds__(256, 5) void k_batch_substep(
     };
     const double m = cp.mass;   // the windows hold sums per unit mass
     if (!F32 || joint) {
-        for (unsigned e = threadIdx.x; e < nodes; e += 256) {
+        for (unsigned e = threadIdx.x; e < nodes; e += 64 * kWaves) {
             unsigned c, r;
             box_node(e, rec.inv, (unsigned)bw, c, r);
             double a, a1, a2;
             if constexpr (F32) {
                 a = a1 = a2 = 0;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
+                for (int q = 0; q < kWaves; ++q) {
                     const unsigned win = rec.win[q], x = c - (win & 0xFFu), y = r - (win >> 8 & 0xFFu);
                     const unsigned w = win >> 16 & 0xFFu, h = win >> 24;
                     if (x < w && y < h) {
@@ -1288,7 +1307,7 @@ __global__ __launch_bounds__(256, 5) void k_batch_substep(
         __syncthreads();
         if (threadIdx.x == 0) {
             unsigned q0 = lim[0], q1 = lim[4], q2 = lim[8], q3 = lim[12];
-            for (int q = 1; q < 4; ++q) {
+            for (int q = 1; q < kWaves; ++q) {
                 q0 = min(q0, lim[q]);
                 q1 = min(q1, lim[4 + q]);
                 q2 = max(q2, lim[8 + q]);
@@ -1298,8 +1317,8 @@ __global__ __launch_bounds__(256, 5) void k_batch_substep(
             if (q2 == 0) {   // no point in the grid
                 out.ext = 0;
                 for (int q = 0; q < 4; ++q) out.win[q] = 0;
-            } else if (set_box(out, (int)q0, (int)q1, (int)q2 - 1, (int)q3 - 1)) {
-                for (int q = 0; q < 4; ++q)
+            } else if (set_box(out, (int)q0, (int)q1, (int)q2 - 1, (int)q3 - 1, kTile)) {
+                for (int q = 0; q < kWaves; ++q)
                     out.win[q] = lim[8 + q] ? win_of(out, (int)lim[q], (int)lim[4 + q], (int)lim[8 + q] - 1,
                                                      (int)lim[12 + q] - 1)
                                             : 0u;
@@ -1318,7 +1337,7 @@ __global__ __launch_bounds__(256, 5) void k_batch_substep(
 template <bool F32>
 __global__ __launch_bounds__(256) void k_chunk_boxes(ChunkRec *recs, int nChunks, const typename Rows<F32>::P *pos,
                                                      size_t pitch, const CaseParams *__restrict__ cases, int4 *bounds,
-                                                     const int *__restrict__ starts) {
+                                                     const int *__restrict__ starts, int waves) {
     const int ch = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, lane = threadIdx.x & 63;
     if (ch >= nChunks) return;
     ChunkRec rec = recs[ch];
@@ -1329,7 +1348,7 @@ __global__ __launch_bounds__(256) void k_chunk_boxes(ChunkRec *recs, int nChunks
         rec.dims = (unsigned)cases[0].gx | (unsigned)cases[0].gy << 16;
     }
     const CaseParams &cp = cases[rec.cs];
-    const int count = F32 ? (int)rec.shape : chunk_count(rec.shape);
+    const int count = band_order(F32, waves) ? (int)rec.shape : chunk_count(rec.shape), space = box_space(waves);
     int wx0[4], wy0[4], wx1[4], wy1[4];   // of each wavefront's points
     int fx = 0, fy = 0, x0 = INT_MAX, y0 = INT_MAX, x1 = -1, y1 = -1;
 #pragma unroll
@@ -1368,12 +1387,12 @@ __global__ __launch_bounds__(256) void k_chunk_boxes(ChunkRec *recs, int nChunks
         rec.ext = 0;
         for (int q = 0; q < 4; ++q) rec.win[q] = 0;
         if (x0 <= x1) widen_bounds(bounds, rec.cs, x0, y0, x1, y1);
-        if (x0 <= x1 && !set_box(rec, x0, y0, x1, y1)) {
+        if (x0 <= x1 && !set_box(rec, x0, y0, x1, y1, space)) {
             x0 = max(fx - 7, x0);
             x1 = min(fx + 7, x1);
             y0 = max(fy - 7, y0);
             y1 = min(fy + 7, y1);
-            if (x0 <= x1 && y0 <= y1) (void)set_box(rec, x0, y0, x1, y1);
+            if (x0 <= x1 && y0 <= y1) (void)set_box(rec, x0, y0, x1, y1, space);
         }
         if (rec.ext) {
 #pragma unroll
@@ -1729,6 +1748,7 @@ struct icempm_batch {
     CaseParams *cases = nullptr;
     ChunkRec *recs = nullptr;   // nChunks records
     int nChunks = 0;
+    int waves = 4;              // wavefronts of a workgroup, for the largest of them
     size_t recCap = 0;
     int2 *nodeBlock = nullptr;
     int nNodeBlocks = 0;
@@ -1779,8 +1799,8 @@ struct icempm_batch {
     hipEvent_t e0 = nullptr, e1 = nullptr;
     float lastMs = 0;
 
-    // tuning: points per chunk (= threads per workgroup of the particle pass)
-    // and the re-sort cadence in substeps (0: never)
+    // tuning: points per chunk (at most; = threads per workgroup of the substep
+    // kernel) and the re-sort cadence in substeps (0: never)
     int chunkPoints = 256;
     int resortEvery = 0;
     std::vector<int> hcstart, hccase;       // the chunk table on the host
@@ -1913,15 +1933,16 @@ struct Pass {
     bool storeVB;
 };
 
-template <bool F32, bool G2P, int RMAP>
-void launch_one(icempm_batch *b, const Pass &p, const LearnArgs &la, const MapQueue &mq) {
+template <bool F32, bool G2P, int RMAP, int kWaves>
+void launch_waves(icempm_batch *b, const Pass &p, const LearnArgs &la, const MapQueue &mq) {
     Rows<F32> S{static_cast<typename Rows<F32>::P *>(b->pos), reinterpret_cast<typename Rows<F32>::V *>(b->rest),
                 b->crushed, b->grain, b->pitch};
     const size_t grid = 3 * b->gpitch;
     const int clear = 3 - p.in - p.out;   // the third grid (unused by a first P2G, where in = out)
     NodeWork nw{b->nodeBlock + p.block0, b->grids + (G2P ? clear * grid : 0), p.hist, b->bins};
     const int groups = ((p.chunks + 7) / 8) * 8;
-    hipLaunchKernelGGL((k_batch_substep<F32, G2P, RMAP>), dim3((unsigned)(groups + (G2P ? p.blocks : 0))), dim3(256), 0,
+    const int blocks = G2P ? p.blocks * (4 / kWaves) : 0;
+    hipLaunchKernelGGL((k_batch_substep<F32, G2P, RMAP, kWaves>), dim3((unsigned)(groups + blocks)), dim3(64 * kWaves), 0,
                        p.stream, b->recs + p.chunk0, b->grids + p.in * grid, p.chunks, groups, S.pos, S.rest, b->gpitch,
                        b->cases, S.crushed, S.pitch, b->grids + p.out * grid, b->bounds, b->err, b->grain,
                        S.rest + 10 * S.pitch, p.tTab, 0.0, p.step, nw, la, mq, p.storeVB ? 1 : 0,
@@ -1933,6 +1954,16 @@ void launch_one(icempm_batch *b, const Pass &p, const LearnArgs &la, const MapQu
                            mq.count == b->mapCount ? b->mapCount + 1 : b->mapCount, b->grids + p.out * grid, b->gpitch,
                            b->err, la);
     }
+}
+
+template <bool F32, bool G2P, int RMAP>
+void launch_one(icempm_batch *b, const Pass &p, const LearnArgs &la, const MapQueue &mq) {
+    if (b->waves == 4)
+        launch_waves<F32, G2P, RMAP, 4>(b, p, la, mq);
+    else if (b->waves == 2)
+        launch_waves<F32, G2P, RMAP, 2>(b, p, la, mq);
+    else
+        launch_waves<F32, G2P, RMAP, 1>(b, p, la, mq);
 }
 
 template <bool F32>
@@ -2067,11 +2098,20 @@ hipError_t launch_boxes(icempm_batch *b) {
     const dim3 nb((unsigned)((b->nChunks + 3) / 4));
     if (b->precision == ICEMPM_BATCH_F32)
         hipLaunchKernelGGL(k_chunk_boxes<true>, nb, dim3(256), 0, b->stream, b->recs, b->nChunks,
-                           static_cast<const unsigned int *>(b->pos), b->pitch, b->cases, b->bounds, nullptr);
+                           static_cast<const unsigned int *>(b->pos), b->pitch, b->cases, b->bounds, nullptr,
+                           b->waves);
     else
         hipLaunchKernelGGL(k_chunk_boxes<false>, nb, dim3(256), 0, b->stream, b->recs, b->nChunks,
-                           static_cast<const double *>(b->pos), b->pitch, b->cases, b->bounds, nullptr);
+                           static_cast<const double *>(b->pos), b->pitch, b->cases, b->bounds, nullptr,
+                           b->waves);
     return hipGetLastError();
+}
+
+// Wavefronts of a workgroup for the host chunk table's chunks.
+int chunk_waves(const icempm_batch *b) {
+    int most = b->chunkPoints;
+    for (size_t c = 0; c < b->hccase.size(); ++c) most = std::max(most, b->hcstart[c + 1] - b->hcstart[c]);
+    return most <= 64 ? 1 : (most <= 128 ? 2 : 4);
 }
 
 // The host chunk table as records on the device (grown when needed).  Boxes
@@ -2080,10 +2120,11 @@ hipError_t launch_boxes(icempm_batch *b) {
 int upload_chunks(icempm_batch *b) {
     const size_t n = b->hccase.size();
     std::vector<ChunkRec> t(n);
+    const int waves = chunk_waves(b);
     for (size_t c = 0; c < n; ++c) {
         const CaseParams &cp = b->hc[(size_t)b->hccase[c]].cp;
         const int count = b->hcstart[c + 1] - b->hcstart[c];
-        t[c] = ChunkRec{b->hcstart[c], b->precision == ICEMPM_BATCH_F32 ? (unsigned)count : chunk_shape(count),
+        t[c] = ChunkRec{b->hcstart[c], band_order(b->precision == ICEMPM_BATCH_F32, waves) ? (unsigned)count : chunk_shape(count),
                         b->hccase[c], cp.gridOffset, (unsigned)cp.gx | (unsigned)cp.gy << 16, 0, 0, 0, {}};
     }
     const ChunkRec *before = b->recs;
@@ -2098,6 +2139,8 @@ int upload_chunks(icempm_batch *b) {
     }
     BCHK(b, hipMemcpy(b->recs, t.data(), n * sizeof(ChunkRec), hipMemcpyHostToDevice), "chunk table");
     b->nChunks = (int)n;
+    const int wavesBefore = b->waves;
+    b->waves = waves;
     // each group's first chunk
     bool splitMoved = false;
     for (int g = 0; g <= b->chains; ++g) {
@@ -2107,10 +2150,10 @@ int upload_chunks(icempm_batch *b) {
         splitMoved = splitMoved || c != b->grpChunk[g];
         b->grpChunk[g] = c;
     }
-    // a captured loop holds the table's address, the chunk count and the
-    // groups' ranges (the grid sizes of its launches); the table's contents
-    // are read at run time
-    if (b->recs != before || b->nChunks != nBefore || splitMoved) drop_graph(b);
+    // a captured loop holds the table's address, the chunk count, the kernel
+    // for their size and the groups' ranges (the grid sizes of its launches);
+    // the table's contents are read at run time
+    if (b->recs != before || b->nChunks != nBefore || b->waves != wavesBefore || splitMoved) drop_graph(b);
     if (b->pending >= 0) BCHK(b, launch_boxes(b), "chunk table");
     return ICEMPM_OK;
 }
@@ -2171,6 +2214,20 @@ size_t rest_elem(const icempm_batch *b, int r, size_t slot) {
     return (size_t)r * b->pitch + slot;
 }
 
+// What a re-sort needs.
+int resort_scratch(icempm_batch *b) {
+    const size_t n = (size_t)b->nPts;
+    BCHK(b, once(b->sKeys2, n * sizeof(int)), "re-sort");
+    BCHK(b, once(b->sVals2, n * sizeof(int)), "re-sort");
+    BCHK(b, once(b->sTmp, radix_tmp_ints(n) * sizeof(int)), "re-sort");
+    BCHK(b, once(b->tpos, pos_bytes(b)), "re-sort");
+    BCHK(b, once(b->trest, rest_bytes(b)), "re-sort");
+    BCHK(b, once(b->tcrushed, b->pitch), "re-sort");
+    BCHK(b, once(b->torig, b->pitch * sizeof(int)), "re-sort");
+    if (b->grain) BCHK(b, once(b->tgrain, b->pitch * sizeof(short)), "re-sort");
+    return ICEMPM_OK;
+}
+
 // Stable re-sort of every case's points by their current cell, then a new
 // chunk table.  The slot -> batch-index map (orig) follows the points, so
 // reads return them in their original order.
@@ -2179,14 +2236,7 @@ int resort(icempm_batch *b) {
     if (n <= 1) return ICEMPM_OK;
     int rc = sort_keys(b);
     if (rc) return rc;
-    BCHK(b, once(b->sKeys2, (size_t)n * sizeof(int)), "re-sort");
-    BCHK(b, once(b->sVals2, (size_t)n * sizeof(int)), "re-sort");
-    BCHK(b, once(b->sTmp, radix_tmp_ints((size_t)n) * sizeof(int)), "re-sort");
-    BCHK(b, once(b->tpos, pos_bytes(b)), "re-sort");
-    BCHK(b, once(b->trest, rest_bytes(b)), "re-sort");
-    BCHK(b, once(b->tcrushed, b->pitch), "re-sort");
-    BCHK(b, once(b->torig, b->pitch * sizeof(int)), "re-sort");
-    if (b->grain) BCHK(b, once(b->tgrain, b->pitch * sizeof(short)), "re-sort");
+    if ((rc = resort_scratch(b))) return rc;
     BCHK(b, radix_sort_pairs(b->sKeys, b->sVals, b->sKeys2, b->sVals2, (size_t)n, b->sTmp, b->stream), "re-sort");
     // the cells in sorted order give the new chunk table, whose chunks then
     // (FP64 storage) arrange their points
@@ -2194,7 +2244,7 @@ int resort(icempm_batch *b) {
     chunk_table(b, b->hcells, b->hcstart, b->hccase);
     if ((rc = upload_chunks(b))) return rc;
     const int *from = b->sVals;
-    if (b->precision != ICEMPM_BATCH_F32) {
+    if (!band_order(b->precision == ICEMPM_BATCH_F32, b->waves)) {
         hipLaunchKernelGGL(k_chunk_order, dim3((unsigned)b->nChunks), dim3(256), 0, b->stream, b->recs, b->nChunks,
                            b->sVals, b->sVals2);
         BCHK(b, hipGetLastError(), "re-sort");
@@ -2311,8 +2361,15 @@ int read_points(icempm_batch *b, int c, double *soa, size_t pitch) {
     return ICEMPM_OK;
 }
 
-// the chunk table for the current slots and chunkPoints
+// The chunk table for chunkPoints.  FP64 storage arranges the points over a
+// chunk's four wavefronts, so that from and to such chunks the points are put in
+// order anew, where there is memory for it: another cut of the same slots has
+// chunks as wide as the former ones.
 int rebuild_chunks(icempm_batch *b) {
+    if (b->precision != ICEMPM_BATCH_F32 && b->nPts > 1 && (b->waves == 4) != (b->chunkPoints == 256)) {
+        if (resort_scratch(b) == ICEMPM_OK) return resort(b);
+        (void)hipGetLastError();
+    }
     int rc = current_cells(b);
     if (rc) return rc;
     chunk_table(b, b->hcells, b->hcstart, b->hccase);
@@ -2505,7 +2562,7 @@ hipError_t enter(const Run &r) {
     hipLaunchKernelGGL(k_reset_bounds, dim3(1), dim3(64), 0, r.stream, bounds, 1);
     hipLaunchKernelGGL(k_chunk_boxes<false>, dim3((unsigned)((r.nChunks + 3) / 4)), dim3(256), 0, r.stream,
                        static_cast<ChunkRec *>(r.recs), r.nChunks, r.rows, r.pp, static_cast<const CaseParams *>(r.cp), bounds,
-                       r.starts);
+                       r.starts, 4);
     return hipGetLastError();
 }
 
@@ -2519,7 +2576,7 @@ hipError_t substep(const Run &r, const double *in, double *out, double *clear, d
     const NodeWork nw{nullptr, clear, hist2, r.bins};
     unsigned char *util = reinterpret_cast<unsigned char *>(r.rows + 7 * r.pp);
     // rows 2-5 of the kernel's 11 are Fe; without storeVB it takes no other
-    hipLaunchKernelGGL((k_batch_substep<false, true, kMapExact>), dim3((unsigned)(groups + blocks)), dim3(256), 0, r.stream,
+    hipLaunchKernelGGL((k_batch_substep<false, true, kMapExact, 4>), dim3((unsigned)(groups + blocks)), dim3(256), 0, r.stream,
                        static_cast<ChunkRec *>(r.recs), in, r.nChunks, groups, r.rows, r.rows, r.gp,
                        static_cast<const CaseParams *>(r.cp), util, r.pp, out, static_cast<int4 *>(r.bounds), r.err,
                        reinterpret_cast<const short *>(util + r.pp), r.rows + 6 * r.pp, nullptr, t, step, nw, LearnArgs{},
@@ -2736,9 +2793,10 @@ int icempm_batch_finalize(icempm_batch *b) {
                 }
             }
             chunk_table(b, cells.data(), b->hcstart, b->hccase);
-            // FP64 storage: every chunk's points in its slot order
+            // every chunk's points in its slot order, where that is not band order
+            const bool inOrder = band_order(b->precision == ICEMPM_BATCH_F32, chunk_waves(b));
             std::vector<int> sorted;
-            for (size_t c = 0; c < b->hccase.size() && b->precision != ICEMPM_BATCH_F32; ++c) {
+            for (size_t c = 0; c < b->hccase.size() && !inOrder; ++c) {
                 std::vector<int> &ord = order[(size_t)b->hccase[c]];
                 const int o = b->hc[(size_t)b->hccase[c]].cp.ptOffset;
                 const int p = b->hcstart[c] - o, n = b->hcstart[c + 1] - b->hcstart[c];

@@ -210,14 +210,14 @@ for call, watch in PRESENT.items():
             rc = calls(b, p)[call]()
             hit = F.fake_hip_pending_failure() < 0
             fail_at(-1)
-            if hit:
-                assert rc == ICEMPM_E_HIP, (call, k, rc)
+            if hit:   # (a chunk table can be had without rearranging the points)
+                assert rc == ICEMPM_E_HIP or call == "chunks", (call, k, rc)
             F.fake_hip_watch(name.encode(), arg)
             before = launches(name)
             assert H.icempm_batch_run(b, 8, 0) == 0
             assert calls(b, p)[call]() == 0, (call, k, H.icempm_batch_last_error(b))
             assert H.icempm_batch_run(b, 8, 0) == 0
-            assert (launches(name) > before or not hit) and F.fake_hip_nulls() == 0, (call, k, name, arg)
+            assert (launches(name) > before or rc == 0) and F.fake_hip_nulls() == 0, (call, k, name, arg)
             H.icempm_batch_destroy(b)
             if not hit:
                 break
