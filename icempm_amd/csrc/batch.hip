@@ -40,10 +40,31 @@
 #include "internal.h"
 #include "mlp_device.h"
 
+namespace icempm {
+namespace batch {
+
+// The substep kernel's device functions, without contraction for the batches and
+// with it for a single case, as their particle passes have always been built.  It
+// matters: without contraction det F = F00 F11 - F10 F01 and J^2 - 1 round twice
+// more at 1e-16 in every substep, of a strain of 1e-5, and the in-cell offset x /
+// h - base at the size of x / h, not of the offset.  Over 2,500 substeps of 2,400
+// points that set the uncontracted Bp apart from the particle pass's by half of
+// what two runs of either differ by (1e-9 of its norm at most); contracted, the
+// means of 24 runs agree to what 24 runs can show.
+struct PlainMath {
+#include "fast_math.inc"
+};
+}  // namespace batch
+}  // namespace icempm
+
 #pragma clang fp contract(fast)
 
 namespace icempm {
 namespace batch {
+
+struct FusedMath {
+#include "fast_math.inc"
+};
 
 struct CaseParams {
     double dt, vol, mass, h, h_inv, Dinv, mu, kappa, gravity, indRsq, indV;
@@ -225,8 +246,8 @@ static __device__ __forceinline__ KParams kp_of(const CaseParams &c, int *err) {
 
 // Return map of crushed points: the exact Drucker-Prager map, the exact map
 // while recording (trial, projected) pairs, or the learned map with the
-// exact one as fallback.
-enum { kMapExact = 0, kMapHarvest = 1, kMapLearned = 2 };
+// exact one as fallback.  kMapSingle: the exact map of a single case (FusedMath).
+enum { kMapExact = 0, kMapHarvest = 1, kMapLearned = 2, kMapSingle = 3 };
 
 struct LearnArgs {
     const unsigned short *wbf;   // MLP weights, BF16 bits
@@ -696,6 +717,7 @@ __global__ __launch_bounds__(64 * kWaves, kWaves == 1 ? 4 : 5) void k_batch_subs
     unsigned char *crushedRow, size_t pitch, double *__restrict__ gridOut, int4 *bounds, int *__restrict__ err,
     const short *__restrict__ grains, typename Rows<F32>::V *jpRow, const double *__restrict__ tTab, double t0, int step,
     NodeWork nw, LearnArgs la, MapQueue mq, int storeVB, int joint) {
+    using M = typename std::conditional<RMAP == kMapSingle, FusedMath, PlainMath>::type;
     constexpr int kWin = box_space(kWaves), kTile = kWin;
     constexpr int kWindows = 3 * (F32 ? kWaves * kWaveWin : kWin);   // doubles
     __shared__ __attribute__((aligned(16))) double smem[kWindows + 2 * kTile + kWaves * (2 * 9 + 1) * kPatch];
@@ -856,8 +878,8 @@ __global__ __launch_bounds__(64 * kWaves, kWaves == 1 ? 4 : 5) void k_batch_subs
                 stencil_cells(px, bx, fx0, wx0, wx1, wx2);
                 stencil_cells(py, by, fx1, wy0, wy1, wy2);
             } else {
-                const bool st = stencil(px, cp.h_inv, bx, fx0, wx0, wx1, wx2) &&
-                                stencil(py, cp.h_inv, by, fx1, wy0, wy1, wy2);
+                const bool st = M::stencil(px, cp.h_inv, bx, fx0, wx0, wx1, wx2) &&
+                                M::stencil(py, cp.h_inv, by, fx1, wy0, wy1, wy2);
                 ok = valid && st;
                 if (valid && !st) flag_error(k);
             }
@@ -963,10 +985,10 @@ __global__ __launch_bounds__(64 * kWaves, kWaves == 1 ? 4 : 5) void k_batch_subs
             vx = v0; vy = v1;
             // p and q^2 of the trial state (q itself is never needed here:
             // every test compares it with a non-negative limit)
-            const InvSq iv = invariants_sq(F00, F01, F10, F11, cp.mu, cp.kappa);
+            const InvSq iv = M::invariants_sq(F00, F01, F10, F11, cp.mu, cp.kappa);
             const unsigned char crushed0 = crushed;
             if (cp.grainVar != 0) {   // GetParametersForGrain's strengths (case-uniform branch)
-                if (crushed == 0) crushed = fails_sq(k, grain, iv.p, iv.q2) ? 1 : 0;
+                if (crushed == 0) crushed = M::fails_sq(k, grain, iv.p, iv.q2) ? 1 : 0;
             } else {
                 // tension line q > slope (p + 3e6), slope >= 0 and p + 3e6 >= 0 there
                 const double ql = cp.slope * (iv.p - -3e6);
@@ -981,9 +1003,9 @@ __global__ __launch_bounds__(64 * kWaves, kWaves == 1 ? 4 : 5) void k_batch_subs
             const bool crushedOk = ok && crushed == 1;
             if (crushedOk) Jp = fe0 + (double)*at(jpRow, u);
             const double Jp0 = Jp;
-            if constexpr (RMAP == kMapExact) {
-                if (crushedOk && dp_projects_sq(k, iv.p, iv.q2, Jp))
-                    dp_return(k, compute_pq_fast(F00, F01, F10, F11, cp.mu, cp.kappa), F00, F01, F10, F11, Jp);
+            if constexpr (RMAP == kMapExact || RMAP == kMapSingle) {
+                if (crushedOk && M::dp_projects_sq(k, iv.p, iv.q2, Jp))
+                    M::dp_return(k, M::compute_pq_fast(F00, F01, F10, F11, cp.mu, cp.kappa), F00, F01, F10, F11, Jp);
             } else if constexpr (RMAP == kMapHarvest) {
                 Trial r{};
                 if (crushedOk) r = compute_pq_fast(F00, F01, F10, F11, cp.mu, cp.kappa);
@@ -1114,8 +1136,8 @@ __global__ __launch_bounds__(64 * kWaves, kWaves == 1 ? 4 : 5) void k_batch_subs
             }
             if (ok && Jp != Jp0 && !defer) *at(jpRow, u) = (V)(Jp - fe0);
             if (!F32 && ok && crushed != crushed0) *at(S.crushed, u) = crushed;   // FP32: in the record
-            kirchhoff_from_inv(iv, t00, t01, t11);
-            if (crushedOk) kirchhoff_rcp(fe0 + F00, F01, F10, fe0 + F11, cp.mu, cp.kappa, t00, t01, t11);
+            M::kirchhoff_from_inv(iv, t00, t01, t11);
+            if (crushedOk) M::kirchhoff_rcp(fe0 + F00, F01, F10, fe0 + F11, cp.mu, cp.kappa, t00, t01, t11);
         } else {
             if constexpr (F32) {
                 px = fix_cells(pr.x, pr.z & 0xFFFFu, cp);
@@ -1142,8 +1164,8 @@ __global__ __launch_bounds__(64 * kWaves, kWaves == 1 ? 4 : 5) void k_batch_subs
             stencil_cells(px, bx, fx0, wx0, wx1, wx2);
             stencil_cells(py, by, fx1, wy0, wy1, wy2);
         } else {
-            const bool st = px == px && py == py && stencil(px, cp.h_inv, bx, fx0, wx0, wx1, wx2) &&
-                            stencil(py, cp.h_inv, by, fx1, wy0, wy1, wy2);
+            const bool st = px == px && py == py && M::stencil(px, cp.h_inv, bx, fx0, wx0, wx1, wx2) &&
+                            M::stencil(py, cp.h_inv, by, fx1, wy0, wy1, wy2);
             ok = valid && st;
             if (valid && !st) flag_error(k);
         }
@@ -2576,7 +2598,7 @@ hipError_t substep(const Run &r, const double *in, double *out, double *clear, d
     const NodeWork nw{nullptr, clear, hist2, r.bins};
     unsigned char *util = reinterpret_cast<unsigned char *>(r.rows + 7 * r.pp);
     // rows 2-5 of the kernel's 11 are Fe; without storeVB it takes no other
-    hipLaunchKernelGGL((k_batch_substep<false, true, kMapExact, 4>), dim3((unsigned)(groups + blocks)), dim3(256), 0, r.stream,
+    hipLaunchKernelGGL((k_batch_substep<false, true, kMapSingle, 4>), dim3((unsigned)(groups + blocks)), dim3(256), 0, r.stream,
                        static_cast<ChunkRec *>(r.recs), in, r.nChunks, groups, r.rows, r.rows, r.gp,
                        static_cast<const CaseParams *>(r.cp), util, r.pp, out, static_cast<int4 *>(r.bounds), r.err,
                        reinterpret_cast<const short *>(util + r.pp), r.rows + 6 * r.pp, nullptr, t, step, nw, LearnArgs{},

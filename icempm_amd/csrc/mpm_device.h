@@ -96,18 +96,6 @@ static __device__ __forceinline__ Svd2 svd2x2(double F00, double F01, double F10
     return r;
 }
 
-// F = U diag(a, b) V^T for the rotation pair of an Svd2.
-static __device__ __forceinline__ void usvt(const Svd2 &r, double a, double b, double &F00, double &F01,
-                                     double &F10, double &F11) {
-    // U = [[uc, us], [-us, uc]], V = [[vc, vs], [-vs, vc]]
-    double U00 = r.uc, U01 = r.us, U10 = -r.us, U11 = r.uc;
-    double V00 = r.vc, V01 = r.vs, V10 = -r.vs, V11 = r.vc;
-    F00 = (U00 * a) * V00 + (U01 * b) * V01;
-    F01 = (U00 * a) * V10 + (U01 * b) * V11;
-    F10 = (U10 * a) * V00 + (U11 * b) * V01;
-    F11 = (U10 * a) * V10 + (U11 * b) * V11;
-}
-
 // ----------------------------------------------------------------------------
 // Kirchhoff stress tau = mu/J dev(F F^T) + kappa (J^2 - 1) I
 // (KirchhoffStress_Wolper, gpu_implementation5.cu:24-34; dev :391-394)
@@ -147,73 +135,6 @@ static __device__ __forceinline__ Trial compute_pq(double F00, double F01, doubl
     r.sh0 = c * (r.ss0 - half_sum);
     r.sh1 = c * (r.ss1 - half_sum);
     r.q = kSqrt2 * sqrt(r.sh0 * r.sh0 + r.sh1 * r.sh1);
-    return r;
-}
-
-// FAST-mode forms of the same quantities (not bit-identical to the
-// reference's operation order): one reciprocal for the polar rotation, and
-// q = 2 |sh0| (in 2D the deviator has sh1 = -sh0, so sqrt2 |sh| = 2 |sh0|).
-static __device__ __forceinline__ Svd2 svd2x2_fast(double F00, double F01, double F10, double F11) {
-    double x0 = F00 + F11;
-    double x1 = F10 - F01;
-    double den2 = x0 * x0 + x1 * x1;
-    double rc = 1.0, rs = 0.0;
-    if (den2 != 0) {
-        const double inv = 1.0 / sqrt(den2);
-        rc = x0 * inv;
-        rs = -x1 * inv;
-    }
-    double S00 = rc * F00 - rs * F10;
-    double S01 = rc * F01 - rs * F11;
-    double S11 = rs * F01 + rc * F11;
-    double cosine, sine, s0, s1;
-    const double y2 = S01 * S01;
-    if (y2 == 0) {
-        cosine = 1;
-        sine = 0;
-        s0 = S00;
-        s1 = S11;
-    } else {
-        double tau = 0.5 * (S00 - S11);
-        double w = sqrt(tau * tau + y2);
-        double t = S01 / ((tau > 0) ? (tau + w) : (tau - w));
-        cosine = 1.0 / sqrt(t * t + 1.0);
-        sine = -t * cosine;
-        double c2 = cosine * cosine;
-        double csy = 2 * cosine * sine * S01;
-        double s2 = sine * sine;
-        s0 = c2 * S00 - csy + s2 * S11;
-        s1 = s2 * S00 + csy + c2 * S11;
-    }
-    Svd2 r;
-    if (s0 < s1) {
-        r.s0 = s1;
-        r.s1 = s0;
-        r.vc = -sine;
-        r.vs = cosine;
-    } else {
-        r.s0 = s0;
-        r.s1 = s1;
-        r.vc = cosine;
-        r.vs = sine;
-    }
-    r.uc = rc * r.vc - rs * r.vs;
-    r.us = rs * r.vc + rc * r.vs;
-    return r;
-}
-
-static __device__ __forceinline__ Trial compute_pq_fast(double F00, double F01, double F10, double F11,
-                                                        double mu, double kappa) {
-    Trial r;
-    r.svd = svd2x2_fast(F00, F01, F10, F11);
-    r.Je = r.svd.s0 * r.svd.s1;
-    r.p = -(kappa / 2.) * (r.Je * r.Je - 1.);
-    r.ss0 = r.svd.s0 * r.svd.s0;
-    r.ss1 = r.svd.s1 * r.svd.s1;
-    const double c = mu / r.Je;
-    r.sh0 = c * (0.5 * (r.ss0 - r.ss1));
-    r.sh1 = -r.sh0;
-    r.q = 2.0 * fabs(r.sh0);
     return r;
 }
 
@@ -261,17 +182,6 @@ static __device__ __forceinline__ void kirchhoff_from_inv(const Inv &v, double &
     t11 = -a - 2. * v.p;
 }
 
-// 1/x for a normal x: the hardware reciprocal (v_rcp_f64) refined by two
-// Newton-Raphson steps, r <- r + r (1 - x r), to within an ulp or two of the
-// correctly rounded quotient.  FAST mode only (not the IEEE division).
-static __device__ __forceinline__ double rcp_nr(double x) {
-    double r = __builtin_amdgcn_rcp(x);
-    double e = fma(-x, r, 1.0);
-    r = fma(r, e, r);
-    e = fma(-x, r, 1.0);
-    return fma(r, e, r);
-}
-
 // The FAST trial invariants with q^2 in place of q: every test on q in the
 // fused passes compares it with a non-negative limit (the NACC ellipse uses
 // q^2 itself), so no square root is taken, and c = mu / J comes from rcp_nr.
@@ -280,56 +190,12 @@ struct InvSq {
     double c, d, b01, p, q2;   // c = mu / J, d = b00 - b11
 };
 
-static __device__ __forceinline__ InvSq invariants_sq(double F00, double F01, double F10, double F11,
-                                                      double mu, double kappa) {
-    InvSq v;
-    const double J = F00 * F11 - F10 * F01;
-    const double b00 = F00 * F00 + F01 * F01, b11 = F10 * F10 + F11 * F11;
-    v.b01 = F00 * F10 + F01 * F11;
-    v.d = b00 - b11;
-    v.c = mu * rcp_nr(J);
-    v.p = -(kappa / 2.) * (J * J - 1.);
-    v.q2 = (v.c * v.c) * (v.d * v.d + 4. * (v.b01 * v.b01));
-    return v;
-}
-
-static __device__ __forceinline__ void kirchhoff_from_inv(const InvSq &v, double &t00, double &t01,
-                                                          double &t11) {
-    const double a = 0.5 * (v.c * v.d);
-    t00 = a - 2. * v.p;
-    t01 = v.c * v.b01;
-    t11 = -a - 2. * v.p;
-}
-
-// KirchhoffStress_Wolper (gpu_implementation5.cu:24-34) with 1/J from rcp_nr
-static __device__ __forceinline__ void kirchhoff_rcp(double F00, double F01, double F10, double F11, double mu,
-                                                     double kappa, double &t00, double &t01, double &t11) {
-    const double Je = F00 * F11 - F10 * F01;
-    const double b00 = F00 * F00 + F01 * F01;
-    const double b01 = F00 * F10 + F01 * F11;
-    const double b11 = F10 * F10 + F11 * F11;
-    const double half_tr = (b00 + b11) / 2;
-    const double c1 = mu * rcp_nr(Je);
-    const double c2 = kappa * (Je * Je - 1.);
-    t00 = c1 * (b00 - half_tr) + c2;
-    t01 = c1 * b01;
-    t11 = c1 * (b11 - half_tr) + c2;
-}
-
 // Whether the Drucker-Prager map (dp_return) changes a crushed trial state
 // with these p and q: the tension branch, or q at or above the cone.
 static __device__ __forceinline__ bool dp_projects(const KParams &k, double p, double q, double Jp_inv) {
     if (p < -k.dpThr || Jp_inv < 1) return true;
     const double q_n_1 = (p > k.ics) ? 0.0 : fmin((p + k.dpThr) * k.tanPhi, k.iss);
     return q >= q_n_1;
-}
-
-// the same from q^2: past the tension test p + p_thr >= 0, so the cone's
-// q_n_1 is >= 0 (for tan(phi), qmax >= 0) and q >= q_n_1 iff q^2 >= q_n_1^2
-static __device__ __forceinline__ bool dp_projects_sq(const KParams &k, double p, double q2, double Jp_inv) {
-    if (p < -k.dpThr || Jp_inv < 1) return true;
-    const double q_n_1 = (p > k.ics) ? 0.0 : fmin((p + k.dpThr) * k.tanPhi, k.iss);
-    return q_n_1 <= 0.0 || q2 >= q_n_1 * q_n_1;
 }
 
 // NACC test with the constants of grain 0 (GrainVariability == 0)
@@ -361,103 +227,7 @@ static __device__ __forceinline__ bool fails_tab(const KParams &k, short grain, 
     return y > 0;
 }
 
-// NACC failure test for intact points with per-grain strengths
-// (CheckIfPointIsInsideFailureSurface :114-141, GetParametersForGrain :97-111)
-static __device__ __forceinline__ bool fails(const KParams &k, short grain, double p, double q) {
-    double var1 = 1.0 + k.grainVar * 0.05 * (-10 + grain % 21);
-    double var2 = 1.0 + k.grainVar * 0.033 * (-15 + (grain + 3) % 30);
-    double var3 = 1.0 + k.grainVar * 0.1 * (-10 + (grain + 4) % 11);
-    double pmax = k.ics * var1;
-    double pmin = -k.its * var2;
-    double qmax = k.iss * var3;
-    double beta = -pmin / pmax;
-    double a = pmax * (1 + beta);
-    double mSq = (4 * qmax * qmax * (1 + 2 * beta)) / (a * a);
-    const double pmin2 = -3e6;
-    if (p < 0) {
-        if (p < pmin2) return true;
-        double q0 = 2 * sqrt(-pmax * pmin) * qmax / (pmax - pmin);
-        double kk = -q0 / pmin2;
-        double q_limit = kk * (p - pmin2);
-        return q > q_limit;
-    }
-    double y = (1. + 2. * beta) * q * q + mSq * (p + beta * pmax) * (p - pmax);
-    return y > 0;
-}
-
-// fails() from q^2 and without its divisions and square root.  With t = -pmin
-// = beta pmax and s = pmax + t, the ellipse is
-//   (1 + 2 beta) (q^2 + 4 qmax^2 (p + t) (p - pmax) / s^2) > 0,
-// and the tension line's q_limit = 2 sqrt(pmax t) qmax / s (p + 3e6) / 3e6 is
-// exceeded iff q^2 > q_limit^2 when it is >= 0, and always when qmax < 0 (a
-// GrainVariability above 1).  A grain whose pmax or t is not positive (nor
-// then 1 + 2 beta) takes the formula as it stands.
-static __device__ __forceinline__ bool fails_sq(const KParams &k, short grain, double p, double q2) {
-    const double var1 = 1.0 + k.grainVar * 0.05 * (-10 + grain % 21);
-    const double var2 = 1.0 + k.grainVar * 0.033 * (-15 + (grain + 3) % 30);
-    const double var3 = 1.0 + k.grainVar * 0.1 * (-10 + (grain + 4) % 11);
-    const double pmax = k.ics * var1, t = k.its * var2, qmax = k.iss * var3;
-    if (!(pmax > 0 && t > 0)) return fails(k, grain, p, sqrt(q2));
-    const double s = pmax + t, qs = q2 * (s * s), m4 = 4. * qmax * qmax;
-    if (p < 0) {
-        const double d = p + 3e6;
-        return d < 0 || qmax < 0 || qs * 9e12 > m4 * (pmax * t) * (d * d);
-    }
-    return qs + m4 * (p + t) * (p - pmax) > 0;
-}
-
-// Drucker-Prager return map for crushed points (Wolper_Drucker_Prager
-// :48-94).  Updates Fe and Jp_inv in place.
-static __device__ __forceinline__ void dp_return(const KParams &k, const Trial &r, double &F00,
-                                          double &F01, double &F10, double &F11,
-                                          double &Jp_inv) {
-    if (r.p < -k.dpThr || Jp_inv < 1) {
-        double p_new = -k.dpThr;
-        double Je_new = sqrt(-2. * p_new / k.kappa + 1.);
-        double sq = sqrt(Je_new);
-        usvt(r.svd, sq, sq, F00, F01, F10, F11);
-        Jp_inv *= Je_new / r.Je;
-    } else {
-        double q_n_1;
-        if (r.p > k.ics) {
-            q_n_1 = 0;
-        } else {
-            double q_from_dp = (r.p + k.dpThr) * k.tanPhi;
-            q_n_1 = fmin(q_from_dp, k.iss);
-        }
-        if (r.q >= q_n_1) {
-            double s_norm = q_n_1 / kSqrt2;
-            double z = r.sh0 * r.sh0 + r.sh1 * r.sh1;
-            double n0 = r.sh0, n1 = r.sh1;
-            if (z > 0) {   // normalising a zero vector leaves it zero
-                double nz = sqrt(z);
-                n0 = n0 / nz;
-                n1 = n1 / nz;
-            }
-            double c = s_norm * (r.Je / k.mu);
-            double m = (r.ss0 + r.ss1) / 2;
-            usvt(r.svd, sqrt(c * n0 + m), sqrt(c * n1 + m), F00, F01, F10, F11);
-        }
-    }
-}
-
-// ----------------------------------------------------------------------------
-// Quadratic B-spline stencil along one axis (gpu_implementation5.cu:185-193)
-// Returns false for a position whose base index cannot be represented.
-static __device__ __forceinline__ bool stencil(double x, double h_inv, int &base, double &fx,
-                                        double &w0, double &w1, double &w2) {
-    double bx = x * h_inv - 0.5;
-    if (!(bx > -1.0 && bx < 2147483000.0)) return false;
-    base = (int)bx;
-    fx = x * h_inv - (double)base;
-    double v0 = 1.5 - fx;
-    double v1 = fx - 1.0;
-    double v2 = fx - 0.5;
-    w0 = 0.5 * v0 * v0;
-    w1 = 0.75 - v1 * v1;
-    w2 = 0.5 * v2 * v2;
-    return true;
-}
+#include "fast_math.inc"
 
 static __device__ __forceinline__ double sel3(int i, double a, double b, double c) {
     return i == 0 ? a : (i == 1 ? b : c);
