@@ -16,9 +16,9 @@ and FP32 storage and the exact map.
 5 m x 2 m, 1,600,000 points, grid 1200 x 500).
 
 Prints one JSON line: particle-updates/s, the roofline of the dominant
-kernel (the fused G2P+P2G pass, timed with HIP events on its stream; the HBM
-traffic per launch from the committed rocprofv3 counter summary), and the
-CPU baseline (the C++ restatement's timing build, OpenMP, on this host's
+kernel (the one-kernel substep or, in short single-case runs, the fused G2P+P2G
+pass, timed with HIP events on its stream; the HBM traffic per launch from the
+committed rocprofv3 counter summary), and the CPU baseline (the C++ restatement's timing build, OpenMP, on this host's
 cores at 1 thread and at 16, on a bounded sample of every case of the same
 workload).
 """
@@ -214,8 +214,9 @@ def run_single(args) -> dict:
     value = n * steps / el
     ms_per_step = el / steps * 1e3
     k_avg_s = (ktot / max(klaunch, 1)) / 1e3
-    # runs of 32 substeps or more do a substep in one kernel, shorter ones in two
-    one_kernel = args.mode == "fast" and args.pass_kind in (None, 2) and steps >= 32
+    # runs of 16 substeps or more (of a million points: 32) do a substep in one
+    # kernel, shorter ones in two
+    one_kernel = args.mode == "fast" and args.pass_kind in (None, 2) and steps >= (16 if n < 1_000_000 else 32)
     prof = f"{'substep' if one_kernel else 'fused_g2p_p2g'}_{case.name}"
     k_bytes = n * FUSED_BYTES_PER_POINT + G * (SUBSTEP_BYTES_PER_NODE if one_kernel else FUSED_BYTES_PER_NODE)
     k_moved = n * FUSED_MOVED_BYTES_PER_POINT + G * (SUBSTEP_MOVED_BYTES_PER_NODE if one_kernel else FUSED_BYTES_PER_NODE)

@@ -1,7 +1,7 @@
 """Batches of independent indentation cases on one GPU (C ABI
-``icempm_batch_*``): many cases of uneven size advanced together, one grid
-update and one particle-pass launch per substep for all of them, the substep
-loop captured in a HIP graph.
+``icempm_batch_*``): many cases of uneven size advanced together, one launch
+per substep for all of them (two side by side when they are large, one more with
+the learned map), the substep loop captured in a HIP graph.
 """
 from __future__ import annotations
 
@@ -112,7 +112,7 @@ class Batch:
         return int(self._H.icempm_batch_num_nodes(self._b))
 
     def kernel_timing(self, stride: int) -> None:
-        """Time every stride-th fused particle pass of stream runs (0: off)."""
+        """Time every stride-th substep kernel of stream runs (0: off)."""
         self._check(self._H.icempm_batch_kernel_timing(self._b, int(stride)))
 
     def kernel_timing_read(self) -> tuple[float, int]:

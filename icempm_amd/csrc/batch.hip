@@ -692,7 +692,8 @@ static __device__ __forceinline__ void quad_scatter(int lane, int e0, int S, dou
 // points the launch and one chain of memory latencies (3.9 us).  Against a grid
 // update of its own and a particle pass that gathered from global memory and
 // found each wavefront's window anew, a substep of 32 cases / 6.98 million points
-// went from 193 to 168 us (FP32 storage), of 12 cases / 81 thousand points from
+// went from 193 to 168 us (FP32 storage, points in mid-run; of cases at rest in
+// their load order both take 165 to 179), of 12 cases / 81 thousand points from
 // 18.4 to 8.2, of 8 cases / 671 thousand points from 35 to 21 (FP64, strengths
 // per grain).  Making a node's velocity in each of the ~2 workgroups that need it
 // costs ~50 instructions per 64 points; it saves a launch, the velocities' trip

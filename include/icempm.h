@@ -223,7 +223,8 @@ int icempm_read_bins(icempm_ctx *ctx, double *out);
 /* -- batches of independent cases (no counterpart) ----------------------
  * Many indentation cases of uneven size advanced together: every substep is
  * one launch over all cases (two groups of cases side by side when they are
- * large; one more launch with the learned map), and the substep loop can be captured in a HIP graph and replayed.  Cases are
+ * large; one more launch with the learned map), and the substep loop can be
+ * captured in a HIP graph and replayed.  Cases are
  * added from the reference SoA layout (16 rows x pitch doubles, as read back
  * by icempm_read_points after LoadRawPoints); all cases share the time step.
  * A case with GrainVariability != 0 takes each point's NACC strengths from
@@ -287,7 +288,7 @@ int icempm_batch_force_bins(icempm_batch *b, int c, double *out, int nbins);
 int icempm_batch_read_points(icempm_batch *b, int c, double *soa, size_t pitch);
 int icempm_batch_error_flag(icempm_batch *b, int *flag);
 /* Tuning knobs: ICEMPM_BATCH_TUNE_CHUNK, points per chunk = threads per
- * workgroup of the particle pass (64, 128 or 256; default 256);
+ * workgroup of the substep kernel (64, 128 or 256; default 256);
  * ICEMPM_BATCH_TUNE_RESORT, re-sort the points by cell every that many
  * substeps within a run (0, the default: never);
  * ICEMPM_BATCH_TUNE_MAP_MIN_ACCEPT, the learned map's acceptance threshold
