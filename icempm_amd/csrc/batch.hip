@@ -49,8 +49,8 @@ namespace batch {
 // more at 1e-16 in every substep, of a strain of 1e-5, and the in-cell offset x /
 // h - base at the size of x / h, not of the offset.  Over 2,500 substeps of 2,400
 // points that set the uncontracted Bp apart from the particle pass's by half of
-// what two runs of either differ by (1e-9 of its norm at most); contracted, the
-// means of 24 runs agree to what 24 runs can show.
+// a run's scatter (2e-10 of its norm in the median, 2e-9 in some inputs);
+// contracted, the means of 24 runs agree to what 24 runs can show.
 struct PlainMath {
 #include "fast_math.inc"
 };
