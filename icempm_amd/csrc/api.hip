@@ -56,6 +56,7 @@ struct icempm_ctx {
     // with its touched nodes
     int *perm = nullptr, *bandStart = nullptr;
     int nBand = 0, bandPoints = 0, bandX = 0, bandY = 0;
+    bool bandInOrder = false;
     double bandCell = 0;
     bool bandDirty = true;
     void *recs = nullptr;
@@ -457,6 +458,7 @@ bool ensure_substep(icempm_ctx *c, double x0, double y0, single::Run &r) {
              get(c->bandStart, starts.size() * sizeof(int)) && get(c->recs, starts.size() * single::kRecBytes) &&
              upload(c->bandStart, starts.data(), starts.size() * sizeof(int));
         c->nBand = (int)starts.size() - 1;
+        c->bandInOrder = r.inOrder;
         r.starts = c->bandStart;
         r.nChunks = c->nBand;
         ok = ok && single::slots(r, c->vals, c->perm) == hipSuccess;
@@ -474,6 +476,7 @@ bool ensure_substep(icempm_ctx *c, double x0, double y0, single::Run &r) {
     r.starts = c->bandStart;
     r.recs = c->recs;
     r.nChunks = c->nBand;
+    r.inOrder = c->bandInOrder;
     r.rows = c->rows;
     r.bins = c->bins;
     r.err = c->dErr;

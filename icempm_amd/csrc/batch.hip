@@ -346,28 +346,33 @@ struct __attribute__((aligned(16))) ChunkRec {
 };
 constexpr int kBoxEvery = 8;
 
-// The points of a chunk, FP32 storage, or workgroups of fewer than four
-// wavefronts: in band order, 64 a wavefront.  The four lanes of a quad mostly hold
-// the points of a cell and add up their contributions before these reach the
-// window (FP32: the wavefront's, which keeps the sums of a node in the order quad,
-// wavefront, grid).
+// The points of a chunk, in one of two layouts.
 //
-// FP64 storage, four wavefronts: in rows of a wavefront each, as few as hold them
+// In order (FP32 storage, workgroups of fewer than four wavefronts, dense clouds):
+// in band order, 64 a wavefront.  The four lanes of a quad mostly hold the points of
+// a cell and add up their contributions before these reach the window (FP32: the
+// wavefront's, which keeps the sums of a node in the order quad, wavefront, grid).
+//
+// In rows (FP64 storage otherwise): in rows of a wavefront each, as few as hold them
 // and filled evenly; slot s holds the point that band order puts at chunk_point(s,
-// shape).  Consecutive points go to the same lane of consecutive rows, so that the 64
-// lanes of a wavefront hold different cells and their LDS atomics, 27 a point
-// into one window for the workgroup, go to different nodes (four lanes of one
-// cell at one node take five times as long).
+// shape).  Consecutive points go to the same lane of consecutive rows, so that the
+// 64 lanes of a wavefront hold different cells, at four points a cell, and their LDS
+// atomics, 27 a point into one window for the workgroup, go to different nodes (four
+// lanes of one cell at one node take five times as long).
 //
-// The latter takes fewer instructions (8 cases FP64, 671 thousand points: 22.6
-// us a substep, 25.0 in band order; 1.6 million points FP64: 50 and 51), but
-// adds the terms in another order.  FP64 points differ by rounding then; the
+// Rows take fewer instructions (8 cases FP64, 671 thousand points: 22.6
+// us a substep, 25.0 in order; 1.6 million points FP64: 50 and 51), but
+// add the terms in another order.  FP64 points differ by rounding then; the
 // rounding of FP32 storage and the yield branches carry a study's points past 1e-5
 // of the other order's within 4000 substeps in most runs, where two runs of one
-// order mostly agree to the bit.  Chunks of 64 points keep band order: in one row
+// order mostly agree to the bit.  Chunks of 64 points are kept in order: in one row
 // their cells' points are neighbours anyway (32 cases, 6.98 million points: 242 us,
-// 480 with an LDS atomic for each of a point's 27 sums).
-constexpr bool band_order(bool f32, int waves) { return f32 || waves < 4; }
+// 480 with an LDS atomic for each of a point's 27 sums).  So are those of clouds
+// with more than kDensePoints a cell, of which a row holds several a cell.  us a
+// substep of 960 thousand points FP64 in rows and in order: 26.9 and 29.2 at 4 a
+// cell, 39.0 and 41.3 at 5.5, 40.8 and 39.7 at 6, 53 and 35 at 9, 75 and 32 at 16,
+// 123 and 30 at 49 (the grid update and pass before: 41, 42, 41, 39, 37 and 37).
+constexpr double kDensePoints = 5.75;
 static __host__ __device__ inline unsigned chunk_shape(int n) {
     const int rows = (n + 63) / 64;
     return (unsigned)(n / rows) | (unsigned)(n % rows) << 8 | (unsigned)rows << 16;
@@ -711,13 +716,14 @@ static __device__ __forceinline__ void quad_scatter(int lane, int e0, int S, dou
 // and 242 (FP64); 12 cases / 81 thousand points 8.2, 8.1 and 9.4, 7.5, 8.1 and 8.4.
 // With four wavefronts for all of them 176, 233 and 356, 212, 287 and 486; 8.1, 8.1
 // and 10.5, 7.5, 8.2 and 13.
-template <bool F32, bool G2P, int RMAP, int kWaves>
+template <bool F32, bool G2P, int RMAP, int kWaves, bool kInOrder>
 __global__ __launch_bounds__(64 * kWaves, kWaves == 1 ? 4 : 5) void k_batch_substep(
     ChunkRec *__restrict__ recs, const double *__restrict__ gridIn, int nChunks, int pGroups,
     typename Rows<F32>::P *pos, typename Rows<F32>::V *rest, size_t gpitch, const CaseParams *__restrict__ cases,
     unsigned char *crushedRow, size_t pitch, double *__restrict__ gridOut, int4 *bounds, int *__restrict__ err,
     const short *__restrict__ grains, typename Rows<F32>::V *jpRow, const double *__restrict__ tTab, double t0, int step,
     NodeWork nw, LearnArgs la, MapQueue mq, int storeVB, int joint) {
+    static_assert(kInOrder || (!F32 && kWaves == 4), "rows are FP64 storage's, four to a workgroup");
     using M = typename std::conditional<RMAP == kMapSingle, FusedMath, PlainMath>::type;
     constexpr int kWin = box_space(kWaves), kTile = kWin;
     constexpr int kWindows = 3 * (F32 ? kWaves * kWaveWin : kWin);   // doubles
@@ -749,7 +755,7 @@ __global__ __launch_bounds__(64 * kWaves, kWaves == 1 ? 4 : 5) void k_batch_subs
     constexpr double fe0 = F32 ? 1.0 : 0.0;   // stored Fe = Fe - fe0 * I, Jp_inv - fe0
     // the wavefront's points: lanes of them (none past the last one)
     int lanes, first;
-    if constexpr (band_order(F32, kWaves)) {
+    if constexpr (kInOrder) {
         lanes = (int)rec.shape - row * 64;
         first = row * 64;
     } else {
@@ -1185,7 +1191,7 @@ __global__ __launch_bounds__(64 * kWaves, kWaves == 1 ? 4 : 5) void k_batch_subs
         const double h = cp.h;
         const double A00 = B00 - cp.scm * t00, A01 = B01 - cp.scm * t01;
         const double A10 = B10 - cp.scm * t01, A11 = B11 - cp.scm * t11;
-        if constexpr (band_order(F32, kWaves)) {
+        if constexpr (kInOrder) {
             // A quad of lanes whose four points share one base cell (in band
             // order most quads, until points cross into other cells) and whose
             // stencil lies in the window sums its contributions in registers
@@ -1360,18 +1366,18 @@ __global__ __launch_bounds__(64 * kWaves, kWaves == 1 ? 4 : 5) void k_batch_subs
 template <bool F32>
 __global__ __launch_bounds__(256) void k_chunk_boxes(ChunkRec *recs, int nChunks, const typename Rows<F32>::P *pos,
                                                      size_t pitch, const CaseParams *__restrict__ cases, int4 *bounds,
-                                                     const int *__restrict__ starts, int waves) {
+                                                     const int *__restrict__ starts, int waves, int inOrder) {
     const int ch = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, lane = threadIdx.x & 63;
     if (ch >= nChunks) return;
     ChunkRec rec = recs[ch];
     if (starts) {
         rec = ChunkRec{};
         rec.beg = starts[ch];
-        rec.shape = chunk_shape(starts[ch + 1] - rec.beg);
+        rec.shape = inOrder ? (unsigned)(starts[ch + 1] - rec.beg) : chunk_shape(starts[ch + 1] - rec.beg);
         rec.dims = (unsigned)cases[0].gx | (unsigned)cases[0].gy << 16;
     }
     const CaseParams &cp = cases[rec.cs];
-    const int count = band_order(F32, waves) ? (int)rec.shape : chunk_count(rec.shape), space = box_space(waves);
+    const int count = inOrder ? (int)rec.shape : chunk_count(rec.shape), space = box_space(waves);
     int wx0[4], wy0[4], wx1[4], wy1[4];   // of each wavefront's points
     int fx = 0, fy = 0, x0 = INT_MAX, y0 = INT_MAX, x1 = -1, y1 = -1;
 #pragma unroll
@@ -1772,6 +1778,7 @@ struct icempm_batch {
     ChunkRec *recs = nullptr;   // nChunks records
     int nChunks = 0;
     int waves = 4;              // wavefronts of a workgroup, for the largest of them
+    bool inOrder = true;        // the points of a chunk are in band order (else in rows)
     size_t recCap = 0;
     int2 *nodeBlock = nullptr;
     int nNodeBlocks = 0;
@@ -1827,6 +1834,7 @@ struct icempm_batch {
     int chunkPoints = 256;
     int resortEvery = 0;
     std::vector<int> hcstart, hccase;       // the chunk table on the host
+    bool hcdense = false;                   // of a dense cloud (kDensePoints)
     int *orig = nullptr;                    // batch index of the point in each slot
     // re-sort scratch
     int *sKeys = nullptr, *sVals = nullptr, *sKeys2 = nullptr, *sVals2 = nullptr, *sTmp = nullptr;
@@ -1848,6 +1856,7 @@ struct icempm_batch {
     double kt = 0;
     int kstep = 0;
     std::vector<int> kcstart, kccase;
+    bool kcdense = false;
     int kChunkPoints = 256;
     double runMs = 0;   // device time of the last run's segments + re-sorts
 
@@ -1956,7 +1965,7 @@ struct Pass {
     bool storeVB;
 };
 
-template <bool F32, bool G2P, int RMAP, int kWaves>
+template <bool F32, bool G2P, int RMAP, int kWaves, bool kInOrder>
 void launch_waves(icempm_batch *b, const Pass &p, const LearnArgs &la, const MapQueue &mq) {
     Rows<F32> S{static_cast<typename Rows<F32>::P *>(b->pos), reinterpret_cast<typename Rows<F32>::V *>(b->rest),
                 b->crushed, b->grain, b->pitch};
@@ -1965,7 +1974,7 @@ void launch_waves(icempm_batch *b, const Pass &p, const LearnArgs &la, const Map
     NodeWork nw{b->nodeBlock + p.block0, b->grids + (G2P ? clear * grid : 0), p.hist, b->bins};
     const int groups = ((p.chunks + 7) / 8) * 8;
     const int blocks = G2P ? p.blocks * (4 / kWaves) : 0;
-    hipLaunchKernelGGL((k_batch_substep<F32, G2P, RMAP, kWaves>), dim3((unsigned)(groups + blocks)), dim3(64 * kWaves), 0,
+    hipLaunchKernelGGL((k_batch_substep<F32, G2P, RMAP, kWaves, kInOrder>), dim3((unsigned)(groups + blocks)), dim3(64 * kWaves), 0,
                        p.stream, b->recs + p.chunk0, b->grids + p.in * grid, p.chunks, groups, S.pos, S.rest, b->gpitch,
                        b->cases, S.crushed, S.pitch, b->grids + p.out * grid, b->bounds, b->err, b->grain,
                        S.rest + 10 * S.pitch, p.tTab, 0.0, p.step, nw, la, mq, p.storeVB ? 1 : 0,
@@ -1981,12 +1990,14 @@ void launch_waves(icempm_batch *b, const Pass &p, const LearnArgs &la, const Map
 
 template <bool F32, bool G2P, int RMAP>
 void launch_one(icempm_batch *b, const Pass &p, const LearnArgs &la, const MapQueue &mq) {
+    if constexpr (!F32)
+        if (!b->inOrder) return launch_waves<F32, G2P, RMAP, 4, false>(b, p, la, mq);
     if (b->waves == 4)
-        launch_waves<F32, G2P, RMAP, 4>(b, p, la, mq);
+        launch_waves<F32, G2P, RMAP, 4, true>(b, p, la, mq);
     else if (b->waves == 2)
-        launch_waves<F32, G2P, RMAP, 2>(b, p, la, mq);
+        launch_waves<F32, G2P, RMAP, 2, true>(b, p, la, mq);
     else
-        launch_waves<F32, G2P, RMAP, 1>(b, p, la, mq);
+        launch_waves<F32, G2P, RMAP, 1, true>(b, p, la, mq);
 }
 
 template <bool F32>
@@ -2029,41 +2040,45 @@ hipError_t launch_pass(icempm_batch *b, bool g2p, const Pass &p) {
 
 // Chunks of n consecutive points with the given base cells (column | row <<
 // 16), the first of them slot o: <= cap points whose cells span at most two
-// cell rows and kChunkCols columns, so that the workgroup's LDS holds all their
+// cell rows and cols (<= kChunkCols) columns, so that the workgroup's LDS holds all their
 // stencils, cut greedily.  A chunk that is cut for its columns alone ends at a
 // wavefront's last point if it can.  Points in band order give chunks of one
-// band each, until they move.
-void cut_chunks(const unsigned *cells, int n, int o, int cap, std::vector<int> &starts) {
+// band each, until they move.  Returns the cells that the chunks span.
+long cut_chunks(const unsigned *cells, int n, int o, int cap, int cols, std::vector<int> &starts) {
     starts.reserve((size_t)n / (size_t)cap + 16);
+    long spanned = 0;
     for (int cs = 0; cs < n;) {
         int c0 = INT_MAX, r0 = INT_MAX, c1 = -1, r1 = -1, i = cs;
         bool wide = false;
+        long area = 0;
         for (; i < n && i - cs < cap; ++i) {
             const int cc = (int)(cells[i] & 0xFFFFu), r = (int)(cells[i] >> 16);
             r0 = std::min(r0, r);
             r1 = std::max(r1, r);
             c0 = std::min(c0, cc);
             c1 = std::max(c1, cc);
-            wide = c1 - c0 > kChunkCols - 1;
+            wide = c1 - c0 > cols - 1;
             if (r1 - r0 > 1 || wide) break;
+            area = (long)(c1 - c0 + 1) * (r1 - r0 + 1);
         }
+        spanned += area;
         if (wide && r1 - r0 <= 1 && i - cs > 64) i = cs + (i - cs) / 64 * 64;
         starts.push_back(o + cs);
         cs = i;
     }
+    return spanned;
 }
 
-// Chunk table from the case-local base cells of the points in slot order, the
-// chunks within one case.  The cases are independent, so they are cut on
+// Every case's chunks, from the case-local base cells of the points in slot order;
+// returns the cells they span.  The cases are independent, so they are cut on
 // several host threads.
-void chunk_table(const icempm_batch *b, const unsigned *cells, std::vector<int> &cstart,
-                 std::vector<int> &ccase) {
+long cut_cases(const icempm_batch *b, const unsigned *cells, int cap, int cols, std::vector<std::vector<int>> &starts) {
     const size_t nc = b->hc.size();
-    const int cap = b->chunkPoints;
-    std::vector<std::vector<int>> starts(nc);
+    std::vector<long> spanned(nc, 0);
     auto cut = [&](size_t ci) {
         const CaseParams &cp = b->hc[ci].cp;
-        if (cp.nPts > 0) cut_chunks(cells + cp.ptOffset, cp.nPts, cp.ptOffset, cap, starts[ci]);
+        starts[ci].clear();
+        if (cp.nPts > 0) spanned[ci] = cut_chunks(cells + cp.ptOffset, cp.nPts, cp.ptOffset, cap, cols, starts[ci]);
     };
     const unsigned hw = std::thread::hardware_concurrency();
     const size_t nt = std::min<size_t>(nc, std::min(16u, std::max(1u, hw)));
@@ -2097,9 +2112,27 @@ void chunk_table(const icempm_batch *b, const unsigned *cells, std::vector<int> 
         for (auto &t : pool) t.join();
         if (failure) std::rethrow_exception(failure);
     }
+    long all = 0;
+    for (long a : spanned) all += a;
+    return all;
+}
+
+// The chunks as b's host table.  A cloud of about a point a cell (kSparsePoints)
+// in FP32 storage has chunks of one wavefront, no wider than its window: of the
+// wider ones half the wavefronts have no points, or points past their window.
+// 960 thousand points at 1, 0.8 and 0.5 a cell: 60 -> 51, 84 -> 55 and 167 -> 74 us a
+// substep (the grid update and pass before: 56, 62 and 148).
+constexpr double kSparsePoints = 1.15;
+void chunk_table(icempm_batch *b, const unsigned *cells) {
+    std::vector<int> &cstart = b->hcstart, &ccase = b->hccase;
+    std::vector<std::vector<int>> starts(b->hc.size());
+    const long spanned = cut_cases(b, cells, b->chunkPoints, kChunkCols, starts);
+    b->hcdense = (double)b->nPts > kDensePoints * (double)spanned;
+    if (b->precision == ICEMPM_BATCH_F32 && (double)b->nPts < kSparsePoints * (double)spanned)
+        cut_cases(b, cells, std::min(b->chunkPoints, 64), kWinCols - 2, starts);
     cstart.clear();
     ccase.clear();
-    for (size_t ci = 0; ci < nc; ++ci)
+    for (size_t ci = 0; ci < starts.size(); ++ci)
         for (int st : starts[ci]) {
             cstart.push_back(st);
             ccase.push_back((int)ci);
@@ -2122,19 +2155,24 @@ hipError_t launch_boxes(icempm_batch *b) {
     if (b->precision == ICEMPM_BATCH_F32)
         hipLaunchKernelGGL(k_chunk_boxes<true>, nb, dim3(256), 0, b->stream, b->recs, b->nChunks,
                            static_cast<const unsigned int *>(b->pos), b->pitch, b->cases, b->bounds, nullptr,
-                           b->waves);
+                           b->waves, b->inOrder ? 1 : 0);
     else
         hipLaunchKernelGGL(k_chunk_boxes<false>, nb, dim3(256), 0, b->stream, b->recs, b->nChunks,
                            static_cast<const double *>(b->pos), b->pitch, b->cases, b->bounds, nullptr,
-                           b->waves);
+                           b->waves, b->inOrder ? 1 : 0);
     return hipGetLastError();
 }
 
 // Wavefronts of a workgroup for the host chunk table's chunks.
 int chunk_waves(const icempm_batch *b) {
-    int most = b->chunkPoints;
+    int most = 0;
     for (size_t c = 0; c < b->hccase.size(); ++c) most = std::max(most, b->hcstart[c + 1] - b->hcstart[c]);
     return most <= 64 ? 1 : (most <= 128 ? 2 : 4);
+}
+
+// Whether its chunks' points are in band order.
+bool chunk_in_order(const icempm_batch *b) {
+    return b->precision == ICEMPM_BATCH_F32 || b->hcdense || chunk_waves(b) < 4;
 }
 
 // The host chunk table as records on the device (grown when needed).  Boxes
@@ -2144,10 +2182,11 @@ int upload_chunks(icempm_batch *b) {
     const size_t n = b->hccase.size();
     std::vector<ChunkRec> t(n);
     const int waves = chunk_waves(b);
+    const bool inOrder = chunk_in_order(b);
     for (size_t c = 0; c < n; ++c) {
         const CaseParams &cp = b->hc[(size_t)b->hccase[c]].cp;
         const int count = b->hcstart[c + 1] - b->hcstart[c];
-        t[c] = ChunkRec{b->hcstart[c], band_order(b->precision == ICEMPM_BATCH_F32, waves) ? (unsigned)count : chunk_shape(count),
+        t[c] = ChunkRec{b->hcstart[c], inOrder ? (unsigned)count : chunk_shape(count),
                         b->hccase[c], cp.gridOffset, (unsigned)cp.gx | (unsigned)cp.gy << 16, 0, 0, 0, {}};
     }
     const ChunkRec *before = b->recs;
@@ -2162,8 +2201,9 @@ int upload_chunks(icempm_batch *b) {
     }
     BCHK(b, hipMemcpy(b->recs, t.data(), n * sizeof(ChunkRec), hipMemcpyHostToDevice), "chunk table");
     b->nChunks = (int)n;
-    const int wavesBefore = b->waves;
+    const bool kernelBefore = b->waves == waves && b->inOrder == inOrder;
     b->waves = waves;
+    b->inOrder = inOrder;
     // each group's first chunk
     bool splitMoved = false;
     for (int g = 0; g <= b->chains; ++g) {
@@ -2176,7 +2216,7 @@ int upload_chunks(icempm_batch *b) {
     // a captured loop holds the table's address, the chunk count, the kernel
     // for their size and the groups' ranges (the grid sizes of its launches);
     // the table's contents are read at run time
-    if (b->recs != before || b->nChunks != nBefore || b->waves != wavesBefore || splitMoved) drop_graph(b);
+    if (b->recs != before || b->nChunks != nBefore || !kernelBefore || splitMoved) drop_graph(b);
     if (b->pending >= 0) BCHK(b, launch_boxes(b), "chunk table");
     return ICEMPM_OK;
 }
@@ -2264,10 +2304,10 @@ int resort(icempm_batch *b) {
     // the cells in sorted order give the new chunk table, whose chunks then
     // (FP64 storage) arrange their points
     if ((rc = current_cells(b, b->sVals))) return rc;
-    chunk_table(b, b->hcells, b->hcstart, b->hccase);
+    chunk_table(b, b->hcells);
     if ((rc = upload_chunks(b))) return rc;
     const int *from = b->sVals;
-    if (!band_order(b->precision == ICEMPM_BATCH_F32, b->waves)) {
+    if (!b->inOrder) {
         hipLaunchKernelGGL(k_chunk_order, dim3((unsigned)b->nChunks), dim3(256), 0, b->stream, b->recs, b->nChunks,
                            b->sVals, b->sVals2);
         BCHK(b, hipGetLastError(), "re-sort");
@@ -2384,18 +2424,17 @@ int read_points(icempm_batch *b, int c, double *soa, size_t pitch) {
     return ICEMPM_OK;
 }
 
-// The chunk table for chunkPoints.  FP64 storage arranges the points over a
-// chunk's four wavefronts, so that from and to such chunks the points are put in
-// order anew, where there is memory for it: another cut of the same slots has
-// chunks as wide as the former ones.
+// The chunk table for chunkPoints.  From rows, and where they may be wanted, the
+// points are put in order anew, if there is memory for it: another cut of the same
+// slots has chunks as wide as the former ones.
 int rebuild_chunks(icempm_batch *b) {
-    if (b->precision != ICEMPM_BATCH_F32 && b->nPts > 1 && (b->waves == 4) != (b->chunkPoints == 256)) {
+    if (b->nPts > 1 && (!b->inOrder || (b->precision != ICEMPM_BATCH_F32 && b->chunkPoints == 256))) {
         if (resort_scratch(b) == ICEMPM_OK) return resort(b);
         (void)hipGetLastError();
     }
     int rc = current_cells(b);
     if (rc) return rc;
-    chunk_table(b, b->hcells, b->hcstart, b->hccase);
+    chunk_table(b, b->hcells);
     return upload_chunks(b);
 }
 
@@ -2501,7 +2540,7 @@ bool case_constants(const icy::SimParams &P, double x0, double y0, void *out) {
     return true;
 }
 
-hipError_t plan(const Run &r, int *keys, int *vals, int *keys2, int *vals2, int *tmp, std::vector<int> &starts) {
+hipError_t plan(Run &r, int *keys, int *vals, int *keys2, int *vals2, int *tmp, std::vector<int> &starts) {
     const int n = r.n;
     hipLaunchKernelGGL(k_batch_keys<double>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, r.stream, r.pts + kRowPosX * r.pp,
                        r.pp, n, static_cast<const CaseParams *>(r.cp), 1, keys, vals);
@@ -2519,6 +2558,7 @@ hipError_t plan(const Run &r, int *keys, int *vals, int *keys2, int *vals2, int 
         band_cell(hk[(size_t)b], r.gx, r.gy, xb, yb);
         return ya >> 1 == yb >> 1 && xb - xa <= kChunkCols - 1;
     };
+    long spanned = 0;   // cells, of the keys from a chunk's first to its last
     for (int cs = 0; cs < n;) {
         starts.push_back(cs);
         int lo = cs + 1, hi = std::min(cs + 256, n);   // the chunk's end lies in [lo, hi]
@@ -2531,20 +2571,23 @@ hipError_t plan(const Run &r, int *keys, int *vals, int *keys2, int *vals2, int 
                     hi = mid;
             }
         }
+        spanned += hk[(size_t)hi - 1] - hk[(size_t)cs] + 1;
         cs = hi;
     }
     starts.push_back(n);
+    r.inOrder = (double)n > kDensePoints * (double)spanned;
     return hipSuccess;
 }
 
 __global__ __launch_bounds__(256) void k_slots(const int *__restrict__ starts, const int *__restrict__ sorted,
-                                               int *__restrict__ perm) {
+                                               int *__restrict__ perm, int inOrder) {
     const int beg = starts[blockIdx.x], n = starts[blockIdx.x + 1] - beg, l = threadIdx.x;
-    if (l < n) perm[beg + l] = sorted[beg + chunk_point(l, chunk_shape(n))];
+    if (l < n) perm[beg + l] = sorted[beg + (inOrder ? l : chunk_point(l, chunk_shape(n)))];
 }
 
 hipError_t slots(const Run &r, const int *sorted, int *perm) {
-    hipLaunchKernelGGL(k_slots, dim3((unsigned)r.nChunks), dim3(256), 0, r.stream, r.starts, sorted, perm);
+    hipLaunchKernelGGL(k_slots, dim3((unsigned)r.nChunks), dim3(256), 0, r.stream, r.starts, sorted, perm,
+                       r.inOrder ? 1 : 0);
     return hipGetLastError();
 }
 
@@ -2585,7 +2628,7 @@ hipError_t enter(const Run &r) {
     hipLaunchKernelGGL(k_reset_bounds, dim3(1), dim3(64), 0, r.stream, bounds, 1);
     hipLaunchKernelGGL(k_chunk_boxes<false>, dim3((unsigned)((r.nChunks + 3) / 4)), dim3(256), 0, r.stream,
                        static_cast<ChunkRec *>(r.recs), r.nChunks, r.rows, r.pp, static_cast<const CaseParams *>(r.cp), bounds,
-                       r.starts, 4);
+                       r.starts, 4, r.inOrder ? 1 : 0);
     return hipGetLastError();
 }
 
@@ -2599,7 +2642,9 @@ hipError_t substep(const Run &r, const double *in, double *out, double *clear, d
     const NodeWork nw{nullptr, clear, hist2, r.bins};
     unsigned char *util = reinterpret_cast<unsigned char *>(r.rows + 7 * r.pp);
     // rows 2-5 of the kernel's 11 are Fe; without storeVB it takes no other
-    hipLaunchKernelGGL((k_batch_substep<false, true, kMapSingle, 4>), dim3((unsigned)(groups + blocks)), dim3(256), 0, r.stream,
+    const auto kernel = r.inOrder ? k_batch_substep<false, true, kMapSingle, 4, true>
+                                  : k_batch_substep<false, true, kMapSingle, 4, false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(groups + blocks)), dim3(256), 0, r.stream,
                        static_cast<ChunkRec *>(r.recs), in, r.nChunks, groups, r.rows, r.rows, r.gp,
                        static_cast<const CaseParams *>(r.cp), util, r.pp, out, static_cast<int4 *>(r.bounds), r.err,
                        reinterpret_cast<const short *>(util + r.pp), r.rows + 6 * r.pp, nullptr, t, step, nw, LearnArgs{},
@@ -2815,9 +2860,9 @@ int icempm_batch_finalize(icempm_batch *b) {
                     cells[(size_t)cp.ptOffset + k] = (unsigned)cx | (unsigned)cy << 16;
                 }
             }
-            chunk_table(b, cells.data(), b->hcstart, b->hccase);
+            chunk_table(b, cells.data());
             // every chunk's points in its slot order, where that is not band order
-            const bool inOrder = band_order(b->precision == ICEMPM_BATCH_F32, chunk_waves(b));
+            const bool inOrder = chunk_in_order(b);
             std::vector<int> sorted;
             for (size_t c = 0; c < b->hccase.size() && !inOrder; ++c) {
                 std::vector<int> &ord = order[(size_t)b->hccase[c]];
@@ -3288,6 +3333,7 @@ int icempm_batch_checkpoint(icempm_batch *b) {
         b->kstep = b->step;
         b->kcstart = b->hcstart;
         b->kccase = b->hccase;
+        b->kcdense = b->hcdense;
         b->kChunkPoints = b->chunkPoints;
         b->haveCheckpoint = true;
         return ICEMPM_OK;
@@ -3312,6 +3358,7 @@ int icempm_batch_restore(icempm_batch *b) {
         b->step = b->kstep;
         b->hcstart = b->kcstart;
         b->hccase = b->kccase;
+        b->hcdense = b->kcdense;
         b->chunkPoints = b->kChunkPoints;
         return upload_chunks(b);
     });

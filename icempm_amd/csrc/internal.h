@@ -126,6 +126,7 @@ struct Run {
     const int *starts;       // nChunks + 1 first slots
     void *recs;              // nChunks records, made by enter
     int nChunks;
+    bool inOrder;            // the layout of their points, chosen by plan
     double *rows;            // the copy
     double *bins;
     int *err;
@@ -135,8 +136,8 @@ struct Run {
 // false where the kernel does not take the case.
 bool case_constants(const icy::SimParams &P, double x0, double y0, void *out);
 // The points' band order as they are (in vals; keys, keys2, vals2: scratch of n
-// ints, tmp: of radix_tmp_ints(n)) and its chunks' first slots.
-hipError_t plan(const Run &r, int *keys, int *vals, int *keys2, int *vals2, int *tmp, std::vector<int> &starts);
+// ints, tmp: of radix_tmp_ints(n)) and its chunks' first slots; sets r.inOrder.
+hipError_t plan(Run &r, int *keys, int *vals, int *keys2, int *vals2, int *tmp, std::vector<int> &starts);
 // The points of the slots, from that order.
 hipError_t slots(const Run &r, const int *sorted, int *perm);
 hipError_t enter(const Run &r);
