@@ -1729,7 +1729,7 @@ using namespace icempm;
 using namespace icempm::batch;
 
 constexpr int kReadGroups = 4;       // groups of rows of a readback
-constexpr int kReadPart = 1 << 20;   // points of a case it brings down at a time (a multiple of 64)
+constexpr int kReadPart = 1 << 16;   // points of a case it brings down at a time (a multiple of 64)
 
 struct icempm_batch {
     int precision = ICEMPM_BATCH_F64;
@@ -2365,7 +2365,11 @@ int read_scratch(icempm_batch *b) {
 // on the host took 192.  (Helper threads copy no faster: 84 ms with eight.)  A
 // case of more than kReadPart points goes by parts of that many, which bounds the
 // scratch (112 bytes a point on either side); the kernel looks at all slots for
-// each, 4 bytes a slot.
+// each, 4 bytes a slot.  The part is as small as costs later reads nothing, for
+// pinning takes a first read longer than the copies: 1.4 million points, first and
+// later read, 57 and 13 ms in parts of 2^20, 25 and 13 of 2^18, 20 and 14 of 2^17,
+// 17 and 14 of 2^16, 16 and 15 of 2^15; 282 thousand 14 and 1.9, 14 and 1.9, 8.8
+// and 1.9, 6.1 and 2.1, 4.7 and 2.4 (a copy per row: 51 and 50, 9 and 10).
 int read_points(icempm_batch *b, int c, double *soa, size_t pitch) {
     const CaseParams &cp = b->hc[c].cp;
     std::lock_guard<std::mutex> lock(b->rbLock);

@@ -1,4 +1,4 @@
-"""Readback of a case of more points than the scratch holds (2^20): part by part,
+"""Readback of a case of more points than the scratch holds (2^16): part by part,
 every point at its own index, the padding zero."""
 import numpy as np
 import pytest
@@ -10,7 +10,8 @@ from icempm_amd.batch import Batch, batch_cases, ingest_cases
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("precision,n", [(BATCH_F64, (1 << 20) + 1), (BATCH_F32, (1 << 21) + 70)], ids=["f64", "f32"])
+@pytest.mark.parametrize("precision,n", [(BATCH_F64, (1 << 20) + 1), (BATCH_F32, (1 << 21) + 70), (BATCH_F64, 1 << 16),
+                                         (BATCH_F32, (1 << 16) + 1)], ids=["f64", "f32", "f64-one", "f32-two"])
 def test_points_come_back_in_parts(gpu_available, precision, n):
     print("read parts", precision, n, flush=True)
     cases = batch_cases(2, 700, 3000, seed=3)
