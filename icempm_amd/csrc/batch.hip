@@ -710,6 +710,9 @@ static __device__ __forceinline__ void quad_scatter(int lane, int e0, int S, dou
 // The records, the grid and the point rows lead the arguments, which the
 // kernel receives preloaded in SGPRs.
 //
+// tAt: where a batch has the substep's time (its runs are captured); null: t0.
+// step: the box is renewed where it is a multiple of kBoxEvery.
+//
 // kWaves: wavefronts of a workgroup, for chunks of at most 64 kWaves points.  Fewer
 // than four only where a caller asks for smaller chunks.  us a substep in chunks of
 // 256, 128 and 64: 32 cases / 6.98 million points 178, 178 and 189 (FP32), 210, 224
@@ -721,7 +724,7 @@ __global__ __launch_bounds__(64 * kWaves, kWaves == 1 ? 4 : 5) void k_batch_subs
     ChunkRec *__restrict__ recs, const double *__restrict__ gridIn, int nChunks, int pGroups,
     typename Rows<F32>::P *pos, typename Rows<F32>::V *rest, size_t gpitch, const CaseParams *__restrict__ cases,
     unsigned char *crushedRow, size_t pitch, double *__restrict__ gridOut, int4 *bounds, int *__restrict__ err,
-    const short *__restrict__ grains, typename Rows<F32>::V *jpRow, const double *__restrict__ tTab, double t0, int step,
+    const short *__restrict__ grains, typename Rows<F32>::V *jpRow, const double *__restrict__ tAt, double t0, int step,
     NodeWork nw, LearnArgs la, MapQueue mq, int storeVB, int joint) {
     static_assert(kInOrder || (!F32 && kWaves == 4), "rows are FP64 storage's, four to a workgroup");
     using M = typename std::conditional<RMAP == kMapSingle, FusedMath, PlainMath>::type;
@@ -730,7 +733,7 @@ __global__ __launch_bounds__(64 * kWaves, kWaves == 1 ? 4 : 5) void k_batch_subs
     __shared__ __attribute__((aligned(16))) double smem[kWindows + 2 * kTile + kWaves * (2 * 9 + 1) * kPatch];
     if constexpr (G2P) {
         if ((int)blockIdx.x >= pGroups) {
-            node_part<kWaves>(nw, (int)blockIdx.x - pGroups, cases, gridIn, gpitch, bounds, tTab ? tTab[step] : t0, smem);
+            node_part<kWaves>(nw, (int)blockIdx.x - pGroups, cases, gridIn, gpitch, bounds, tAt ? *tAt : t0, smem);
             return;
         }
     }
@@ -793,7 +796,7 @@ __global__ __launch_bounds__(64 * kWaves, kWaves == 1 ? 4 : 5) void k_batch_subs
     const int wsh = ww <= 16 ? 4 : (ww <= 32 ? 5 : 6);
     const int wcol = lane & ((1 << wsh) - 1), wrow0 = lane >> wsh, wstep = 64 >> wsh;
     double2 *tile = reinterpret_cast<double2 *>(smem + kWindows);
-    const double ind_x = cp.x0 + (G2P ? (tTab ? tTab[step] : t0) : 0.0) * cp.indV;
+    const double ind_x = cp.x0 + (G2P ? (tAt ? *tAt : t0) : 0.0) * cp.indV;
 
     // The state of the points, read once per substep.  FP32 records
     // non-temporally, so the grid keeps the L2 (167 us for 6.98 million points,
@@ -1809,9 +1812,10 @@ struct icempm_batch {
 
     // executable graphs of the substep loop, two per start (of different
     // step counts, the least recently used replaced): fresh (row 0), or the
-    // first substep's P2G already in grid 0, 1 or 2 (rows 1-3); each
-    // with the step count, time table and history rows it was captured
-    // with, and the grid that holds the next P2G after it
+    // first substep's P2G already in grid 0, 1 or 2 (rows 1-3, and 4-6 where
+    // the boxes are not renewed); each with the step count, time table and
+    // history rows it was captured with, and the grid that holds the next P2G
+    // after it
     struct GraphSlot {
         hipGraphExec_t exec = nullptr;
         int steps = 0;
@@ -1820,12 +1824,13 @@ struct icempm_batch {
         int end = -1;
         unsigned long long used = 0;
     };
-    GraphSlot graphs[4][2];
+    GraphSlot graphs[7][2];
     unsigned long long graphTick = 0;
     // the grid (0, 1 or 2) that holds the P2G of the next substep, made
     // from the current points by the last pass of the previous run; -1 when
     // there is none, or the points have changed since (restore, re-sort)
     int pending = -1;
+    int boxAge = 0;   // substeps of the last runs since one of them renewed the chunks' boxes
     hipEvent_t e0 = nullptr, e1 = nullptr;
     float lastMs = 0;
 
@@ -1959,9 +1964,9 @@ struct Pass {
     int in, out;              // grids
     int chunk0, chunks;
     int block0, blocks;       // node blocks
-    const double *tTab;
+    const double *t;          // the substep's time
     double *hist;             // of this substep
-    int step;
+    int step;                 // its place in the renewals of the boxes
     bool storeVB;
 };
 
@@ -1977,7 +1982,7 @@ void launch_waves(icempm_batch *b, const Pass &p, const LearnArgs &la, const Map
     hipLaunchKernelGGL((k_batch_substep<F32, G2P, RMAP, kWaves, kInOrder>), dim3((unsigned)(groups + blocks)), dim3(64 * kWaves), 0,
                        p.stream, b->recs + p.chunk0, b->grids + p.in * grid, p.chunks, groups, S.pos, S.rest, b->gpitch,
                        b->cases, S.crushed, S.pitch, b->grids + p.out * grid, b->bounds, b->err, b->grain,
-                       S.rest + 10 * S.pitch, p.tTab, 0.0, p.step, nw, la, mq, p.storeVB ? 1 : 0,
+                       S.rest + 10 * S.pitch, p.t, 0.0, p.step, nw, la, mq, p.storeVB ? 1 : 0,
                        b->nChunks < kJointChunks ? 1 : 0);
     if (b->evAfter) (void)hipEventRecord(b->evAfter, p.stream);
     if (G2P && RMAP == kMapLearned && la.branches != 0) {
@@ -2446,9 +2451,10 @@ int rebuild_chunks(icempm_batch *b) {
 // fresh start (start < 0) clears the grids and scatters the points into grid 0
 // first; start = 0, 1 or 2 takes the P2G that the previous run's last pass
 // left in that grid.  Substep i reads grid start + i, scatters into the next
-// and clears the one after (mod 3).  *end receives the grid that then holds
-// the next substep's P2G.
-hipError_t enqueue_loop(icempm_batch *b, int n, const double *tTab, double *hist, int start, int *end) {
+// and clears the one after (mod 3).  renew: the boxes are renewed by the first
+// substep and every kBoxEvery-th after it; else n is less than kBoxEvery and none
+// does.  *end receives the grid that then holds the next substep's P2G.
+hipError_t enqueue_loop(icempm_batch *b, int n, const double *tTab, double *hist, int start, bool renew, int *end) {
     hipError_t e;
     const size_t nc = b->hc.size();
     if ((e = launch_fill_f64(hist, 2 * (size_t)n * nc, 0.0, b->stream)) != hipSuccess) return e;
@@ -2478,7 +2484,6 @@ hipError_t enqueue_loop(icempm_batch *b, int n, const double *tTab, double *hist
         for (int g = 1; g < groups; ++g)
             if ((e = hipStreamWaitEvent(b->side[g - 1], b->evFork, 0)) != hipSuccess) return e;
     }
-    p.tTab = tTab;
     for (int g = 0; g < groups; ++g) {
         hipStream_t st = p.stream = g == 0 ? b->stream : b->side[g - 1];
         p.chunk0 = groups > 1 ? b->grpChunk[g] : 0;
@@ -2488,8 +2493,9 @@ hipError_t enqueue_loop(icempm_batch *b, int n, const double *tTab, double *hist
         for (int i = 0; i < n; ++i) {
             p.in = (start + i) % 3;
             p.out = (start + i + 1) % 3;
+            p.t = tTab + i;
             p.hist = hist + 2 * nc * (size_t)i;
-            p.step = i;
+            p.step = renew ? i : i + 1;
             const bool timeIt = b->timingStride > 0 && i % b->timingStride == 0;
             hipEvent_t t0 = nullptr, t1 = nullptr;
             if (timeIt) {
@@ -2972,11 +2978,12 @@ namespace {
 // launch (captured when the start, the step count or the pointers change)
 // or as stream launches; returns the device time in ms.
 // The executable graph of n substeps from the given start (-1 fresh, 0, 1 or
-// 2: the P2G in that grid) with these time-table and history rows, captured,
-// instantiated and put on the device unless its slot already holds it.
+// 2: the P2G in that grid, the boxes renewed or not) with these time-table and
+// history rows, captured, instantiated and put on the device unless its slot
+// already holds it.
 int ensure_graph(icempm_batch *b, int n, const double *tTab, double *hist, int start,
-                 const icempm_batch::GraphSlot **out) {
-    icempm_batch::GraphSlot *row = b->graphs[start + 1];
+                 bool renew, const icempm_batch::GraphSlot **out) {
+    icempm_batch::GraphSlot *row = b->graphs[renew ? start + 1 : start + 4];
     for (int w = 0; w < 2; ++w)
         if (row[w].exec && row[w].steps == n && row[w].T == tTab && row[w].H == hist) {
             row[w].used = ++b->graphTick;
@@ -2989,7 +2996,7 @@ int ensure_graph(icempm_batch *b, int n, const double *tTab, double *hist, int s
     hipGraph_t graph = nullptr;
     int end = -1;
     BCHK(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal), "batch capture");
-    hipError_t e = enqueue_loop(b, n, tTab, hist, start, &end);
+    hipError_t e = enqueue_loop(b, n, tTab, hist, start, renew, &end);
     hipError_t e2 = hipStreamEndCapture(b->stream, &graph);
     if (e != hipSuccess) {
         if (graph) (void)hipGraphDestroy(graph);
@@ -3025,14 +3032,20 @@ int ensure_capacity(icempm_batch *b, int n) {
     return ICEMPM_OK;
 }
 
+// Runs this short may leave the boxes to a later one: renewing them costs a
+// substep of 6.4M points 25 us, each time for runs of one substep.  A longer run
+// gains less than the second set of graphs costs it.
+constexpr int kShortRun = kBoxEvery / 2;
+
 int run_segment(icempm_batch *b, int n, int use_graph, const double *tTab, double *hist, float *ms) {
     b->tevNext = 0;
     const int start = b->pending;
+    const bool renew = start < 0 || n > kShortRun || b->boxAge + n > kBoxEvery;
     b->pending = -1;   // until the loop below is enqueued whole
     int end = -1;
     if (use_graph) {
         const icempm_batch::GraphSlot *g = nullptr;
-        const int rc = ensure_graph(b, n, tTab, hist, start, &g);
+        const int rc = ensure_graph(b, n, tTab, hist, start, renew, &g);
         if (rc) return rc;
         end = g->end;
         // timed from here: capture and instantiation are host work before it
@@ -3040,11 +3053,12 @@ int run_segment(icempm_batch *b, int n, int use_graph, const double *tTab, doubl
         BCHK(b, hipGraphLaunch(g->exec, b->stream), "batch graph launch");
     } else {
         BCHK(b, hipEventRecord(b->e0, b->stream), "batch run");
-        BCHK(b, enqueue_loop(b, n, tTab, hist, start, &end), "batch run");
+        BCHK(b, enqueue_loop(b, n, tTab, hist, start, renew, &end), "batch run");
     }
     BCHK(b, hipEventRecord(b->e1, b->stream), "batch run");
     BCHK(b, hipEventSynchronize(b->e1), "batch run");
     b->pending = end;
+    b->boxAge = renew ? (n - 1) % kBoxEvery + 1 : b->boxAge + n;
     BCHK(b, hipEventElapsedTime(ms, b->e0, b->e1), "batch run");
     for (size_t q = 0; q + 1 < b->tevNext; q += 2) {
         float kms = 0;
@@ -3116,8 +3130,10 @@ int icempm_batch_prepare(icempm_batch *b, int n) {
         if (rc) return rc;
         // the first segment of such a run, from each of the four starts
         const int len = b->resortEvery > 0 ? std::min(b->resortEvery, n) : n;
-        for (int start = -1; start <= 2; ++start)
-            if ((rc = ensure_graph(b, len, b->tTab, b->hist, start, nullptr))) return rc;
+        for (int start = -1; start <= 2; ++start) {
+            if ((rc = ensure_graph(b, len, b->tTab, b->hist, start, true, nullptr))) return rc;
+            if (start >= 0 && len <= kShortRun && (rc = ensure_graph(b, len, b->tTab, b->hist, start, false, nullptr))) return rc;
+        }
         return ICEMPM_OK;
     });
 }
